@@ -95,10 +95,13 @@ class Linear:
         ep = hip.make_epi(keys=keys, bias=bias, col_offset=col_offset, **kw)
         if self.f32:
             _req(x.dtype == torch.float32 and x.is_cuda and keys is None, "linear: fp32 cuda input")
-            if ws is None:
+            # a graph is replayed on other streams than the one it was captured on: without a workspace of its own, in whole tiles
+            if ws is None and not torch.cuda.is_current_stream_capturing():
                 ws = hip.default_workspace(x.device)
-            _check(lib().lsa_linear_f32(_p(x), x.stride(0), _p(self.w), rows, self.n, self.k, epi, ctypes.byref(ep), _p(ws.slab),
-                                        ws.slab.numel(), _p(ws.counters), ws.counters.numel(), _stream()), "lsa_linear_f32")
+            slab, counters = (None, None) if ws is None else (ws.slab, ws.counters)
+            _check(lib().lsa_linear_f32(_p(x), x.stride(0), _p(self.w), rows, self.n, self.k, epi, ctypes.byref(ep), _p(slab),
+                                        0 if ws is None else slab.numel(), _p(counters), 0 if ws is None else counters.numel(),
+                                        _stream()), "lsa_linear_f32")
         elif rows <= 128:
             hip.gemv(x, self.w, rows, self.n, self.k, epi, ep, ws=ws)
         else:

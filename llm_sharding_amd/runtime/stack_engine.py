@@ -471,7 +471,7 @@ class StackEngine(StageEngine):
         xn = self._normed(h, rows, a_rows)
         if self.dtype == torch.float32:
             lg = torch.empty((rows, self.lm_head.n), dtype=torch.float32, device=self.device)
-            self.lm_head(xn, rows, lg)
+            self.lm_head(xn, rows, lg, ws=self.coop_ws)
             L.logits_argmax(lg, rows, self.head_vocab, keys, offset=self.head_v0)
             return
         self.lm_head(xn, rows, None, ws=self.coop_ws, sk_ws=self.sk_ws, keys=keys, bias=self.head_bias,

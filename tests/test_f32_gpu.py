@@ -146,3 +146,67 @@ def test_paged_attention_of_many_rows(name):
             got[i].append(o)
     for i in range(3):
         rows_close(torch.cat(got[i]).flatten(1), case.want(i).flatten(1), 1e-5, f"{name}: {i}")
+
+
+def _engine_with_a_parted_head(slots):
+    """One layer of a real width; 40 rows of its head are 32 tiles, whose K is shared out."""
+    import dataclasses
+    from llm_sharding_amd.config import get_preset
+    from llm_sharding_amd.runtime.registry import make_engine, random_source
+    cfg = get_preset("deretar-2k")
+    cfg = dataclasses.replace(cfg, layers=cfg.layers[:1], vocab_size=2048)
+    return make_engine(cfg, 0, 1, torch.device(DEV, 0), torch.float32, has_embed=True, has_head=True, source=random_source(cfg, 3),
+                       max_slots=slots, max_seq=16, max_prefill_rows=slots)
+
+
+@torch.inference_mode()
+def test_captured_heads_share_no_workspace(monkeypatch):
+    """Two graphs with scratch sets of their own, side by side: the tokens and sums of each by itself, and those of an eager
+    step; no workspace but the sets'."""
+    from llm_sharding_amd.runtime.engine import DecodeGraph
+    n, steps = 40, 6
+    monkeypatch.setattr(hip, "_WS", {})
+    eng = _engine_with_a_parted_head(2 * n)
+    graphs = [DecodeGraph(eng, n, "full", slots=list(range(i * n, i * n + n)), scratch=i).capture() for i in range(2)]
+    ids = torch.randint(3, 2048, (2, n), generator=torch.Generator().manual_seed(1), dtype=torch.int32).to(DEV)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+
+    def run(together):
+        eng.reset()
+        got = [[], []]
+        for i, g in enumerate(graphs):
+            g.set_positions()
+            g.tokens.copy_(ids[i])
+        torch.cuda.synchronize()
+        for _ in range(steps):
+            for i, g in enumerate(graphs):
+                with torch.cuda.stream(streams[i if together else 0]):
+                    g.replay()
+                    got[i].append((g.out_hidden.clone(), g.tokens.clone()))
+        torch.cuda.synchronize()
+        return got
+    alone, both = run(False), run(True)
+    for a, b in zip(alone[0] + alone[1], both[0] + both[1]):
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    for i in range(2):
+        for h, t in alone[i]:
+            assert torch.equal(eng.head(h, list(range(n))).to(torch.int32), t)
+    assert not hip._WS
+
+
+@torch.inference_mode()
+def test_captured_product_without_a_workspace():
+    """In a graph, a product that is given no workspace takes none: its replays may run beside others of any stream."""
+    k, n, rows = 2048, 2048, 40
+    x, lin = _rand(rows, k, seed=1).to(DEV), Linear(_rand(n, k, seed=2, scale=k ** -0.5).to(DEV))
+    out, want = torch.zeros(rows, n, device=DEV), torch.zeros(rows, n, device=DEV)
+    lin(x, rows, want)
+    before, s, g = set(hip._WS), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        lin(x, rows, out)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        rows_close(out, want.double().cpu(), 2 * sum_tol(k), "replay")
+    assert set(hip._WS) == before

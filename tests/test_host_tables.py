@@ -92,3 +92,22 @@ def test_coop_choice_without_a_table_entry(even, monkeypatch):
                 mb = packing.row_blocks(lo)
                 assert all(packing.coop_cost(n // 16, k, mb, cfg) <= packing.coop_cost(n // 16, k, mb, c)
                            for c in full if c[3] <= 8)
+
+
+def test_fp32_head_takes_the_workspace_of_its_scratch_set(monkeypatch):
+    """A captured head is replayed beside other graphs: scratch of its own set, not what belongs to the capturing stream."""
+    from types import SimpleNamespace
+    from llm_sharding_amd.ops import stream
+    from llm_sharding_amd.runtime.stack_engine import StackEngine
+    got = {}
+
+    class Head:
+        n = 128
+
+        def __call__(self, x, rows, out, **kw):
+            got.update(kw)
+    eng = SimpleNamespace(dtype=torch.float32, device="cpu", lm_head=Head(), head_vocab=100, head_v0=0, coop_ws=object(),
+                          _normed=lambda h, rows, a_rows: h)
+    monkeypatch.setattr(stream, "logits_argmax", lambda *a, **kw: None)
+    StackEngine.head_gemv(eng, torch.zeros(4, 128), 4, torch.zeros(4, dtype=torch.int64))
+    assert got.get("ws") is eng.coop_ws
