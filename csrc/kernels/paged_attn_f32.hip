@@ -9,6 +9,7 @@
 // they meet in LDS at the end; no barrier in the loop. Bound by the latency of its reads; at 2567 rows of up to 200 keys, 16
 // heads of 128 over 4 kv heads, it takes 82 us (softmax) and 92 us (sigmoids), at 16 rows 19 and 23. The plain kernel, a
 // workgroup per row and head, took 1952, 2003, 51 and 50.
+#include <type_traits>
 #include "paged_attn.h"
 
 namespace {
@@ -61,90 +62,117 @@ __global__ __launch_bounds__(256, 2) void attend_f32_kernel(AttnArgs a, int n, i
     const AttBlocks blocks(a, lo, hi);
     const int pooled = att_pooled(a, hi), mine_pooled = att_pooled(a, p);
     f32x4_t o[4 * DV];
+    float m, l;
+    // A value that a pair does not see, or whose weight is 0, has no part in its sums, whatever it is: a tile's product is 0
+    // times it, which an infinity or a NaN would make a NaN of. A wave whose sums are not all finite takes its keys once more,
+    // each pair without what it gives no weight to. (The check is 1 to 3 % of 16 to 67 us: one row of 64 to 256 sequences.)
+    auto sums = [&](auto apart) {
 #pragma unroll
-    for (int t = 0; t < 4 * DV; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-    for (int i = w; i < 2 * blocks.n; i += 4) {
-      const bool pool = blocks.is_pooled(i >> 1);
-      const int half = 32 * (i & 1), key0 = blocks.at(i >> 1) * ATT_PAGE + half;
-      const int last = pool ? pooled - 1 : hi;  // behind it nothing was written
-      if (key0 > last) continue;
-      const AttKv kv = att_kv(a, blocks, slot, i >> 1);
-      const size_t page = (size_t)kv.page * a.kv_heads + kvh;
-      const float* kb = (const float*)kv.k + page * ATT_PAGE * a.dkp + 4 * g4;
-      const float* k0 = kb + (size_t)(half + min(c, last - key0)) * a.dkp;
-      const float* k1 = kb + (size_t)(half + min(c + 16, last - key0)) * a.dkp;
-      f32x4_t sc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
-      for (int d = 0; d < a.dkp; d += 64) {  // dkp % 64 == 0
-        f32x4_t x[4], y[4], z[4];
+      for (int t = 0; t < 4 * DV; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      m = -INFINITY, l = 0.f;
+      for (int i = w; i < 2 * blocks.n; i += 4) {
+        const bool pool = blocks.is_pooled(i >> 1);
+        const int half = 32 * (i & 1), key0 = blocks.at(i >> 1) * ATT_PAGE + half;
+        const int last = pool ? pooled - 1 : hi;  // behind it nothing was written
+        if (key0 > last) continue;
+        const AttKv kv = att_kv(a, blocks, slot, i >> 1);
+        const size_t page = (size_t)kv.page * a.kv_heads + kvh;
+        const float* kb = (const float*)kv.k + page * ATT_PAGE * a.dkp + 4 * g4;
+        const float* k0 = kb + (size_t)(half + min(c, last - key0)) * a.dkp;
+        const float* k1 = kb + (size_t)(half + min(c + 16, last - key0)) * a.dkp;
+        f32x4_t sc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+        for (int d = 0; d < a.dkp; d += 64) {  // dkp % 64 == 0
+          f32x4_t x[4], y[4], z[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          x[u] = ldf4(k0 + d + 16 * u);
-          y[u] = ldf4(k1 + d + 16 * u);
-          z[u] = ldf4(sq + d + 16 * u);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            sc[0] = mfma(x[u][j], z[u][j], sc[0]);
-            sc[1] = mfma(y[u][j], z[u][j], sc[1]);
+          for (int u = 0; u < 4; ++u) {
+            x[u] = ldf4(k0 + d + 16 * u);
+            y[u] = ldf4(k1 + d + 16 * u);
+            z[u] = ldf4(sq + d + 16 * u);
           }
-      }
-      float wt[2][4], mx = -INFINITY;
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+          for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = key0 + 16 * u + 4 * g4 + r;
-          const bool sees = pool ? key < mine_pooled : att_sees(a, p, key);
-          float s = sc[u][r] * hs;
-          if (a.softcap > 0.f) s = a.softcap * tanhf(s / a.softcap);
-          if constexpr (SIG) {
-            s += b2 - r1 * log1pf(r2 * (float)(p - key));
-            wt[u][r] = sees ? 1.f / (1.f + expf(-s)) : 0.f;
-          } else {
-            wt[u][r] = sees ? s : -INFINITY;
-            mx = fmaxf(mx, wt[u][r]);
-          }
+            for (int j = 0; j < 4; ++j) {
+              sc[0] = mfma(x[u][j], z[u][j], sc[0]);
+              sc[1] = mfma(y[u][j], z[u][j], sc[1]);
+            }
         }
-      float alpha = 1.f;
-      if constexpr (!SIG) {
-        mx = fmaxf(mx, lane_xor<16>(mx));
-        mx = fmaxf(mx, lane_xor<32>(mx));
-        const float mn = fmaxf(m, mx), at = mn == -INFINITY ? 0.f : mn;  // (no key of these 32 or before is this pair's)
-        alpha = __builtin_amdgcn_exp2f((m - at) * LOG2E);
-        float sum = 0.f;
+        float wt[2][4], mx = -INFINITY;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            wt[u][r] = __builtin_amdgcn_exp2f((wt[u][r] - at) * LOG2E);
-            sum += wt[u][r];
+            const int key = key0 + 16 * u + 4 * g4 + r;
+            const bool sees = pool ? key < mine_pooled : att_sees(a, p, key);
+            float s = sc[u][r] * hs;
+            if (a.softcap > 0.f) s = a.softcap * tanhf(s / a.softcap);
+            if constexpr (SIG) {
+              s += b2 - r1 * log1pf(r2 * (float)(p - key));
+              wt[u][r] = sees ? 1.f / (1.f + expf(-s)) : 0.f;
+            } else {
+              wt[u][r] = sees ? s : -INFINITY;
+              mx = fmaxf(mx, wt[u][r]);
+            }
           }
-        l = l * alpha + sum;
-        m = mn;
-      }
-      // tokens half + 16 u + 4 g4 + r of a channel lie at half + 8 g4 + 4 u + r
-      const float* vb = (const float*)kv.v + page * a.dvp * ATT_PAGE + (size_t)c * ATT_PAGE + half + 8 * g4;
-      const bool cut = key0 + 31 > last;
-#pragma unroll
-      for (int t = 0; t < 4 * DV; ++t) {
-        f32x4_t v[2] = {ldf4(vb + (size_t)t * 16 * ATT_PAGE), ldf4(vb + (size_t)t * 16 * ATT_PAGE + 4)};
-        if (cut) {
+        float alpha = 1.f;
+        if constexpr (!SIG) {
+          mx = fmaxf(mx, lane_xor<16>(mx));
+          mx = fmaxf(mx, lane_xor<32>(mx));
+          const float mn = fmaxf(m, mx), at = mn == -INFINITY ? 0.f : mn;  // (no key of these 32 or before is this pair's)
+          alpha = __builtin_amdgcn_exp2f((m - at) * LOG2E);
+          float sum = 0.f;
 #pragma unroll
           for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (key0 + 16 * u + 4 * g4 + r > last) v[u][r] = 0.f;
+            for (int r = 0; r < 4; ++r) {
+              wt[u][r] = __builtin_amdgcn_exp2f((wt[u][r] - at) * LOG2E);
+              sum += wt[u][r];
+            }
+          l = l * alpha + sum;
+          m = mn;
         }
-        if constexpr (!SIG) o[t] *= alpha;
+        // tokens half + 16 u + 4 g4 + r of a channel lie at half + 8 g4 + 4 u + r
+        const float* vb = (const float*)kv.v + page * a.dvp * ATT_PAGE + (size_t)c * ATT_PAGE + half + 8 * g4;
+        const bool cut = key0 + 31 > last;
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int t = 0; t < 4 * DV; ++t) {
+          f32x4_t v[2] = {ldf4(vb + (size_t)t * 16 * ATT_PAGE), ldf4(vb + (size_t)t * 16 * ATT_PAGE + 4)};
+          if (cut) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) o[t] = mfma(v[u][r], wt[u][r], o[t]);
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                if (key0 + 16 * u + 4 * g4 + r > last) v[u][r] = 0.f;
+          }
+          if constexpr (!SIG) o[t] *= alpha;
+          if constexpr (decltype(apart)::value) {
+            f32x4_t own = o[t];
+            for (int x = 0; x < cols; ++x) {
+              f32x4_t y = o[t];
+#pragma unroll
+              for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                  y = mfma(__shfl(wt[u][r], (lane & 48) | x, 64) != 0.f ? v[u][r] : 0.f, wt[u][r], y);
+              if (c == x) own = y;
+            }
+            o[t] = own;
+          } else {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) o[t] = mfma(v[u][r], wt[u][r], o[t]);
+          }
+        }
       }
-    }
+    };
+    sums(std::false_type{});
+    bool finite = true;
+#pragma unroll
+    for (int t = 0; t < 4 * DV; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) finite = finite && fabsf(o[t][r]) < INFINITY;
+    if (!__all(finite)) sums(std::true_type{});
     float f = 1.f, F = a.oscale;
     if constexpr (!SIG) {
       l += lane_xor<16>(l);

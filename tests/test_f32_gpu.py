@@ -210,3 +210,37 @@ def test_captured_product_without_a_workspace():
         g.replay()
         rows_close(out, want.double().cpu(), 2 * sum_tol(k), "replay")
     assert set(hip._WS) == before
+
+
+@pytest.mark.parametrize("name", ["one_group", "small", "wide_values"])
+@pytest.mark.parametrize("loud", [False, True])
+def test_paged_attention_of_values_that_are_no_numbers(name, loud):
+    """An infinity and a NaN among the values reach the rows that give their tokens a weight, and no other, also where rows
+    share a workgroup: not those before, not those whose window has passed, and (``loud``) not those whose scores leave the
+    tokens' weights at 0."""
+    from test_gupuvik_gpu import SIZES, Case
+    from llm_sharding_amd.ops import paged_attn as A
+    s, n, bad = SIZES[name], 1030, [201, 202]
+    case = Case(s, [n], torch.float32)
+    case.v[0][bad[0]], case.v[0][bad[1]] = float("inf"), float("nan")
+    if loud:
+        case.k[0][bad] *= 2000
+    case.fill()
+    q = _rand(n, s.heads, s.dim, seed=7)
+    out = torch.full((n, s.heads * s.dvp), 9.0, device=DEV)
+    A.plain(case.args([0] * n, list(range(n))), n, case.padded(q, s.dkp).to(DEV), None, out)
+    got = case.unpad(out).double().cpu()
+    i, j = torch.arange(n)[:, None], torch.arange(n)[None]
+    see = (j <= i) & ((i - j < (s.window or n)) | (j < s.keep_first))
+    k, v = (x.double().repeat_interleave(s.group, 1) for x in (case.k[0], case.v[0].nan_to_num(0, 0, 0)))
+    sc = torch.einsum("ihd,jhd->hij", q.double(), k) * s.scale * case.temp.double()[:, None, None]
+    if s.softcap:
+        sc = s.softcap * torch.tanh(sc / s.softcap)
+    sc = sc.masked_fill(~see, -float("inf"))
+    far = (sc[..., bad] - sc.amax(-1, keepdim=True)).amax(-1).T  # the louder one's distance below the top
+    none, some = far < -120, far > -80  # weights below 2^-150 are 0 in fp32, above 2^-126 they are not
+    assert none.any() and some.any()
+    want = torch.einsum("hij,jhd->ihd", torch.softmax(sc, -1), v)
+    off = (got - want).norm(dim=-1) / want.norm(dim=-1)
+    assert off[none].max() < 1e-5, f"{name}: {off[none].max():.2e}"
+    assert not torch.isfinite(got[some]).any()
