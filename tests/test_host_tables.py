@@ -46,6 +46,25 @@ def test_host_numbers_are_read_as_before():
     assert torch.equal(hip.to_device(rows, "cpu"), torch.tensor(rows, dtype=torch.int32))
 
 
+@pytest.mark.parametrize("x", [2 ** 31, 2 ** 32 + 1, -2 ** 31 - 1, 2 ** 70])
+def test_numbers_past_32_bits_are_refused(x):
+    """A position that int32 does not hold is an error as it is for torch, not another position."""
+    with pytest.raises((RuntimeError, OverflowError, ValueError)):
+        torch.tensor([x], dtype=torch.int32)
+    for rows in ([x], [3, x, 5]):
+        with pytest.raises((RuntimeError, OverflowError, ValueError)):
+            hip.to_device(rows, "cpu")
+        with pytest.raises((RuntimeError, OverflowError, ValueError)):
+            hip.to_device(hip.host_ints(rows), "cpu")
+        with pytest.raises((RuntimeError, OverflowError, ValueError)):
+            hip.build_prefill_tiles([0] * len(rows), rows)
+    for bad in (float("nan"), float("inf")):
+        for rows in ([bad], np.array([1.0, bad]), torch.tensor([bad])):
+            with pytest.raises((ValueError, OverflowError)):
+                hip.host_ints(rows)
+    assert hip.to_device(np.array([2 ** 31 - 1, -2 ** 31]), "cpu").tolist() == [2 ** 31 - 1, -2 ** 31]
+
+
 def test_remembered_candidates_are_not_shared():
     a = packing.coop_candidates(768, 4096, 64)
     a.append("more")
