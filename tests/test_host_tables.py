@@ -91,6 +91,24 @@ def test_copies_are_not_overtaken():
         assert t.tolist() == [i] * (1 + i % 70)
 
 
+@pytest.mark.gpu
+def test_no_copy_from_the_host_inside_a_capture():
+    """A graph would keep the address of pinned memory that the next tables are written to: refused, and the capture goes on."""
+    x, g = torch.zeros(4, device="cuda"), torch.cuda.CUDAGraph()
+    x += 0
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        with pytest.raises(RuntimeError):
+            hip.to_device([1, 2, 3], "cuda")
+        with pytest.raises(RuntimeError):
+            hip.to_device(torch.tensor([1, 2, 3]), "cuda")
+        x += 1
+    assert hip.to_device([1, 2, 3], "cuda").tolist() == [1, 2, 3]
+    for _ in range(3):
+        g.replay()
+    assert x.tolist() == [3.0] * 4
+
+
 @pytest.mark.parametrize("even", [False, True])
 def test_coop_choice_without_a_table_entry(even, monkeypatch):
     """Every choice is a candidate, the same for all rows of a block (the workspace is sized at 32, 64 and 128 rows), and no
