@@ -44,6 +44,15 @@ def embed_rows(cfg: StackConfig, table: torch.Tensor, ids: torch.Tensor) -> torc
     return h
 
 
+def _host_rows(x) -> torch.Tensor:
+    """Slots or positions of a forward pass -> int64 on the host, one after another."""
+    from ..ops import hip
+    try:
+        return torch.from_numpy(hip.host_ints(x)).reshape(-1)
+    except TypeError:  # one number
+        return torch.as_tensor(x, dtype=torch.int64).reshape(-1)
+
+
 class StackEngine(StageEngine):
     GPU_DTYPES = (torch.bfloat16, torch.float32)
     SCRATCH_ATTRS = ("buf_h", "buf_x", "buf_y", "flat", "qt", "part_o", "part_ml", "coop_ws", "sk_ws", "keys", "tokens",
@@ -381,8 +390,7 @@ class StackEngine(StageEngine):
         if kv_len is not None:
             raise ValueError("stack engines attend causally (no kv_len)")
         rows = h.shape[0]
-        from ..ops import hip
-        sl, ps = (torch.from_numpy(hip.host_ints(t)).reshape(-1) for t in (slot, pos))
+        sl, ps = _host_rows(slot), _host_rows(pos)
         if sl.numel() != rows or ps.numel() != rows or rows < 1:
             raise ValueError("forward: one slot and one position per row")
         if int(sl.min()) < 0 or int(sl.max()) >= self.max_slots or int(ps.min()) < 0 or int(ps.max()) >= self.max_seq:

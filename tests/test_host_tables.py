@@ -44,6 +44,9 @@ def test_host_numbers_are_read_as_before():
         assert hip.host_ints(x).tolist() == want.tolist()
     rows = [(0, 3, 1, 5), (3, 1, 0, 0)]
     assert torch.equal(hip.to_device(rows, "cpu"), torch.tensor(rows, dtype=torch.int32))
+    assert hip.host_ints(rows).tolist() == [list(r) for r in rows]
+    with pytest.raises(TypeError):
+        hip.host_ints(3)
 
 
 @pytest.mark.parametrize("x", [2 ** 31, 2 ** 32 + 1, -2 ** 31 - 1, 2 ** 70])
@@ -60,7 +63,7 @@ def test_numbers_past_32_bits_are_refused(x):
             hip.build_prefill_tiles([0] * len(rows), rows)
     for bad in (float("nan"), float("inf")):
         for rows in ([bad], np.array([1.0, bad]), torch.tensor([bad])):
-            with pytest.raises((ValueError, OverflowError)):
+            with pytest.raises((RuntimeError, OverflowError, ValueError)):
                 hip.host_ints(rows)
     assert hip.to_device(np.array([2 ** 31 - 1, -2 ** 31]), "cpu").tolist() == [2 ** 31 - 1, -2 ** 31]
 
@@ -73,6 +76,19 @@ def test_remembered_candidates_are_not_shared():
     b = packing.gemv_candidates(768, 4096, 8)
     b.clear()
     assert packing.gemv_candidates(768, 4096, 8)
+
+
+@pytest.mark.parametrize("slot,pos", [([0, 0, 0], [0, 1, 2]), ([[0], [0], [0]], torch.tensor([[0], [1], [2]])),
+                                      (torch.zeros(1, 3), np.array([[0, 1, 2]])), (range(0, 1), 0), (torch.tensor(0), (0,))])
+def test_rows_of_a_stack_in_any_shape(slot, pos):
+    """Slots and positions come as lists, arrays or tensors, flat or not, one row also as a number."""
+    from deretar_models import engine, stack
+    eng = engine(stack(), "cpu", torch.float32)
+    n = torch.as_tensor(pos).numel()
+    h = eng.embed(torch.tensor([3, 4, 5][:n], dtype=torch.int32))
+    got = eng.forward(h.clone(), slot, pos)
+    eng.reset()
+    assert torch.equal(got, eng.forward(h.clone(), [0] * n, list(range(n))))
 
 
 @pytest.mark.gpu
