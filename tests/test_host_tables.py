@@ -164,3 +164,14 @@ def test_fp32_head_takes_the_workspace_of_its_scratch_set(monkeypatch):
     monkeypatch.setattr(stream, "logits_argmax", lambda *a, **kw: None)
     StackEngine.head_gemv(eng, torch.zeros(4, 128), 4, torch.zeros(4, dtype=torch.int64))
     assert got.get("ws") is eng.coop_ws
+
+
+@pytest.mark.parametrize("n,k", [(1152, 3072), (2304, 2048), (6144, 3072), (8192, 8192)])
+def test_workspace_of_a_size_with_and_without_gates(n, k):
+    """Two projections of one size, one of them gated: scratch for what either takes, by the table and by the cost model."""
+    floats, groups = packing.coop_workspace_need([(n, k), (n, k)], 128, [(n, k)])
+    for rows in (17, 32, 33, 64, 65, 128):
+        for even in (False, True):
+            algo, cfg = packing.proj_config(n // 16, rows, need_even=even, k=k)
+            if algo == "coop":
+                assert floats >= packing.coop_slab_floats(n, rows, *cfg[:4]) and groups >= n // 16 // (cfg[0] * cfg[1])
