@@ -168,6 +168,12 @@ def _kernels(text: str):
         yield name, ins
 
 
+def _target(addr: int, operand: str) -> int:
+    """Where the branch at ``addr`` goes."""
+    off = int(operand, 0)
+    return addr + 4 + 4 * (off - 0x10000 if off >= 0x8000 else off)
+
+
 def audit_mfma(text: str, slots: int = MFMA_SLOTS) -> list:
     """Findings of rule ``mfma``: every path from an MFMA, its branches taken and not."""
     findings = []
@@ -202,8 +208,7 @@ def audit_mfma(text: str, slots: int = MFMA_SLOTS) -> list:
                     if not store and o2:
                         live = live - _regs(o2[0])
                 if op2 == "s_branch" or op2.startswith("s_cbranch"):
-                    off = int(o2[0], 0)
-                    todo.append((at.get(addr + 4 + 4 * (off - 0x10000 if off >= 0x8000 else off), len(ins)), d + 1, live))
+                    todo.append((at.get(_target(addr, o2[0]), len(ins)), d + 1, live))
                     if op2 == "s_branch":
                         continue
                 todo.append((j + 1, d + 1, live))
@@ -211,20 +216,30 @@ def audit_mfma(text: str, slots: int = MFMA_SLOTS) -> list:
 
 
 def audit_stores(text: str, slots: int = STORE_SLOTS) -> list:
-    """Findings of rule ``store``, in program order (a branch ends the search)."""
+    """Findings of rule ``store``: every path from a store, its branches (a slot each) taken and not."""
     findings = []
     for kernel, ins in _kernels(text):
+        at = {a: i for i, (a, *_) in enumerate(ins)}
         for i, (_, writer, op, ops) in enumerate(ins):
             if not op.startswith(("buffer_store_dwordx3", "buffer_store_dwordx4")) or not re.match(r"s\d+\b|m0\b", ops[3]):
                 continue
-            data, d = _regs(ops[0]), 0
-            for _, s, op2, o2 in ins[i + 1:i + 1 + slots]:
-                if d >= slots or op2.startswith(("s_branch", "s_cbranch", "s_endpgm")):
-                    break
-                d += int(o2[0], 0) + 1 if op2 == "s_nop" else 1
-                if op2.startswith("v_") and o2 and _regs(o2[0]) & data and d <= slots:
+            data, seen, todo = _regs(ops[0]), {}, [(i + 1, 0)]
+            while todo:
+                j, d = todo.pop()
+                if j >= len(ins) or d >= slots or seen.get(j, slots) <= d:
+                    continue
+                seen[j] = d
+                addr, s, op2, o2 = ins[j]
+                if op2 in ("s_endpgm", "s_setpc_b64"):
+                    continue
+                if op2.startswith("v_") and o2 and _regs(o2[0]) & data:
                     findings.append(("store", kernel, writer, s))
-                    break
+                    continue
+                if op2 == "s_branch" or op2.startswith("s_cbranch"):
+                    todo.append((at.get(_target(addr, o2[0]), len(ins)), d + 1))
+                    if op2 == "s_branch":
+                        continue
+                todo.append((j + 1, d + (int(o2[0], 0) + 1 if op2 == "s_nop" else 1)))
     return findings
 
 

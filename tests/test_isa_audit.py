@@ -108,6 +108,15 @@ def test_a_store_whose_data_is_written_at_once():
                      ([store, write.replace("v12", "v14")], 0)):
         assert len(audit_stores(text(ins + ["s_endpgm"]))) == bad, ins
 
+    # behind a branch, whichever way it goes, and at the head of the loop that the store ends; another's way out is its own
+    for ins, bad in (([store, "s_cbranch_scc1 4", write], 1), ([store, "s_cbranch_scc1 1", "s_endpgm", write], 1),
+                     ([store, "s_branch 1", write, other], 0), ([store, "s_branch 0", write], 1),
+                     ([store, other, "s_cbranch_scc1 1", write], 0),
+                     ([write, other, store, "s_cbranch_scc1 65532", "s_endpgm"], 1),
+                     ([other, write, other, store, "s_cbranch_scc1 65531", "s_endpgm"], 0),
+                     ([store, "s_setpc_b64 s[30:31]", write], 0)):
+        assert len(audit_stores(text(ins + ["s_endpgm"]))) == bad, ins
+
 
 def test_rules_match_the_hardware(tmp_path):
     """Rebuild the probe from its generator, audit its ISA, and map every finding back to its case:
