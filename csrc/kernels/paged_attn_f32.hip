@@ -16,7 +16,6 @@ namespace {
 
 LSA_DEVICE f32x4_t mfma(float a, float b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 LSA_DEVICE f32x4_t ldf4(const float* p) { return *reinterpret_cast<const f32x4_t*>(p); }
-constexpr float LOG2E = 1.4426950408889634f;
 
 template <int DV, bool SIG>  // dvp / 64
 __global__ __launch_bounds__(256, 2) void attend_f32_kernel(AttnArgs a, int n, int per, const float* __restrict__ q, int ldq,
@@ -80,7 +79,10 @@ __global__ __launch_bounds__(256, 2) void attend_f32_kernel(AttnArgs a, int n, i
         const float* kb = (const float*)kv.k + page * ATT_PAGE * a.dkp + 4 * g4;
         const float* k0 = kb + (size_t)(half + min(c, last - key0)) * a.dkp;
         const float* k1 = kb + (size_t)(half + min(c + 16, last - key0)) * a.dkp;
-        f32x4_t sc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+        // four sums a score, each of every fourth value, as the plain kernel has them: a single one rounds twice as much
+        f32x4_t part[2][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) part[0][u] = part[1][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         for (int d = 0; d < a.dkp; d += 64) {  // dkp % 64 == 0
           f32x4_t x[4], y[4], z[4];
 #pragma unroll
@@ -89,14 +91,18 @@ __global__ __launch_bounds__(256, 2) void attend_f32_kernel(AttnArgs a, int n, i
             y[u] = ldf4(k1 + d + 16 * u);
             z[u] = ldf4(sq + d + 16 * u);
           }
+          __builtin_amdgcn_sched_barrier(0);  // all requested before the first is waited for
 #pragma unroll
           for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              sc[0] = mfma(x[u][j], z[u][j], sc[0]);
-              sc[1] = mfma(y[u][j], z[u][j], sc[1]);
+              part[0][j] = mfma(x[u][j], z[u][j], part[0][j]);
+              part[1][j] = mfma(y[u][j], z[u][j], part[1][j]);
             }
         }
+        f32x4_t sc[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) sc[u] = (part[u][0] + part[u][1]) + (part[u][2] + part[u][3]);
         float wt[2][4], mx = -INFINITY;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
@@ -119,13 +125,13 @@ __global__ __launch_bounds__(256, 2) void attend_f32_kernel(AttnArgs a, int n, i
           mx = fmaxf(mx, lane_xor<16>(mx));
           mx = fmaxf(mx, lane_xor<32>(mx));
           const float mn = fmaxf(m, mx), at = mn == -INFINITY ? 0.f : mn;  // (no key of these 32 or before is this pair's)
-          alpha = __builtin_amdgcn_exp2f((m - at) * LOG2E);
+          alpha = expf(m - at);
           float sum = 0.f;
 #pragma unroll
           for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              wt[u][r] = __builtin_amdgcn_exp2f((wt[u][r] - at) * LOG2E);
+              wt[u][r] = expf(wt[u][r] - at);
               sum += wt[u][r];
             }
           l = l * alpha + sum;
@@ -187,10 +193,10 @@ __global__ __launch_bounds__(256, 2) void attend_f32_kernel(AttnArgs a, int n, i
       for (int x = 0; x < 4; ++x) M = fmaxf(M, s_ml[0][x][c]);
 #pragma unroll
       for (int x = 0; x < 4; ++x)
-        if (s_ml[0][x][c] != -INFINITY) L += s_ml[1][x][c] * __builtin_amdgcn_exp2f((s_ml[0][x][c] - M) * LOG2E);
-      f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - M) * LOG2E);
-      const float t = a.sink ? fmaxf(M, 0.f) : M, e = __builtin_amdgcn_exp2f((M - t) * LOG2E);
-      F *= e / (L * e + (a.sink ? __builtin_amdgcn_exp2f(-t * LOG2E) : 0.f));
+        if (s_ml[0][x][c] != -INFINITY) L += s_ml[1][x][c] * expf(s_ml[0][x][c] - M);
+      f = m == -INFINITY ? 0.f : expf(m - M);
+      const float t = a.sink ? fmaxf(M, 0.f) : M, e = expf(M - t);
+      F *= e / (L * e + (a.sink ? expf(-t) : 0.f));
     }
     f *= F;
     // waves 0 and 1 write, 2 and 3 add: channels 16 t + 4 g4 + r of pair c

@@ -244,3 +244,30 @@ def test_paged_attention_of_values_that_are_no_numbers(name, loud):
     off = (got - want).norm(dim=-1) / want.norm(dim=-1)
     assert off[none].max() < 1e-5, f"{name}: {off[none].max():.2e}"
     assert not torch.isfinite(got[some]).any()
+
+
+@pytest.mark.parametrize("name", ["one_group", "small", "wide_values"])
+def test_paged_attention_rounds_no_more_than_four_sums_a_score(name):
+    """Large scores, whose rounding the softmax passes on: against float64 no further off than scores that are added up in fp32
+    as four sums of every fourth value (what the plain kernel does), everything behind them in float64, and an eighth for
+    that; a single sum is about twice as far."""
+    import dataclasses
+    from test_gupuvik_gpu import SIZES, Case
+    from llm_sharding_amd.ops import paged_attn as A
+    s, n = dataclasses.replace(SIZES[name], scale=10 * SIZES[name].scale, softcap=0.0), 400
+    case = Case(s, [n], torch.float32).fill()
+    q = _rand(n, s.heads, s.dim, seed=7)
+    out = torch.full((n, s.heads * s.dvp), 9.0, device=DEV)
+    A.plain(case.args([0] * n, list(range(n))), n, case.padded(q, s.dkp).to(DEV), None, out)
+    got, want = case.unpad(out).double().cpu(), case.want(q, [0] * n, list(range(n)))
+    i, j = torch.arange(n)[:, None], torch.arange(n)[None]
+    see = (j <= i) & ((i - j < (s.window or n)) | (j < s.keep_first))
+    k, v = (x.repeat_interleave(s.group, 1) for x in (case.k[0], case.v[0]))
+    parts = torch.zeros(4, s.heads, n, n)
+    for d in range(s.dim):
+        parts[d % 4] += q[:, None, :, d].permute(2, 0, 1) * k[None, :, :, d].permute(2, 0, 1)
+    sc = ((parts[0] + parts[1]) + (parts[2] + parts[3])) * case.hscale.cpu()[:, None, None]
+    four = torch.einsum("hij,jhd->ihd", torch.softmax(sc.double().masked_fill(~see, -float("inf")), -1), v.double())
+    ours, theirs = (float((x - want).norm() / want.norm()) for x in (got, four))
+    print(f"{name}: {ours:.2e}, four sums a score {theirs:.2e}")
+    assert ours < 1.125 * theirs
