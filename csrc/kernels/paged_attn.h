@@ -157,4 +157,5 @@ LSA_DEVICE float att_cap(float s, float cap, float icap) {
 }
 
 // lsa_attn_plain's work in fp32 (paged_attn_f32.hip); false: not a size or alignment for it, nothing launched.
-bool attn_f32(const AttnArgs& a, int n, const float* q, int ldq, const float* gate, int ldg, float* out, int ldo, hipStream_t s);
+bool attn_f32(const AttnArgs& a, int n, bool singles, const float* q, int ldq, const float* gate, int ldg, float* out, int ldo,
+              hipStream_t s);

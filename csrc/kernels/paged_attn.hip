@@ -196,12 +196,13 @@ extern "C" int lsa_attn_append_tiles(int f32, const AttnArgs* a, const void* til
   return LSA_OK;
 }
 
-extern "C" int lsa_attn_plain(int f32, const AttnArgs* a, int n, const void* q, int ldq, const void* gate, int ldg,
-                              void* out, int ldo, hipStream_t s) {
+// singles: the rows are of as many sequences
+extern "C" int lsa_attn_plain(int f32, const AttnArgs* a, int n, int singles, const void* q, int ldq, const void* gate,
+                              int ldg, void* out, int ldo, hipStream_t s) {
   if (bad_args(a) || !a->slot || !a->pos || n < 1 || ldq < a->heads * a->dkp || ldo < a->heads * a->dvp ||
       (gate && ldg < a->heads * (a->elem_gate ? a->dvp : 1)) || a->dkp + a->dvp > 8192)
     return LSA_BAD_SHAPE;
-  if (f32 && attn_f32(*a, n, (const float*)q, ldq, (const float*)gate, ldg, (float*)out, ldo, s)) {
+  if (f32 && attn_f32(*a, n, singles != 0, (const float*)q, ldq, (const float*)gate, ldg, (float*)out, ldo, s)) {
     LSA_CHECK_LAUNCH();
     return LSA_OK;
   }

@@ -224,14 +224,17 @@ __global__ __launch_bounds__(256, 2) void attend_f32_kernel(AttnArgs a, int n, i
 
 }  // namespace
 
-bool attn_f32(const AttnArgs& a, int n, const float* q, int ldq, const float* gate, int ldg, float* out, int ldo, hipStream_t s) {
+bool attn_f32(const AttnArgs& a, int n, bool singles, const float* q, int ldq, const float* gate, int ldg, float* out, int ldo,
+              hipStream_t s) {
   const int G = a.heads / a.kv_heads;
   if (G > 16 || a.dkp > 256 || (a.dvp != 64 && a.dvp != 128 && a.dvp != 256) ||
       ((uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.pk | (uintptr_t)a.pv) % 16)
     return false;
-  // Rows of one sequence share its keys' reads where that leaves a workgroup per CU (16 columns of at least one head each);
-  // else, and so in decode, a row has a workgroup of its own: rows of several sequences would run one after another.
-  const int per = (long)n * a.kv_heads >= 1024 ? 16 / G : 1;
+  // Rows of one sequence share its keys' reads once there are 1024 workgroups of a row each: 128 rows of a sequence, 8 heads
+  // over 8 kv heads 18.0 us, with a row each 24.8; 256 rows, 16 heads over 4 14.8 and 26.5. Rows of as many sequences would
+  // run one after another in a workgroup: up to 200 keys, 128 rows of 8 over 8 219 us, with a row each 46; 256 of 16 over 4 57
+  // and 45 (the plain kernel 122 and 303).
+  const int per = !singles && (long)n * a.kv_heads >= 1024 ? 16 / G : 1;
   const dim3 grid((n + per - 1) / per, a.kv_heads);
   const size_t lds = (size_t)16 * (a.dkp + 4) * 4;
 #define LSA_A(DV)                                                                                                          \

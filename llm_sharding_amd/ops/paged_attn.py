@@ -151,10 +151,10 @@ def _shapes(a: AttnArgs, q, gate, out, dtype=None) -> tuple:
     return _p(q), q.stride(0), _p(gate), 0 if gate is None else gate.stride(0), _p(out), out.stride(0)
 
 
-def plain(a: AttnArgs, n: int, q, gate, out) -> None:
+def plain(a: AttnArgs, n: int, q, gate, out, singles: bool = False) -> None:
     """Attention of n rows (or a.index' rows), any size, both types. ``gate`` [rows, >= heads, or heads x dvp] or
-    None."""
-    _check(lib().lsa_attn_plain(is_f32(q.dtype), ctypes.byref(a), n, *_shapes(a, q, gate, out), _stream()),
+    None. ``singles``: they are of as many sequences."""
+    _check(lib().lsa_attn_plain(is_f32(q.dtype), ctypes.byref(a), n, int(singles), *_shapes(a, q, gate, out), _stream()),
            "lsa_attn_plain")
 
 
@@ -187,7 +187,7 @@ def declare(L: ctypes.CDLL) -> None:
         "lsa_attn_append_tiles": [i, aa, vp, i, vp, i, i, i, vp],
         "lsa_attn_prep": [i, aa, ctypes.POINTER(PrepArgs), i, vp],
         "lsa_attn_pool": [i, aa, i, vp],
-        "lsa_attn_plain": [i, aa, i] + io + [vp],
+        "lsa_attn_plain": [i, aa, i, i] + io + [vp],
         "lsa_attn_rows": [aa, i] + io + [i, vp, vp, vp],
         "lsa_attn_merge": [aa, i, vp, vp, i, vp, i, vp, i, vp],
         "lsa_attn_tiles": [aa, vp, i] + io + [vp],

@@ -133,7 +133,7 @@ class Attention:
         if n and self.tuned:
             A.rows(b, n, q, gate, ao, self.key_splits(eng, n, plan.longest), eng.part_o, eng.part_ml)
         elif n:
-            A.plain(b, n, q, gate, ao)
+            A.plain(b, n, q, gate, ao, singles=plan.singles)
         return ao
 
     @staticmethod

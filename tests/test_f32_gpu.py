@@ -271,3 +271,35 @@ def test_paged_attention_rounds_no_more_than_four_sums_a_score(name):
     ours, theirs = (float((x - want).norm() / want.norm()) for x in (got, four))
     print(f"{name}: {ours:.2e}, four sums a score {theirs:.2e}")
     assert ours < 1.125 * theirs
+
+
+@torch.inference_mode()
+def test_paged_attention_of_many_single_rows(monkeypatch):
+    """One row of each of 130 sequences: the same from workgroups of a row each and from shared ones; a decode step asks for
+    the former, a prompt's rows share."""
+    from test_gupuvik_gpu import SIZES, Case
+    from llm_sharding_amd.ops import paged_attn as A
+    s, n = SIZES["wide_values"], 130
+    case = Case(s, [1 + (37 * i) % 150 for i in range(n)], torch.float32).fill()
+    slot, pos = list(range(n)), [x - 1 for x in case.lens]
+    pos[5] = -1  # idle
+    q = _rand(n, s.heads, s.dim, seed=7)
+    live = [i for i in range(n) if pos[i] >= 0]
+    want = case.want(q[live], live, [pos[i] for i in live])
+    for singles in (False, True):
+        out = torch.full((n, s.heads * s.dvp), 9.0, device=DEV)
+        A.plain(case.args(slot, pos), n, case.padded(q, s.dkp).to(DEV), None, out, singles=singles)
+        rows_close(case.unpad(out)[live].flatten(1), want.flatten(1), 1e-5, f"singles {singles}")
+        assert not out[5].any()
+    import dumizen_models as M
+    from llm_sharding_amd.runtime.engine import DecodeGraph
+    asked, plain = [], A.plain
+    monkeypatch.setattr(A, "plain", lambda *a, singles=False: (asked.append(singles), plain(*a, singles=singles)))
+    eng = M.engine(M.stack(), DEV, torch.float32)
+    sl, po = eng.prefill_rows([0, 1], [9, 4])
+    eng.forward(eng.embed(torch.arange(13, dtype=torch.int32, device=DEV)), sl, po)
+    eng.advance([0, 1], [9, 4])
+    assert asked and not any(asked)
+    asked.clear()
+    DecodeGraph(eng, 2, "first").capture()
+    assert asked and all(asked)
