@@ -330,12 +330,14 @@ def coop_cost(n_tiles: int, k: int, mb: int, cfg: tuple) -> float:
     """Modelled us of the cooperative GEMV with ``cfg`` (one tile per wave, whole splits) at ``mb`` row blocks, least squares
     over cold products: the weights at 8.2 TB/s and every workgroup's read of the activations at 27 (from L2), over how evenly
     workgroups fill the CUs and whether a CU has four waves; not faster than memory; and a split's partial sums, written and
-    read at 4.7 TB/s."""
+    read at 4.7 TB/s. More than 130 MB of weights push the activations out of L2 between two workgroups' reads: 11 TB/s. (16384 x
+    28672 at 64 rows: 512 workgroups of two waves 223 us, 256 of four 169, 256 of eight in two splits 147.)"""
     _, nw, _, sk, kw, _ = cfg
     n, mr, wg = 16 * n_tiles, 16 * mb, n_tiles // nw * sk
     load = -(-wg // N_CU) * N_CU / wg if wg > N_CU else (N_CU / wg) ** 0.62
     weights, acts = n * k * 2e-6, wg * mr * k // sk * 2e-6
-    us = 4.0 + max(weights / 4.9, (weights / 8.2 + acts / 27) * load * max(1.0, 4 * N_CU / (wg * nw * kw)) ** 0.3)
+    rate = 27 if weights <= 130 else 11
+    us = 4.0 + max(weights / 4.9, (weights / 8.2 + acts / rate) * load * max(1.0, 4 * N_CU / (wg * nw * kw)) ** 0.3)
     return us if sk == 1 else us + 2.2 + sk * mr * n * 8e-6 / 4.7
 
 
@@ -343,9 +345,10 @@ def coop_cost(n_tiles: int, k: int, mb: int, cfg: tuple) -> float:
 def _coop_choice(n_tiles: int, k: int, mb: int, need_even: bool) -> tuple | None:
     """A configuration for a product that no table entry covers.
 
-    One tile per wave and the K chunk of the row block's register budget: of these the cheapest takes 1.02, 1.07 and 1.05
-    times the fastest of all configurations at 24, 48 and 96 rows (geometric mean over 53 products of 1024 to 28672 columns,
-    K 1024 to 11008); the smallest split that fills the CUs takes 1.53, 1.54 and 1.57 times and is what is left where K or N
+    One tile per wave and the K chunk of the row block's register budget: of these the cheapest takes 1.02, 1.06 and 1.04
+    times the fastest of all configurations at 24, 48 and 96 rows (geometric mean over 62 products of 1024 to 28672 columns,
+    K 1024 to 11008; worst 1.48), 1.03 times over 42 larger ones (4096 to 57344 columns, K to 28672, 32 to 128 rows; worst 1.28); the
+    smallest split that fills the CUs takes 1.53, 1.54 and 1.57 times, of the larger 1.14, and is what is left where K or N
     allows none of them. Four layers of Llama 3.2 3B at 47 sequences: 8 steps 5374 -> 4259 us; at 21 4171 -> 3215."""
     allc = _coop_candidates(n_tiles, k, mb, need_even)
     cands = [c for c in allc if c[0] == 1 and c[2] == (2 if mb == 8 else 4) and 1 <= c[3] <= 8 and c[4] <= 2 and c[5] == 3]

@@ -175,3 +175,24 @@ def test_workspace_of_a_size_with_and_without_gates(n, k):
             algo, cfg = packing.proj_config(n // 16, rows, need_even=even, k=k)
             if algo == "coop":
                 assert floats >= packing.coop_slab_floats(n, rows, *cfg[:4]) and groups >= n // 16 // (cfg[0] * cfg[1])
+
+
+# us of products whose weights are 360 to 940 MB on MI355X, each read from memory: what the cost model chose before it knew
+# that such weights push the activations out of L2, the smallest split that fills the chip, and the fastest that it may choose
+LARGE = {
+    (8192, 22016, 64): {(1, 2, 4, 1, 2, 3): 82.3, (1, 8, 8, 4, 1, 3): 70.3, (1, 4, 4, 2, 1, 3): 73.2, (1, 8, 4, 4, 1, 3): 66.4},
+    (8192, 22016, 128): {(1, 4, 2, 2, 1, 3): 103.3, (1, 8, 4, 4, 1, 3): 80.3, (1, 8, 2, 4, 1, 3): 79.2},
+    (8192, 28672, 64): {(1, 2, 4, 1, 2, 3): 101.7, (1, 8, 8, 4, 1, 3): 82.2, (1, 4, 4, 2, 1, 3): 86.1, (1, 8, 4, 4, 1, 3): 78.8},
+    (8192, 28672, 128): {(1, 4, 2, 2, 1, 3): 129.6, (1, 8, 4, 4, 1, 3): 96.0, (1, 8, 2, 4, 1, 3): 98.7},
+    (16384, 28672, 64): {(1, 2, 4, 1, 1, 3): 223.2, (1, 8, 8, 2, 1, 3): 147.5, (1, 4, 4, 1, 1, 3): 168.5, (1, 8, 4, 2, 1, 3): 145.7},
+}
+
+
+@pytest.mark.parametrize("n,k,rows", list(LARGE))
+def test_coop_choice_of_large_products(n, k, rows, monkeypatch):
+    """No slower than the smallest split that fills the chip by more than a box's products differ between runs (5 %)."""
+    monkeypatch.setattr(packing, "_TUNED", {})
+    us, cfg = LARGE[n, k, rows], packing.proj_config(n // 16, rows, k=k)[1]
+    fills = next(c for c in packing.coop_candidates(n // 16, k, rows)
+                 if c[:3] == (1, 8, 4 if rows > 64 else 8) and c[3] >= 1 and c[4:] == (1, 3) and n // 128 * c[3] >= 256)
+    assert us[cfg] <= 1.05 * us[fills], (cfg, fills)
