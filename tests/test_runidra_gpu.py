@@ -484,6 +484,18 @@ def test_matrix_memory(name, dtype, wide):
     assert not rest.any() and not case.state[1][..., s.dim:].any()
 
 
+@pytest.mark.parametrize("dtype", [BF, F32])
+@pytest.mark.parametrize("name", list(ML))
+def test_matrix_memory_at_the_ends_of_batches(name, dtype):
+    """Step by step, in portions that end before, at and behind a batch of 16 rows or two, from a start and from a state."""
+    parts = [(15, 33), (16, 32), (17, 31), (31, 17), (32, 16), (33, 15), (1, 2), (2, 1)]
+    case = MlCase(ML[name], [sum(a for a, _ in parts), sum(b for _, b in parts)], dtype)
+    for a, b in parts:
+        case.step([(1, b), (0, a)], "steps")
+    for i in (0, 1):
+        case.check(i, f"{name} {i}")
+
+
 @pytest.mark.parametrize("how,wide", [("chunks", 1), ("chunks", 1000), ("steps", 1)])
 @pytest.mark.parametrize("bias,spread", [((0.0, -30.0), 1.0), ((30.0, 2.0), 1.0), ((-30.0, 30.0), 1.0), ((0.0, 0.0), 40.0), ((10.0, 6.0), 8.0)])
 def test_matrix_memory_with_gates_at_their_ends(how, wide, bias, spread):
