@@ -196,3 +196,14 @@ def test_coop_choice_of_large_products(n, k, rows, monkeypatch):
     fills = next(c for c in packing.coop_candidates(n // 16, k, rows)
                  if c[:3] == (1, 8, 4 if rows > 64 else 8) and c[3] >= 1 and c[4:] == (1, 3) and n // 128 * c[3] >= 256)
     assert us[cfg] <= 1.05 * us[fills], (cfg, fills)
+
+
+def test_stream_handle_with_and_without_the_raw_call(monkeypatch):
+    """The raw handle of the current device's stream where torch has the call, the Stream object's elsewhere."""
+    from types import SimpleNamespace
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=7))
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda d: 100 + d, raising=False)
+    assert hip._stream().value == 103
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert hip._stream().value == 7
