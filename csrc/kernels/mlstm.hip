@@ -36,10 +36,10 @@ LSA_DEVICE float lane_at(float x, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
 }
 
-// A single row per sequence (decoding): all threads share the key channels, one wave norms the read-out. 4 sequences, 16
-// heads of 128 x 128: 5.4 us; as a batch of one row below 7.4.
+// Row by row: all threads share the key channels, one wave norms the read-out, the next row's operands are requested while
+// this one is computed. A single row (decoding) of 4 sequences, 16 heads of 128 x 128: 5.4 us.
 template <typename T, int DK, int DV>
-__global__ __launch_bounds__(256) void ml_one_kernel(MlArgs a) {
+__global__ __launch_bounds__(256) void ml_rows_kernel(MlArgs a) {
   // a thread holds RPT rows x 4 value channels of S and the same rows of n
   constexpr int NG = 1024 / DV, RPT = DK / NG, NX = (2 * DK + DV + 255) / 256;
   constexpr int NO = (DV + 63) / 64;  // channels per lane of the wave that stores
@@ -51,18 +51,25 @@ __global__ __launch_bounds__(256) void ml_one_kernel(MlArgs a) {
   const size_t head = (size_t)r.slot * a.heads + h;
   float* st = a.S + head * DK * DV + (size_t)d0 * DV + v;
   float* sn = a.n + head * a.copies * DK;
-  const T* in = (const T*)a.in + (size_t)r.row0 * a.ldi;
-  float x[NX], gate[NO];
+  struct Row {
+    float x[NX], gate[NO], i, f;
+  };
+  auto load = [&](int row, Row& y) {
+    const T* in = (const T*)a.in + (size_t)row * a.ldi;
 #pragma unroll
-  for (int u = 0; u < NX; ++u) {
-    const int c = tid + 256 * u;
-    x[u] = ld1(in + (c < DK ? a.oq + h * DK + c : c < 2 * DK ? a.ok + h * DK + c - DK : a.ov + h * DV + min(c - 2 * DK, DV - 1)));
-  }
+    for (int u = 0; u < NX; ++u) {
+      const int c = tid + 256 * u;
+      y.x[u] = ld1(in + (c < DK ? a.oq + h * DK + c : c < 2 * DK ? a.ok + h * DK + c - DK : a.ov + h * DV + min(c - 2 * DK, DV - 1)));
+    }
 #pragma unroll
-  for (int u = 0; u < NO; ++u) gate[u] = ml_out_gate<T>(a, r.row0, h, ((tid & 63) + 64 * u) % DV);
-  const float i = ml_input_gate(a, r.row0, h), f = ml_forget_gate(a, r.row0, h);
+    for (int u = 0; u < NO; ++u) y.gate[u] = ml_out_gate<T>(a, row, h, ((tid & 63) + 64 * u) % DV);
+    y.i = ml_input_gate(a, row, h);
+    y.f = ml_forget_gate(a, row, h);
+  };
+  Row y;
+  load(r.row0, y);
   const bool fresh = r.pos0 == 0;
-  const float m0 = fresh ? 0.f : a.m[head * a.copies];
+  float m = fresh ? 0.f : a.m[head * a.copies];
   f32x4_t S[RPT];
   float n[RPT];
 #pragma unroll
@@ -70,28 +77,58 @@ __global__ __launch_bounds__(256) void ml_one_kernel(MlArgs a) {
     S[j] = fresh ? f32x4_t{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4_t*>(st + (size_t)j * DV);
     n[j] = fresh ? 0.f : sn[d0 + j];
   }
-  const float m = fmaxf(f + m0, i), keep = expf(f + m0 - m), add = expf(i - m);
+  for (int t = 0; t < r.n; ++t) {
+    const bool last = t + 1 == r.n;
+    const float i = y.i, fm = y.f + m;
+    m = fmaxf(fm, i);
+    const float keep = expf(fm - m), add = expf(i - m);
+    float gate[NO];
 #pragma unroll
-  for (int u = 0; u < NX; ++u) {
-    const int c = tid + 256 * u;
-    if (c < 2 * DK + DV) s_in[c] = c < DK ? x[u] * a.q_scale : x[u];
-  }
-  __syncthreads();
-  const f32x4_t u4 = *reinterpret_cast<const f32x4_t*>(&s_in[2 * DK + v]) * add;
-  f32x4_t o = {0.f, 0.f, 0.f, 0.f};
-  float nq = 0.f;
+    for (int u = 0; u < NO; ++u) gate[u] = y.gate[u];
 #pragma unroll
-  for (int j = 0; j < RPT; ++j) {
-    const float q = s_in[d0 + j], k = s_in[DK + d0 + j];
-    S[j] = S[j] * keep + u4 * k;
-    o += S[j] * q;
-    n[j] = n[j] * keep + add * k;
-    nq += n[j] * q;
-    *reinterpret_cast<f32x4_t*>(st + (size_t)j * DV) = S[j];
+    for (int u = 0; u < NX; ++u) {
+      const int c = tid + 256 * u;
+      if (c < 2 * DK + DV) s_in[c] = c < DK ? y.x[u] * a.q_scale : y.x[u];
+    }
+    __syncthreads();
+    if (!last) load(r.row0 + t + 1, y);
+    __builtin_amdgcn_sched_barrier(0);  // requested here, not where it is first used
+    const f32x4_t u4 = *reinterpret_cast<const f32x4_t*>(&s_in[2 * DK + v]) * add;
+    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+    float nq = 0.f;
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      const float q = s_in[d0 + j], k = s_in[DK + d0 + j];
+      S[j] = S[j] * keep + u4 * k;
+      o += S[j] * q;
+      n[j] = n[j] * keep + add * k;
+      nq += n[j] * q;
+      if (last) *reinterpret_cast<f32x4_t*>(st + (size_t)j * DV) = S[j];
+    }
+    *reinterpret_cast<f32x4_t*>(&s_b[grp][v]) = o;
+    if (v == 0) s_n[grp] = nq;
+    __syncthreads();
+    if (tid >= 64) continue;  // s_in is written again by now, s_b and s_n behind the next row's first barrier
+    float z = 0.f, x[NO], ss = 0.f;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) z += s_n[g];
+    const float den = ml_denominator(z, m);
+#pragma unroll
+    for (int u = 0; u < NO; ++u) {
+      const int d = tid + 64 * u;
+      x[u] = 0.f;
+      if (d < DV) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) x[u] += s_b[g][d];
+        x[u] /= den;
+      }
+      ss += x[u] * x[u];
+    }
+    const float rs = 1.f / sqrtf(wave_sum(ss) / (float)a.vdim + a.eps);
+#pragma unroll
+    for (int u = 0; u < NO; ++u)
+      if (tid + 64 * u < DV) ml_store<T>(a, r.row0 + t, h, tid + 64 * u, x[u], rs, gate[u]);
   }
-  *reinterpret_cast<f32x4_t*>(&s_b[grp][v]) = o;
-  if (v == 0) s_n[grp] = nq;
-  __syncthreads();
   for (int c = 0; c < a.copies; ++c) {
     if (v == 0) {
 #pragma unroll
@@ -99,26 +136,6 @@ __global__ __launch_bounds__(256) void ml_one_kernel(MlArgs a) {
     }
     if (tid == 0) a.m[head * a.copies + c] = m;
   }
-  if (tid >= 64) return;
-  float z = 0.f, y[NO], ss = 0.f;
-#pragma unroll
-  for (int g = 0; g < NG; ++g) z += s_n[g];
-  const float den = ml_denominator(z, m);
-#pragma unroll
-  for (int u = 0; u < NO; ++u) {
-    const int d = tid + 64 * u;
-    y[u] = 0.f;
-    if (d < DV) {
-#pragma unroll
-      for (int g = 0; g < NG; ++g) y[u] += s_b[g][d];
-      y[u] /= den;
-    }
-    ss += y[u] * y[u];
-  }
-  const float rs = 1.f / sqrtf(wave_sum(ss) / (float)a.vdim + a.eps);
-#pragma unroll
-  for (int u = 0; u < NO; ++u)
-    if (tid + 64 * u < DV) ml_store<T>(a, r.row0, h, tid + 64 * u, y[u], rs, gate[u]);
 }
 
 // over the lanes with the same lane % 4
@@ -314,16 +331,30 @@ __global__ __launch_bounds__(256) void ml_plain_kernel(MlArgs a) {
   if (tid == 0) a.m[head] = m;  // read before the first barrier
 }
 
+// Up to how many rows of the longest run go row by row. A batch costs its filling however few rows it has, and of many
+// workgroups one's rows fill another's waits. us row by row and in batches, 16 heads: 128 x 128, 4 runs of 2 rows 8.2 and 8.4,
+// of 3 10.1 and 9.2; 128 x 32 (three times the operands a thread), 4 runs of 4 rows 9.7 and 11.5, of 6 13.3 and 12.5;
+// 128 x 128, 32 runs of 8 rows 30.6 and 29.8 (fp32), 28.7 and 31.4 (bf16), of 12 39.1 and 39.5 (bf16); 64 of 12 77.6 and
+// 69.7 (fp32), 75.2 and 78.9 (bf16); 128 of 24 252 and 250 (bf16). 8 heads of 64 x 64, 64 runs of 4 rows 11 and 9.3, 128
+// 14.5 and 16.
+int few_rows(int f32, const MlArgs& a, int n) {
+  const int wg = n * a.heads, fill = 4 * (2 * a.dk + a.dv) / a.dv;  // operands a thread stages for a batch
+  if (wg < 512) return fill >= 20 ? 4 : 2;
+  if (a.dk < 128) return 4;
+  return f32 || wg < 1024 ? 8 : wg < 2048 ? 16 : 24;
+}
+
 }  // namespace
 
 // n runs (a->runs), or n single rows (a->slot / a->pos)
-extern "C" int lsa_ml_steps(int f32, const MlArgs* a, int n, hipStream_t s) {
-  if (bad_ml(a) || n < 1) return LSA_BAD_SHAPE;
+extern "C" int lsa_ml_steps(int f32, const MlArgs* a, int n, int longest, hipStream_t s) {
+  if (bad_ml(a) || n < 1 || longest < 0) return LSA_BAD_SHAPE;
   const dim3 grid(n, a->heads);
+  const bool few = !a->runs || (longest > 0 && longest <= few_rows(f32, *a, n));
 #define LSA_D(K, V)                                                   \
   if (a->dk == K && a->dv == V) {                                     \
-    if (!a->runs && f32) ml_one_kernel<float, K, V><<<grid, 256, 0, s>>>(*a);     \
-    else if (!a->runs) ml_one_kernel<bf16_raw, K, V><<<grid, 256, 0, s>>>(*a);    \
+    if (few && f32) ml_rows_kernel<float, K, V><<<grid, 256, 0, s>>>(*a);         \
+    else if (few) ml_rows_kernel<bf16_raw, K, V><<<grid, 256, 0, s>>>(*a);        \
     else if (f32) ml_steps_kernel<float, K, V><<<grid, V * 4, 0, s>>>(*a);        \
     else ml_steps_kernel<bf16_raw, K, V><<<grid, V * 4, 0, s>>>(*a);              \
     LSA_CHECK_LAUNCH();                                               \

@@ -57,10 +57,11 @@ class Mlstm:
         if plan.runs is None:
             X.steps(args(slot=slot, pos=pos), self.dtype, rows)
             return ao
-        short, long = plan.memo(("mlstm", s, self.chunks),
-                                lambda: split_runs(plan, rows, state[0].shape[0], s, self.chunk_min if self.chunks else 0))
+        least = self.chunk_min if self.chunks else 0
+        short, long = plan.memo(("mlstm", s, self.chunks), lambda: split_runs(plan, rows, state[0].shape[0], s, least))
         if short is not None:
-            X.steps(args(runs=short), self.dtype, short.shape[0])
+            longest = max(r[1] for r in plan.runs if not least or r[1] < least)
+            X.steps(args(runs=short), self.dtype, short.shape[0], longest)
         if long is not None:
             items, entries, longest, several = long
             (dk, dv), f32, H = s.state_dims, torch.float32, s.heads

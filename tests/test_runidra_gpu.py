@@ -431,8 +431,9 @@ class MlCase:
         if how == "rows":
             slot, pos = (torch.tensor([r[j] for r in runs], dtype=torch.int32, device=DEV) for j in (2, 3))
             X.steps(args(slot=slot, pos=pos), self.dtype, rows)
-        elif how == "steps":
-            X.steps(args(runs=torch.tensor(runs, dtype=torch.int32, device=DEV)), self.dtype, len(runs))
+        elif how in ("steps", "known"):  # (how long the longest run is decides between two kernels)
+            X.steps(args(runs=torch.tensor(runs, dtype=torch.int32, device=DEV)), self.dtype, len(runs),
+                    max(n for _, n, *_ in runs) if how == "known" else 0)
         else:
             items, entries, longest, several = X.segments(s, runs, wide, least=64)
 
@@ -494,6 +495,29 @@ def test_matrix_memory_at_the_ends_of_batches(name, dtype):
         case.step([(1, b), (0, a)], "steps")
     for i in (0, 1):
         case.check(i, f"{name} {i}")
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+@pytest.mark.parametrize("name,count", [(n, 2) for n in ML] + [("square", 130), ("middle", 260), ("square", 260)])
+def test_matrix_memory_in_short_runs(name, count, dtype):
+    """Runs of a few rows go row by row, longer ones in batches, of few sequences and of so many that more rows do; all carry
+    the state on, and from position 0 on start anew."""
+    lens = [3 + 8 + 1 + 9 + 2 + i % 3 for i in range(count)]
+    case = MlCase(ML[name], lens, dtype)
+    case.step([(i, 3) for i in range(count)], "known")
+    case.step([(i, 8 if i % 2 else 1) for i in range(count)], "known")
+    case.step([(i, 1) for i in range(count)], "known")
+    case.step([(i, 2 if i % 2 else 9) for i in range(count)], "known")
+    case.step([(i, lens[i] - case.at[i]) for i in range(count)], "known")
+    for i in (0, 1, count // 2, count - 1):
+        case.check(i, f"{name} {i}")
+    if count > 2:  # the state's other slots too: against the batches' kernel
+        other = MlCase(ML[name], lens, dtype)
+        other.step([(i, lens[i]) for i in range(count)], "steps")
+        for i in range(count):
+            close(case.got[i], other.got[i], 1e-2 if dtype == BF else 2e-5, f"{name} {i}")
+        for a, b in zip(case.state, other.state):
+            close(a, b, 1e-5, name)
 
 
 @pytest.mark.parametrize("how,wide", [("chunks", 1), ("chunks", 1000), ("steps", 1)])
