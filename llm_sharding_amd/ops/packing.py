@@ -347,9 +347,9 @@ def _coop_choice(n_tiles: int, k: int, mb: int, need_even: bool) -> tuple | None
 
     One tile per wave and the K chunk of the row block's register budget: of these the cheapest takes 1.02, 1.06 and 1.04
     times the fastest of all configurations at 24, 48 and 96 rows (geometric mean over 62 products of 1024 to 28672 columns,
-    K 1024 to 11008; worst 1.48), 1.03 times over 42 larger ones (4096 to 57344 columns, K to 28672, 32 to 128 rows; worst 1.28); the
-    smallest split that fills the CUs takes 1.53, 1.54 and 1.57 times, of the larger 1.14, and is what is left where K or N
-    allows none of them. Four layers of Llama 3.2 3B at 47 sequences: 8 steps 5374 -> 4259 us; at 21 4171 -> 3215."""
+    K 1024 to 11008; worst 1.48), 1.03 times over 42 larger ones (4096 to 57344 columns, K to 28672, 32 to 128 rows; worst 1.27); the
+    smallest split that fills the CUs takes 1.51, 1.53 and 1.58 times, of the larger 1.14, and is what is left where K or N
+    allows none of them (profiles/cost_models.md, scripts/cost_models.py). Four layers of Llama 3.2 3B at 47 sequences: 8 steps 5374 -> 4259 us; at 21 4171 -> 3215."""
     allc = _coop_candidates(n_tiles, k, mb, need_even)
     cands = [c for c in allc if c[0] == 1 and c[2] == (2 if mb == 8 else 4) and 1 <= c[3] <= 8 and c[4] <= 2 and c[5] == 3]
     if cands:

@@ -1,0 +1,111 @@
+"""The planners' cost models against the products they were fitted to (profiles/cost_*.csv, MI355X, weights read from memory):
+how much slower than the fastest measured configuration the model's choice is, as a geometric mean and at worst, and with
+``--fit`` the cooperative GEMV's constants by least squares again. On the CPU.
+
+usage: cost_models.py [--fit]"""
+import csv
+import math
+import os
+import sys
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, ROOT)
+from llm_sharding_amd.ops import hip, packing  # noqa: E402
+
+
+def load(name, key):
+    """{values of the first ``key`` columns: [(us, the columns between)]}"""
+    out = {}
+    with open(os.path.join(ROOT, "profiles", name)) as fh:
+        rows = csv.reader(fh)
+        next(rows)
+        for r in rows:
+            out.setdefault(tuple(map(int, r[:key])), []).append((float(r[-1]), tuple(map(int, r[key:-1]))))
+    return out
+
+
+def regret(products, choose) -> str:
+    off = []
+    for k, res in products.items():
+        times = {c: us for us, c in res}
+        c = choose(k, times)
+        if c in times:
+            off.append(times[c] / min(times.values()))
+    return f"{math.exp(sum(map(math.log, off)) / len(off)):.3f}, worst {max(off):.2f}, {len(off)} products"
+
+
+def sk(k, times):
+    n, kk, m = k
+    return min((c for c in times if c[2] == 1), key=lambda c: hip.gemm_sk_cost(m, n, kk, c[0], c[1], c[3]))
+
+
+def coop(k, times):
+    return packing._coop_choice(k[0] // 16, k[1], packing.row_blocks(k[2]), False)
+
+
+def fills(k, times):
+    """The smallest split that fills the chip."""
+    for kf in (8, 4, 2):
+        c = sorted(c for c in times if c[:3] == (1, 8, kf) and c[4:] == (1, 3) and c[3] >= 1)
+        if c:
+            return next((x for x in c if k[0] // 128 * x[3] >= hip.N_CU), c[-1])
+
+
+def parts_us(rem, whole, k, s):
+    """csrc/kernels/linear_f32.hip parts_of_k"""
+    n = -(-rem * s // 256)
+    return n * -(-k // 32 // s) * 0.45 * (0.95 if n > 1 or whole else 1) \
+        + ((2.0 + 0.6 * s + 0.005 * rem * s) * (0.2 if whole else 1) if s > 1 else 0)
+
+
+def parts(k, times):
+    n, kk, rows = k
+    tiles = -(-rows // 64) * -(-n // 64)
+    whole = tiles // 256 * 256
+    if rows <= 32 or whole == tiles:
+        return None
+    have = [c for c in times if c[0] == whole and c[1] <= 16 and (c[1] == 1 or (kk >= 64 * c[1] and (tiles - whole) * c[1] <= 768))]
+    return min(have, key=lambda c: parts_us(tiles - whole, whole, kk, c[1])) if have else None
+
+
+def fit(products):
+    import numpy as np
+    from scipy.optimize import least_squares
+    data = []
+    for k, res in products.items():
+        best = min(us for us, _ in res)
+        data += [(k, c, us, best) for us, c in res if c[0] == 1 and c[2] == (2 if k[2] > 64 else 4) and 1 <= c[3] <= 8
+                 and c[4] <= 2 and c[5] == 3 and us < 2 * best]
+
+    def model(p, k, c):
+        fixed, stream, l2, far, meet, merge, fill, waves = p
+        n, kk, rows = k
+        mr, wg = 16 * packing.row_blocks(rows), n // 16 // c[1] * c[3]
+        load = -(-wg // 256) * 256 / wg if wg > 256 else (256 / wg) ** fill
+        w, a = n * kk * 2e-6, wg * mr * kk / c[3] * 2e-6
+        us = fixed + max(w / 4.9, (w / stream + a / (l2 if w <= 130 else far)) * load * max(1, waves * 256 / (wg * c[1] * c[4])) ** 0.3)
+        return us if c[3] == 1 else us + meet + c[3] * mr * n * 8e-6 / merge
+    sol = least_squares(lambda p: [math.log(model(p, k, c) / us) * (best / us) ** 2 for k, c, us, best in data],
+                        [4, 8, 27, 11, 2.2, 4.7, 0.6, 4], loss="soft_l1", f_scale=0.1)
+    print("us fixed, TB/s weights, TB/s activations (L2, beyond it), us and TB/s of a split, power of idle CUs, waves a CU wants:",
+          np.round(sol.x, 2), f"{len(data)} points, rms of the logarithm {math.sqrt(2 * sol.cost / len(data)):.3f}")
+
+
+def main() -> None:
+    packing._TUNED = {}
+    print("gemm_sk:", regret(load("cost_gemm_sk.csv", 3), sk))
+    products = load("cost_coop.csv", 3)
+    for name, pick in (("the model", coop), ("smallest split that fills", fills)):
+        for rows in (24, 48, 96):
+            print(f"cooperative GEMV, {name}, {rows} rows:", regret({k: r for k, r in products.items() if k[2] == rows}, pick))
+        print(f"cooperative GEMV, {name}, larger products at 32, 64 and 128:",
+              regret({k: r for k, r in products.items() if k[2] in (32, 64, 128)}, pick))
+    print("fp32 tiles in parts of K:", regret(
+        {k: [x for x in r if x[1][0] == -(-k[2] // 64) * -(-k[0] // 64) // 256 * 256]
+         for k, r in load("cost_f32_parts.csv", 3).items() if parts(k, {c: us for us, c in r})}, parts))
+    if "--fit" in sys.argv:
+        fit(products)
+
+
+if __name__ == "__main__":
+    main()
