@@ -230,11 +230,12 @@ bool attn_f32(const AttnArgs& a, int n, bool singles, const float* q, int ldq, c
   if (G > 16 || a.dkp > 256 || (a.dvp != 64 && a.dvp != 128 && a.dvp != 256) ||
       ((uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.pk | (uintptr_t)a.pv) % 16)
     return false;
-  // Rows of one sequence share its keys' reads once there are 1024 workgroups of a row each: 128 rows of a sequence, 8 heads
-  // over 8 kv heads 18.0 us, with a row each 24.8; 256 rows, 16 heads over 4 14.8 and 26.5. Rows of as many sequences would
-  // run one after another in a workgroup: up to 200 keys, 128 rows of 8 over 8 219 us, with a row each 46; 256 of 16 over 4 57
-  // and 45 (the plain kernel 122 and 303).
-  const int per = !singles && (long)n * a.kv_heads >= 1024 ? 16 / G : 1;
+  // Rows of one sequence share its keys' reads once there are 1024 workgroups of a row each, as many as leave one for every CU:
+  // 128 rows of a sequence, 8 heads over 8 kv heads 12.1 us, with a row each 24.8, with 16 each 18.1; 256 rows, 16 heads over 4
+  // 14.8 and with a row each 26.5. Rows of as many sequences would run one after another in a workgroup: up to 200 keys, 128 rows
+  // of 8 over 8 219 us with 16 each, 46 with one; 256 of 16 over 4 57 and 45 (the plain kernel 122 and 303).
+  const long all = (long)n * a.kv_heads;
+  const int per = singles || all < 1024 ? 1 : (int)min(16L / G, all / 256);
   const dim3 grid((n + per - 1) / per, a.kv_heads);
   const size_t lds = (size_t)16 * (a.dkp + 4) * 4;
 #define LSA_A(DV)                                                                                                          \
