@@ -6,9 +6,9 @@
 // lane's four weights are operands of the value product as they are (step r: key 4 g + r of lane = 16 g + c), and a pair's
 // numbers stay in its lanes. Keys lie token by token, values channel by channel with four tokens of a lane side by side
 // (att_vidx): both go to registers in 16-byte pieces. Each of four waves takes 32 keys at a time with sums of its own, and
-// they meet in LDS at the end; no barrier in the loop. Bound by the latency of its reads; at 2567 rows of up to 200 keys, 16
-// heads of 128 over 4 kv heads, it takes 82 us (softmax) and 92 us (sigmoids), at 16 rows 19 and 23. The plain kernel, a
-// workgroup per row and head, took 1952, 2003, 51 and 50.
+// they meet in LDS at the end; no barrier in the loop. Bound by the latency of its reads; at 2560 rows of up to 200 keys, 16
+// heads of 128 over 4 kv heads, it takes 84 us (softmax) and 97 us (sigmoids), at 16 rows 15 and 20. The plain kernel, a
+// workgroup per row and head, takes 2300 at 2560 rows.
 #include <type_traits>
 #include "paged_attn.h"
 
@@ -17,10 +17,13 @@ namespace {
 LSA_DEVICE f32x4_t mfma(float a, float b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 LSA_DEVICE f32x4_t ldf4(const float* p) { return *reinterpret_cast<const f32x4_t*>(p); }
 
-template <int DV, bool SIG>  // dvp / 64
-__global__ __launch_bounds__(256, 2) void attend_f32_kernel(AttnArgs a, int n, int per, const float* __restrict__ q, int ldq,
-                                                            const float* __restrict__ gate, int ldg, float* __restrict__ out,
-                                                            int ldo) {
+// DV: dvp / 64. U: scores' operands are requested for 16 U channels together: 4 for as few workgroups as have a CU's registers
+// to themselves (16 rows, 16 heads of 128 over 4: 15.0 us, with 2 15.8), else 2 and a wave more per SIMD (256 rows 35 us, with
+// 4 45).
+template <int DV, bool SIG, int U>
+__global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void attend_f32_kernel(
+    AttnArgs a, int n, int per, const float* __restrict__ q, int ldq, const float* __restrict__ gate, int ldg,
+    float* __restrict__ out, int ldo) {
   constexpr int DVP = 64 * DV, LO = DVP + 4;
   extern __shared__ __attribute__((aligned(16))) float s_q[];  // [16][dkp + 4]
   __shared__ __attribute__((aligned(16))) float s_o[2][16 * LO], s_ml[2][4][16];
@@ -79,30 +82,38 @@ __global__ __launch_bounds__(256, 2) void attend_f32_kernel(AttnArgs a, int n, i
         const float* kb = (const float*)kv.k + page * ATT_PAGE * a.dkp + 4 * g4;
         const float* k0 = kb + (size_t)(half + min(c, last - key0)) * a.dkp;
         const float* k1 = kb + (size_t)(half + min(c + 16, last - key0)) * a.dkp;
-        // four sums a score, each of every fourth value, as the plain kernel has them: a single one rounds twice as much
-        f32x4_t part[2][4];
+        // A score is added up from sums of every fourth of 16 U values, pair by pair: in one sum of all its rounding is twice
+        // the plain kernel's, so it is nine tenths of it.
+        f32x4_t sc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+        for (int d = 0; d < a.dkp; d += 16 * U) {  // dkp % 64 == 0
+          f32x4_t x[U], y[U], z[U];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) part[0][u] = part[1][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        for (int d = 0; d < a.dkp; d += 64) {  // dkp % 64 == 0
-          f32x4_t x[4], y[4], z[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
+          for (int u = 0; u < U; ++u) {
             x[u] = ldf4(k0 + d + 16 * u);
             y[u] = ldf4(k1 + d + 16 * u);
             z[u] = ldf4(sq + d + 16 * u);
           }
           __builtin_amdgcn_sched_barrier(0);  // all requested before the first is waited for
+          f32x4_t sum[2];
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
+          for (int h = 0; h < 2; ++h) {
+            f32x4_t p[2][2];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              part[0][j] = mfma(x[u][j], z[u][j], part[0][j]);
-              part[1][j] = mfma(y[u][j], z[u][j], part[1][j]);
+            for (int j = 0; j < 2; ++j) {
+              p[0][j] = p[1][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+              for (int u = 0; u < U; ++u) {
+                p[0][j] = mfma(x[u][2 * h + j], z[u][2 * h + j], p[0][j]);
+                p[1][j] = mfma(y[u][2 * h + j], z[u][2 * h + j], p[1][j]);
+              }
             }
-        }
-        f32x4_t sc[2];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) sc[u] = (part[u][0] + part[u][1]) + (part[u][2] + part[u][3]);
+            for (int k = 0; k < 2; ++k) sum[k] = h ? sum[k] + (p[k][0] + p[k][1]) : p[k][0] + p[k][1];
+            if constexpr (U == 2) __builtin_amdgcn_sched_barrier(0);  // (else all eight are kept)
+          }
+          sc[0] += sum[0];
+          sc[1] += sum[1];
+        }
         float wt[2][4], mx = -INFINITY;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
@@ -233,17 +244,22 @@ bool attn_f32(const AttnArgs& a, int n, bool singles, const float* q, int ldq, c
   // Rows of one sequence share its keys' reads once there are 1024 workgroups of a row each, as many as leave one for every CU:
   // 128 rows of a sequence, 8 heads over 8 kv heads 12.1 us, with a row each 24.8, with 16 each 18.1; 256 rows, 16 heads over 4
   // 14.8 and with a row each 26.5. Rows of as many sequences would run one after another in a workgroup: up to 200 keys, 128 rows
-  // of 8 over 8 219 us with 16 each, 46 with one; 256 of 16 over 4 57 and 45 (the plain kernel 122 and 303).
+  // of 8 over 8 219 us with 16 each, 46 with one; 256 of 16 over 4 57 and 35 (the plain kernel 122 and 303).
   const long all = (long)n * a.kv_heads;
   const int per = singles || all < 1024 ? 1 : (int)min(16L / G, all / 256);
   const dim3 grid((n + per - 1) / per, a.kv_heads);
   const size_t lds = (size_t)16 * (a.dkp + 4) * 4;
-#define LSA_A(DV)                                                                                                          \
-  {                                                                                                                        \
-    if (a.sig) attend_f32_kernel<DV, true><<<grid, 256, lds, s>>>(a, n, per, q, ldq, gate, ldg, out, ldo);                 \
-    else attend_f32_kernel<DV, false><<<grid, 256, lds, s>>>(a, n, per, q, ldq, gate, ldg, out, ldo);                      \
+  const bool few = all <= 512;
+#define LSA_K(DV, SIG, U) attend_f32_kernel<DV, SIG, U><<<grid, 256, lds, s>>>(a, n, per, q, ldq, gate, ldg, out, ldo)
+#define LSA_A(DV)                         \
+  {                                       \
+    if (a.sig && few) LSA_K(DV, true, 4); \
+    else if (a.sig) LSA_K(DV, true, 2);   \
+    else if (few) LSA_K(DV, false, 4);    \
+    else LSA_K(DV, false, 2);             \
   }
   if (a.dvp == 64) LSA_A(1) else if (a.dvp == 128) LSA_A(2) else LSA_A(4)
 #undef LSA_A
+#undef LSA_K
   return true;
 }

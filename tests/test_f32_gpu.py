@@ -214,13 +214,14 @@ def test_captured_product_without_a_workspace():
 
 @pytest.mark.parametrize("name", ["one_group", "small", "wide_values"])
 @pytest.mark.parametrize("loud", [False, True])
-def test_paged_attention_of_values_that_are_no_numbers(name, loud):
+@pytest.mark.parametrize("n", [1030, 120])
+def test_paged_attention_of_values_that_are_no_numbers(name, loud, n):
     """An infinity and a NaN among the values reach the rows that give their tokens a weight, and no other, also where rows
     share a workgroup: not those before, not those whose window has passed, and (``loud``) not those whose scores leave the
     tokens' weights at 0."""
     from test_gupuvik_gpu import SIZES, Case
     from llm_sharding_amd.ops import paged_attn as A
-    s, n, bad = SIZES[name], 1030, [201, 202]
+    s, bad = SIZES[name], [n // 5, n // 5 + 1]
     case = Case(s, [n], torch.float32)
     case.v[0][bad[0]], case.v[0][bad[1]] = float("inf"), float("nan")
     if loud:
