@@ -37,9 +37,11 @@ LSA_DEVICE float lane_at(float x, int lane) {
 }
 
 // Row by row: all threads share the key channels, one wave norms the read-out, the next row's operands are requested while
-// this one is computed. A single row (decoding) of 4 sequences, 16 heads of 128 x 128: 5.4 us.
-template <typename T, int DK, int DV>
-__global__ __launch_bounds__(256) void ml_rows_kernel(MlArgs a) {
+// this one is computed. ONE: a launch of single rows (decoding) has a kernel without the loop, whose operands took a 128 x 128
+// state's workgroups from four to two waves per SIMD: 4 sequences, 16 heads 5.1 us, with the loop 5.8; 64 sequences 21.8 and 24.3.
+// With it, such a state is bounded to three: 128 runs of 4 rows 68 -> 59 us, of 8 106 -> 86.
+template <typename T, int DK, int DV, bool ONE>
+__global__ __launch_bounds__(256, !ONE && DK * DV == 128 * 128 ? 3 : 1) void ml_rows_kernel(MlArgs a) {
   // a thread holds RPT rows x 4 value channels of S and the same rows of n
   constexpr int NG = 1024 / DV, RPT = DK / NG, NX = (2 * DK + DV + 255) / 256;
   constexpr int NO = (DV + 63) / 64;  // channels per lane of the wave that stores
@@ -77,8 +79,8 @@ __global__ __launch_bounds__(256) void ml_rows_kernel(MlArgs a) {
     S[j] = fresh ? f32x4_t{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4_t*>(st + (size_t)j * DV);
     n[j] = fresh ? 0.f : sn[d0 + j];
   }
-  for (int t = 0; t < r.n; ++t) {
-    const bool last = t + 1 == r.n;
+  for (int t = 0; t < (ONE ? 1 : r.n); ++t) {
+    const bool last = ONE || t + 1 == r.n;
     const float i = y.i, fm = y.f + m;
     m = fmaxf(fm, i);
     const float keep = expf(fm - m), add = expf(i - m);
@@ -332,16 +334,18 @@ __global__ __launch_bounds__(256) void ml_plain_kernel(MlArgs a) {
 }
 
 // Up to how many rows of the longest run go row by row. A batch costs its filling however few rows it has, and of many
-// workgroups one's rows fill another's waits. us row by row and in batches, 16 heads: 128 x 128, 4 runs of 2 rows 8.2 and 8.4,
-// of 3 10.1 and 9.2; 128 x 32 (three times the operands a thread), 4 runs of 4 rows 9.7 and 11.5, of 6 13.3 and 12.5;
-// 128 x 128, 32 runs of 8 rows 30.6 and 29.8 (fp32), 28.7 and 31.4 (bf16), of 12 39.1 and 39.5 (bf16); 64 of 12 77.6 and
-// 69.7 (fp32), 75.2 and 78.9 (bf16); 128 of 24 252 and 250 (bf16). 8 heads of 64 x 64, 64 runs of 4 rows 11 and 9.3, 128
-// 14.5 and 16.
+// workgroups one's rows fill another's waits. us row by row and in batches: 16 heads, 4 runs: 128 x 128, 2 rows 7.7 and 8.1, 3
+// 9.7 and 8.9; 128 x 64 (twice the operands a thread), 3 rows 7.9 and 8, 4 9.6 and 8.5; 128 x 32 (three times), 4 rows 9.4 and
+// 11.2, 6 13 and 12.2. 128 x 128, 32 runs of 8 rows 29.6 and 28.9 (fp32), 27.4 and 30.5 (bf16), of 12 39.5 and 36.3, 38.1 and
+// 38.9; 64 of 12 68.9 and 68.2 (fp32), of 24 118 and 128 (bf16); 128 of 24 204 and 214 (fp32), of 32 287 and 269, 253 and 305.
+// Fewer keys: 8 heads of 64 x 64, 64 runs of 2 rows 7 and 7.8, 3 8.7 and 8.2, 128 of 4 14.2 and 14.2, 6 19.1 and 16.5; 4 heads of
+// 32 x 128, 128 runs of 3 rows 9.1 and 9.9, 4 11 and 10.7.
 int few_rows(int f32, const MlArgs& a, int n) {
   const int wg = n * a.heads, fill = 4 * (2 * a.dk + a.dv) / a.dv;  // operands a thread stages for a batch
-  if (wg < 512) return fill >= 20 ? 4 : 2;
-  if (a.dk < 128) return 4;
-  return f32 || wg < 1024 ? 8 : wg < 2048 ? 16 : 24;
+  if (wg < 512) return fill >= 36 ? 4 : fill >= 20 ? 3 : 2;
+  if (a.dk < 128) return wg >= 1024 ? 4 : a.dv > a.dk ? 3 : 2;
+  if (f32) return wg < 2048 ? 8 : 24;
+  return wg < 1024 ? 12 : wg < 2048 ? 24 : 32;
 }
 
 }  // namespace
@@ -350,15 +354,17 @@ int few_rows(int f32, const MlArgs& a, int n) {
 extern "C" int lsa_ml_steps(int f32, const MlArgs* a, int n, int longest, hipStream_t s) {
   if (bad_ml(a) || n < 1 || longest < 0) return LSA_BAD_SHAPE;
   const dim3 grid(n, a->heads);
-  const bool few = !a->runs || (longest > 0 && longest <= few_rows(f32, *a, n));
-#define LSA_D(K, V)                                                   \
-  if (a->dk == K && a->dv == V) {                                     \
-    if (few && f32) ml_rows_kernel<float, K, V><<<grid, 256, 0, s>>>(*a);         \
-    else if (few) ml_rows_kernel<bf16_raw, K, V><<<grid, 256, 0, s>>>(*a);        \
-    else if (f32) ml_steps_kernel<float, K, V><<<grid, V * 4, 0, s>>>(*a);        \
-    else ml_steps_kernel<bf16_raw, K, V><<<grid, V * 4, 0, s>>>(*a);              \
-    LSA_CHECK_LAUNCH();                                               \
-    return LSA_OK;                                                    \
+  const bool few = longest > 0 && longest <= few_rows(f32, *a, n);
+#define LSA_D(K, V)                                                                      \
+  if (a->dk == K && a->dv == V) {                                                        \
+    if (!a->runs && f32) ml_rows_kernel<float, K, V, true><<<grid, 256, 0, s>>>(*a);     \
+    else if (!a->runs) ml_rows_kernel<bf16_raw, K, V, true><<<grid, 256, 0, s>>>(*a);    \
+    else if (few && f32) ml_rows_kernel<float, K, V, false><<<grid, 256, 0, s>>>(*a);    \
+    else if (few) ml_rows_kernel<bf16_raw, K, V, false><<<grid, 256, 0, s>>>(*a);        \
+    else if (f32) ml_steps_kernel<float, K, V><<<grid, V * 4, 0, s>>>(*a);               \
+    else ml_steps_kernel<bf16_raw, K, V><<<grid, V * 4, 0, s>>>(*a);                     \
+    LSA_CHECK_LAUNCH();                                                                  \
+    return LSA_OK;                                                                       \
   }
   LSA_D(32, 32) LSA_D(32, 64) LSA_D(32, 128) LSA_D(64, 32) LSA_D(64, 64) LSA_D(64, 128) LSA_D(128, 32) LSA_D(128, 64)
   LSA_D(128, 128)

@@ -179,3 +179,19 @@ def test_fdot2_repro_isa(tmp_path):
     if len({(a, b) for _, a, b in bc}) == 4:
         pytest.skip("this hipcc compiles the bit_cast form correctly (miscompile fixed)")
     assert len({(a, b) for _, a, b in bc}) == 1, bc  # all four dot products on dword 0
+
+
+@pytest.mark.skipif(not shutil.which("/opt/rocm/bin/hipcc"), reason="hipcc not available")
+def test_matrix_memory_row_by_row_keeps_its_waves(tmp_path):
+    """A 128 x 128 state's registers leave single rows four waves per SIMD and runs three, without spills."""
+    r = subprocess.run(["/opt/rocm/bin/hipcc", "-O3", "-std=c++17", "--offload-arch=gfx950", "--cuda-device-only", "-c",
+                        "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Rpass-analysis=kernel-resource-usage",
+                        os.path.join(ROOT, "csrc", "kernels", "mlstm.hip"), "-o", str(tmp_path / "o")],
+                       check=True, capture_output=True, text=True).stderr
+    got = {}
+    for part in r.split("Function Name: ")[1:]:
+        got[part.split()[0]] = [int(re.search(re.escape(k) + r": (\d+)", part).group(1))
+                                for k in ("Occupancy [waves/SIMD]", "ScratchSize [bytes/lane]")]
+    for one, waves in ((1, 4), (0, 3)):
+        of = [v for k, v in got.items() if "ml_rows_kernel" in k and f"Li128ELi128ELb{one}" in k]
+        assert len(of) == 2 and all(w >= waves and spill == 0 for w, spill in of), got
