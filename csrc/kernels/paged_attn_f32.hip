@@ -67,11 +67,12 @@ __global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void 
     float m, l;
     // A value that a pair does not see, or whose weight is 0, has no part in its sums, whatever it is: a tile's product is 0
     // times it, which an infinity or a NaN would make a NaN of. A wave whose sums are not all finite takes its keys once more,
-    // each pair without what it gives no weight to. (The check is 1 to 3 % of 16 to 67 us: one row of 64 to 256 sequences.)
-    auto sums = [&](auto apart) {
+    // each pair without what it gives no weight to, by the maximum of all waves' keys (m0; a sum that is an infinity is not
+    // scaled down to 0). (The check is 1 to 3 % of 16 to 67 us: one row of 64 to 256 sequences.)
+    auto sums = [&](auto apart, float m0) {
 #pragma unroll
       for (int t = 0; t < 4 * DV; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      m = -INFINITY, l = 0.f;
+      m = m0, l = 0.f;
       for (int i = w; i < 2 * blocks.n; i += 4) {
         const bool pool = blocks.is_pooled(i >> 1);
         const int half = 32 * (i & 1), key0 = blocks.at(i >> 1) * ATT_PAGE + half;
@@ -183,14 +184,14 @@ __global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void 
         }
       }
     };
-    sums(std::false_type{});
+    sums(std::false_type{}, -INFINITY);
     bool finite = true;
 #pragma unroll
     for (int t = 0; t < 4 * DV; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) finite = finite && fabsf(o[t][r]) < INFINITY;
-    if (!__all(finite)) sums(std::true_type{});
-    float f = 1.f, F = a.oscale;
+    const bool again = !__all(finite);
+    float f = 1.f, F = a.oscale, M = -INFINITY;
     if constexpr (!SIG) {
       l += lane_xor<16>(l);
       l += lane_xor<32>(l);
@@ -199,16 +200,17 @@ __global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void 
         s_ml[1][w][c] = l;
       }
       __syncthreads();
-      float M = -INFINITY, L = 0.f;
+      float L = 0.f;
 #pragma unroll
       for (int x = 0; x < 4; ++x) M = fmaxf(M, s_ml[0][x][c]);
 #pragma unroll
       for (int x = 0; x < 4; ++x)
         if (s_ml[0][x][c] != -INFINITY) L += s_ml[1][x][c] * expf(s_ml[0][x][c] - M);
-      f = m == -INFINITY ? 0.f : expf(m - M);
+      f = again ? 1.f : m == -INFINITY ? 0.f : expf(m - M);
       const float t = a.sink ? fmaxf(M, 0.f) : M, e = expf(M - t);
       F *= e / (L * e + (a.sink ? expf(-t) : 0.f));
     }
+    if (again) sums(std::true_type{}, M);
     f *= F;
     // waves 0 and 1 write, 2 and 3 add: channels 16 t + 4 g4 + r of pair c
     float* so = s_o[w & 1] + c * LO + 4 * g4;

@@ -248,6 +248,29 @@ def test_paged_attention_of_values_that_are_no_numbers(name, loud, n):
 
 
 @pytest.mark.parametrize("name", ["one_group", "small", "wide_values"])
+@pytest.mark.parametrize("bad", [5, 40, 70, 100])
+def test_paged_attention_of_a_value_far_below_the_top(name, bad):
+    """A token that outweighs all others leaves an infinity's weight at 0, also where another wave has it: its rows' sums are
+    those without the infinity."""
+    import dataclasses
+    from test_gupuvik_gpu import SIZES, Case
+    from llm_sharding_amd.ops import paged_attn as A
+    s, n, top = dataclasses.replace(SIZES[name], softcap=0.0, window=0, keep_first=0), 128, 20
+    case = Case(s, [n], torch.float32)
+    q = torch.ones(n, s.heads, s.dim)
+    case.k[0][top] = 2000 / s.scale / s.dim  # a score of 2000 times a head's factor
+    case.k[0][bad] = 0
+    case.fill()
+    want = case.want(q, [0] * n, list(range(n)))
+    case.v[0][bad] = float("inf")
+    case.fill()
+    out = torch.full((n, s.heads * s.dvp), 9.0, device=DEV)
+    A.plain(case.args([0] * n, list(range(n))), n, case.padded(q, s.dkp).to(DEV), None, out)
+    got = case.unpad(out).double().cpu()
+    rows_close(got[max(top, bad):].flatten(1), want[max(top, bad):].flatten(1), 1e-5, f"{name}: {bad}")
+
+
+@pytest.mark.parametrize("name", ["one_group", "small", "wide_values"])
 def test_paged_attention_rounds_no_more_than_four_sums_a_score(name):
     """Large scores, whose rounding the softmax passes on: against float64 no further off than scores that are added up in fp32
     as four sums of every fourth value (what the plain kernel does), everything behind them in float64, and an eighth for
