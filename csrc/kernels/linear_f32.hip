@@ -1,4 +1,4 @@
-// Projections of the fp32 engine: C[M][N] = A[M][K] . W[N][K]^T with true fp32 products and sums (f32_core.h). Epilogues:
+// Projections of the fp32 engine: C[M][N] = A[M][K] . W[N][K]^T with products and sums of fp32 accuracy (f32_core.h). Epilogues:
 // store, or the gated unit over interleaved 16-row gate / up blocks (ops/packing.py fuse_gate_up), as EPI_STORE /
 // EPI_SWIGLU / EPI_GEGLU of the bf16 GEMMs.
 #include "epilogue.h"
@@ -52,61 +52,66 @@ __global__ __launch_bounds__(NW * 64) void stream_f32_kernel(const float* __rest
   }
 }
 
-template <int EPI, int BM, int BN>
-__global__ __launch_bounds__(256) void tile_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int M,
-                                                       int N, int K, int mt, int nt, int whole, int S, float* slab,
-                                                       unsigned* counters, EpiArgs ep) {
-  using T = F32Tile<BM, BN>;
-  __shared__ __attribute__((aligned(16))) float lds[T::LDS];
+template <int EPI, int MT, int NW, int KG>
+__global__ __launch_bounds__(NW * KG * 64) void tile_f32_kernel(
+    const float* __restrict__ A, int lda, const float* __restrict__ W, int M, int N, int K, int mt, int nt, int whole, int S,
+    float* slab, unsigned* counters, EpiArgs ep) {
+  using T = F32Split<MT, NW, KG>;
+  __shared__ u32x4_t lds[T::LDS];
   __shared__ int s_last;
   // workgroups of one XCD get consecutive work; 8 row tiles share a sweep over the columns
   const int part = (int)blockIdx.x - whole, q = whole / 8, r = whole % 8, x = blockIdx.x % 8;
   const int g = part >= 0 ? whole + part / S : (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + blockIdx.x / 8;
   const int first = g / (8 * nt) * 8, gm = min(mt - first, 8), in = g - first * nt;
-  const int m0 = (first + in % gm) * BM, n0 = in / gm * BN;
-  const int tid = threadIdx.x;
-  const float *ar[T::RA], *wr[T::RW];
+  const int m0 = (first + in % gm) * T::BM, n0 = in / gm * T::BN;
+  const int p = part >= 0 ? part % S : 0, u0 = part >= 0 ? K / 32 * p / S : 0, u1 = part >= 0 ? K / 32 * (p + 1) / S : K / 32;
+  const float* wr[T::NT];
 #pragma unroll
-  for (int i = 0; i < T::RA; ++i) ar[i] = A + (size_t)min(m0 + (tid >> 3) + 32 * i, M - 1) * lda + (tid & 7) * 4;
-#pragma unroll
-  for (int i = 0; i < T::RW; ++i) wr[i] = T::tile_block(W, n0 / 16, i, N / 16, K);
-  T t;
-  if (part >= 0) {  // one of the S parts of K of a tile past the whole ones
-    const int p = part % S, u0 = K / 32 * p / S, u1 = K / 32 * (p + 1) / S;
-#pragma unroll
-    for (int i = 0; i < T::RA; ++i) ar[i] += u0 * 32;
-#pragma unroll
-    for (int i = 0; i < T::RW; ++i) wr[i] += u0 * 512;
-    t.run(ar, wr, (u1 - u0) * 32, lds);
-    if (!t.meet(p, S, slab + (size_t)(part / S) * S * (BM * BN), counters + part / S, &s_last)) return;
-  } else {
-    t.run(ar, wr, K, lds);
-  }
-  t.each([&](int m, int n, float v) {
+  for (int n = 0; n < T::NT; ++n) wr[n] = f32_block(W, min(n0 / 16 + T::wave() * T::NT + n, N / 16 - 1), K) + u0 * 512;
+  T t;  // of a tile past the whole ones one of the S parts of K
+  t.run([&](int i) { return A + (size_t)min(m0 + i, M - 1) * lda + u0 * 32; }, wr, (u1 - u0) * 32, lds);
+  if (part >= 0 && !t.meet(p, S, slab + (size_t)(part / S) * S * (T::BM * T::BN), counters + part / S, &s_last)) return;
+  t.each([&](int m, int n, float v, float u) {
+    if (m0 + m >= M || n0 + n >= N) return;
     if constexpr (epi_gated(EPI)) {
-      const float u = lane_xor<16>(v);  // gate columns sit 16 lanes below their up columns
-      if (!(n & 16) && m0 + m < M && n0 + n < N) store_glu<EPI>(ep, m0 + m, n0 + n, v, u);
+      store_glu<EPI>(ep, m0 + m, n0 + n, v, u);
     } else {
-      if (m0 + m < M && n0 + n < N) store_f32(ep, m0 + m, n0 + n, v);
+      store_f32(ep, m0 + m, n0 + n, v);
+      if (n0 + n + 16 < N) store_f32(ep, m0 + m, n0 + n + 16, u);
     }
   });
 }
 
-// How many parts of K for each of the last `rem` 64 x 64 tiles, which fill the CUs only in part; `whole` before them that
-// fill them. Modelled us: 0.45 for a part's 32 k, times the parts that a CU gets, and the meeting: 2, 0.6 for each part of a
-// tile and 0.005 for each part of all, of which a fifth shows where whole tiles run beside it. Of all splits it takes one
-// that is 1.003 times the fastest (geometric mean, 8 products of 128 to 8320 columns at 40 to 2567 rows; worst 1.07). Against
-// whole tiles: N = K = 2048 64 rows 37 -> 16 us, 200 rows 38 -> 25, 700 rows 68 -> 51, 2567 rows 195 -> 169; K = 8192 at 128
-// rows 128 -> 44.
-int parts_of_k(int rem, int whole, int K, long long slab_floats, int counters) {
-  int best = 1;
+// A product's tiles, and how many parts of K for each of the last `rem` ones, which fill the CUs only in part (S; `whole` before
+// them that fill them). Modelled us: a round of tiles its steps of 32 k and 5.2 to begin and end, a part its share of the steps;
+// the meeting by the parts of a tile and by their bytes. Fitted to 176 products (11 of 512 to 8192 k by 640 to 16384 columns at 20
+// to 2567 rows, all forms and splits): what it takes is 1.005 times the fastest (geometric mean; worst 1.08). The largest tiles
+// split least and read least (1.04 us for 128 x 128 of 32 k against 1.52 of the smallest), the smallest leave the fewest CUs idle.
+struct Plan {
+  int rows, cols, whole, S;
+};
+Plan plan(int M, int N, int K, long long slab_floats, int counters) {
+  struct Form {
+    int rows, cols;
+    double busy, idle;  // us for 32 k: all CUs at it, few
+  };
+  constexpr Form forms[] = {{128, 256, 2.08, 1.74}, {128, 128, 1.14, 0.92}, {64, 128, 0.635, 0.525}, {64, 64, 0.38, 0.31}};
+  Plan best{};
   double least = 0;
-  for (int S : {1, 2, 3, 4, 6, 8, 12, 16}) {
-    if (S > 1 && (K / 32 < 2 * S || rem * S > 768 || (long long)rem * S * 4096 > slab_floats || rem > counters)) continue;
-    const int per = (K / 32 + S - 1) / S, n = (rem * S + 255) / 256;
-    const double us = n * per * 0.45 * (n > 1 || whole ? 0.95 : 1.0) +
-                      (S > 1 ? (2.0 + 0.6 * S + 0.005 * rem * S) * (whole ? 0.2 : 1.0) : 0.0);
-    if (S == 1 || us < least) best = S, least = us;
+  for (const Form& f : forms) {
+    const int tiles = ((M + f.rows - 1) / f.rows) * ((N + f.cols - 1) / f.cols), rem = tiles % 256, rounds = tiles / 256;
+    const double kb = f.rows * f.cols / 256.0;
+    for (int S : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      const long long parts = (long long)rem * S;
+      if (S > 1 && (!rem || K / 32 < 2 * S || parts > 1024 || parts * f.rows * f.cols > slab_floats || rem > counters)) continue;
+      double us = rounds * (K / 32 * f.busy + 5.2);
+      if (rem) {
+        const int n = (int)((parts + 255) / 256), per = (K / 32 + S - 1) / S;
+        us += n * (per * (rounds || n > 1 ? f.busy : f.idle + (f.busy - f.idle) * parts / 256) + 5.2);
+        if (S > 1) us += (0.28 + S * (0.22 + 0.0065 * kb) + 0.00051 * kb * parts) * (rounds ? 1.42 : 1.0);
+      }
+      if (!best.rows || us < least) best = Plan{f.rows, f.cols, S > 1 ? tiles - rem : tiles, S}, least = us;
+    }
   }
   return best;
 }
@@ -116,16 +121,17 @@ void launch(const float* a, int lda, const float* w, int M, int N, int K, const 
             unsigned* counters, int n_counters, hipStream_t s) {
 #define LSA_STREAM(MT, NT) \
   stream_f32_kernel<EPI, MT, NT, 8><<<dim3((t + NT - 1) / NT, (M + MT * 16 - 1) / (MT * 16)), 512, 0, s>>>(a, lda, w, M, N, K, ep)
-  // Up to 32 rows, and where one 16 x 16 tile per workgroup (one pair of columns of them if gated) does not fill the CUs: the
-  // stream form, us at K = 2048 against 64 x 64 tiles: N = 128 48 rows 7 and 13, N = 2048 20 rows 9 and 15, N = 8448 20 rows 28
-  // and 30, N = 16384 32 rows 36 and 40; 48 rows N = 2048 15 and 16, N = 4352 27 and 20.
+  // The stream form: up to 16 rows; up to 32 of a product that is not large (20 rows, K = 2048, N = 4352 16 against 19 us of tiles,
+  // N = 8448 28 and 25, N = 16384 35 and 31; 4096 x 4096 19 and 25); where one 16 x 16 tile per workgroup does not fill the CUs
+  // (N = 128 48 rows 7 against 13 us), or a pair of columns of them does not and K is not long (N = 2048 64 rows: K = 2048 12
+  // against 16, K = 4096 20 and 20, K = 8192 36 and 26; K = 1024, N = 1024, 128 rows 8 and 14).
   // A CU takes 3 us for a tile's products, so that the tiles are as many per workgroup as the fullest CU has anyway:
   // N = 4352 (272 tiles) two 12.2, one 14.8; N = 8448 (528) two 26.5, one 21.4; from N = 8192 on one streams better up to 8 rows
   // (N = 16384, 8 rows 24.6 against 28.4, 16 rows 28.5 and 28.7).
   const int t = N / 16, mt16 = (M + 15) / 16, g = epi_gated(EPI) ? 2 : 1;
-  const bool alone = t / g * mt16 <= 256;
-  if (K % 32 || M <= 32 || alone) {
-    const int m = M <= 16 || alone ? 1 : 2, rows = (mt16 + m - 1) / m;
+  const bool alone = (long long)t / g * mt16 <= 256, pairs = (long long)(t + 1) / 2 * mt16 <= 256 && K <= 4096;
+  if (K % 32 || M <= 16 || (M <= 32 && (long long)N * K <= 1 << 24) || alone || pairs) {
+    const int m = M <= 16 || alone || pairs ? 1 : 2, rows = (mt16 + m - 1) / m;
     const int one = (t * rows + 255) / 256, two = ((t + 1) / 2 * rows + 255) / 256 * 2;
     if constexpr (epi_gated(EPI)) {
       if (m == 1) LSA_STREAM(1, 2);
@@ -140,18 +146,15 @@ void launch(const float* a, int lda, const float* w, int M, int N, int K, const 
     return;
   }
 #undef LSA_STREAM
-  // 128 x 64 tiles (two thirds of the operand traffic) pay from 16 tiles per CU on (963 rows, N = 16384: 521 against 539 us;
-  // 2567 rows, N = 4352, 11 tiles per CU: 392 against 394); such a grid's last round is not worth parting.
-  const int tiles = ((M + 63) / 64) * ((N + 63) / 64);
-  if (tiles >= 4096) {
-    const int mt = (M + 127) / 128, nt = (N + 63) / 64;
-    tile_f32_kernel<EPI, 128, 64><<<mt * nt, 256, 0, s>>>(a, lda, w, M, N, K, mt, nt, mt * nt, 1, nullptr, nullptr, ep);
-    return;
-  }
-  const int rem = tiles % 256, S = rem ? parts_of_k(rem, tiles - rem, K, slab_floats, n_counters) : 1;
-  const int whole = S > 1 ? tiles - rem : tiles;
-  tile_f32_kernel<EPI, 64, 64><<<whole + (tiles - whole) * S, 256, 0, s>>>(a, lda, w, M, N, K, (M + 63) / 64, (N + 63) / 64, whole,
-                                                                           S, slab, counters, ep);
+  const Plan p = plan(M, N, K, slab_floats, n_counters);
+  const int mt = (M + p.rows - 1) / p.rows, nt = (N + p.cols - 1) / p.cols, grid = p.whole + (mt * nt - p.whole) * p.S;
+#define LSA_TILE(MT, NW, KG)                                                                                               \
+  tile_f32_kernel<EPI, MT, NW, KG><<<grid, NW * KG * 64, 0, s>>>(a, lda, w, M, N, K, mt, nt, p.whole, p.S, slab, counters, ep)
+  if (p.cols == 256) LSA_TILE(8, 8, 1);
+  else if (p.rows == 128) LSA_TILE(8, 4, 2);
+  else if (p.cols == 128) LSA_TILE(4, 4, 2);
+  else LSA_TILE(4, 2, 4);
+#undef LSA_TILE
 }
 
 }  // namespace

@@ -1,5 +1,5 @@
-// Mixture of experts (moe.h): routing, grouping and the expert products (bf16 on MFMA, and plain fp32
-// for the fp32 engine).
+// Mixture of experts (moe.h): routing, grouping and the expert products (bf16 on MFMA, and fp32 for the
+// fp32 engine).
 #include "f32_core.h"
 #include "moe.h"
 
@@ -289,16 +289,16 @@ __global__ __launch_bounds__(NW * 64) void moe_stream_f32_kernel(const MoeTile* 
   }
 }
 
-// many: 64 pairs x 64 columns
-template <int UP>
-__global__ __launch_bounds__(256) void moe_tile_f32_kernel(const MoeTile* __restrict__ tiles, const int* __restrict__ order,
-                                                           int top, const float* __restrict__ A, int lda,
-                                                           const float* __restrict__ W, int N, int K,
-                                                           float* __restrict__ out, int ldo) {
-  using T = F32Tile<64, 64>;
-  __shared__ __attribute__((aligned(16))) float lds[T::LDS];
-  // Workgroups of one XCD get consecutive work, 8 tiles (mostly of one expert) share a sweep over the columns: with every XCD
-  // reading all rows instead, 20536 pairs, 32 experts of 2048 x 1024 took 793 us up and 788 down, now 776 and 769.
+// many: MT x 16 pairs x NW x 32 columns. 20536 pairs, 32 experts of 2048 x 1024: up 776 -> 477, down 769 -> 465 us (64 x 64 tiles
+// on the fp32 matrix instructions before); about 90 pairs an expert, gated, of 1024 columns 509 -> 346 in 64 x 128 tiles.
+template <int UP, int MT, int NW, int KG>
+__global__ __launch_bounds__(NW * KG * 64) void moe_tile_f32_kernel(const MoeTile* __restrict__ tiles, const int* __restrict__ order,
+                                                                    int top, const float* __restrict__ A, int lda,
+                                                                    const float* __restrict__ W, int N, int K,
+                                                                    float* __restrict__ out, int ldo) {
+  using T = F32Split<MT, NW, KG>;
+  __shared__ u32x4_t lds[T::LDS];
+  // Workgroups of one XCD get consecutive work, 8 tiles (mostly of one expert) share a sweep over the columns.
   const int nx = gridDim.x, b = blockIdx.y * nx + blockIdx.x, told = tiles[0].used;
   const int used = told > 0 ? min(told, (int)gridDim.y) : gridDim.y;
   const int G = used * nx, q = G / 8, r = G % 8, x = b % 8;
@@ -307,22 +307,25 @@ __global__ __launch_bounds__(256) void moe_tile_f32_kernel(const MoeTile* __rest
   const int first = g / (8 * nx) * 8, gm = min(used - first, 8), in = g - first * nx;
   const MoeTile tile = tiles[first + in % gm];
   if (tile.expert < 0) return;
-  const int tid = threadIdx.x, n0 = in / gm * 64;
-  const float *ar[T::RA], *wr[T::RW];
+  const int n0 = in / gm * T::BN;
+  const float* wr[T::NT];
 #pragma unroll
-  for (int i = 0; i < T::RA; ++i) {
-    const int at = tile.start + min((tid >> 3) + 32 * i, tile.count - 1);
-    ar[i] = A + (size_t)(UP ? order[at] / top : at) * lda + (tid & 7) * 4;
-  }
-#pragma unroll
-  for (int i = 0; i < T::RW; ++i)
-    wr[i] = T::tile_block(W + (size_t)tile.expert * N * K, n0 / 16, i, N / 16, K);
+  for (int n = 0; n < T::NT; ++n)
+    wr[n] = f32_block(W + (size_t)tile.expert * N * K, min(n0 / 16 + T::wave() * T::NT + n, N / 16 - 1), K);
   T t;
-  t.run(ar, wr, K, lds);
-  t.each([&](int m, int n, float v) {
-    const float u = UP == MOE_GLU ? lane_xor<16>(v) : 0.f;  // up columns sit 16 lanes above their gate columns
-    if (m >= tile.count || n0 + n >= N || (UP == MOE_GLU && (n & 16))) return;
-    out[(size_t)(tile.start + m) * ldo + (UP == MOE_GLU ? n0 / 2 + (n >> 5) * 16 + (n & 15) : n0 + n)] = up_f32<UP>(v, u);
+  t.run([&](int i) {
+    const int at = tile.start + min(i, tile.count - 1);  // rows past the count are not stored
+    return A + (size_t)(UP ? order[at] / top : at) * lda;
+  }, wr, K, lds);
+  t.each([&](int m, int n, float v, float u) {
+    if (m >= tile.count || n0 + n >= N) return;
+    float* o = out + (size_t)(tile.start + m) * ldo;
+    if (UP == MOE_GLU) {
+      o[((n0 + n) >> 5) * 16 + (n & 15)] = up_f32<UP>(v, u);
+    } else {
+      o[n0 + n] = up_f32<UP>(v, 0.f);
+      o[n0 + n + 16] = up_f32<UP>(u, 0.f);  // N % 32 == 0
+    }
   });
 }
 
@@ -334,7 +337,9 @@ int launch_f32(const MoeTile* t, int max_tiles, int tile_rows, const int* order,
   if (tile_rows <= 16) moe_stream_f32_kernel<UP, 1, NT, 8><<<grid, 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
   else if (tile_rows <= 32) moe_stream_f32_kernel<UP, 2, NT, 8><<<grid, 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
   else if (tile_rows <= 64)
-    moe_tile_f32_kernel<UP><<<dim3((N + 63) / 64, max_tiles), 256, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
+    moe_tile_f32_kernel<UP, 4, 4, 2><<<dim3((N + 127) / 128, max_tiles), 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
+  else if (tile_rows <= 128)
+    moe_tile_f32_kernel<UP, 8, 8, 1><<<dim3((N + 255) / 256, max_tiles), 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
   else return LSA_UNSUPPORTED;
   LSA_CHECK_LAUNCH();
   return LSA_OK;

@@ -256,8 +256,8 @@ class StackEngine(StageEngine):
                                                          even_n=[(n, k) for n, k, even in shapes if even])
             out["coop_ws"] = hip.CoopWorkspace(dev, slab_floats=max(floats, 1 << 20), groups=max(groups, 4096))
             out["sk_ws"] = hip.SkWorkspace(dev)
-        else:  # 64 x 64 tiles of an fp32 product in up to 768 parts of K
-            out["coop_ws"] = hip.CoopWorkspace(dev, slab_floats=768 * 64 * 64, groups=256)
+        else:  # the largest tiles of an fp32 product, one of a part of K for each CU
+            out["coop_ws"] = hip.CoopWorkspace(dev, slab_floats=256 * 128 * 256, groups=256)
         return out
 
     ATTEND_ITEMS = 1024  # (row, key split) pairs of one absorbed-attention launch

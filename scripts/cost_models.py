@@ -51,21 +51,22 @@ def fills(k, times):
             return next((x for x in c if k[0] // 128 * x[3] >= hip.N_CU), c[-1])
 
 
-def parts_us(rem, whole, k, s):
-    """csrc/kernels/linear_f32.hip parts_of_k"""
-    n = -(-rem * s // 256)
-    return n * -(-k // 32 // s) * 0.45 * (0.95 if n > 1 or whole else 1) \
-        + ((2.0 + 0.6 * s + 0.005 * rem * s) * (0.2 if whole else 1) if s > 1 else 0)
+def tiles_us(k, c):
+    """csrc/kernels/linear_f32.hip plan"""
+    (n, kk, rows), (bm, bn, s) = k, c
+    busy, idle = {(128, 256): (2.08, 1.74), (128, 128): (1.14, 0.92), (64, 128): (0.635, 0.525), (64, 64): (0.38, 0.31)}[bm, bn]
+    rounds, rem = divmod(-(-rows // bm) * -(-n // bn), 256)
+    us, kb, part = rounds * (kk // 32 * busy + 5.2), bm * bn / 256, rem * s
+    if rem:
+        m = -(-part // 256)
+        us += m * (-(-kk // 32 // s) * (busy if rounds or m > 1 else idle + (busy - idle) * part / 256) + 5.2)
+        if s > 1:
+            us += (0.28 + s * (0.22 + 0.0065 * kb) + 0.00051 * kb * part) * (1.42 if rounds else 1)
+    return us
 
 
-def parts(k, times):
-    n, kk, rows = k
-    tiles = -(-rows // 64) * -(-n // 64)
-    whole = tiles // 256 * 256
-    if rows <= 32 or whole == tiles:
-        return None
-    have = [c for c in times if c[0] == whole and c[1] <= 16 and (c[1] == 1 or (kk >= 64 * c[1] and (tiles - whole) * c[1] <= 768))]
-    return min(have, key=lambda c: parts_us(tiles - whole, whole, kk, c[1])) if have else None
+def tiles(k, times):
+    return min(times, key=lambda c: tiles_us(k, c))
 
 
 def fit(products):
@@ -100,9 +101,7 @@ def main() -> None:
             print(f"cooperative GEMV, {name}, {rows} rows:", regret({k: r for k, r in products.items() if k[2] == rows}, pick))
         print(f"cooperative GEMV, {name}, larger products at 32, 64 and 128:",
               regret({k: r for k, r in products.items() if k[2] in (32, 64, 128)}, pick))
-    print("fp32 tiles in parts of K:", regret(
-        {k: [x for x in r if x[1][0] == -(-k[2] // 64) * -(-k[0] // 64) // 256 * 256]
-         for k, r in load("cost_f32_parts.csv", 3).items() if parts(k, {c: us for us, c in r})}, parts))
+    print("fp32 tiles and parts of K:", regret(load("cost_f32_tiles.csv", 3), tiles))
     if "--fit" in sys.argv:
         fit(products)
 

@@ -67,6 +67,57 @@ def test_linear_in_parts(rows, n, k, slab):
     assert not cnt.any() and bool((part[slab:] == 7).all())
 
 
+def product(x, w):
+    """x w^T by the kernel itself (Linear fills k up), 16 columns of 7 beside it."""
+    (rows, k), n, xd, wd = x.shape, w.shape[0], x.to(DEV), pack_f32(w).to(DEV)
+    out, part = torch.full((rows, n + 16), 7.0, device=DEV), torch.empty(256 * 128 * 256, device=DEV)
+    cnt = torch.zeros(256, dtype=torch.int32, device=DEV)
+    assert hip.lib().lsa_linear_f32(xd.data_ptr(), k, wd.data_ptr(), rows, n, k, hip.EPI_STORE, hip.make_epi(out=out, ldo=n + 16),
+                                    part.data_ptr(), part.numel(), cnt.data_ptr(), 256,
+                                    torch.cuda.current_stream().cuda_stream) == 0
+    assert bool((out[:, n:] == 7).all())
+    return out[:, :n].double().cpu()
+
+
+@pytest.mark.parametrize("rows,n,k", [(33, 8464, 64), (65, 16400, 32), (100, 4112, 96), (129, 16400, 224), (257, 4368, 544),
+                                      (960, 8208, 128), (2100, 2064, 160)])
+def test_linear_tiles(rows, n, k):
+    """Every size of tiles, with rows, columns and groups' parts of k that fill none; values of very different sizes, which a
+    product of only the leading pieces would miss."""
+    x, w = _rand(rows, k, seed=1), _rand(n, k, seed=2, scale=k ** -0.5)
+    x *= torch.exp2(torch.randint(-90, 60, (rows, 1), generator=torch.Generator().manual_seed(3)).float())
+    w *= torch.exp2(torch.randint(-30, 30, (n, 1), generator=torch.Generator().manual_seed(4)).float())
+    want = x.double() @ w.double().T
+    scale = x.double().norm(dim=1)[:, None] * w.double().norm(dim=1)[None]
+    off = ((product(x, w) - want).abs() / scale).max()  # of every value by itself
+    assert off < sum_tol(k)
+
+
+@pytest.mark.parametrize("rows,n,k", [(40, 4112, 64), (200, 2064, 2048), (600, 8464, 96)])
+def test_linear_values_that_are_no_numbers(rows, n, k):
+    """Infinities, NaN and values that round to an infinity in bf16 give what fp32 products of them give, and leave all other
+    results as they are without them; zeros meet infinities. Of a value below 2^-109 what is smaller than 2^-133 is lost."""
+    x, w = _rand(rows, k, seed=1), _rand(n, k, seed=2, scale=k ** -0.5)
+    w[::7, 5] = 0
+    w[3::16] = w[3::16].bfloat16().float()  # second and third pieces that are zero
+    clean = x.double() @ w.double().T
+    x[1, 5], x[rows - 1, 5], x[2, 7], x[17, 5], x[17, 6], x[30, 9] = [float(v) for v in ("inf", "-inf", "nan", "inf", "-inf", 3.4e38)]
+    x[33] = torch.rand(k) * 1e-38
+    x[34] = 1e-41
+    want = x.double() @ w.double().T
+    got = product(x, w)
+    fine = torch.ones(rows, dtype=torch.bool)
+    fine[[1, 2, 17, 30, 33, 34, rows - 1]] = False
+    rows_close(got[fine], clean[fine], sum_tol(k), "rows beside")
+    for r in (1, 2, 17, rows - 1):
+        assert torch.equal(got[r].isnan(), want[r].isnan()) and torch.equal(got[r][got[r].isinf()], want[r][want[r].isinf()]), r
+        assert not got[r].isfinite().any()
+    over = want[30].abs() > 3.402823e38
+    assert torch.equal(got[30].isinf(), over) or (got[30].isinf() ^ over).sum() <= 1
+    assert ((got[30] - want[30]).abs()[~over & got[30].isfinite()] < 1e-5 * 3.4e38).all()
+    assert (got[33:35] - want[33:35]).abs().max() < sum_tol(k) * want[33].abs().max() + k * 2.0 ** -133 * float(w.abs().max())
+
+
 @pytest.mark.parametrize("kind", ["store", "silu", "gelu"])
 @pytest.mark.parametrize("rows", [20, 64, 700])
 def test_parts_beside_each_other_on_a_cu(kind, rows):
