@@ -280,6 +280,177 @@ __global__ __launch_bounds__(DV * 4) void ml_steps_kernel(MlArgs a) {
   }
 }
 
+// the sum of a and that of b over both halves of the wave (of each 32 lanes): a's in the lower one, b's in the upper one
+LSA_DEVICE float halves(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+LSA_DEVICE float quarters(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// As above for runs that leave CUs idle: 32 value channels a workgroup, a wave 8 of them, so that a head has DV / 32 workgroups
+// of one wave per SIMD, and a lane 16 elements of the state instead of 32. The four sums over 32 lanes are halved with their
+// lanes. Read-outs go out as they are; n and m, which every workgroup reads and only the first writes, go to nm
+// [run][head][DK + 1]; ml_finish_kernel norms the ones and puts the others in their place.
+// Bound by the vector unit, some 100 instructions a row and 700 a batch for its gates and operands: 0.35 us a row. 4 portions
+// of 300 rows, 16 heads of 128 x 128: 267 -> 117 us (ml_steps_kernel, these two kernels).
+template <int DK, int DV>
+__global__ __launch_bounds__(256) void ml_split_kernel(MlArgs a, float* __restrict__ nm) {
+  constexpr int BR = 16, V = 32, W = 2 * DK + V, Q = W / 4, NX = (BR * Q + 255) / 256, KPL = DK / 32;
+  __shared__ __attribute__((aligned(16))) float s_in[BR][W], so[BR][V];  // q, k, v
+  __shared__ float s_nq[BR], s_m[BR];
+  const MlRun r = ml_run(a, blockIdx.x);
+  const int h = blockIdx.y, v0 = blockIdx.z * V, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, kg = lane >> 1;
+  if (!r.n) return;
+  const size_t head = (size_t)r.slot * a.heads + h;
+  const int v = w * 8 + (lane & 1) * 4;
+  float* const st = a.S + head * DK * DV + v0 + v;
+  const float* const sn = a.n + head * a.copies * DK;
+  const bool fresh = r.pos0 == 0;
+  f32x4_t S[KPL];
+  float n[KPL], m = fresh ? 0.f : a.m[head * a.copies];
+#pragma unroll
+  for (int j = 0; j < KPL; ++j) {
+    S[j] = fresh ? f32x4_t{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4_t*>(st + (size_t)(kg * KPL + j) * DV);
+    n[j] = fresh ? 0.f : sn[kg * KPL + j];
+  }
+  const float* const in = (const float*)a.in + (size_t)r.row0 * a.ldi;
+  f32x4_t x[NX];
+  float zi, zf;
+  auto load = [&](int t0) {
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      const int e = tid + 256 * u, t = min(t0 + e / Q, r.n - 1), c = e % Q * 4;
+      const int at = c < DK ? a.oq + h * DK + c : c < 2 * DK ? a.ok + h * DK + c - DK : a.ov + h * DV + v0 + c - 2 * DK;
+      x[u] = *reinterpret_cast<const f32x4_t*>(in + (size_t)t * a.ldi + at);
+    }
+    const float* z = a.in32 + (size_t)(r.row0 + min(t0 + (lane & (BR - 1)), r.n - 1)) * a.ldi32 + h;
+    zi = z[a.oi];
+    zf = z[a.of];
+  };
+  load(0);
+  for (int t0 = 0; t0 < r.n; t0 += BR) {
+    const int nb = min(BR, r.n - t0);
+#pragma unroll
+    for (int u = 0; u < NX; ++u) {
+      const int e = tid + 256 * u, c = e % Q * 4;
+      if (e >= BR * Q) continue;
+      f32x4_t y = c < DK ? x[u] * a.q_scale : x[u];
+      if (e / Q >= nb) y = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<f32x4_t*>(&s_in[0][0] + 4 * e) = y;
+    }
+    // a lane's gates, the running maximum of its row, and from these what its step keeps and adds
+    const float i = ml_in(a, zi), f = ml_forget(a, zf);
+    float fm = 0.f, mx = 0.f;
+    for (int t = 0; t < nb; ++t) {
+      const float y = lane_at(f, t) + m;
+      m = fmaxf(y, lane_at(i, t));
+      if ((lane & (BR - 1)) == t) fm = y, mx = m;
+    }
+    const float keep = expf(fm - mx), add = (lane & (BR - 1)) < nb ? expf(i - mx) : 0.f;  // rows past the batch change nothing
+    __syncthreads();
+    if (tid < BR) s_m[tid] = mx;
+    if (t0 + BR < r.n) load(t0 + BR);
+    __builtin_amdgcn_sched_barrier(0);  // requested here, not where they are first used
+    typedef float kvec __attribute__((ext_vector_type(KPL)));
+    struct Row {
+      kvec q, k;
+      f32x4_t v;
+    };
+    auto fetch = [&](int t, Row& y) {
+      y.q = *reinterpret_cast<const kvec*>(&s_in[t][kg * KPL]);
+      y.k = *reinterpret_cast<const kvec*>(&s_in[t][DK + kg * KPL]);
+      y.v = *reinterpret_cast<const f32x4_t*>(&s_in[t][2 * DK + v]);
+    };
+    auto step = [&](int t, const Row& y) {
+      const float kp = lane_at(keep, t), ad = lane_at(add, t);
+      const f32x4_t u = y.v * ad;
+      f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+      float nq = 0.f;
+#pragma unroll
+      for (int j = 0; j < KPL; ++j) {
+        const float q = y.q[j], k = y.k[j];
+        S[j] = S[j] * kp + u * k;
+        o += S[j] * q;
+        n[j] = n[j] * kp + ad * k;
+        nq += n[j] * q;
+      }
+      float z = quarters(halves(o[0], o[1]), halves(o[2], o[3]));
+      z += dpp_mov<0x4E>(z);
+      z += dpp_mov<0x124>(z);
+      z += dpp_mov<0x128>(z);
+      nq += dpp_mov<0x4E>(nq);
+      nq += dpp_mov<0x124>(nq);
+      nq += dpp_mov<0x128>(nq);
+      nq += lane_xor<16>(nq);
+      nq += lane_xor<32>(nq);
+      so[t][v + (lane >> 3 & 2) + (lane >> 5)] = z;  // lanes with the same sum store it all: no branch
+      s_nq[t] = nq;
+    };
+    Row y[2][2];  // two rows in one block of code: the sums of one are made beside the products of the other
+    fetch(0, y[0][0]);
+    fetch(1, y[0][1]);
+    for (int t = 0; t < nb; t += 4) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int u = t + 2 * p;
+        fetch((u + 2) % BR, y[1 - p][0]);
+        fetch((u + 3) % BR, y[1 - p][1]);
+        step(u, y[p][0]);
+        step(u + 1, y[p][1]);
+      }
+    }
+    __syncthreads();
+    const int rt = tid / 16, c = tid % 16 * 2;
+    if (rt >= nb) continue;  // s_in and so are written again behind this barrier and the next
+    const float den = ml_denominator(s_nq[rt], s_m[rt]);
+    *reinterpret_cast<float2*>((float*)a.out + (size_t)(r.row0 + t0 + rt) * a.ldo + h * DV + v0 + c) =
+        make_float2(so[rt][c] / den, so[rt][c + 1] / den);
+  }
+#pragma unroll
+  for (int j = 0; j < KPL; ++j) *reinterpret_cast<f32x4_t*>(st + (size_t)(kg * KPL + j) * DV) = S[j];
+  if (blockIdx.z) return;
+  float* to = nm + ((size_t)blockIdx.x * a.heads + h) * (DK + 1);
+  if (w == 0 && (lane & 1) == 0) {
+#pragma unroll
+    for (int j = 0; j < KPL; ++j) to[kg * KPL + j] = n[j];
+  }
+  if (tid == 0) to[DK] = m;
+}
+
+// What ml_split_kernel left: rows of a run by blockIdx.y, dv / 4 lanes per head, in place; n and m into all their copies.
+__global__ __launch_bounds__(256) void ml_finish_kernel(MlArgs a, const float* __restrict__ nm) {
+  const MlRun r = ml_run(a, blockIdx.x);
+  const int g4 = a.dv / 4, n = a.heads * g4;
+  for (int t = blockIdx.y; t < r.n; t += gridDim.y) {
+    const size_t row = r.row0 + t;
+    for (int c = threadIdx.x; c < n; c += 256) {  // whole heads leave together
+      float* const o = (float*)a.out + row * a.ldo + 4 * c;
+      const f32x4_t y = *reinterpret_cast<const f32x4_t*>(o), nw = *reinterpret_cast<const f32x4_t*>(a.norm + 4 * c);
+      const f32x4_t g = *reinterpret_cast<const f32x4_t*>((const float*)a.in + row * a.ldi + a.og + 4 * c);
+      float ss = y[0] * y[0] + y[1] * y[1] + y[2] * y[2] + y[3] * y[3];
+      for (int s = g4 / 2; s > 0; s >>= 1) ss += __shfl_xor(ss, s, 64);
+      const float rs = 1.f / sqrtf(ss / (float)a.vdim + a.eps);
+      f32x4_t z;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) z[j] = y[j] * rs * nw[j] * sigmoid(g[j]);
+      *reinterpret_cast<f32x4_t*>(o) = z;
+    }
+  }
+  if (blockIdx.y || !r.n) return;
+  for (int e = threadIdx.x; e < a.heads * (a.dk + 1); e += 256) {
+    const int h = e / (a.dk + 1), d = e % (a.dk + 1);
+    const size_t head = (size_t)r.slot * a.heads + h;
+    const float x = nm[((size_t)blockIdx.x * a.heads + h) * (a.dk + 1) + d];
+    for (int c = 0; c < a.copies; ++c) {
+      if (d < a.dk) a.n[(head * a.copies + c) * a.dk + d] = x;
+      else a.m[head * a.copies + c] = x;
+    }
+  }
+}
+
 // any size (one copy): the state stays in memory; thread <-> value channels, and key channels of n
 template <typename T>
 __global__ __launch_bounds__(256) void ml_plain_kernel(MlArgs a) {
@@ -348,20 +519,32 @@ int few_rows(int f32, const MlArgs& a, int n) {
   return wg < 1024 ? 12 : wg < 2048 ? 24 : 32;
 }
 
+// Runs for the split form: its second launch takes 6 us, and a CU that two of its workgroups share gains nothing. us in batches
+// and split, 16 heads of 128 x 128: 4 runs of 12 rows 17 and 15.5, of 8 13.9 and 14.5, of 60 59 and 33; 8 runs of 12 rows 17.6 and
+// 17.1, of 300 268 and 160; 16 of 60 63 and 67, of 300 270 and 270; 64 of 60 227 and 208. 8 heads of 64 x 64, 4 of 100 57 and 33.
+bool split_form(const MlArgs& a, int n, int longest) { return longest >= 12 && (long long)n * a.heads * (a.dv / 32) <= 512; }
+
 }  // namespace
 
-// n runs (a->runs), or n single rows (a->slot / a->pos)
-extern "C" int lsa_ml_steps(int f32, const MlArgs* a, int n, int longest, hipStream_t s) {
-  if (bad_ml(a) || n < 1 || longest < 0) return LSA_BAD_SHAPE;
+// n runs (a->runs), or n single rows (a->slot / a->pos); longest: none has more rows (0: not known); nm: scratch, nm_floats
+// n heads (dk + 1) or no form that needs it
+extern "C" int lsa_ml_steps(int f32, const MlArgs* a, int n, int longest, float* nm, long long nm_floats, hipStream_t s) {
+  if (bad_ml(a) || n < 1 || longest < 0 || (!nm && nm_floats)) return LSA_BAD_SHAPE;
   const dim3 grid(n, a->heads);
   const bool few = longest > 0 && longest <= few_rows(f32, *a, n);
+  const bool split = f32 && a->runs && !few && split_form(*a, n, longest) &&
+                     nm_floats >= (long long)n * a->heads * (a->dk + 1) && !((a->ldi | a->ldo | a->oq | a->ok | a->ov | a->og) % 4) &&
+                     !(((uintptr_t)a->in | (uintptr_t)a->out | (uintptr_t)a->norm | (uintptr_t)a->S) % 16);
 #define LSA_D(K, V)                                                                      \
   if (a->dk == K && a->dv == V) {                                                        \
     if (!a->runs && f32) ml_rows_kernel<float, K, V, true><<<grid, 256, 0, s>>>(*a);     \
     else if (!a->runs) ml_rows_kernel<bf16_raw, K, V, true><<<grid, 256, 0, s>>>(*a);    \
     else if (few && f32) ml_rows_kernel<float, K, V, false><<<grid, 256, 0, s>>>(*a);    \
     else if (few) ml_rows_kernel<bf16_raw, K, V, false><<<grid, 256, 0, s>>>(*a);        \
-    else if (f32) ml_steps_kernel<float, K, V><<<grid, V * 4, 0, s>>>(*a);               \
+    else if (split) {                                                                    \
+      ml_split_kernel<K, V><<<dim3(n, a->heads, V / 32), 256, 0, s>>>(*a, nm);           \
+      ml_finish_kernel<<<dim3(n, longest < 512 ? longest : 512), 256, 0, s>>>(*a, nm);   \
+    } else if (f32) ml_steps_kernel<float, K, V><<<grid, V * 4, 0, s>>>(*a);               \
     else ml_steps_kernel<bf16_raw, K, V><<<grid, V * 4, 0, s>>>(*a);                     \
     LSA_CHECK_LAUNCH();                                                                  \
     return LSA_OK;                                                                       \

@@ -65,14 +65,17 @@ def chunked(a: MlArgs, s, items, longest: int, several: bool, gates, rows: int, 
            "lsa_ml_chunked")
 
 
-def steps(a: MlArgs, dtype, n: int, longest: int = 0) -> None:
-    """n runs (or rows), step by step; ``longest``: none has more rows (0: not known)."""
-    _check(lib().lsa_ml_steps(is_f32(dtype), ctypes.byref(a), n, longest, _stream()), "lsa_ml_steps")
+def steps(a: MlArgs, dtype, n: int, longest: int = 0, nm=None) -> None:
+    """n runs (or rows), step by step; ``longest``: none has more rows (0: not known); ``nm``: fp32 scratch of n heads (dk + 1)
+    values for the form that gives a head several workgroups (none: another form)."""
+    _req(nm is None or (nm.dtype == torch.float32 and nm.is_contiguous()), "mlstm: scratch")
+    _check(lib().lsa_ml_steps(is_f32(dtype), ctypes.byref(a), n, longest, _p(nm), 0 if nm is None else nm.numel(), _stream()),
+           "lsa_ml_steps")
 
 
 def declare(L: ctypes.CDLL) -> None:
     """Signatures of these entry points (called by hip.load_library)."""
     vp, i = ctypes.c_void_p, ctypes.c_int
     ma = ctypes.POINTER(MlArgs)
-    hip.set_signatures(L, {"lsa_ml_steps": [i, ma, i, i, vp],
+    hip.set_signatures(L, {"lsa_ml_steps": [i, ma, i, i, vp, ctypes.c_longlong, vp],
                            "lsa_ml_chunked": [ma, vp, i, i, i, vp, i, vp, vp, vp, vp, i, vp]})

@@ -57,17 +57,17 @@ class Mlstm:
         if plan.runs is None:
             X.steps(args(slot=slot, pos=pos), self.dtype, rows)
             return ao
+        def ws(name, n):
+            return eng.workspace(name, 4 * n).view(torch.float32)[:n]
         least = self.chunk_min if self.chunks else 0
         short, long = plan.memo(("mlstm", s, self.chunks), lambda: split_runs(plan, rows, state[0].shape[0], s, least))
         if short is not None:
             longest = max(r[1] for r in plan.runs if not least or r[1] < least)
-            X.steps(args(runs=short), self.dtype, short.shape[0], longest)
+            X.steps(args(runs=short), self.dtype, short.shape[0], longest,
+                    ws("ml_nm", short.shape[0] * s.heads * (s.state_dims[0] + 1)) if self.dtype == torch.float32 else None)
         if long is not None:
             items, entries, longest, several = long
-            (dk, dv), f32, H = s.state_dims, torch.float32, s.heads
-
-            def ws(name, n):
-                return eng.workspace(name, 4 * n).view(f32)[:n]
+            (dk, dv), H = s.state_dims, s.heads
             o32, gates = ws("ml_o", rows * H * dv).view(rows, -1), ws("ml_g", 3 * H * rows)
             parts = tuple(ws(f"ml_{k}", entries * H * n) for k, n in (("S", dk * dv), ("n", s.copies * dk), ("m", 2 * s.copies))) \
                 if several else None

@@ -431,9 +431,10 @@ class MlCase:
         if how == "rows":
             slot, pos = (torch.tensor([r[j] for r in runs], dtype=torch.int32, device=DEV) for j in (2, 3))
             X.steps(args(slot=slot, pos=pos), self.dtype, rows)
-        elif how in ("steps", "known"):  # (how long the longest run is decides between two kernels)
-            X.steps(args(runs=torch.tensor(runs, dtype=torch.int32, device=DEV)), self.dtype, len(runs),
-                    max(n for _, n, *_ in runs) if how == "known" else 0)
+        elif how in ("steps", "known", "split"):  # (how long the longest run is, and scratch, decide between kernels)
+            table = torch.tensor(runs, dtype=torch.int32, device=DEV)  # held: the arguments have its address alone
+            nm = torch.full((len(runs) * H * (dk + 1),), float("nan"), device=DEV) if how == "split" else None
+            X.steps(args(runs=table), self.dtype, len(runs), max(n for _, n, *_ in runs) if how != "steps" else 0, nm)
         else:
             items, entries, longest, several = X.segments(s, runs, wide, least=64)
 
@@ -518,6 +519,26 @@ def test_matrix_memory_in_short_runs(name, count, dtype):
             close(case.got[i], other.got[i], 1e-2 if dtype == BF else 2e-5, f"{name} {i}")
         for a, b in zip(case.state, other.state):
             close(a, b, 1e-5, name)
+
+
+@pytest.mark.parametrize("name,count", [(n, 2) for n in ML] + [("square", 32), ("square", 33), ("narrow", 102)])
+def test_matrix_memory_with_several_workgroups_a_head(name, count):
+    """Runs around batches of 16 rows, from a start and from a state; as many as the form takes, and one more.
+    The state is that of the other form."""
+    lens = [12 + 33 + 1 + i % 18 for i in range(count)]
+    case = MlCase(ML[name], lens, F32)
+    case.step([(i, 12 - i % 3) for i in reversed(range(count))], "split")
+    case.step([(i, 33 if i % 2 else 16) for i in range(count)], "split")
+    case.step([(i, 1) for i in range(count)], "split")
+    case.step([(i, lens[i] - case.at[i]) for i in range(count)], "split")
+    for i in {0, 1, count // 2, count - 1}:
+        case.check(i, f"{name} {i}")
+    other = MlCase(ML[name], lens, F32)
+    other.step([(i, lens[i]) for i in range(count)], "steps")
+    for i in range(count):
+        close(case.got[i], other.got[i], 2e-5, f"{name} {i}")
+    for a, b in zip(case.state, other.state):
+        close(a, b, 1e-5, name)
 
 
 @pytest.mark.parametrize("how,wide", [("chunks", 1), ("chunks", 1000), ("steps", 1)])
