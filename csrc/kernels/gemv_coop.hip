@@ -588,7 +588,7 @@ int launch(bool norm, const bf16_raw* x, int ldx, const int* a_rows, const bf16_
   X(8, 1, 4, 4, 2, 3) X(4, 1, 4, 4, 4, 3) X(4, 1, 2, 4, 2, 3) X(4, 1, 2, 4, 1, 3) X(2, 1, 2, 4, 2, 3) X(8, 1, 2, 2, 2, 3) \
   X(8, 1, 3, 2, 1, 3) X(8, 1, 3, 2, 2, 3) X(8, 1, 6, 2, 1, 3) X(8, 1, 1, 2, 2, 3) X(8, 1, 1, 2, 4, 3) X(8, 1, 2, 2, 1, 3) \
   X(4, 1, 3, 4, 1, 3) X(4, 1, 3, 4, 2, 3) \
-  X(8, 1, 8, 2, 1, 4) X(8, 1, 8, 4, 1, 4) X(4, 1, 8, 4, 1, 4) X(2, 1, 8, 4, 1, 4) X(2, 1, 4, 4, 1, 4)
+  X(8, 1, 8, 2, 1, 4) X(8, 1, 8, 4, 1, 4) X(4, 1, 8, 4, 1, 4) X(2, 1, 8, 4, 1, 4) X(2, 1, 4, 4, 1, 4) X(8, 2, 2, 2, 4, 2)
 
 // fp8-weight instantiations (subset; KF even so one 16-B load carries two k-fragments; d = 3)
 #define LSA_COOP_FP8_CONFIGS(X) \

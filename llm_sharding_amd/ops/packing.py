@@ -196,9 +196,12 @@ COOP_CONFIGS = [(2, 1, 8, 8, 1, 3), (4, 1, 8, 8, 1, 3), (2, 1, 8, 4, 1, 3), (4, 
                 (2, 1, 2, 4, 2, 3), (8, 1, 2, 2, 2, 3),
                 (8, 1, 3, 2, 1, 3), (8, 1, 3, 2, 2, 3), (8, 1, 6, 2, 1, 3), (8, 1, 1, 2, 2, 3), (8, 1, 1, 2, 4, 3),
                 (8, 1, 2, 2, 1, 3), (4, 1, 3, 4, 1, 3), (4, 1, 3, 4, 2, 3),
-                (8, 1, 8, 2, 1, 4), (8, 1, 8, 4, 1, 4), (4, 1, 8, 4, 1, 4), (2, 1, 8, 4, 1, 4), (2, 1, 4, 4, 1, 4)]
+                (8, 1, 8, 2, 1, 4), (8, 1, 8, 4, 1, 4), (4, 1, 8, 4, 1, 4), (2, 1, 8, 4, 1, 4), (2, 1, 4, 4, 1, 4),
+                (8, 2, 2, 2, 4, 2)]
 GEMV_MAX_ROWS = 128  # rows 65..128 are served by the coop kernel only
 COOP_SPLITS = (1, 2, 4, 8, 16)
+# 65 rows and more also in three parts (5120 x 13824, 100 rows: four waves' columns in two 45, in three 38.5 us)
+COOP_SPLITS_128 = (1, 2, 3, 4, 8, 16)
 
 
 def coop_candidates(n_tiles: int, k: int, rows: int, need_even: bool = False) -> list:
@@ -221,7 +224,7 @@ def _coop_candidates(n_tiles: int, k: int, mb: int, need_even: bool) -> dict:
         if b != mb or n_tiles % (tnw * nw) or k % (32 * kf) or (need_even and (tnw * nw) % 2):
             continue
         nch = k // (32 * kf)
-        for sk in COOP_SPLITS:
+        for sk in COOP_SPLITS_128 if mb == 8 else COOP_SPLITS:
             if nch < sk * kw or (kw > 1 and nch % (sk * kw)):
                 continue
             if (n_tiles // (tnw * nw)) * sk <= 4 * N_CU:
@@ -327,31 +330,36 @@ def partial_config(n_tiles: int, rows: int, k: int = 4096) -> Optional[tuple]:
 
 
 def coop_cost(n_tiles: int, k: int, mb: int, cfg: tuple) -> float:
-    """Modelled us of the cooperative GEMV with ``cfg`` (one tile per wave, whole splits) at ``mb`` row blocks, least squares
+    """Modelled us of the cooperative GEMV with ``cfg`` (whole splits) at ``mb`` row blocks, one tile per wave by least squares
     over cold products: the weights at 8.2 TB/s and every workgroup's read of the activations at 27 (from L2), over how evenly
     workgroups fill the CUs and whether a CU has four waves; not faster than memory; and a split's partial sums, written and
     read at 4.7 TB/s. More than 130 MB of weights push the activations out of L2 between two workgroups' reads: 11 TB/s. (16384 x
-    28672 at 64 rows: 512 workgroups of two waves 223 us, 256 of four 169, 256 of eight in two splits 147.)"""
-    _, nw, _, sk, kw, _ = cfg
-    n, mr, wg = 16 * n_tiles, 16 * mb, n_tiles // nw * sk
-    load = -(-wg // N_CU) * N_CU / wg if wg > N_CU else (N_CU / wg) ** 0.62
+    28672 at 64 rows: 512 workgroups of two waves 223 us, 256 of four 169, 256 of eight in two splits 147.) Two tiles per wave
+    read the activations from LDS half as often: 4 % less, and more where CUs stay idle (65 products at 100 rows)."""
+    tnw, nw, _, sk, kw, _ = cfg
+    n, mr, wg = 16 * n_tiles, 16 * mb, n_tiles // (nw * tnw) * sk
+    load = -(-wg // N_CU) * N_CU / wg if wg > N_CU else (N_CU / wg) ** (0.62 if tnw == 1 else 0.8)
     weights, acts = n * k * 2e-6, wg * mr * k // sk * 2e-6
     rate = 27 if weights <= 130 else 11
     us = 4.0 + max(weights / 4.9, (weights / 8.2 + acts / rate) * load * max(1.0, 4 * N_CU / (wg * nw * kw)) ** 0.3)
-    return us if sk == 1 else us + 2.2 + sk * mr * n * 8e-6 / 4.7
+    us = us if sk == 1 else us + 2.2 + sk * mr * n * 8e-6 / 4.7
+    return us if tnw == 1 else 0.96 * us
 
 
 @functools.lru_cache(maxsize=4096)
 def _coop_choice(n_tiles: int, k: int, mb: int, need_even: bool) -> tuple | None:
     """A configuration for a product that no table entry covers.
 
-    One tile per wave and the K chunk of the row block's register budget: of these the cheapest takes 1.02, 1.06 and 1.04
+    One tile per wave and the K chunk of the row block's register budget, from 65 rows on also two tiles per wave and four groups
+    of them along K (65 products at 100 rows: a geometric mean of 1.025 times the fastest, 1.050 without these and without
+    three parts; 4096 x 3072 16.3 -> 14.1 us, 4096 x 8192 26.5 -> 23.2, 10240 x 8192 51 -> 44.6): of the first the cheapest takes 1.02, 1.06 and 1.04
     times the fastest of all configurations at 24, 48 and 96 rows (geometric mean over 62 products of 1024 to 28672 columns,
     K 1024 to 11008; worst 1.48), 1.03 times over 42 larger ones (4096 to 57344 columns, K to 28672, 32 to 128 rows; worst 1.27); the
     smallest split that fills the CUs takes 1.51, 1.53 and 1.58 times, of the larger 1.14, and is what is left where K or N
     allows none of them (profiles/cost_models.md, scripts/cost_models.py). Four layers of Llama 3.2 3B at 47 sequences: 8 steps 5374 -> 4259 us; at 21 4171 -> 3215."""
     allc = _coop_candidates(n_tiles, k, mb, need_even)
     cands = [c for c in allc if c[0] == 1 and c[2] == (2 if mb == 8 else 4) and 1 <= c[3] <= 8 and c[4] <= 2 and c[5] == 3]
+    cands += [c for c in allc if c[:3] == (2, 2, 2) and 1 <= c[3] <= 8 and c[4:] == (4, 2)]
     if cands:
         return min(cands, key=lambda c: (coop_cost(n_tiles, k, mb, c), c[1] * c[4]))
     cands = [c for c in allc if c[3] >= 1]
