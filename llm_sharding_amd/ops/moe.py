@@ -81,23 +81,25 @@ def route(logits, rows: int, experts: int, top: int, expert, weight, how: Option
            "lsa_moe_route")
 
 
-def group(expert, pairs: int, experts: int, rows: int, order, place, tiles) -> int:
-    """Pairs sorted by expert (``order``; ``place`` is its inverse) and their tiles; returns the table's length."""
+def group(expert, pairs: int, experts: int, rows: int, order, place, tiles, spare=None) -> int:
+    """Pairs sorted by expert (``order``; ``place`` is its inverse) and their tiles; returns the table's length. ``spare``: int32
+    scratch, as long as the pairs, that lets many of them have several workgroups."""
     n = max_tiles(pairs, experts, rows)
     _req(all(t.dtype == torch.int32 for t in (expert, order, place, tiles)) and tiles.numel() >= 4 * n
          and min(expert.numel(), order.numel(), place.numel()) >= pairs, "group: shapes")
-    _check(lib().lsa_moe_group(_p(expert), pairs, experts, rows, n, _p(order), _p(place), _p(tiles), _stream()),
-           "lsa_moe_group")
+    _req(spare is None or (spare.dtype == torch.int32 and spare.is_contiguous()), "group: scratch")
+    _check(lib().lsa_moe_group(_p(expert), pairs, experts, rows, n, _p(order), _p(place), _p(tiles), _p(spare),
+                               0 if spare is None else spare.numel(), _stream()), "lsa_moe_group")
     return n
 
 
 def route_group(logits, rows: int, experts: int, top: int, tile: int, expert, weight, order, place, tiles,
-                how: Optional[RouteArgs] = None) -> int:
+                how: Optional[RouteArgs] = None, spare=None) -> int:
     """:func:`route` and :func:`group`, in one launch where there are few rows."""
     pairs, how = rows * top, how or route_args()
     if rows > 16 or experts > 256:
         route(logits, rows, experts, top, expert, weight, how)
-        return group(expert, pairs, experts, tile, order, place, tiles)
+        return group(expert, pairs, experts, tile, order, place, tiles, spare)
     n = max_tiles(pairs, experts, tile)
     _req(logits.dtype == torch.float32 and logits.stride(1) == 1 and logits.shape[0] >= rows
          and logits.shape[1] >= experts and weight.dtype == torch.float32 and weight.numel() >= pairs, "route: shapes")
@@ -128,7 +130,7 @@ def declare(L: ctypes.CDLL) -> None:
     vp, i, ra = ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(RouteArgs)
     hip.set_signatures(L, {
         "lsa_moe_route": [ra, vp, i, i, i, i, vp, vp, vp],
-        "lsa_moe_group": [vp, i, i, i, i, vp, vp, vp, vp],
+        "lsa_moe_group": [vp, i, i, i, i, vp, vp, vp, vp, i, vp],
         "lsa_moe_route_group": [ra, vp, i, i, i, i, vp, vp, i, i, vp, vp, vp, vp],
         "lsa_moe_gemm_big": [i, vp, i, i, vp, i, vp, i, i, vp, i, i, vp, i, vp],
         "lsa_moe_gemm": [i, i, vp, i, i, vp, i, vp, i, vp, i, i, vp, i, vp],

@@ -726,3 +726,25 @@ def test_experts_share_out_the_tiles_there_are(pairs, experts, rows):
         X.gemm(table, nt, rows, order, 1, a, w, n, k, out, pairs, X.DOWN)
         outs.append(out)
     assert torch.equal(*outs) and bool((outs[0].abs().sum(1) > 0).all())
+
+
+@pytest.mark.parametrize("pairs", [5119, 5120, 6143, 6144, 6145, 40961])
+@pytest.mark.parametrize("experts", [1, 7, 32, 1024])
+def test_many_pairs_are_sorted_by_several_workgroups(pairs, experts):
+    """With scratch the order is a sort by expert, ``place`` its inverse, and the tiles are those of one workgroup; one expert
+    has none. Too little scratch is none."""
+    from llm_sharding_amd.ops import moe as X
+    g = torch.Generator().manual_seed(pairs + experts)
+    e = (torch.rand(pairs, generator=g).square() * experts).int()
+    if experts > 1:
+        e[e == 3] = 1
+    expert, tables = e.to(DEV), []
+    for spare in (None, torch.full((pairs,), -9, dtype=torch.int32, device=DEV), torch.zeros(3, dtype=torch.int32, device=DEV)):
+        order, place = (torch.full((pairs,), -5, dtype=torch.int32, device=DEV) for _ in range(2))
+        tiles = torch.full((X.max_tiles(pairs, experts, 64), 4), -7, dtype=torch.int32, device=DEV)
+        X.group(expert, pairs, experts, 64, order, place, tiles, spare)
+        o = order.cpu().long()
+        assert torch.equal(o.sort().values, torch.arange(pairs)) and torch.equal(e[o], e.sort().values)
+        assert torch.equal(place.cpu().long()[o], torch.arange(pairs))
+        tables.append(tiles)
+    assert torch.equal(tables[0], tables[1]) and torch.equal(tables[0], tables[2])
