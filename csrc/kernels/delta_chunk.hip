@@ -121,10 +121,14 @@ template <int DK, int DV>
 __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const DeltaChunk* __restrict__ chunks,
                                                           unsigned char* __restrict__ ws) {
   using PC = Pieces<DK>;
-  constexpr int KF = DK / 32, LD = DK + 4, LA = C + 4;
+  constexpr int KF = DK / 32;
   constexpr size_t STRIDE = (size_t)(PC::U + DV / 8) * 1024;
-  __shared__ __attribute__((aligned(16))) float sq[C][LD], sk[C][LD], sg[C][LD], sA[C][LA], sP[C][LA];
+  // Rows without padding, their 16-byte pieces exchanged by the row (at); A below the diagonal of one square, P's columns as
+  // its rows on and above it: 53632 bytes, so that three workgroups share a CU.
+  __shared__ __attribute__((aligned(16))) float sq[C][DK], sk[C][DK], sg[C][DK], sAP[C][C];
   __shared__ float su[2 * C], sb[C];
+  const auto at = [](int t, int d) { return d ^ ((t & (DK / 4 < 16 ? DK / 4 - 1 : 15)) << 2); };
+  const auto four = [&](float (*x)[DK], int t, int d) { return *reinterpret_cast<const f32x4_t*>(&x[t][at(t, d)]); };
   const DeltaChunk ck = chunks[blockIdx.x];
   const int h = blockIdx.y, kb = h / (a.heads / a.kv_heads), kc = a.kv_heads * a.dim;
   const int channels = 2 * kc + a.heads * a.vdim;
@@ -149,31 +153,30 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
   }
   if (tid < 2 * DK) {
     auto& dst = isk ? sk : sq;
-    qk.run(a, ck, channels, [&](int t, float y) { dst[t][cd] = cd < a.dim ? y : 0.f; });
+    qk.run(a, ck, channels, [&](int t, float y) { dst[t][at(t, cd)] = cd < a.dim ? y : 0.f; });
     const float A = cd < a.dim ? -a.decay[h] * 1.4426950408889634f : 0.f, bias = cd < a.dim ? a.dt_bias[h * a.dim + cd] : 0.f;
     float g = 0.f;  // sums of log2 decays, 16 rows at a time
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
       g = isk * 16 + t < ck.n ? fmaf(A, softplus_fast(zz[t] + bias), g) : g;
-      sg[isk * 16 + t][cd] = g;
+      sg[isk * 16 + t][at(t, cd)] = g;
     }
   }
   if (tid < C) sb[tid] = tid < ck.n ? 1.f / (1.f + __expf(-a.in32[(size_t)(ck.row0 + tid) * a.ld32 + a.ob + h])) : 0.f;
-  for (int e = tid; e < C * LA; e += 256) (&sA[0][0])[e] = (&sP[0][0])[e] = 0.f;
   __syncthreads();
   {  // unit vectors: four threads per vector
     const int v = tid >> 2, t = v & (C - 1);
-    const float* x = v < C ? sq[t] : sk[t];
+    const float(*x)[DK] = v < C ? sq : sk;
     float ss = 0.f;
-    for (int d = tid & 3; d < DK; d += 4) ss = fmaf(x[d], x[d], ss);
+    for (int d = tid & 3; d < DK; d += 4) ss = fmaf(x[t][at(t, d)], x[t][at(t, d)], ss);
     ss += __shfl_xor(ss, 1, 64);
     ss += __shfl_xor(ss, 2, 64);
     if ((tid & 3) == 0) su[v] = (v < C ? a.q_scale : 1.f) / sqrtf(ss + a.unit_eps);
   }
-  for (int e = tid; e < 16 * DK; e += 256) sg[16 + e / DK][e % DK] += sg[15][e % DK];
+  for (int e = tid; e < 16 * DK; e += 256) sg[16 + e / DK][at(e / DK, e % DK)] += sg[15][at(15, e % DK)];
   __syncthreads();
   for (int e = tid; e < C * DK; e += 256) {
-    const int t = e / DK, d = e % DK;
+    const int t = e / DK, d = e % DK;  // (whole rows: the order of their pieces does not matter)
     sq[t][d] *= su[t];
     sk[t][d] *= su[C + t];
   }
@@ -185,9 +188,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
     float x = 0.f, y = 0.f;
 #pragma unroll 4
     for (int d = 0; d < DK; d += 4) {
-      const f32x4_t gi = *reinterpret_cast<const f32x4_t*>(&sg[i][d]), gj = *reinterpret_cast<const f32x4_t*>(&sg[j][d]);
-      const f32x4_t ki = *reinterpret_cast<const f32x4_t*>(&sk[i][d]), kj = *reinterpret_cast<const f32x4_t*>(&sk[j][d]);
-      const f32x4_t qi = *reinterpret_cast<const f32x4_t*>(&sq[i][d]);
+      const f32x4_t gi = four(sg, i, d), gj = four(sg, j, d), ki = four(sk, i, d), kj = four(sk, j, d), qi = four(sq, i, d);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float z = kj[e] * __builtin_amdgcn_exp2f(gi[e] - gj[e]);
@@ -195,26 +196,30 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
         y = fmaf(qi[e], z, y);
       }
     }
-    if (i != j) sA[i][j] = sb[i] * x;
-    sP[i][j] = y;
+    if (i != j) sAP[i][j] = sb[i] * x;
+    sAP[j][i] = y;
     if (tid < 16) {  // the second block's diagonal
       float p = 0.f;
-      for (int d = 0; d < DK; ++d) p = fmaf(sq[16 + tid][d], sk[16 + tid][d], p);
-      sP[16 + tid][16 + tid] = p;
+      for (int d = 0; d < DK; ++d) p = fmaf(sq[16 + tid][at(tid, d)], sk[16 + tid][at(tid, d)], p);
+      sAP[16 + tid][16 + tid] = p;
     }
   }
   if (w < 2) {  // the block below, through row 15: wave 0 A, wave 1 P
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    const auto& sx = w ? sq : sk;
+    float(*sx)[DK] = w ? sq : sk;
 #pragma unroll
     for (int kf = 0; kf < KF; ++kf) {
       float x[8], y[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int d = kf * 32 + q4 * 8 + e;
-        const float g = sg[15][d];
-        x[e] = sx[16 + l16][d] * __builtin_amdgcn_exp2f(sg[16 + l16][d] - g);
-        y[e] = sk[l16][d] * __builtin_amdgcn_exp2f(g - sg[l16][d]);
+      for (int p = 0; p < 2; ++p) {
+        const int d = kf * 32 + q4 * 8 + 4 * p;
+        const f32x4_t g = four(sg, 15, d), gi = four(sg, 16 + l16, d), gj = four(sg, l16, d), xi = four(sx, 16 + l16, d),
+                      kj = four(sk, l16, d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[4 * p + e] = xi[e] * __builtin_amdgcn_exp2f(gi[e] - g[e]);
+          y[4 * p + e] = kj[e] * __builtin_amdgcn_exp2f(g[e] - gj[e]);
+        }
       }
       u32x4_t xh, xl, yh, yl;
       split_pair(x, xh, xl);
@@ -224,8 +229,8 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = 16 + q4 * 4 + r;
-      if (w) sP[i][l16] = acc[r];
-      else sA[i][l16] = sb[i] * acc[r];
+      if (w) sAP[l16][i] = acc[r];
+      else sAP[i][l16] = sb[i] * acc[r];
     }
   }
   // q e^G (rows x key channels) and k e^(G_31 - G) (key channels x rows)
@@ -233,9 +238,10 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
     const int ln = e & 63, kf = (e >> 6) % KF, t = (e >> 6) / KF * 16 + (ln & 15), d0 = kf * 32 + (ln >> 4) * 4;
     float f[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int d = d0 + (j & 4) * 4 + (j & 3);
-      f[j] = sq[t][d] * __builtin_amdgcn_exp2f(sg[t][d]);
+    for (int p = 0; p < 2; ++p) {
+      const f32x4_t y = four(sq, t, d0 + 16 * p), g = four(sg, t, d0 + 16 * p);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[4 * p + j] = y[j] * __builtin_amdgcn_exp2f(g[j]);
     }
     put_pair(out + PC::Q * 1024, out + (PC::Q + 2 * KF) * 1024, e, f);
   }
@@ -245,17 +251,20 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int t = t0 + (j & 4) * 4 + (j & 3);
-      f[j] = sk[t][d] * __builtin_amdgcn_exp2f(sg[C - 1][d] - sg[t][d]);
+      f[j] = sk[t][at(t, d)] * __builtin_amdgcn_exp2f(sg[C - 1][at(C - 1, d)] - sg[t][at(t, d)]);
     }
     put_pair(out + PC::K * 1024, out + (PC::K + 2 * KF) * 1024, e, f);
   }
-  for (int d = tid; d < DK; d += 256) reinterpret_cast<float*>(out + PC::E * 1024)[d] = __builtin_amdgcn_exp2f(sg[C - 1][d]);
+  for (int d = tid; d < DK; d += 256) reinterpret_cast<float*>(out + PC::E * 1024)[d] = __builtin_amdgcn_exp2f(sg[C - 1][at(C - 1, d)]);
   __syncthreads();
   if (tid < 128) {  // P (rows x rows)
     const int t = (tid >> 6) * 16 + l16;
     float f[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = sP[t][q4 * 4 + (j & 4) * 4 + (j & 3)];
+    for (int j = 0; j < 8; ++j) {
+      const int i = q4 * 4 + (j & 4) * 4 + (j & 3);
+      f[j] = i <= t ? sAP[i][t] : 0.f;
+    }
     put_pair(out + PC::P * 1024, out + (PC::P + 2) * 1024, tid, f);
   }
   // (1 + A) x = b, one column per thread: beta v -> U, beta k e^G -> W
@@ -266,14 +275,14 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
       vc.run(a, ck, channels, [&](int t, float y) { x[t] = c < a.vdim ? y * sb[t] : 0.f; });
     } else {
 #pragma unroll
-      for (int t = 0; t < C; ++t) x[t] = sb[t] * sk[t][c - DV] * __builtin_amdgcn_exp2f(sg[t][c - DV]);
+      for (int t = 0; t < C; ++t) x[t] = sb[t] * sk[t][at(t, c - DV)] * __builtin_amdgcn_exp2f(sg[t][at(t, c - DV)]);
     }
 #pragma unroll
     for (int i = 1; i < C; ++i) {
       float s = x[i];
 #pragma unroll
       for (int j = 0; j < i; j += 4) {
-        const f32x4_t r = *reinterpret_cast<const f32x4_t*>(&sA[i][j]);
+        const f32x4_t r = *reinterpret_cast<const f32x4_t*>(&sAP[i][j]);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           if (j + e < i) s = fmaf(-r[e], x[j + e], s);
@@ -286,7 +295,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
       for (int e = 0; e < 8; ++e) u[e * 16 + (c & 15)] = f32x4_t{x[4 * e], x[4 * e + 1], x[4 * e + 2], x[4 * e + 3]};
     } else {
 #pragma unroll
-      for (int t = 0; t < C; ++t) sq[t][c - DV] = x[t];  // q is in memory already
+      for (int t = 0; t < C; ++t) sq[t][at(t, c - DV)] = x[t];  // q is in memory already
     }
   }
   __syncthreads();
@@ -294,7 +303,11 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
     const int ln = e & 63, kf = (e >> 6) % KF, t = (e >> 6) / KF * 16 + (ln & 15), d0 = kf * 32 + (ln >> 4) * 4;
     float f[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = sq[t][d0 + (j & 4) * 4 + (j & 3)];
+    for (int p = 0; p < 2; ++p) {
+      const f32x4_t y = four(sq, t, d0 + 16 * p);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[4 * p + j] = y[j];
+    }
     put_pair(out, out + 2 * KF * 1024, e, f);
   }
 }
