@@ -5,9 +5,10 @@
 // as many rows of one sequence as fit. Scores are keys (rows of a tile) by pairs, values channels by pairs, so that a
 // lane's four weights are operands of the value product as they are (step r: key 4 g + r of lane = 16 g + c), and a pair's
 // numbers stay in its lanes. Keys lie token by token, values channel by channel with four tokens of a lane side by side
-// (att_vidx): both go to registers in 16-byte pieces. Each of four waves takes 32 keys at a time with sums of its own, and
-// they meet in LDS at the end; no barrier in the loop. Bound by the latency of its reads; at 2560 rows of up to 200 keys, 16
-// heads of 128 over 4 kv heads, it takes 84 us (softmax) and 97 us (sigmoids), at 16 rows 15 and 20. The plain kernel, a
+// (att_vidx): both go to registers in 16-byte pieces. Each wave takes 32 keys at a time with sums of its own, and
+// they meet in LDS at the end; no barrier in the loop. Where every workgroup has a CU to itself there are eight waves.
+// Bound by the latency of its reads; at 2560 rows of up to 200 keys, 16 heads of 128 over 4 kv heads, it takes 84 us (softmax)
+// and 97 us (sigmoids), at 16 rows in a decoding step 15.2 and 18 (19.5 and 23.9 with four waves and pages looked up one by one). The plain kernel, a
 // workgroup per row and head, takes 2300 at 2560 rows.
 #include <type_traits>
 #include "paged_attn.h"
@@ -20,22 +21,42 @@ LSA_DEVICE f32x4_t ldf4(const float* p) { return *reinterpret_cast<const f32x4_t
 // DV: dvp / 64. U: scores' operands are requested for 16 U channels together: 4 for as few workgroups as have a CU's registers
 // to themselves (16 rows, 16 heads of 128 over 4: 15.0 us, with 2 15.8), else 2 and a wave more per SIMD (256 rows 35 us, with
 // 4 45).
-template <int DV, bool SIG, int U>
-__global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void attend_f32_kernel(
+template <int DV, bool SIG, int U, int NW>
+__global__ __launch_bounds__(NW * 64, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void attend_f32_kernel(
     AttnArgs a, int n, int per, const float* __restrict__ q, int ldq, const float* __restrict__ gate, int ldg,
     float* __restrict__ out, int ldo) {
-  constexpr int DVP = 64 * DV, LO = DVP + 4;
+  constexpr int DVP = 64 * DV, LO = DVP + 4, NT = NW * 64, NO = NW / 2;
   extern __shared__ __attribute__((aligned(16))) float s_q[];  // [16][dkp + 4]
-  __shared__ __attribute__((aligned(16))) float s_o[2][16 * LO], s_ml[2][4][16];
+  __shared__ __attribute__((aligned(16))) float s_o[NO][16 * LO], s_ml[2][NW][16];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g4 = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int G = a.heads / a.kv_heads, kvh = blockIdx.y, lq = a.dkp + 4;
   const int e0 = blockIdx.x * per, ne = min(per, n - e0);
   for (int s0 = 0, s1; s0 < ne; s0 = s1) {
-    const int row0 = a.index ? a.index[e0 + s0] : e0 + s0, p0 = att_pos(a, row0), slot = a.slot[row0];
+    const int row0 = a.index ? a.index[e0 + s0] : e0 + s0, slot = __builtin_amdgcn_readfirstlane(a.slot[row0]);
+    const int pos0 = __builtin_amdgcn_readfirstlane(a.pos[row0]);
+    auto queries = [&](int cols) {
+      for (int t = tid; t < cols * a.dkp; t += NT) {
+        const int x = t / a.dkp, d = t % a.dkp, e = e0 + s0 + x / G;
+        s_q[x * lq + d] = q[(size_t)(a.index ? a.index[e] : e) * ldq + (size_t)(kvh * G + x % G) * a.dkp + d];
+      }
+    };
+    // Reads that wait for one another are most of a few rows' time: the first 64 pages of the sequence come in one, beside a
+    // single row's queries.
+    const bool live = pos0 >= 0 && pos0 < a.max_pages * ATT_PAGE;
+    const int first_pages = live ? a.table[(size_t)slot * a.max_pages + min(lane, a.max_pages - 1)] : -1;
+    if (per == 1) queries(G);
+    auto table = [&](int b) {
+      return b < 64 ? __builtin_amdgcn_readlane(first_pages, b) : a.table[(size_t)slot * a.max_pages + b];
+    };
+    int p0 = -1;
+    if (live) {
+      const int pg = table(pos0 / ATT_PAGE);
+      if (pg >= 0 && pg < a.n_pages) p0 = pos0;
+    }
     s1 = s0 + 1;
     if (p0 < 0) {  // an idle row
-      for (int d = tid; d < G * a.dvp; d += 256) out[(size_t)row0 * ldo + (size_t)kvh * G * a.dvp + d] = 0.f;
+      for (int d = tid; d < G * a.dvp; d += NT) out[(size_t)row0 * ldo + (size_t)kvh * G * a.dvp + d] = 0.f;
       continue;
     }
     int lo = p0, hi = p0;
@@ -55,10 +76,7 @@ __global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void 
       r2 = a.sig[a.heads + h];
       b2 = a.sig[2 * a.heads + h];
     }
-    for (int t = tid; t < cols * a.dkp; t += 256) {
-      const int x = t / a.dkp, d = t % a.dkp, e = e0 + s0 + x / G;
-      s_q[x * lq + d] = q[(size_t)(a.index ? a.index[e] : e) * ldq + (size_t)(kvh * G + x % G) * a.dkp + d];
-    }
+    if (per != 1) queries(cols);
     __syncthreads();
     const float* sq = s_q + min(c, cols - 1) * lq + 4 * g4;
     const AttBlocks blocks(a, lo, hi);
@@ -73,12 +91,18 @@ __global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void 
 #pragma unroll
       for (int t = 0; t < 4 * DV; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       m = m0, l = 0.f;
-      for (int i = w; i < 2 * blocks.n; i += 4) {
+      for (int i = w; i < 2 * blocks.n; i += NW) {
         const bool pool = blocks.is_pooled(i >> 1);
         const int half = 32 * (i & 1), key0 = blocks.at(i >> 1) * ATT_PAGE + half;
         const int last = pool ? pooled - 1 : hi;  // behind it nothing was written
         if (key0 > last) continue;
-        const AttKv kv = att_kv(a, blocks, slot, i >> 1);
+        AttKv kv;
+        if (pool) {
+          kv = att_kv(a, blocks, slot, i >> 1);
+        } else {
+          const int pg = table(__builtin_amdgcn_readfirstlane(blocks.at(i >> 1)));
+          kv = AttKv{a.k, a.v, pg < 0 || pg >= a.n_pages ? 0 : pg};
+        }
         const size_t page = (size_t)kv.page * a.kv_heads + kvh;
         const float* kb = (const float*)kv.k + page * ATT_PAGE * a.dkp + 4 * g4;
         const float* k0 = kb + (size_t)(half + min(c, last - key0)) * a.dkp;
@@ -202,9 +226,9 @@ __global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void 
       __syncthreads();
       float L = 0.f;
 #pragma unroll
-      for (int x = 0; x < 4; ++x) M = fmaxf(M, s_ml[0][x][c]);
+      for (int x = 0; x < NW; ++x) M = fmaxf(M, s_ml[0][x][c]);
 #pragma unroll
-      for (int x = 0; x < 4; ++x)
+      for (int x = 0; x < NW; ++x)
         if (s_ml[0][x][c] != -INFINITY) L += s_ml[1][x][c] * expf(s_ml[0][x][c] - M);
       f = again ? 1.f : m == -INFINITY ? 0.f : expf(m - M);
       const float t = a.sink ? fmaxf(M, 0.f) : M, e = expf(M - t);
@@ -212,11 +236,11 @@ __global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void 
     }
     if (again) sums(std::true_type{}, M);
     f *= F;
-    // waves 0 and 1 write, 2 and 3 add: channels 16 t + 4 g4 + r of pair c
-    float* so = s_o[w & 1] + c * LO + 4 * g4;
+    // the first half of the waves write, the others add: channels 16 t + 4 g4 + r of pair c
+    float* so = s_o[w % NO] + c * LO + 4 * g4;
 #pragma unroll
     for (int turn = 0; turn < 2; ++turn) {
-      if (w >> 1 == turn) {
+      if (w / NO == turn) {
 #pragma unroll
         for (int t = 0; t < 4 * DV; ++t) {
           f32x4_t v = o[t] * f;
@@ -227,9 +251,12 @@ __global__ __launch_bounds__(256, U == 4 || DV == 1 ? 2 : DV == 2 ? 4 : 3) void 
       }
       __syncthreads();
     }
-    for (int t = tid; t < cols * a.dvp; t += 256) {
+    for (int t = tid; t < cols * a.dvp; t += NT) {
       const int x = t / a.dvp, d = t % a.dvp, e = e0 + s0 + x / G, r = a.index ? a.index[e] : e, hh = kvh * G + x % G;
-      out[(size_t)r * ldo + (size_t)hh * a.dvp + d] = (s_o[0][x * LO + d] + s_o[1][x * LO + d]) * att_gate(a, gate, r, ldg, hh, d);
+      float y = s_o[0][x * LO + d];
+#pragma unroll
+      for (int k = 1; k < NO; ++k) y += s_o[k][x * LO + d];
+      out[(size_t)r * ldo + (size_t)hh * a.dvp + d] = y * att_gate(a, gate, r, ldg, hh, d);
     }
     __syncthreads();  // s_q, s_o and s_ml serve the next sequence
   }
@@ -251,17 +278,27 @@ bool attn_f32(const AttnArgs& a, int n, bool singles, const float* q, int ldq, c
   const int per = singles || all < 1024 ? 1 : (int)min(16L / G, all / 256);
   const dim3 grid((n + per - 1) / per, a.kv_heads);
   const size_t lds = (size_t)16 * (a.dkp + 4) * 4;
-  const bool few = all <= 512;
-#define LSA_K(DV, SIG, U) attend_f32_kernel<DV, SIG, U><<<grid, 256, lds, s>>>(a, n, per, q, ldq, gate, ldg, out, ldo)
-#define LSA_A(DV)                         \
-  {                                       \
-    if (a.sig && few) LSA_K(DV, true, 4); \
-    else if (a.sig) LSA_K(DV, true, 2);   \
-    else if (few) LSA_K(DV, false, 4);    \
-    else LSA_K(DV, false, 2);             \
+  const bool few = all <= 512, alone = all <= 256;
+#define LSA_K(DV, SIG, U, NW) attend_f32_kernel<DV, SIG, U, NW><<<grid, NW * 64, lds, s>>>(a, n, per, q, ldq, gate, ldg, out, ldo)
+#define LSA_S(DV, SIG)                 \
+  if (alone) LSA_K(DV, SIG, 4, 8);     \
+  else if (few) LSA_K(DV, SIG, 4, 4);  \
+  else LSA_K(DV, SIG, 2, 4)
+#define LSA_A(DV)                              \
+  if (a.sig) {                                 \
+    LSA_S(DV, true);                           \
+  } else {                                     \
+    LSA_S(DV, false);                          \
   }
-  if (a.dvp == 64) LSA_A(1) else if (a.dvp == 128) LSA_A(2) else LSA_A(4)
+  if (a.dvp == 64) {
+    LSA_A(1)
+  } else if (a.dvp == 128) {
+    LSA_A(2)
+  } else {
+    LSA_A(4)
+  }
 #undef LSA_A
+#undef LSA_S
 #undef LSA_K
   return true;
 }

@@ -199,6 +199,21 @@ def test_paged_attention_of_many_rows(name):
         rows_close(torch.cat(got[i]).flatten(1), case.want(i).flatten(1), 1e-5, f"{name}: {i}")
 
 
+@pytest.mark.parametrize("name", ["sink", "sigmoid"])
+def test_paged_attention_behind_the_first_64_pages(name):
+    """Single rows of a sequence whose page table is longer than what a wave reads of it at once, beside a short one."""
+    from test_dumizen_gpu import SPECS, Case
+    case = Case(SPECS[name], [4163, 70], torch.float32)
+    case.step([(0, 4094), (1, 60)])
+    got = {0: [], 1: []}
+    for parts in ([(0, 1), (1, 1)], [(1, 1), (0, 1)], [(0, 1)], [(0, 64), (1, 6)], [(0, 1), (1, 1)], [(0, 1)]):
+        for i, o in case.step(parts).items():
+            got[i].append(o)
+    for i, first in ((0, 4094), (1, 60)):
+        o = torch.cat(got[i]).flatten(1)
+        rows_close(o, case.want(i).flatten(1)[first:first + len(o)], 1e-5, f"{name}: {i}")
+
+
 def _engine_with_a_parted_head(slots):
     """One layer of a real width; 40 rows of its head are 32 tiles, whose K is shared out."""
     import dataclasses
