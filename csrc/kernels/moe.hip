@@ -188,8 +188,9 @@ __global__ __launch_bounds__(1024) void group_kernel(RouteArgs ra, const float* 
 // The same of many pairs in two launches of a workgroup for every GROUP_PAIRS: counts [workgroups][E] and ranks within a
 // workgroup's pairs, then the sums over the workgroups (each makes them for itself) and the places. One workgroup is bound by its
 // pairs' turns at the counters and at memory; here a thread has two of them. us, 32 experts: 4096 pairs 5.3 and 5.8, 6000 6.2 and
-// 5.9, 25512 17.2 and 6.7, 65536 38 and 8; 8 experts 4096 5.7 and 6.2, 25512 19 and 8.7; 256 experts 25512 22 and 7.5.
-constexpr int GROUP_PAIRS = 2048, GROUP_MANY = 5120;
+// 5.9, 12000 9.6 and 6.4, 25512 17.2 and 6.7, 65536 38 and 8; 8 experts 25512 19 and 8.7; 256 experts 22 and 7.5 (graphs; in a
+// prompt's stream 5868 pairs 7.6 and 10.2, 25512 25 and 9.5).
+constexpr int GROUP_PAIRS = 2048, GROUP_MANY = 10240;
 __global__ __launch_bounds__(1024) void count_kernel(const int* __restrict__ expert, int pairs, int E, int* __restrict__ place,
                                                      int* __restrict__ counts) {
   __shared__ int s_cnt[MAX_E];

@@ -61,8 +61,9 @@ class Experts:
 def tile_rows(pairs: int, experts: int, f32: bool) -> int:
     """Pairs per tile: what an expert gets on average, rounded to a kernel's size."""
     mean = pairs / experts  # (a second tile of an expert reads its weights again)
-    if f32:  # 128 rows x 256 columns take 0.84 of the time of four tiles of 64 x 128, and an expert leaves half a tile empty
-        return next((n for n in (16, 32) if mean <= 0.75 * n), 64 if mean <= 192 else 128)
+    if f32:  # 64 x 128 and 128 rows x 256 columns: 90 pairs an expert 3907 and 4155 us a pass (Runidra 2k), 183 6000 and 5662, 104
+        # 3780 and 3804 (Dumizen 2k), 141 4568 and 4440
+        return next((n for n in (16, 32) if mean <= 0.75 * n), 64 if mean <= 112 else 128)
     return next((n for n in (16, 32, 64) if mean <= 0.75 * n), 128 if mean <= 320 else 256)
 
 

@@ -728,7 +728,7 @@ def test_experts_share_out_the_tiles_there_are(pairs, experts, rows):
     assert torch.equal(*outs) and bool((outs[0].abs().sum(1) > 0).all())
 
 
-@pytest.mark.parametrize("pairs", [5119, 5120, 6143, 6144, 6145, 40961])
+@pytest.mark.parametrize("pairs", [10239, 10240, 12287, 12288, 12289, 40961])
 @pytest.mark.parametrize("experts", [1, 7, 32, 1024])
 def test_many_pairs_are_sorted_by_several_workgroups(pairs, experts):
     """With scratch the order is a sort by expert, ``place`` its inverse, and the tiles are those of one workgroup; one expert
