@@ -100,7 +100,8 @@ __global__ __launch_bounds__(256) void absorb_f32_kernel(LatentArgs a, int n, co
 // (columns), so that a lane's weights are operands of the value product as they are, and the value product is
 // latent dimensions by heads: a head's numbers stay in its lanes. A key's latent is read twice, from L2 the second time.
 // Bound by those reads: 963 rows of up to 500 keys, 16 heads, krp 256: the plain kernel, a workgroup per row and head
-// with one key per thread, took 1216 us, this 96 (four times the time of its products).
+// with one key per thread, took 1216 us, this 81 (three times the time of its products; 102 with the first rows first, whose
+// last ones ran alone; with two neighbouring rows to a workgroup and one read for both 103).
 template <int KR>  // krp / 64; rp == 64
 __global__ __launch_bounds__(256, KR <= 4 ? 2 : 1) void attend_f32_kernel(LatentArgs a, const float* __restrict__ qt, int ns,
                                                          float* __restrict__ po, float* __restrict__ pm) {
@@ -108,7 +109,8 @@ __global__ __launch_bounds__(256, KR <= 4 ? 2 : 1) void attend_f32_kernel(Latent
   __shared__ __attribute__((aligned(16))) float s_q[16 * LQ], s_o[2][16 * LO], s_ml[2][4][16];
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int e = blockIdx.x, h0 = blockIdx.y * 16, s = blockIdx.z, row = a.index ? a.index[e] : e;
+  const int e = gridDim.x - 1 - blockIdx.x;  // a prompt's last rows see most keys: they begin
+  const int h0 = blockIdx.y * 16, s = blockIdx.z, row = a.index ? a.index[e] : e;
   const int len = lat_keys(a, row), first = lat_first(a, len), slot = a.slot[row];
   const int fb = first / LAT_PAGE, nb = (len + LAT_PAGE - 1) / LAT_PAGE - fb;
   const int k0 = max(first, (fb + nb * s / ns) * LAT_PAGE), k1 = min(len, (fb + nb * (s + 1) / ns) * LAT_PAGE);
