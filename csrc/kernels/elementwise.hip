@@ -334,6 +334,58 @@ extern "C" int lsa_layernorm(void* x, int ldx, const void* pe, const int* pos, c
   return LSA_OK;
 }
 
+// Small tables from the host in the kernel's arguments. A copy from pinned memory is a launch of 4 us too, and 6 us more pass
+// before the next kernel begins (it has read memory that the host writes); a prompt sends 6 to 12 of them.
+constexpr int UPLOAD_INTS = 896;
+struct UploadInts {
+  int v[UPLOAD_INTS];
+};
+// the argument at ``offset`` where the launch put it (indexed by thread a copy of it would be made in scratch memory)
+LSA_DEVICE const __attribute__((address_space(4))) int* kernel_argument(int offset) {
+  return (const __attribute__((address_space(4))) int*)((const __attribute__((address_space(4))) char*)
+                                                            __builtin_amdgcn_kernarg_segment_ptr() + offset);
+}
+__global__ __launch_bounds__(UPLOAD_INTS) void upload_kernel(int* __restrict__ dst, int n, int unused, UploadInts) {
+  const auto* v = kernel_argument(16);
+  if ((int)threadIdx.x < n) dst[threadIdx.x] = v[threadIdx.x];
+}
+// Rows in runs of one slot's consecutive positions: run i has the first row, slot and first position v[i], v[N + i], v[2 N + i]
+// (N = UPLOAD_INTS / 3).
+__global__ __launch_bounds__(256) void run_rows_kernel(int* __restrict__ slot, int* __restrict__ pos, int n, int rows, UploadInts) {
+  constexpr int N = UPLOAD_INTS / 3;
+  const auto* v = kernel_argument(24);
+  const int row = blockIdx.x * 256 + threadIdx.x;
+  if (row >= rows) return;
+  int i = 0;  // the last run that begins at this row or before
+  for (int step = 256; step > 0; step >>= 1)
+    if (i + step < n && v[i + step] <= row) i += step;
+  slot[row] = v[N + i];
+  pos[row] = v[2 * N + i] + row - v[i];
+}
+
+extern "C" int lsa_upload(const int* host, int n, int* dst, hipStream_t stream) {
+  if (!host || !dst || n < 1) return LSA_BAD_SHAPE;
+  for (int at = 0; at < n; at += UPLOAD_INTS) {
+    UploadInts b;
+    const int m = n - at < UPLOAD_INTS ? n - at : UPLOAD_INTS;
+    __builtin_memcpy(b.v, host + at, (size_t)m * 4);
+    upload_kernel<<<1, (m + 63) / 64 * 64, 0, stream>>>(dst + at, m, 0, b);
+  }
+  LSA_CHECK_LAUNCH();
+  return LSA_OK;
+}
+
+// runs (host): [3][n] first rows (rising from 0), slots, first positions
+extern "C" int lsa_run_rows(const int* runs, int n, int rows, int* slot, int* pos, hipStream_t stream) {
+  constexpr int N = UPLOAD_INTS / 3;
+  if (!runs || !slot || !pos || n < 1 || n > N || rows < n || runs[0] != 0) return LSA_BAD_SHAPE;
+  UploadInts b;
+  for (int k = 0; k < 3; ++k) __builtin_memcpy(b.v + k * N, runs + k * n, (size_t)n * 4);
+  run_rows_kernel<<<(rows + 255) / 256, 256, 0, stream>>>(slot, pos, n, rows, b);
+  LSA_CHECK_LAUNCH();
+  return LSA_OK;
+}
+
 extern "C" int lsa_argmax_finalize(unsigned long long* keys, int rows, int* tokens, int* pos,
                                    int pos_inc, int* history, int hist_stride, int hist_len,
                                    int* step_ctr, hipStream_t stream) {

@@ -604,7 +604,10 @@ class StageEngine:
         if self.gpu:  # lists are read once
             from ..ops import hip
             slot, pos = (x if torch.is_tensor(x) else hip.host_ints(x) for x in (slot, pos))
-        slot_t, pos_t = self._i32(slot), self._i32(pos)
+        if self.gpu and not torch.is_tensor(slot) and not torch.is_tensor(pos):
+            slot_t, pos_t = hip.row_tables(slot, pos, self.device)
+        else:
+            slot_t, pos_t = self._i32(slot), self._i32(pos)
         kvl_t = None if kv_len is None else self._i32(kv_len)
         if self.gpu:
             tiles = None
@@ -1157,8 +1160,9 @@ class DecodeGraph:
         self._host_pos[i] = p
 
     def set_positions(self) -> None:
-        self.pos.copy_(torch.tensor([self.eng.seq_len[s] for s in self.slots], dtype=torch.int32))
         self._host_pos = [self.eng.seq_len[s] for s in self.slots]
+        from ..ops import hip
+        hip.send(self._host_pos, self.pos)  # (a plain copy would wait for the device, and leave it without work meanwhile)
 
     def sync_positions(self) -> None:
         p = self.pos.tolist()

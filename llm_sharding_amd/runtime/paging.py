@@ -47,7 +47,7 @@ class PagePool:
         new = [self.free.pop() for _ in range(need - have)]
         self.held[slot] += new
         from ..ops import hip
-        self.table[slot, have:need] = hip.to_device(new, self.table.device)
+        hip.send(new, self.table[slot, have:need])
 
     def release(self, slot: int) -> None:
         """Every page of ``slot`` back to the pool."""

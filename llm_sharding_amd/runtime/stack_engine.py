@@ -400,7 +400,8 @@ class StackEngine(StageEngine):
             self._ensure(s, p + n)
         if not self.gpu:
             return self._forward_stack_torch(h, sl, ps)
-        return self._forward_hip(h, self._i32(sl), self._i32(ps), None, rows, runs=runs)
+        from ..ops import hip
+        return self._forward_hip(h, *hip.row_tables(sl.numpy(), ps.numpy(), self.device), None, rows, runs=runs)
 
     def latent_nsplit(self, s, entries: int, longest: int) -> int:
         """Key splits of the absorbed attention: about one workgroup per CU (each fills a CU's

@@ -207,3 +207,37 @@ def test_stream_handle_with_and_without_the_raw_call(monkeypatch):
     assert hip._stream().value == 103
     monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
     assert hip._stream().value == 7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 64, 895, 896, 897, 1792, 1793, 5000])
+def test_small_tables_are_kernel_arguments(n):
+    """As lists, arrays and tensors, into tensors of their own and into part of another; numbers past 32 bits are refused."""
+    x = np.random.default_rng(n).integers(-2 ** 31, 2 ** 31, n)
+    for kind in (list, lambda v: v, torch.from_numpy, lambda v: torch.from_numpy(v).to(torch.int32)):
+        got = hip.to_device(kind(x), "cuda")
+        assert got.dtype == torch.int32 and got.is_cuda and got.tolist() == x.tolist()
+    table = torch.full((3, n + 7), -5, dtype=torch.int32, device="cuda")
+    hip.send(x.tolist(), table[1, 4:n + 4])
+    assert table[1, 4:n + 4].tolist() == x.tolist()
+    table[1, 4:n + 4] = -5
+    assert bool((table == -5).all())
+    with pytest.raises(RuntimeError):
+        hip.send([2 ** 31] + [0] * (n - 1), table[1, 4:n + 4])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("runs", [1, 2, 3, 64, 255, 256, 257, 297, 298, 299, 700])
+def test_row_tables_from_runs(runs):
+    """Rows in as many runs of a slot's consecutive positions as one launch takes, and more; neighbouring runs of one slot."""
+    g = np.random.default_rng(runs)
+    slot, pos = [], []
+    for i in range(runs):
+        n, p = int(g.integers(1, 9 if runs > 3 else 900)), int(g.integers(0, 5000))
+        slot += [i // 2] * n
+        pos += range(p, p + n)
+    s, p = hip.row_tables(np.array(slot), np.array(pos), "cuda")
+    assert s.dtype == p.dtype == torch.int32 and s.is_contiguous() and p.is_contiguous()
+    assert s.tolist() == slot and p.tolist() == pos
+    with pytest.raises(RuntimeError):
+        hip.row_tables(np.array([0, 0]), np.array([5, 2 ** 31]), "cuda")
