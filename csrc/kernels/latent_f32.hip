@@ -244,7 +244,8 @@ __global__ __launch_bounds__(256) void value_f32_kernel(LatentArgs a, int n, con
 #pragma unroll
       for (int j = 0; j < 4; ++j) y[u][j] = ldf4(wh + (size_t)(16 * u + j) * a.dvp + 64 * b);
   };
-  load_w(0);
+  const int step = gridDim.z;  // columns 64 b ..: all of them, or each 64 a workgroup's
+  load_w(blockIdx.z);
   __builtin_amdgcn_sched_barrier(0);  // requested here, not where it is used
   if (tid < 16) {
     const float* pe = pm + ((size_t)min(e0 + tid, n - 1) * a.heads + h) * ns * 2;
@@ -266,7 +267,7 @@ __global__ __launch_bounds__(256) void value_f32_kernel(LatentArgs a, int n, con
 #pragma unroll
     for (int u = 0; u < KR; ++u) x[u] += ldf4(pr + (size_t)s * KRP + 16 * u) * f;
   }
-  for (int b = 0; b < a.dvp / 64; ++b) {
+  for (int b = blockIdx.z; b < a.dvp / 64; b += step) {
     f32x4_t acc[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[t] = ZERO4;
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(256) void value_f32_kernel(LatentArgs a, int n, con
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc[t] = mfma(x[u][j], y[u][j][t], acc[t]);
-    if (b + 1 < a.dvp / 64) load_w(b + 1);
+    if (b + step < a.dvp / 64) load_w(b + step);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       *reinterpret_cast<f32x4_t*>(&s_acc[w][4 * g + r][4 * c]) = f32x4_t{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
@@ -328,6 +329,7 @@ bool latent_value_f32(const LatentArgs& a, int n, const float* po, const float* 
   if (!latent_size(a) || !aligned(po, 0) || !aligned(wv, 0)) return false;
   auto* f = a.krp == 64 ? value_f32_kernel<1> : a.krp == 128 ? value_f32_kernel<2> : a.krp == 256 ? value_f32_kernel<4>
                                                                                                : value_f32_kernel<8>;
-  f<<<dim3((n + 15) / 16, a.heads), 256, 0, s>>>(a, n, po, pm, ns, wv, gate, ldg, out, ldo);
+  const int wg = (n + 15) / 16 * a.heads, blocks = a.dvp / 64;
+  f<<<dim3((n + 15) / 16, a.heads, wg * blocks <= 256 ? blocks : 1), 256, 0, s>>>(a, n, po, pm, ns, wv, gate, ldg, out, ldo);
   return true;
 }
