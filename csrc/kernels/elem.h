@@ -15,3 +15,13 @@ LSA_DEVICE void st4(bf16_raw* p, f32x4_t v) {
 }
 
 LSA_DEVICE float sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
+
+// the sum of a and that of b over both halves of the wave (of each 32 lanes): a's in the lower one, b's in the upper one
+LSA_DEVICE float halves(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+LSA_DEVICE float quarters(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}

@@ -280,16 +280,6 @@ __global__ __launch_bounds__(DV * 4) void ml_steps_kernel(MlArgs a) {
   }
 }
 
-// the sum of a and that of b over both halves of the wave (of each 32 lanes): a's in the lower one, b's in the upper one
-LSA_DEVICE float halves(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-LSA_DEVICE float quarters(float a, float b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
 // As above for runs that leave CUs idle: 32 value channels a workgroup, a wave 8 of them, so that a head has DV / 32 workgroups
 // of one wave per SIMD, and a lane 16 elements of the state instead of 32. The four sums over 32 lanes are halved with their
 // lanes. Read-outs go out as they are; n and m, which every workgroup reads and only the first writes, go to nm

@@ -80,13 +80,13 @@ def chunked(a: RetArgs, s, items, longest: int, several: bool, ws, o32) -> None:
                                  o32.stride(0), _stream()), "lsa_ret_chunked")
 
 
-def steps(a: RetArgs, dtype, n: int) -> None:
-    """n runs (or rows), step by step."""
-    _check(lib().lsa_ret_steps(is_f32(dtype), ctypes.byref(a), n, _stream()), "lsa_ret_steps")
+def steps(a: RetArgs, dtype, n: int, longest: int = 0) -> None:
+    """n runs (or rows), step by step; ``longest``: none has more rows (0: not known)."""
+    _check(lib().lsa_ret_steps(is_f32(dtype), ctypes.byref(a), n, longest, _stream()), "lsa_ret_steps")
 
 
 def declare(L: ctypes.CDLL) -> None:
     """Signatures of these entry points (called by hip.load_library)."""
     vp, i = ctypes.c_void_p, ctypes.c_int
     ra = ctypes.POINTER(RetArgs)
-    hip.set_signatures(L, {"lsa_ret_steps": [i, ra, i, vp], "lsa_ret_chunked": [ra, vp, i, i, i, vp, vp, i, vp]})
+    hip.set_signatures(L, {"lsa_ret_steps": [i, ra, i, i, vp], "lsa_ret_chunked": [ra, vp, i, i, i, vp, vp, i, vp]})

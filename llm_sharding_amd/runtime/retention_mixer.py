@@ -83,7 +83,8 @@ class Retention:
         short, long = plan.memo(("retention", s, self.chunks),
                                 lambda: split_runs(plan, rows, state[0].shape[0], s, self.chunk_min if self.chunks else 0))
         if short is not None:
-            X.steps(args(runs=short), self.dtype, short.shape[0])
+            least = self.chunk_min if self.chunks else 0
+            X.steps(args(runs=short), self.dtype, short.shape[0], max(r[1] for r in plan.runs if not least or r[1] < least))
         if long is not None:
             items, entries, longest, several = long
             (dk, dv), f32 = s.state_dims, torch.float32

@@ -464,8 +464,9 @@ class RetCase:
         if how == "rows":
             slot, pos = (torch.tensor([r[j] for r in runs], dtype=torch.int32, device=DEV) for j in (2, 3))
             X.steps(args(slot=slot, pos=pos), self.dtype, rows)
-        elif how == "steps":
-            X.steps(args(runs=torch.tensor(runs, dtype=torch.int32, device=DEV)), self.dtype, len(runs))
+        elif how in ("steps", "known"):  # (how long the longest run is decides between kernels)
+            X.steps(args(runs=torch.tensor(runs, dtype=torch.int32, device=DEV)), self.dtype, len(runs),
+                    max(n for _, n, *_ in runs) if how == "known" else 0)
         else:
             items, entries, longest, several = X.segments(s, runs, wide, least=64)
             ws = torch.full((entries, H, dk, dv), float("nan"), device=DEV)
@@ -503,6 +504,26 @@ def test_retention(name, dtype, wide):
     rest = case.state.clone()
     rest[:, :, :s.dim, :s.vdim] = 0
     assert not rest.any()
+
+
+@pytest.mark.parametrize("name,count", [(n, 2) for n in RET] + [("square", 32), ("square", 33), ("part", 130)])
+def test_retention_with_several_workgroups_a_head(name, count):
+    """Runs around batches of 16 rows, from a start and from a state; as many as the form takes, and one more. The state is that
+    of the other form."""
+    lens = [12 + 33 + 1 + i % 18 for i in range(count)]
+    case, other = RetCase(RET[name], lens, F32), RetCase(RET[name], lens, F32)
+    case.step([(i, 12 - i % 3) for i in reversed(range(count))], "known")
+    case.step([(i, 33 if i % 2 else 16) for i in range(count)], "known")
+    case.step([(i, 1) for i in range(count)], "known")
+    case.step([(i, lens[i] - case.at[i]) for i in range(count)], "known")
+    other.step([(i, lens[i]) for i in range(count)], "steps")
+    for i in range(count):
+        close(case.got[i], other.got[i], 2e-5, f"{name} {i}")
+    for i in {0, 1, count // 2, count - 1}:
+        out, S = case.want(i)
+        close(case.got[i], out, 2e-5, f"{name}: outputs of {i}")
+        close(case.state[i, :, :RET[name].dim, :RET[name].vdim], S, 3e-5, f"{name}: state of {i}")
+    close(case.state, other.state, 1e-5, name)
 
 
 def test_a_portion_from_the_start_ignores_what_the_slot_held():
