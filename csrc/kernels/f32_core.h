@@ -12,7 +12,7 @@
 //   F32Split   many rows, on the bf16 matrix instructions, which are 16 times as fast: each operand is taken apart into three
 //              bf16 (8 + 8 + 8 bits of its 24), and of their nine products the six of more than 2^-24 of the whole are made.
 //              Bound by the matrix unit: what its clock allows with six full-width products (random operands: 1750 of 2500
-//              TFLOP/s, 290 of fp32 product), and for a third of that by the splitting, 5.5 vector instructions a value, two of
+//              TFLOP/s, 290 of fp32 product), and for a third of that by the splitting, 6.5 vector instructions a value, two of
 //              which fit beside a matrix instruction. 2567 rows, N = 16384, K = 2048 1371 -> 800 us (215 TFLOP/s; the fp32
 //              instructions reach 157 at best and did 126), 963 rows, N = 16384 520 -> 301, N = 2048 71 -> 51, K = 8192
 //              265 -> 165, 64 rows, N = 2048 17.3 -> 16.5.
@@ -97,8 +97,12 @@ struct F32Stream {
 // MT x 16 rows by NW x 32 columns of C; KG groups of NW waves, each with its part of K, every wave 32 columns of all rows. A
 // wave splits its columns for itself, from memory to operand registers, and an NW-th of the rows for all, through LDS: were the
 // columns shared too, twice as much would go through LDS. The pieces are rounded to nearest, so that they hold 24 bits and the
-// dropped products have either sign; what is below 2^-133 is lost, so that values under 2^-109 have
-// fewer bits (measured: full accuracy at 2^-109, 1e-6 at 2^-115). Tile sizes (linear_f32.hip plan) by how many there are of them.
+// dropped products have either sign. Operands are split 2^16 times as large: the last bit of an fp32 number, 2^-149 for
+// the smallest, is then one that a bf16 holds (2^-133), and every finite value is the sum of its pieces. The sums are 2^32 times as
+// large in turn: values from 2^112 and results from 2^96 on give infinities in them and are made again from the values
+// (whole). Unscaled, values under 2^-109 had fewer bits (1e-6 off at 2^-115, nothing left at 2^-134); the two products with 2^16 of
+// a pair of values take 2 % of a product's time (2567 rows, N = 16384, K = 2048 797 -> 812 us, 963 rows 300 -> 307). Tile sizes
+// (linear_f32.hip plan) by how many there are of them.
 template <int MT, int NW, int KG>
 struct F32Split {
   static_assert(MT % NW == 0 && MT % KG == 0);
@@ -107,6 +111,7 @@ struct F32Split {
   static constexpr int BUF = MT * 3 * 64;  // 32 k of the rows: fragments of three pieces, 16 bytes a lane
   static constexpr int LDS = KG * 2 * BUF;
   static constexpr int MO = MT / KG;       // fragments that a wave holds in the end: from MO * group on
+  static constexpr float UP = 0x1p16f, DOWN = 0x1p-32f;
   f32x4_t acc[MT][NT];
 
   LSA_DEVICE static int group() { return KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / NW; }
@@ -177,7 +182,7 @@ struct F32Split {
     auto third = [&](int s, int k0, u32x4_t* nxt, u32x4_t (&bn)[NT][3]) {
       const int i = s / 12, j = s / 3 % 4, x = s % 3;
       u32x4_t(&to)[3] = i < SF ? sa : bn[i < SF ? 0 : i - SF];
-      if (x == 0) u = g[i][j >> 1][2 * j & 3], v = g[i][j >> 1][(2 * j & 3) + 1];
+      if (x == 0) u = g[i][j >> 1][2 * j & 3] * UP, v = g[i][j >> 1][(2 * j & 3) + 1] * UP;
       const unsigned h = pack2(u, v);
       to[x][j] = h;
       if (x < 2) u -= __uint_as_float(h << 16), v -= __uint_as_float(h & 0xffff0000u);
@@ -227,7 +232,7 @@ struct F32Split {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int n = 0; n < NT; ++n) acc[m][n] += low[m][n];
+      for (int n = 0; n < NT; ++n) acc[m][n] = (acc[m][n] + low[m][n]) * DOWN;
   }
 
   // Sums that are no finite numbers again from the values as they are: the pieces of an infinity, and of a value that rounds

@@ -96,7 +96,7 @@ def test_linear_tiles(rows, n, k):
 @pytest.mark.parametrize("rows,n,k", [(40, 4112, 64), (200, 2064, 2048), (600, 8464, 96)])
 def test_linear_values_that_are_no_numbers(rows, n, k):
     """Infinities, NaN and values that round to an infinity in bf16 give what fp32 products of them give, and leave all other
-    results as they are without them; zeros meet infinities. Of a value below 2^-109 what is smaller than 2^-133 is lost."""
+    results as they are without them; zeros meet infinities, and values at the lower end keep all their bits."""
     x, w = _rand(rows, k, seed=1), _rand(n, k, seed=2, scale=k ** -0.5)
     w[::7, 5] = 0
     w[3::16] = w[3::16].bfloat16().float()  # second and third pieces that are zero
@@ -115,7 +115,26 @@ def test_linear_values_that_are_no_numbers(rows, n, k):
     over = want[30].abs() > 3.402823e38
     assert torch.equal(got[30].isinf(), over) or (got[30].isinf() ^ over).sum() <= 1
     assert ((got[30] - want[30]).abs()[~over & got[30].isfinite()] < 1e-5 * 3.4e38).all()
-    assert (got[33:35] - want[33:35]).abs().max() < sum_tol(k) * want[33].abs().max() + k * 2.0 ** -133 * float(w.abs().max())
+    rows_close(got[33:34], want[33:34], sum_tol(k) + 2.0 ** -20, "small values")  # (results down to 2^-130, of 19 bits)
+    assert (got[34] - want[34]).abs().max() < sum_tol(k) * want[34].abs().max() + 2.0 ** -145  # up to 20 sums' last bits of 2^-149
+
+
+@pytest.mark.parametrize("rows,n,k", [(33, 8464, 64), (100, 4112, 96), (200, 2064, 2048), (257, 4368, 544), (960, 8208, 128)])
+def test_linear_tiles_at_the_ends_of_the_range(rows, n, k):
+    """Rows of values from fp32's last bit to 2^120, as exact as any; and values of both kinds in one row, where the small ones'
+    weights are as much larger."""
+    x, w = _rand(rows, k, seed=1), _rand(n, k, seed=2, scale=k ** -0.5)
+    e = torch.arange(rows)[:, None].remainder(270).double() - 150
+    lo = (x.double() * torch.exp2(e)).float()
+    a, b = (e < -50)[:, 0], (e >= -50)[:, 0]
+    for r, f in ((a, 2.0 ** 40), (b, 2.0 ** -40)):
+        if r.any():
+            some = lo[r].any(1)
+            rows_close(product(lo[r], w * f)[some], (lo[r].double() @ (w * f).double().T)[some], sum_tol(k), "rows")
+    x[:, ::2] *= 2.0 ** -125
+    w[:, ::2] *= 2.0 ** 95
+    w[:, 1::2] *= 2.0 ** -30
+    rows_close(product(x, w), x.double() @ w.double().T, sum_tol(k), "in one row")
 
 
 @pytest.mark.parametrize("kind", ["store", "silu", "gelu"])
