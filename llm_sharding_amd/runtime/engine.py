@@ -1066,6 +1066,7 @@ class DecodeGraph:
         self.keys = torch.zeros(rows, dtype=torch.int64, device=dev)
         self.h_in = torch.zeros((rows, eng.cfg.stream_width), dtype=eng.hidden_dtype, device=dev)
         self._host_pos = [eng.seq_len[s] for s in self.slots]  # paged caches: where the next tokens go
+        self._sent = None  # positions on their way: the stream that brings them, and the event behind them
         self.history = torch.zeros((max(1, history_len), rows), dtype=torch.int32, device=dev) if history_len else None
         self.step_ctr = torch.zeros(1, dtype=torch.int32, device=dev)
         self.graph = None
@@ -1152,6 +1153,7 @@ class DecodeGraph:
             for i, s in enumerate(self.slots):
                 self.eng.grow(s, self._host_pos[i] + 1)
                 self._host_pos[i] += 1
+        self._behind_positions()
         self.graph.replay()
 
     def set_pos(self, i: int, p: int) -> None:
@@ -1160,11 +1162,28 @@ class DecodeGraph:
         self._host_pos[i] = p
 
     def set_positions(self) -> None:
+        """The engine's positions for the next tokens, sent in the current stream's order and without waiting for the device (a plain
+        copy would, and leave it without work meanwhile). Replays and :meth:`sync_positions` come behind them on every stream;
+        other work on ``pos`` only on this one."""
         self._host_pos = [self.eng.seq_len[s] for s in self.slots]
-        from ..ops import hip
-        hip.send(self._host_pos, self.pos)  # (a plain copy would wait for the device, and leave it without work meanwhile)
+        self._hip.send(self._host_pos, self.pos)
+        stream = torch.cuda.current_stream(self.eng.device)
+        self._sent = stream, stream.record_event()
+
+    def _behind_positions(self) -> None:
+        """The current stream waits for positions that another one brings."""
+        if self._sent is None:
+            return
+        stream, event = self._sent
+        now = torch.cuda.current_stream(self.eng.device)
+        if now != stream:
+            if event.query():
+                self._sent = None
+            else:
+                now.wait_event(event)
 
     def sync_positions(self) -> None:
+        self._behind_positions()
         p = self.pos.tolist()
         for s, v in zip(self.slots, p):
             self.eng.seq_len[s] = int(v)

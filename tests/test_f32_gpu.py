@@ -280,6 +280,36 @@ def test_captured_heads_share_no_workspace(monkeypatch):
 
 
 @torch.inference_mode()
+def test_positions_arrive_before_replays_of_other_streams():
+    """Positions that a busy stream is yet to bring: a replay and a read of another stream come behind them."""
+    from llm_sharding_amd.runtime.engine import DecodeGraph
+    eng = _engine_with_a_parted_head(4)
+    g = DecodeGraph(eng, 4, "full").capture()
+    ids, busy, other = torch.tensor([5, 9, 11, 300], dtype=torch.int32, device=DEV), torch.cuda.Stream(), torch.cuda.Stream()
+    outs = []
+    for late in (False, True):
+        eng.reset()
+        g.set_positions()
+        for _ in range(2):
+            g.tokens.copy_(ids)
+            g.replay()
+        eng.advance([0, 1, 2, 3], [1] * 4)  # back by a token: the next replay is the second one again
+        g.tokens.copy_(ids)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(busy):
+            if late:
+                torch.cuda._sleep(20_000_000)
+            g.set_positions()
+        with torch.cuda.stream(other):
+            g.replay()
+            g.sync_positions()
+        assert [eng.seq_len[i] for i in range(4)] == [2] * 4
+        torch.cuda.synchronize()
+        outs.append((g.out_hidden.clone(), g.tokens.clone()))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@torch.inference_mode()
 def test_captured_product_without_a_workspace():
     """In a graph, a product that is given no workspace takes none: its replays may run beside others of any stream."""
     k, n, rows = 2048, 2048, 40
