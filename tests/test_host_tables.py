@@ -78,6 +78,20 @@ def test_remembered_candidates_are_not_shared():
     assert packing.gemv_candidates(768, 4096, 8)
 
 
+def test_sent_numbers_fill_their_places():
+    """As many int32 as there are places, on the way that takes no launch as on the others."""
+    out = torch.full((2, 3), -5, dtype=torch.int32)
+    hip.send([4, 5, 6], out[0])
+    hip.send(np.array([7]), out[1, 2:])
+    hip.send([], out[1, :0])
+    assert out.tolist() == [[4, 5, 6], [-5, -5, 7]]
+    hip.send(list(range(6)), out.t())  # places in the order of the shape
+    assert out.t().flatten().tolist() == list(range(6))
+    for x, to in (([1], out[0]), ([1, 2], out[0]), ([1, 2, 3], torch.zeros(3, dtype=torch.int64)), ([1.0], torch.zeros(1))):
+        with pytest.raises(ValueError):
+            hip.send(x, to)
+
+
 @pytest.mark.parametrize("slot,pos", [([0, 0, 0], [0, 1, 2]), ([[0], [0], [0]], torch.tensor([[0], [1], [2]])),
                                       (torch.zeros(1, 3), np.array([[0, 1, 2]])), (range(0, 1), 0), (torch.tensor(0), (0,))])
 def test_rows_of_a_stack_in_any_shape(slot, pos):
