@@ -116,22 +116,29 @@ Plan plan(int M, int N, int K, long long slab_floats, int counters) {
   return best;
 }
 
+// The stream form: up to 16 rows; up to 32 of a product that is not large (20 rows, K = 2048, N = 4352 16 against 19 us of tiles,
+// N = 8448 28 and 25, N = 16384 35 and 31; 4096 x 4096 19 and 25); where one 16 x 16 tile per workgroup does not fill the CUs
+// (N = 128 48 rows 7 against 13 us), or a pair of columns of them does not and K is not long (N = 2048 64 rows: K = 2048 12
+// against 16, K = 4096 20 and 20, K = 8192 36 and 26; K = 1024, N = 1024, 128 rows 8 and 14).
+// Tiles of 16 rows that a workgroup of that form has; 0: not that form.
+int stream_tiles(int M, int N, int K, bool gated) {
+  const int t = N / 16, mt16 = (M + 15) / 16;
+  const bool alone = (long long)(gated ? t / 2 : t) * mt16 <= 256, pairs = (long long)(t + 1) / 2 * mt16 <= 256 && K <= 4096;
+  if (M <= 16 || alone || pairs) return 1;
+  return K % 32 || (M <= 32 && (long long)N * K <= 1 << 24) ? 2 : 0;
+}
+
 template <int EPI>
 void launch(const float* a, int lda, const float* w, int M, int N, int K, const EpiArgs& ep, float* slab, long long slab_floats,
             unsigned* counters, int n_counters, hipStream_t s) {
 #define LSA_STREAM(MT, NT) \
   stream_f32_kernel<EPI, MT, NT, 8><<<dim3((t + NT - 1) / NT, (M + MT * 16 - 1) / (MT * 16)), 512, 0, s>>>(a, lda, w, M, N, K, ep)
-  // The stream form: up to 16 rows; up to 32 of a product that is not large (20 rows, K = 2048, N = 4352 16 against 19 us of tiles,
-  // N = 8448 28 and 25, N = 16384 35 and 31; 4096 x 4096 19 and 25); where one 16 x 16 tile per workgroup does not fill the CUs
-  // (N = 128 48 rows 7 against 13 us), or a pair of columns of them does not and K is not long (N = 2048 64 rows: K = 2048 12
-  // against 16, K = 4096 20 and 20, K = 8192 36 and 26; K = 1024, N = 1024, 128 rows 8 and 14).
   // A CU takes 3 us for a tile's products, so that the tiles are as many per workgroup as the fullest CU has anyway:
   // N = 4352 (272 tiles) two 12.2, one 14.8; N = 8448 (528) two 26.5, one 21.4; from N = 8192 on one streams better up to 8 rows
   // (N = 16384, 8 rows 24.6 against 28.4, 16 rows 28.5 and 28.7).
-  const int t = N / 16, mt16 = (M + 15) / 16, g = epi_gated(EPI) ? 2 : 1;
-  const bool alone = (long long)t / g * mt16 <= 256, pairs = (long long)(t + 1) / 2 * mt16 <= 256 && K <= 4096;
-  if (K % 32 || M <= 16 || (M <= 32 && (long long)N * K <= 1 << 24) || alone || pairs) {
-    const int m = M <= 16 || alone || pairs ? 1 : 2, rows = (mt16 + m - 1) / m;
+  const int t = N / 16;
+  if (const int m = stream_tiles(M, N, K, epi_gated(EPI))) {
+    const int rows = (M + 16 * m - 1) / (16 * m);
     const int one = (t * rows + 255) / 256, two = ((t + 1) / 2 * rows + 255) / 256 * 2;
     if constexpr (epi_gated(EPI)) {
       if (m == 1) LSA_STREAM(1, 2);
@@ -176,5 +183,18 @@ extern "C" int lsa_linear_f32(const float* a, int lda, const float* w, int M, in
     return LSA_UNSUPPORTED;
   }
   LSA_CHECK_LAUNCH();
+  return LSA_OK;
+}
+
+// What a product becomes: form[0..3] = rows and columns of a tile, tiles in one piece, parts of K of each tile past those; rows 16 or
+// 32 with no columns: the stream form
+extern "C" int lsa_linear_f32_form(int M, int N, int K, int gated, long long slab_floats, int n_counters, int* form) {
+  if (M < 1 || N < 16 || N % 16 || K < 16 || K % 16 || (gated && N % 32) || !form) return LSA_BAD_SHAPE;
+  const int m = stream_tiles(M, N, K, gated);
+  const Plan p = m ? Plan{16 * m, 0, 0, 1} : plan(M, N, K, slab_floats, n_counters);
+  form[0] = p.rows;
+  form[1] = p.cols;
+  form[2] = p.whole;
+  form[3] = p.S;
   return LSA_OK;
 }

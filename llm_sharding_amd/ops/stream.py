@@ -108,6 +108,14 @@ class Linear:
             hip.gemm_sk(x, self.w, rows, self.n, self.k, epi, ep, ws=sk_ws)
 
 
+def linear_f32_form(rows: int, n: int, k: int, gated: bool = False, slab: int = 256 * 128 * 256, counters: int = 256) -> tuple:
+    """What an fp32 product becomes: (rows and columns of a tile, tiles in one piece, parts of K of each tile past those); 16 or 32
+    rows and no columns: the form that streams the weights."""
+    form = (ctypes.c_int * 4)()
+    _check(lib().lsa_linear_f32_form(rows, n, k, int(gated), slab, counters, form), "lsa_linear_f32_form")
+    return tuple(form)
+
+
 # ------------------------------------------------------------------------------ fp32 stream
 def stream_embed(ids, table, scale: float, x, xc, rows: int, copies: int = 1) -> None:
     """x = table[ids] * scale, ``copies`` of it side by side; ``xc`` (or None): one in the projections' type."""
@@ -283,5 +291,6 @@ def declare(L: ctypes.CDLL) -> None:
         "lsa_stream_join": [i, ctypes.POINTER(JoinArgs), i, i, vp, i, vp, i, vp],
         "lsa_stream_renorm": [i, ctypes.POINTER(RenormArgs), i, i, vp, i, vp, i, vp],
         "lsa_logits_argmax": [vp, i, i, i, i, vp, vp],
+        "lsa_linear_f32_form": [i, i, i, i, ctypes.c_longlong, i, vp],
         "lsa_linear_f32": [vp, i, vp, i, i, i, i, ctypes.POINTER(hip.EpiArgs), vp, ctypes.c_longlong, vp, i, vp],
     })

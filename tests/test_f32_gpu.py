@@ -6,7 +6,7 @@ import torch
 from llm_sharding_amd.models.stack import GluSpec
 from llm_sharding_amd.ops import hip
 from llm_sharding_amd.ops.packing import pack_f32
-from llm_sharding_amd.ops.stream import Linear
+from llm_sharding_amd.ops.stream import Linear, linear_f32_form
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -48,22 +48,47 @@ def test_linear_store(rows, n, k):
                                       (700, 2048, 2048), (1030, 1024, 4096)])
 @pytest.mark.parametrize("slab", [0, 70000, 768 * 4096])
 def test_linear_in_parts(rows, n, k, slab):
-    """K in parts: of all tiles and of the last ones, uneven, two at least, fewer where the scratch is small, none without;
-    the same bits each time, the counters left at zero, and nothing written past the scratch."""
+    """Products of short and long K around the border between streamed weights and tiles, with scratch and without: the same bits
+    each time, the counters left at zero, and nothing written past the scratch."""
+    in_parts(rows, n, k, slab)
+
+
+SLAB = 256 * 128 * 256  # an engine's
+
+
+@pytest.mark.parametrize("rows,n,k,slab,form", [
+    (70, 2080, 2144, SLAB, (64, 64, 0, 3)), (70, 2080, 2144, 600000, (64, 64, 0, 2)), (283, 4096, 8192, 1000000, (64, 64, 256, 3)),
+    (283, 4096, 8192, 768 * 4096, (64, 64, 256, 4)), (283, 4096, 8192, 0, (64, 128, 160, 1)), (283, 4096, 8192, SLAB, (64, 128, 0, 3)),
+    (70, 4128, 2080, SLAB, (64, 128, 0, 3)), (505, 4128, 2144, SLAB, (64, 128, 256, 8)), (505, 2080, 2144, SLAB, (128, 128, 0, 3)),
+    (505, 8224, 2080, SLAB, (128, 128, 256, 8)), (505, 4416, 4064, SLAB, (128, 256, 0, 3)), (900, 8224, 2080, SLAB, (128, 256, 256, 6))])
+@pytest.mark.parametrize("gated", [False, True])
+def test_linear_in_parts_of_every_form(rows, n, k, slab, form, gated):
+    """K in parts of each size of tiles: of all tiles and of those past the ones that fill the CUs, uneven, fewer where the
+    scratch is small, none without it; rows and columns that fill no tile."""
+    n -= 16 if n % 64 and not gated else 0
+    assert linear_f32_form(rows, n, k, gated, slab) == form
+    in_parts(rows, n, k, slab, gated)
+
+
+def in_parts(rows, n, k, slab, gated=False):
     x, w, b = _rand(rows, k, seed=1).to(DEV), _rand(n, k, seed=2, scale=k ** -0.5).to(DEV), _rand(n, seed=3).to(DEV)
     wd = pack_f32(w)
     part, cnt = torch.full((slab + 64,), 7.0, device=DEV), torch.zeros(256, dtype=torch.int32, device=DEV)
     outs = []
     for _ in range(3):
         out = torch.full((rows, n + 16 - n % 8), 7.0, device=DEV)
-        ep = hip.make_epi(out=out, ldo=out.stride(0), bias=b)
-        st = hip.lib().lsa_linear_f32(x.data_ptr(), k, wd.data_ptr(), rows, n, k, hip.EPI_STORE, ep,
+        ep = hip.make_epi(**{"out32" if gated else "out": out}, ldo=out.stride(0), bias=b)
+        st = hip.lib().lsa_linear_f32(x.data_ptr(), k, wd.data_ptr(), rows, n, k, hip.EPI_GEGLU if gated else hip.EPI_STORE, ep,
                                       part.data_ptr() if slab else None, slab, cnt.data_ptr(), 256,
                                       torch.cuda.current_stream().cuda_stream)
         assert st == 0
         outs.append(out)
-    rows_close(outs[0][:, :n], x.double().cpu() @ w.double().cpu().T + b.double().cpu(), sum_tol(k), "parts")
-    assert all(torch.equal(outs[0], o) for o in outs[1:]) and bool((outs[0][:, n:] == 7).all())
+    want = (x.double() @ w.double().T + b.double()).cpu()
+    if gated:  # 16 columns of gates, 16 of what they open
+        want = want.view(rows, -1, 2, 16)
+        want = (torch.nn.functional.gelu(want[:, :, 0], approximate="tanh") * want[:, :, 1]).flatten(1)
+    rows_close(outs[0][:, :want.shape[1]], want, 2 * sum_tol(k) + 1e-6 if gated else sum_tol(k), "parts")
+    assert all(torch.equal(outs[0], o) for o in outs[1:]) and bool((outs[0][:, want.shape[1]:] == 7).all())
     assert not cnt.any() and bool((part[slab:] == 7).all())
 
 
@@ -138,10 +163,13 @@ def test_linear_tiles_at_the_ends_of_the_range(rows, n, k):
 
 
 @pytest.mark.parametrize("kind", ["store", "silu", "gelu"])
-@pytest.mark.parametrize("rows", [20, 64, 700])
-def test_parts_beside_each_other_on_a_cu(kind, rows):
-    """More parts than CUs: one writes its sums while another of the same CU keeps the memory pipe busy."""
-    n, k = 8448, 2048
+@pytest.mark.parametrize("rows,n,k", [(20, 8448, 2048), (64, 8448, 2048), (700, 8448, 2048), (283, 4096, 8192), (2500, 4352, 2048)])
+def test_parts_beside_each_other_on_a_cu(kind, rows, n, k):
+    """More parts than CUs, or whole tiles for all CUs and parts (the two largest products; the others have one for a CU at most): one
+    writes its sums while another of the same CU keeps the memory pipe busy."""
+    bm, bn, whole, parts = linear_f32_form(rows, n, k, kind != "store")
+    if n < 8448:
+        assert parts > 1 and whole + (-(-rows // bm) * -(-n // bn) - whole) * parts > 256
     x, w = _rand(rows, k, seed=1).to(DEV), _rand(n, k, seed=2, scale=k ** -0.5).to(DEV)
     if kind == "store":
         lin, glu, want = Linear(w), None, x.double() @ w.double().T
@@ -234,12 +262,13 @@ def test_paged_attention_behind_the_first_64_pages(name):
 
 
 def _engine_with_a_parted_head(slots):
-    """One layer of a real width; 40 rows of its head are 32 tiles, whose K is shared out."""
+    """One layer of a real width; 40 rows of its head are 64 tiles, whose K is shared out."""
+    assert linear_f32_form(40, 4096, 2048) == (64, 64, 0, 4)
     import dataclasses
     from llm_sharding_amd.config import get_preset
     from llm_sharding_amd.runtime.registry import make_engine, random_source
     cfg = get_preset("deretar-2k")
-    cfg = dataclasses.replace(cfg, layers=cfg.layers[:1], vocab_size=2048)
+    cfg = dataclasses.replace(cfg, layers=cfg.layers[:1], vocab_size=4096)
     return make_engine(cfg, 0, 1, torch.device(DEV, 0), torch.float32, has_embed=True, has_head=True, source=random_source(cfg, 3),
                        max_slots=slots, max_seq=16, max_prefill_rows=slots)
 
@@ -309,10 +338,12 @@ def test_positions_arrive_before_replays_of_other_streams():
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
 
 
+@pytest.mark.parametrize("n", [2048, 4096])  # streamed; in parts of K where there is a workspace
 @torch.inference_mode()
-def test_captured_product_without_a_workspace():
+def test_captured_product_without_a_workspace(n):
     """In a graph, a product that is given no workspace takes none: its replays may run beside others of any stream."""
-    k, n, rows = 2048, 2048, 40
+    k, rows = 2048, 40
+    assert linear_f32_form(rows, n, k)[3] == (4 if n == 4096 else 1)
     x, lin = _rand(rows, k, seed=1).to(DEV), Linear(_rand(n, k, seed=2, scale=k ** -0.5).to(DEV))
     out, want = torch.zeros(rows, n, device=DEV), torch.zeros(rows, n, device=DEV)
     lin(x, rows, want)
