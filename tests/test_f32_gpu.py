@@ -104,6 +104,17 @@ def product(x, w):
     return out[:, :n].double().cpu()
 
 
+@pytest.mark.parametrize("rows", [4, 33, 64])
+@pytest.mark.parametrize("k", [2048, 4096])
+def test_streamed_products_are_sums_of_sixteenths(rows, k):
+    """Of random operands. k / 16 roundings in each of 16 sums, of partial sums that grow as the root of their number: each off by
+    2^-24 / 3^0.5 of its value on average, together by the root of k / 32 times that."""
+    assert linear_f32_form(rows, 2048, k) == (16, 0, 0, 1)
+    x, w = _rand(rows, k, seed=1), _rand(2048, k, seed=2, scale=k ** -0.5)
+    want = x.double() @ w.double().T
+    assert (product(x, w) - want).norm() / want.norm() < 2.0 ** -24 / 3 ** 0.5 * (k / 32) ** 0.5
+
+
 @pytest.mark.parametrize("rows,n,k", [(33, 8464, 64), (65, 16400, 32), (100, 4112, 96), (129, 16400, 224), (257, 4368, 544),
                                       (960, 8208, 128), (2100, 2064, 160)])
 def test_linear_tiles(rows, n, k):
