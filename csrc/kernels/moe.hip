@@ -357,7 +357,8 @@ __global__ __launch_bounds__(NW * 64) void moe_stream_f32_kernel(const MoeTile* 
 }
 
 // many: MT x 16 pairs x NW x 32 columns. 20536 pairs, 32 experts of 2048 x 1024: up 776 -> 477, down 769 -> 465 us (64 x 64 tiles
-// on the fp32 matrix instructions before); about 90 pairs an expert, gated, of 1024 columns 509 -> 346 in 64 x 128 tiles.
+// on the fp32 matrix instructions before); about 90 pairs an expert, gated, of 1024 columns 509 -> 346 in 64 x 128 tiles; 8 experts
+// of 1024 x 2048, 40 pairs each 35 -> 29 in 64 x 64 (64 x 128 44, 128 x 256 117: which of them, ops/moe.py).
 template <int UP, int MT, int NW, int KG>
 __global__ __launch_bounds__(NW * KG * 64) void moe_tile_f32_kernel(const MoeTile* __restrict__ tiles, const int* __restrict__ order,
                                                                     int top, const float* __restrict__ A, int lda,
@@ -397,12 +398,14 @@ __global__ __launch_bounds__(NW * KG * 64) void moe_tile_f32_kernel(const MoeTil
 }
 
 template <int UP>
-int launch_f32(const MoeTile* t, int max_tiles, int tile_rows, const int* order, int top, const float* A, int lda, const float* W,
-               int N, int K, float* out, int ldo, hipStream_t s) {
+int launch_f32(const MoeTile* t, int max_tiles, int tile_rows, bool narrow, const int* order, int top, const float* A, int lda,
+               const float* W, int N, int K, float* out, int ldo, hipStream_t s) {
   constexpr int NT = UP == MOE_GLU ? 2 : 1;
   const dim3 grid((N + NT * 16 - 1) / (NT * 16), max_tiles);
   if (tile_rows <= 16) moe_stream_f32_kernel<UP, 1, NT, 8><<<grid, 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
   else if (tile_rows <= 32) moe_stream_f32_kernel<UP, 2, NT, 8><<<grid, 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
+  else if (tile_rows <= 64 && narrow)
+    moe_tile_f32_kernel<UP, 4, 2, 4><<<dim3((N + 63) / 64, max_tiles), 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
   else if (tile_rows <= 64)
     moe_tile_f32_kernel<UP, 4, 4, 2><<<dim3((N + 127) / 128, max_tiles), 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
   else if (tile_rows <= 128)
@@ -470,7 +473,8 @@ extern "C" int lsa_moe_route_group(const RouteArgs* ra, const float* logits, int
 }
 
 // up (MoeUp): A = h rows, out [pairs][ldo >= N / 2 (glu) or N]; down: A = act [pairs], out [pairs][ldo >= N]
-extern "C" int lsa_moe_gemm(int f32, int up, const void* tiles, int max_tiles, int tile_rows, const int* order, int top,
+// narrow (fp32, tiles of 64 rows): 64 columns a workgroup instead of 128
+extern "C" int lsa_moe_gemm(int f32, int up, const void* tiles, int max_tiles, int tile_rows, int narrow, const int* order, int top,
                             const void* A, int lda, const void* W, int N, int K, void* out, int ldo, hipStream_t s) {
   if (max_tiles < 1 || max_tiles > 65535 || top < 1 || N < 32 || N % 32 || K < 32 || K % 32 || lda < K || lda % 8 ||
       up < MOE_DOWN || up > MOE_RELU2 || ldo < (up == MOE_GLU ? N / 2 : N) || ldo % 4 ||
@@ -480,7 +484,7 @@ extern "C" int lsa_moe_gemm(int f32, int up, const void* tiles, int max_tiles, i
   const MoeTile* t = (const MoeTile*)tiles;
   if (f32) {
     auto* f = up == MOE_GLU ? launch_f32<MOE_GLU> : up ? launch_f32<MOE_RELU2> : launch_f32<MOE_DOWN>;
-    return f(t, max_tiles, tile_rows, order, top, (const float*)A, lda, (const float*)W, N, K, (float*)out, ldo, s);
+    return f(t, max_tiles, tile_rows, narrow, order, top, (const float*)A, lda, (const float*)W, N, K, (float*)out, ldo, s);
   }
 #define LSA_M(MT)                                                                                                     \
   if (tile_rows == MT * 16) {                                                                                         \

@@ -58,13 +58,26 @@ class Experts:
         return [self.up, self.down]
 
 
-def tile_rows(pairs: int, experts: int, f32: bool) -> int:
-    """Pairs per tile: what an expert gets on average, rounded to a kernel's size."""
+def tile_rows(pairs: int, experts: int, f32: bool, cols: Optional[int] = None) -> int:
+    """Pairs per tile: what an expert gets on average, rounded to a kernel's size. ``cols``: of the narrower of the two products (None:
+    wide enough)."""
     mean = pairs / experts  # (a second tile of an expert reads its weights again)
     if f32:  # 64 x 128 and 128 rows x 256 columns: 90 pairs an expert 3907 and 4155 us a pass (Runidra 2k), 183 6000 and 5662, 104
-        # 3780 and 3804 (Dumizen 2k), 141 4568 and 4440
-        return next((n for n in (16, 32) if mean <= 0.75 * n), 64 if mean <= 112 else 128)
+        # 3780 and 3804 (Dumizen 2k), 141 4568 and 4440. The large ones keep a CU for more than twice as long and are for products with as
+        # many as 160 of them: 8 experts of 1024 x 2048, 136 pairs each 51 and 122 us, 32 experts 145 and 138. With narrow ones (gemm)
+        # 1.02 times the fastest of all three, worst 1.45 (just under 112 pairs); by the pairs alone 1.37, worst 4.0 (270 products
+        # of 2 to 32 experts, 768 to 4096 columns and 26 to 400 pairs evenly drawn, profiles/cost_moe_f32.csv).
+        if mean > 112 and (cols is None or experts * max(1.0, mean / 128 + 0.5) * -(-cols // 256) >= 160):
+            return 128
+        return next((n for n in (16, 32) if mean <= 0.75 * n), 64)
     return next((n for n in (16, 32, 64) if mean <= 0.75 * n), 128 if mean <= 320 else 256)
+
+
+def narrow_tiles(pairs: int, experts: int, rows: int, cols: int) -> bool:
+    """Whether tiles of 64 rows have 64 columns instead of 128 (fp32): where there are no more of those than CUs, with 3/8 of a tile
+    more per expert than its pairs fill. 1024 x 2048: 128 tiles 30 and 46 us, 256 33 and 48, 288 58 and 50."""
+    n = min(experts, pairs)
+    return rows == 64 and n * max(1.0, pairs / n / 64 + 0.375) * -(-cols // 64) <= 256
 
 
 def max_tiles(pairs: int, experts: int, rows: int) -> int:
@@ -122,7 +135,7 @@ def gemm(tiles, n_tiles: int, rows: int, order, top: int, a, w, n: int, k: int, 
         _check(lib().lsa_moe_gemm_big(up, _p(tiles), n_tiles, rows, _p(order), top, _p(a), a.shape[0] if up else 0,
                                       a.stride(0), _p(w), n, k, _p(out), out.stride(0), _stream()), "lsa_moe_gemm_big")
         return
-    _check(lib().lsa_moe_gemm(is_f32(a.dtype), up, _p(tiles), n_tiles, rows, _p(order), top, _p(a), a.stride(0), _p(w),
+    _check(lib().lsa_moe_gemm(is_f32(a.dtype), up, _p(tiles), n_tiles, rows, narrow_tiles(pairs, w.shape[0], rows, n), _p(order), top, _p(a), a.stride(0), _p(w),
                               n, k, _p(out), out.stride(0), _stream()), "lsa_moe_gemm")
 
 
@@ -134,5 +147,5 @@ def declare(L: ctypes.CDLL) -> None:
         "lsa_moe_group": [vp, i, i, i, i, vp, vp, vp, vp, i, vp],
         "lsa_moe_route_group": [ra, vp, i, i, i, i, vp, vp, i, i, vp, vp, vp, vp],
         "lsa_moe_gemm_big": [i, vp, i, i, vp, i, vp, i, i, vp, i, i, vp, i, vp],
-        "lsa_moe_gemm": [i, i, vp, i, i, vp, i, vp, i, vp, i, i, vp, i, vp],
+        "lsa_moe_gemm": [i, i, vp, i, i, i, vp, i, vp, i, vp, i, i, vp, i, vp],
     })

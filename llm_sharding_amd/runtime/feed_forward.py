@@ -142,7 +142,7 @@ class Moe:
         expert, order, place, spare = eng.scratch_view("pairs", rows, 4 * s.top).reshape(4, pairs)
         weight, tiles = eng.scratch_view("pair_w", rows, s.top).reshape(-1), eng.scratch_view("tiles", rows, 8 * s.top)
         act, ye = eng.scratch_view("act", pairs, x.ff), eng.scratch_view("ye", pairs, x.width)
-        tr = X.tile_rows(pairs, s.experts, x.f32)
+        tr = X.tile_rows(pairs, s.experts, x.f32, min(x.up_n, x.width))
         nt = X.route_group(in32[:, col["router"]:], rows, s.experts, s.top, tr, expert, weight, order, place, tiles,
                            self.how, spare)
         X.gemm(tiles, nt, tr, order, s.top, h, x.up, x.up_n, x.width, act, pairs, x.kind)

@@ -748,3 +748,33 @@ def test_many_pairs_are_sorted_by_several_workgroups(pairs, experts):
         assert torch.equal(place.cpu().long()[o], torch.arange(pairs))
         tables.append(tiles)
     assert torch.equal(tables[0], tables[1]) and torch.equal(tables[0], tables[2])
+
+
+@pytest.mark.parametrize("kind", ["down", "glu", "relu2"])
+@pytest.mark.parametrize("n,k", [(32, 32), (96, 160), (160, 64), (256, 96)])
+@pytest.mark.parametrize("narrow", [False, True])
+def test_fp32_tiles_of_both_widths(kind, n, k, narrow, monkeypatch):
+    """64 pairs by 64 and by 128 columns: columns and pairs that fill no tile, experts with one pair, none, and a tile and two more;
+    nothing written beside the result."""
+    from llm_sharding_amd.ops import moe as X
+    from llm_sharding_amd.ops.packing import pack_f32
+    up = {"down": X.DOWN, "glu": X.GLU, "relu2": X.RELU2}[kind]
+    monkeypatch.setattr(X, "narrow_tiles", lambda *a: narrow)
+    e = torch.tensor([0] * 66 + [2] + [3] * 64).int()[torch.randperm(131, generator=torch.Generator().manual_seed(1))]
+    pairs, experts, cols = 131, 4, n // 2 if up == X.GLU else n
+    w, a = _rand(experts, n, k, seed=2, scale=k ** -0.5, dtype=F32), _rand(pairs, k, seed=3, dtype=F32)
+    order, place = (torch.zeros(pairs, dtype=torch.int32, device=DEV) for _ in range(2))
+    tiles = torch.zeros((X.max_tiles(pairs, experts, 64), 4), dtype=torch.int32, device=DEV)
+    nt = X.group(e.to(DEV), pairs, experts, 64, order, place, tiles)
+    at = order.cpu().long()
+    rows = a if up else a[at]  # down reads the sorted pairs
+    out = torch.full((pairs + 1, cols + 4), 7.0, device=DEV)
+    X.gemm(tiles, nt, 64, order, 1, rows.to(DEV), torch.stack([pack_f32(x) for x in w]).to(DEV), n, k, out, pairs, up)
+    y = torch.einsum("pnk,pk->pn", w.double()[e[at].long()], a.double()[at])
+    if up == X.GLU:
+        y = y.view(pairs, -1, 2, 16)
+        y = (torch.nn.functional.silu(y[:, :, 0]) * y[:, :, 1]).flatten(1)
+    elif up == X.RELU2:
+        y = y.relu().square()
+    close(out[:pairs, :cols], y, 2e-6, kind)
+    assert bool((out[pairs:] == 7).all()) and bool((out[:, cols:] == 7).all())

@@ -212,6 +212,23 @@ def test_coop_choice_of_large_products(n, k, rows, monkeypatch):
     assert us[cfg] <= 1.05 * us[fills], (cfg, fills)
 
 
+@pytest.mark.parametrize("experts,mean,cols,rows", [
+    (8, 136, 1024, 64), (8, 208, 768, 64), (8, 250, 2048, 64), (8, 256, 2048, 128), (8, 640, 4096, 128), (32, 112, 4096, 64),
+    (32, 113, 2048, 128), (32, 136, 1024, 128), (32, 400, 256, 64), (1, 5000, 1024, 64), (1, 5000, 1024 + 4096, 128), (64, 20, 4096, 32)])
+def test_fp32_experts_have_large_tiles_where_these_fill_the_chip(experts, mean, cols, rows):
+    from llm_sharding_amd.ops import moe
+    assert moe.tile_rows(mean * experts, experts, True, cols) == rows
+    assert moe.tile_rows(mean * experts, experts, True) == (128 if mean > 112 else rows)
+
+
+@pytest.mark.parametrize("pairs,experts,rows,cols,narrow", [
+    (320, 8, 64, 1024, True), (640, 8, 64, 1024, True), (896, 8, 64, 1024, False), (1400, 8, 64, 768, False), (328, 8, 64, 2048, False),
+    (40, 1000, 64, 384, True), (40, 1000, 64, 448, False), (320, 8, 32, 1024, False), (5120, 8, 128, 1024, False)])
+def test_fp32_experts_have_narrow_tiles_where_these_leave_cus(pairs, experts, rows, cols, narrow):
+    from llm_sharding_amd.ops import moe
+    assert moe.narrow_tiles(pairs, experts, rows, cols) == narrow
+
+
 def test_stream_handle_with_and_without_the_raw_call(monkeypatch):
     """The raw handle of the current device's stream where torch has the call, the Stream object's elsewhere."""
     from types import SimpleNamespace
