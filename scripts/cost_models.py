@@ -43,6 +43,12 @@ def coop(k, times):
     return packing._coop_choice(k[0] // 16, k[1], packing.row_blocks(k[2]), False)
 
 
+def one_tile(k, times):
+    """The model's choice without two tiles per wave and three parts."""
+    c = [c for c in times if c[0] == 1 and c[2] == 2 and c[3] in (1, 2, 4, 8) and c[4] <= 2 and c[5] == 3]
+    return min(c, key=lambda c: (packing.coop_cost(k[0] // 16, k[1], packing.row_blocks(k[2]), c), c[1] * c[4]), default=None)
+
+
 def fills(k, times):
     """The smallest split that fills the chip."""
     for kf in (8, 4, 2):
@@ -97,10 +103,13 @@ def main() -> None:
     print("gemm_sk:", regret(load("cost_gemm_sk.csv", 3), sk))
     products = load("cost_coop.csv", 3)
     for name, pick in (("the model", coop), ("smallest split that fills", fills)):
-        for rows in (24, 48, 96, 100):  # (of 96 rows the present choice is measured for some, of 100 for all)
+        for rows in (24, 48, 65, 96, 100, 128):
             print(f"cooperative GEMV, {name}, {rows} rows:", regret({k: r for k, r in products.items() if k[2] == rows}, pick))
-        print(f"cooperative GEMV, {name}, larger products at 32, 64 and 128:",
-              regret({k: r for k, r in products.items() if k[2] in (32, 64, 128)}, pick))
+        print(f"cooperative GEMV, {name}, larger products at 32 and 64:",
+              regret({k: r for k, r in products.items() if k[2] in (32, 64)}, pick))
+    for rows in (65, 96, 128):
+        print(f"cooperative GEMV, one tile per wave and no three parts, {rows} rows:",
+              regret({k: r for k, r in products.items() if k[2] == rows}, one_tile))
     print("fp32 tiles and parts of K:", regret(load("cost_f32_tiles.csv", 3), tiles))
     if "--fit" in sys.argv:
         fit(products)
