@@ -11,14 +11,13 @@
 //              8 rows, N = K = 2048 7 us (2.4 TB/s), N = 16384 25 us (5.5 TB/s).
 //   F32Split   many rows, on the bf16 matrix instructions, which are 16 times as fast: each operand is taken apart into three
 //              bf16 (8 + 8 + 8 bits of its 24), and of their nine products the six of more than 2^-24 of the whole are made.
-//              Bound by the matrix unit: what its clock allows with six full-width products (random operands: 1750 of 2500
-//              TFLOP/s, 290 of fp32 product), and for a third of that by the splitting, 6.5 vector instructions a value, two of
-//              which fit beside a matrix instruction. 2567 rows, N = 16384, K = 2048 1371 -> 800 us (215 TFLOP/s; the fp32
-//              instructions reach 157 at best and did 126), 963 rows, N = 16384 520 -> 301, N = 2048 71 -> 51, K = 8192
-//              265 -> 165, 64 rows, N = 2048 17.3 -> 16.5.
+//              Bound by the matrix unit and by the splitting, which take turns: at 2567 rows, N = 16384, K = 2048 the one is busy
+//              for 66 % of the time, at the 1.75 GHz that its six products leave it (1835 of 2500 TFLOP/s, 306 of fp32 product), and 1.9
+//              other vector instructions for each of its take 31 %. That product 1343 -> 806 us (214 TFLOP/s; the fp32 instructions
+//              reach 157 at best), 963 rows, N = 16384 512 -> 302, N = 2048 78 -> 54, K = 8192 257 -> 171.
 //              Errors against 64 bits are lower than those of fp32 instructions, since a sum is rounded once for 32 k instead
-//              of once for 2 (the five smaller products have sums of their own): K = 2048 5.7e-7 -> 1.9e-7 to 2.7e-7 of the
-//              result's norm, K = 8192 1.15e-6 -> 2.8e-7 to 5.7e-7. With all six in one sum it was 7e-7.
+//              of once for 2 (the five smaller products have sums of their own): K = 2048 3.3e-7 to 5.7e-7 -> 1.1e-7 to 2.7e-7 of the
+//              result's norm, K = 8192 6.6e-7 to 1.15e-6 -> 2.2e-7 to 5.7e-7. With all six in one sum it was 7e-7.
 #pragma once
 #include "elem.h"
 #include "mfma_pair.h"

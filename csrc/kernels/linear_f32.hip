@@ -85,8 +85,9 @@ __global__ __launch_bounds__(NW * KG * 64) void tile_f32_kernel(
 // A product's tiles, and how many parts of K for each of the last `rem` ones, which fill the CUs only in part (S; `whole` before
 // them that fill them). Modelled us: a round of tiles its steps of 32 k and 5.2 to begin and end, a part its share of the steps;
 // the meeting by the parts of a tile and by their bytes. Fitted to 176 products (11 of 512 to 8192 k by 640 to 16384 columns at 20
-// to 2567 rows, all forms and splits): what it takes is 1.005 times the fastest (geometric mean; worst 1.08). The largest tiles
-// split least and read least (1.04 us for 128 x 128 of 32 k against 1.52 of the smallest), the smallest leave the fewest CUs idle.
+// to 2567 rows, all forms and splits): what it takes is 1.005 times the fastest (geometric mean; worst 1.08; timed without the operands' scaling, which adds 2 %
+// to the large tiles' products and up to 9 % to the others). The largest tiles
+// split least and read least (1.14 us for 128 x 128 of 32 k against 1.52 of the smallest), the smallest leave the fewest CUs idle.
 struct Plan {
   int rows, cols, whole, S;
 };

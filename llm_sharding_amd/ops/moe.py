@@ -131,11 +131,13 @@ def gemm(tiles, n_tiles: int, rows: int, order, top: int, a, w, n: int, k: int, 
          and out.shape[0] >= pairs and out.shape[1] >= (n // 2 if up == GLU else n) and order.numel() >= pairs
          and (a.shape[0] * top >= pairs if up else a.shape[0] >= pairs), "moe: shapes")
     _req(w[0].numel() == n * k and w.is_contiguous(), "moe: weights")
-    if rows > 64 and not is_f32(a.dtype):
+    f32 = is_f32(a.dtype)
+    if rows > 64 and not f32:
         _check(lib().lsa_moe_gemm_big(up, _p(tiles), n_tiles, rows, _p(order), top, _p(a), a.shape[0] if up else 0,
                                       a.stride(0), _p(w), n, k, _p(out), out.stride(0), _stream()), "lsa_moe_gemm_big")
         return
-    _check(lib().lsa_moe_gemm(is_f32(a.dtype), up, _p(tiles), n_tiles, rows, narrow_tiles(pairs, w.shape[0], rows, n), _p(order), top, _p(a), a.stride(0), _p(w),
+    narrow = bool(f32) and narrow_tiles(pairs, w.shape[0], rows, n)
+    _check(lib().lsa_moe_gemm(f32, up, _p(tiles), n_tiles, rows, narrow, _p(order), top, _p(a), a.stride(0), _p(w),
                               n, k, _p(out), out.stride(0), _stream()), "lsa_moe_gemm")
 
 

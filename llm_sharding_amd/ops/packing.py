@@ -351,12 +351,12 @@ def _coop_choice(n_tiles: int, k: int, mb: int, need_even: bool) -> tuple | None
     """A configuration for a product that no table entry covers.
 
     One tile per wave and the K chunk of the row block's register budget, from 65 rows on also two tiles per wave and four groups
-    of them along K (65 products at 100 rows: a geometric mean of 1.025 times the fastest, 1.050 without these and without
-    three parts; 4096 x 3072 16.3 -> 14.1 us, 4096 x 8192 26.5 -> 23.2, 10240 x 8192 51 -> 44.6): of the first the cheapest takes 1.02, 1.06 and 1.04
-    times the fastest of all configurations at 24, 48 and 96 rows (geometric mean over 62 products of 1024 to 28672 columns,
-    K 1024 to 11008; worst 1.48), 1.03 times over 42 larger ones (4096 to 57344 columns, K to 28672, 32 to 128 rows; worst 1.27); the
-    smallest split that fills the CUs takes 1.51, 1.53 and 1.58 times, of the larger 1.14, and is what is left where K or N
-    allows none of them (profiles/cost_models.md, scripts/cost_models.py). Four layers of Llama 3.2 3B at 47 sequences: 8 steps 5374 -> 4259 us; at 21 4171 -> 3215."""
+    of them along K (at 100 rows 4096 x 3072 16.3 -> 14.1 us, 4096 x 8192 26.5 -> 23.2, 10240 x 8192 51 -> 44.6). The cheapest
+    takes 1.02 and 1.06 times the fastest of all configurations at 24 and 48 rows (geometric mean over 62 products of 1024 to 28672
+    columns, K 1024 to 11008; worst 1.48), 1.04 times over 28 larger ones at 32 and 64 rows (to 57344 columns, K to 28672; worst
+    1.27), and 1.04, 1.03 and 1.03 times over 74 of both kinds at 65, 96 and 128 rows (worst 1.22; 1.07, 1.05 and 1.05 without
+    two tiles per wave and three parts); the smallest split that fills the CUs takes 1.51, 1.53, of the larger 1.16, 1.67, 1.65
+    and 1.62 times, and is what is left where K or N allows none of them (profiles/cost_models.md, scripts/cost_models.py). Four layers of Llama 3.2 3B at 47 sequences: 8 steps 5374 -> 4259 us; at 21 4171 -> 3215."""
     allc = _coop_candidates(n_tiles, k, mb, need_even)
     cands = [c for c in allc if c[0] == 1 and c[2] == (2 if mb == 8 else 4) and 1 <= c[3] <= 8 and c[4] <= 2 and c[5] == 3]
     cands += [c for c in allc if c[:3] == (2, 2, 2) and 1 <= c[3] <= 8 and c[4:] == (4, 2)]
