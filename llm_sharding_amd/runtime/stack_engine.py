@@ -12,7 +12,7 @@ decoders that differ from Llama / GPT-2 in what a layer is made of:
 * layers that run several times in a row are as many entries of the stack, with one layer's weights and caches
   of their own; what a pass starts from reads the embedding output, so they begin on the first stage;
 * projections run the framework's GEMV / GEMM kernels on padded weights (ops/stream.Linear); fp32
-  engines run every product in true fp32.
+  engines run every product at fp32 accuracy.
 """
 from __future__ import annotations
 
