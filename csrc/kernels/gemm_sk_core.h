@@ -97,17 +97,28 @@ LSA_DEVICE void loop_barrier() {
   if constexpr (LSA_SK_ABLATE != 4) barrier();
 }
 
-LSA_DEVICE void glds16(const void* src, unsigned char* lds_base) {
+// v, as far as the compiler knows another value each time: what is computed from it is not kept in registers over the main loop
+LSA_DEVICE int fresh(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// 16 bytes a lane from base + off + at to LDS: the descriptor and ``at`` are scalars and off is one register (pointers took two a
+// block, two more to add the K offset in, and vector additions for that)
+LSA_DEVICE __amdgpu_buffer_rsrc_t dma_src(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, -1, 0x00020000);
+}
+LSA_DEVICE void glds16(__amdgpu_buffer_rsrc_t src, unsigned off, unsigned at, unsigned char* lds_base) {
   if constexpr (LSA_SK_ABLATE != 2 && LSA_SK_ABLATE != 11)
-    __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)lds_base, 16, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)lds_base, 16, off, at, 0, 0);
 }
 // weight stream: default cache policy (non-temporal weight DMA measured no better in the headline
 // step, profiles/r3_gemm_nt_retune.jsonl; ablation build 9 keeps it for probes)
-LSA_DEVICE void glds16_w(const void* src, unsigned char* lds_base) {
+LSA_DEVICE void glds16_w(__amdgpu_buffer_rsrc_t src, unsigned off, unsigned at, unsigned char* lds_base) {
   if constexpr (LSA_SK_ABLATE == 9)
-    __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)lds_base, 16, 0, 2 /* nt */);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)lds_base, 16, off, at, 0, 2 /* nt */);
   else
-    glds16(src, lds_base);
+    glds16(src, off, at, lds_base);
 }
 
 // tile id -> (row tile, col tile): group_m row tiles sweep the column tiles together so the
@@ -142,24 +153,20 @@ struct Kern {
   // ---- DMA staging of one LDS region of local K-tile t ------------------------------------------
   // A region mh: the 128 rows wr'*TM + mh*TM/2 + i*16 + r16 (ordered (wr', i, r16)), 128 B each,
   // 16-B chunks XOR-swizzled by row%8; each DMA instruction fetches 8 whole rows (full lines)
-  // Sources = wave-uniform segment base (SGPRs) + 32-bit per-lane offset (one VGPR per block
-  // instead of a 64-bit pointer: the 256-wide tile needs every register it can keep).
-  const unsigned char* a_seg;
-  const unsigned char* b_seg;
+  // Sources = wave-uniform segment base (SGPRs) + 32-bit per-lane offset (one VGPR per block).
+  __amdgpu_buffer_rsrc_t a_seg, b_seg;
   LSA_DEVICE void stage_a(int buf, int mh, const unsigned (&aoff)[2][AGL], int kt) {
     unsigned char* dst = smem + buf * BUF + mh * AREG;
-    const unsigned char* base = a_seg + (size_t)kt * (BK * 2);
     if constexpr (LSA_SK_ABLATE == 6) return;
 #pragma unroll
-    for (int s = 0; s < AGL; ++s) glds16(base + aoff[mh][s], dst + (w * AGL + s) * 1024);
+    for (int s = 0; s < AGL; ++s) glds16(a_seg, aoff[mh][s], kt * (BK * 2), dst + (w * AGL + s) * 1024);
   }
   LSA_DEVICE void stage_b(int buf, int nh, const unsigned (&boff)[2][BGL], int kt) {
     unsigned char* dst = smem + buf * BUF + 2 * AREG + nh * BREG;
-    const unsigned char* base = b_seg + (size_t)kt * 2048;
     if constexpr (LSA_SK_ABLATE == 7) return;
 #pragma unroll
     for (int s = 0; s < BGL; ++s)
-      if (s < BGL_LO || w < BHI_WAVES) glds16_w(base + boff[nh][s], dst + (s * 8 + w) * 1024);
+      if (s < BGL_LO || w < BHI_WAVES) glds16_w(b_seg, boff[nh][s], kt * 2048, dst + (s * 8 + w) * 1024);
   }
   // the same for a wave group known at compile time (HI: a wave w < BHI_WAVES, which issues
   // BGL B blocks per region; else BGL_LO): the main loop is instantiated per group, so neither
@@ -167,11 +174,10 @@ struct Kern {
   template <bool HI>
   LSA_DEVICE void stage_b_g(int buf, int nh, const unsigned (&boff)[2][BGL], int kt) {
     unsigned char* dst = smem + buf * BUF + 2 * AREG + nh * BREG;
-    const unsigned char* base = b_seg + (size_t)kt * 2048;
     if constexpr (LSA_SK_ABLATE == 7) return;
 #pragma unroll
     for (int s = 0; s < BGL; ++s)
-      if (s < BGL_LO || HI) glds16_w(base + boff[nh][s], dst + (s * 8 + w) * 1024);
+      if (s < BGL_LO || HI) glds16_w(b_seg, boff[nh][s], kt * 2048, dst + (s * 8 + w) * 1024);
   }
   template <bool HI>
   LSA_DEVICE void wait_tile_g() {
@@ -203,8 +209,8 @@ struct Kern {
     const int n = kb - ka;
     const int n0 = nt * BN;
     const int KT32 = P.K >> 5;
-    a_seg = reinterpret_cast<const unsigned char*>(A + (GATHER ? 0 : (size_t)m0 * P.lda) + ka * BK);
-    b_seg = reinterpret_cast<const unsigned char*>(W) + ((size_t)(n0 >> 4) * KT32 + ka * 2) * 1024;
+    a_seg = dma_src(A + (GATHER ? 0 : (size_t)m0 * P.lda) + ka * BK);
+    b_seg = dma_src(reinterpret_cast<const unsigned char*>(W) + ((size_t)(n0 >> 4) * KT32 + ka * 2) * 1024);
     unsigned aoff[2][AGL], boff[2][BGL];
 #pragma unroll
     for (int mh = 0; mh < 2; ++mh)
@@ -392,6 +398,7 @@ struct Kern {
 
   // ---- fp32 partial slab (fragment-native, write-through) ------------------------------------
   LSA_DEVICE void slab_store(float* slab, size_t slot, const f32x4_t (&acc)[FM][FN]) {
+    const int lane = fresh(this->lane);
     const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(slab + slot * (size_t)(BM * BN), (short)0,
                                                                          BM * BN * 4, 0x00020000);
 #pragma unroll
@@ -407,6 +414,7 @@ struct Kern {
   // read sc1: they bypass this CU's L1, which may hold stale copies). Caller: every wave, LDS
   // free (and a barrier before the LDS is reused by other waves).
   LSA_DEVICE void slab_add(const float* slab, size_t slot, f32x4_t (&acc)[FM][FN]) {
+    const int lane = fresh(this->lane);
     // RP tile rows (PB blocks) per pass, NP passes, DB ring buffers per wave: as much in flight
     // as this geometry's LDS allows (the ring must stay below the flag word at SMEM - 16)
     constexpr int AVAIL = G_::SMEM - 16;
@@ -443,8 +451,31 @@ struct Kern {
     }
   }
 
+  // One pass of an EPI_STORE product whose columns of this wave all go to out32: four columns a lane, so that the lanes of a
+  // store have whole rows of the wave's tile (256 or 384 bytes) and not 16 bytes of every 64. 3189 x 4096 x 256 31.5 -> 20.0 us
+  // (bf16 18.2), 3189 x 2048 x 2048 41 -> 33. What gates (reads and writes 10 bytes a value, in all workgroups at once) is bound by
+  // memory and no faster this way (24.9 and 23.9; 204 and 212 us).
+  LSA_DEVICE void store32(const EpiArgs& ep, const float* img, int lane, int row_base, int col_base) {
+    constexpr int QPR = TN / 4, UNITS = G_::EROWS * QPR / 64;
+    static_assert(G_::EROWS * QPR % 64 == 0, "whole waves of quads");
+#pragma unroll
+    for (int s = 0; s < UNITS; ++s) {
+      const int u = lane + 64 * s, row = u / QPR, q = u % QPR, c = col_base + q * 4;
+      f32x4_t v = *reinterpret_cast<const f32x4_t*>(img + row * G_::ELD + q * 4);
+      if (row_base + row < p->M && (BN != 192 || c < p->N)) {
+        if (ep.bias) v += *reinterpret_cast<const f32x4_t*>(ep.bias + c);
+        if (ep.act && epi_acts(ep, c)) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = epi_activate(ep.act, v[j]);
+        }
+        *reinterpret_cast<f32x4_t*>(ep.out32 + (size_t)(row_base + row) * ep.ldo32 + (c - ep.col32)) = v;
+      }
+    }
+  }
+
   // ---- fused epilogue through an LDS transpose -------------------------------------------------
   LSA_DEVICE void epilogue(const EpiArgs& ep, const f32x4_t (&acc)[FM][FN], int m0, int nt, int sp) {
+    const int lane = fresh(this->lane), tid = fresh(this->tid);
     const SkParams& P = *p;
     constexpr int EROWS = G_::EROWS, ELD = G_::ELD, FPP = EROWS / 16;  // rows / fragments per pass
     float* img = reinterpret_cast<float*>(smem) + w * (EROWS * ELD);
@@ -524,6 +555,8 @@ struct Kern {
           }
           __builtin_amdgcn_sched_barrier(0);
         }
+      } else if (EPI == EPI_STORE && ep.out32 && !ep.gate && col_base >= ep.col32) {
+        store32(ep, img, lane, row_base, col_base);
       } else {
 #pragma unroll
         for (int s = 0; s < (EROWS * FN) / 64; ++s) {
