@@ -4,8 +4,8 @@
 // nn.Linear calls inside HF LlamaDecoderLayer (/root/reference/utils/shard_loader.py:66-74).
 //
 // Structure (cdna_hip_programming.md §5 "The 256² 8-phase template", T1-T5):
-//  * 256 x BN output tile (BN = 256 or 128) per 512-thread workgroup (8 waves, 2 per SIMD),
-//    K step 64, one workgroup per CU, all LDS in ONE __shared__ array.
+//  * 256 x BN output tile (BN = 256 or 128; 128 to 384 rows) per 512-thread workgroup (8 waves, 2 per
+//    SIMD), K step 64, one workgroup per CU, all LDS in ONE __shared__ array.
 //  * Both operands reach LDS by LDS-DMA (global_load_lds_dwordx4): the packed-16x32 weights
 //    (common.h) are already one lane-linear 1 KiB block per (16 cols, 32 k) fragment; the A
 //    tile is fetched as whole 128-B rows (full cache lines: 5-12 % faster than gathering
@@ -109,12 +109,11 @@ __global__ __launch_bounds__(NTHR) void gemm_sk_kernel(const bf16_raw* __restric
     LSA_STAMP(k.stamp_base + 2);
     bool do_epi = true;
     if (partial && EPI != EPI_PARTIAL) {
-      // contributors of this tile, in K order: split mode - workgroups ts + s * sk_tiles
-      // (slot 0); stream-K - the workgroups whose iteration ranges intersect the tile's
+      // contributors of this tile, in K order: split mode - workgroups ts + s * sk_tiles; stream-K - the workgroups whose iteration ranges intersect the tile's
       const long long t0 = (long long)ts * prm.NKT, t1 = t0 + prm.NKT;
       const int g_first = prm.split ? 0 : (int)(((t0 + 1) * G - 1) / S);
       const int g_last = prm.split ? prm.split - 1 : (int)((t1 * G - 1) / S);
-      k.slab_store(slab, prm.split ? (size_t)su * 2 : (size_t)g * 2 + (it == lo ? 0 : 1), acc);
+      k.slab_store(slab, prm.split ? (size_t)su : (size_t)g * 2 + (it == lo ? 0 : 1), acc);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       if (k.tid == 0) {
@@ -130,16 +129,17 @@ __global__ __launch_bounds__(NTHR) void gemm_sk_kernel(const bf16_raw* __restric
         const bool all = g_last - g_first > 1;
         if (all) zero();
         for (int ci = g_first; ci <= g_last; ++ci) {
-          int c, slot;
+          int c;
+          size_t slot;
           if (prm.split) {
             c = ts + ci * prm.sk_tiles;
-            slot = 0;
+            slot = c;
           } else {
             c = ci;
-            slot = (long long)c * S / G >= t0 ? 0 : 1;  // slot 0: c's range starts in this tile
+            slot = (size_t)c * 2 + ((long long)c * S / G >= t0 ? 0 : 1);  // the first of two: c's range starts in this tile
           }
           if (c == (prm.split ? su : g) && !all) continue;
-          k.slab_add(slab, (size_t)c * 2 + slot, acc);
+          k.slab_add(slab, slot, acc);
         }
         if (k.tid == 0) __hip_atomic_store(&counters[ts], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();  // every wave's slab ring reads are done before the epilogue reuses LDS
@@ -165,20 +165,26 @@ int launch(const bf16_raw* A, const bf16_raw* W, const SkParams& prm, const EpiA
 template <int BM, int EPI>
 int dispatch(const bf16_raw* A, const bf16_raw* W, const SkParams& prm, const EpiArgs& ep, float* slab,
              unsigned* cnt, int bn, int nb, hipStream_t s) {
-  if (bn == 256) {
-    if constexpr (BM == 128) {
-      if (nb == 3) return launch<BM, 256, EPI, 3>(A, W, prm, ep, slab, cnt, s);
-    }
+  if constexpr (BM == 320 || BM == 192) {
     return launch<BM, 256, EPI, 2>(A, W, prm, ep, slab, cnt, s);
+  } else if constexpr (BM == 384) {
+    return bn == 192 ? launch<BM, 192, EPI, 2>(A, W, prm, ep, slab, cnt, s) : launch<BM, 128, EPI, 2>(A, W, prm, ep, slab, cnt, s);
+  } else {
+    if (bn == 256) {
+      if constexpr (BM == 128) {
+        if (nb == 3) return launch<BM, 256, EPI, 3>(A, W, prm, ep, slab, cnt, s);
+      }
+      return launch<BM, 256, EPI, 2>(A, W, prm, ep, slab, cnt, s);
+    }
+    if (bn == 192) return launch<BM, 192, EPI, 2>(A, W, prm, ep, slab, cnt, s);
+    return nb == 3 ? launch<BM, 128, EPI, 3>(A, W, prm, ep, slab, cnt, s)
+                   : launch<BM, 128, EPI, 2>(A, W, prm, ep, slab, cnt, s);
   }
-  if (bn == 192) return launch<BM, 192, EPI, 2>(A, W, prm, ep, slab, cnt, s);
-  return nb == 3 ? launch<BM, 128, EPI, 3>(A, W, prm, ep, slab, cnt, s)
-                 : launch<BM, 128, EPI, 2>(A, W, prm, ep, slab, cnt, s);
 }
 
 }  // namespace
 
-// bm: tile height 256 or 128. bn: tile width 256 / 192 (192: N % 16 == 0, partial last tile) / 128.
+// bm: tile height 256 or 128, and 320 / 192 for bn 256, 384 for bn 192 / 128. bn: tile width 256 / 192 (192: N % 16 == 0, partial last tile) / 128.
 // nb: DMA ring buffers, 2 or 3 (3 for bn 128, and bn 256 at bm 128; 0 = the default: 3 where
 // allowed). grid: workgroups (<= 1024); dp: 1 = whole tiles in data-parallel rounds first (0 =
 // all tiles are remainder).
@@ -186,17 +192,18 @@ int dispatch(const bf16_raw* A, const bf16_raw* W, const SkParams& prm, const Ep
 // partial k stored to ((float*)ep->out)[k][M][ldo], no slabs or tickets (lsa_resid_rmsnorm_partials sums them).
 // split: 0 = remainder by stream-K, S >= 1 = remainder tiles split into up to S K ranges
 // (clamped to NKT and to grid / remainder tiles; stream-K when the remainder exceeds the grid).
-// slab: >= 2 * grid * bm * bn floats and counters: >= remainder tiles (zeroed) when any tile is
+// slab: >= 2 * grid * bm * bn floats (split tiles larger than 256 x 256: grid * bm * bn) and counters: >= remainder tiles (zeroed) when any tile is
 // split. Returns LSA_BAD_SHAPE on any shape the kernel's indexing cannot take.
 extern "C" int lsa_gemm_sk(const void* a, int lda, const void* wp, int M, int N, int K, int epi,
                            const EpiArgs* ep, int bm, int bn, int nb, int grid, int dp, int split, int group_m, float* slab,
                            unsigned* counters, long long slab_floats, int n_counters, hipStream_t stream) {
   if (M < 1 || K < BK || K % BK || lda < K || lda % 8 || !ep) return LSA_BAD_SHAPE;
   if (bn != 256 && bn != 192 && bn != 128) return LSA_UNSUPPORTED;
-  if (bm != 256 && bm != 128) return LSA_UNSUPPORTED;
+  if (bm != 256 && bm != 128 && !((bm == 320 || bm == 192) && bn == 256) && !(bm == 384 && bn != 256)) return LSA_UNSUPPORTED;
   const int BM = bm;
-  if (nb == 0) nb = (bn == 128 || (bm == 128 && bn == 256)) ? 3 : 2;
-  if (nb != 2 && !(nb == 3 && (bn == 128 || (bm == 128 && bn == 256)))) return LSA_UNSUPPORTED;
+  const bool three = bm <= 256 && bn == 128 || (bm == 128 && bn == 256);
+  if (nb == 0) nb = three ? 3 : 2;
+  if (nb != 2 && !(nb == 3 && three)) return LSA_UNSUPPORTED;
   if (bn == 192 ? (N % 16 || (epi_gated(epi) && N % 32)) : N % bn) return LSA_BAD_SHAPE;
   if (grid < 1 || grid > 1024 || group_m < 1) return LSA_BAD_SHAPE;
   if (epi == EPI_RESID && !ep->resid) return LSA_BAD_SHAPE;
@@ -244,12 +251,15 @@ extern "C" int lsa_gemm_sk(const void* a, int lda, const void* wp, int M, int N,
     }
   }
   if (epi != EPI_PARTIAL && prm.sk_tiles > 0 &&
-      (!slab || !counters || slab_floats < 2LL * prm.G * BM * bn || n_counters < prm.sk_tiles))
+      (!slab || !counters || slab_floats < (prm.split && BM * bn > 256 * 256 ? 1LL : 2LL) * prm.G * BM * bn || n_counters < prm.sk_tiles))
     return LSA_BAD_SHAPE;
   const bf16_raw* A = static_cast<const bf16_raw*>(a);
   const bf16_raw* W = static_cast<const bf16_raw*>(wp);
-#define LSA_G(E) (bm == 256 ? dispatch<256, E>(A, W, prm, *ep, slab, counters, bn, nb, stream) \
-                    : dispatch<128, E>(A, W, prm, *ep, slab, counters, bn, nb, stream))
+#define LSA_G(E) (bm == 256   ? dispatch<256, E>(A, W, prm, *ep, slab, counters, bn, nb, stream) \
+                  : bm == 128 ? dispatch<128, E>(A, W, prm, *ep, slab, counters, bn, nb, stream) \
+                  : bm == 320 ? dispatch<320, E>(A, W, prm, *ep, slab, counters, bn, nb, stream) \
+                  : bm == 192 ? dispatch<192, E>(A, W, prm, *ep, slab, counters, bn, nb, stream) \
+                              : dispatch<384, E>(A, W, prm, *ep, slab, counters, bn, nb, stream))
   switch (epi) {
     case EPI_STORE: return LSA_G(EPI_STORE);
     case EPI_RESID: return LSA_G(EPI_RESID);

@@ -10,9 +10,9 @@ namespace {
 
 constexpr int BK = 64, NTHR = 512;
 
-// BM x BN tile, BM = 256 or 128 (decode batches of <= 128 rows and M = 384 / 640 ...: no
-// MFMA or A traffic on rows past M). BN = 256: 2 x 4 waves of BM/2 x 64; BN = 192 / 128: 4 x 2
-// waves of BM/4 x 96 / BM/4 x 64.
+// BM x BN tile, BM = 384 (BN 128 / 192), 320 or 192 (BN 256), 256 or 128 (no MFMA or A traffic on
+// rows past the last tile). BN = 256: 2 x 4 waves of BM/2 x 64; BN = 192 / 128: 4 x 2 waves of
+// BM/4 x 96 / BM/4 x 64.
 // BN = 192 exists for shapes where 256-wide tiles leave CUs idle or need split-K fixups
 // (Llama-2-7B qkv N=12288 at M=512: 2 x 64 = 128 tiles; gate_up N=22016: 230 tiles in one
 // round at full K); N need not be a multiple of 192 (the last column tile is partial).
@@ -25,22 +25,24 @@ struct Geo {
   static constexpr int AREG = (BM / 2) * BK * 2;    // bytes of one A region (16 / 8 KiB)
   static constexpr int BREG = (BN / 2) * BK * 2;    // bytes of one B region
   static constexpr int BUF = 2 * AREG + 2 * BREG;   // one K-tile
-  static constexpr int AGL = AREG / 1024 / 8;       // DMA instructions per wave per A region
-  static constexpr int BBLK = BREG / 1024;          // 1 KiB blocks per B region (16 / 12 / 8)
-  // block b of a B region is issued by wave b % 8: with 12 blocks waves 0-3 issue 2 per
-  // region and waves 4-7 one, so the per-wave counts (and counted waits) depend on the wave
+  static constexpr int ABLK = AREG / 1024;          // 1 KiB blocks per A region (24 / 20 / 16 / 12 / 8)
+  static constexpr int BBLK = BREG / 1024;          // and per B region (16 / 12 / 8)
+  // block b of a region is issued by wave b % 8: with 12 or 20 blocks waves 0-3 issue one more
+  // per region than waves 4-7, so the per-wave counts (and counted waits) depend on the wave
+  static constexpr int AGL = (ABLK + 7) / 8, AGL_LO = ABLK / 8, AHI_WAVES = ABLK % 8;
   static constexpr int BGL = (BBLK + 7) / 8, BGL_LO = BBLK / 8, BHI_WAVES = BBLK % 8;
-  static constexpr int NPT = 2 * AGL + 2 * BGL;     // DMA instructions per K-tile, waves < BHI_WAVES
-  static constexpr int NPT_LO = 2 * AGL + 2 * BGL_LO;  // ... the other waves
-  static constexpr int EROWS = (TN > 64 || TM < 64) ? 32 : 64;  // rows per epilogue transpose pass
+  static constexpr int HI_WAVES = AHI_WAVES > BHI_WAVES ? AHI_WAVES : BHI_WAVES;
+  static constexpr int NPT = 2 * AGL + 2 * BGL;     // DMA instructions per K-tile, waves < HI_WAVES
+  static constexpr int NPT_LO = 2 * AGL_LO + 2 * BGL_LO;  // ... the other waves
+  static constexpr int EROWS = (TN > 64 || TM % 64) ? 32 : 64;  // rows per epilogue transpose pass
   static constexpr int ELD = TN + 4;                // fp32 row stride of the transpose image
   static constexpr int EPI_BYTES = 8 * EROWS * ELD * 4;
   static constexpr int RS_OFF = (NB * BUF > EPI_BYTES ? NB * BUF : EPI_BYTES);  // row rstd of the tile [BM]
   static constexpr int SMEM = RS_OFF + BM * 4 + 16;
   static_assert(SMEM <= 160 * 1024, "LDS budget");
-  static_assert(BHI_WAVES == 0 || BGL_LO == 0 || BHI_WAVES == 4, "B blocks per wave");
-  static_assert(AGL >= 1 && TM % EROWS == 0 && FM % 2 == 0, "tile geometry");
-  static_assert(NB == 2 || BHI_WAVES == 0, "3-buffer ring needs the same DMA count in every wave");
+  static_assert((AHI_WAVES == 0 || AHI_WAVES == 4) && (BHI_WAVES == 0 || BHI_WAVES == 4), "blocks per wave");
+  static_assert(AGL_LO >= 1 && BGL_LO >= 1 && TM % EROWS == 0 && FM % 2 == 0, "tile geometry");
+  static_assert(NB == 2 || HI_WAVES == 0, "3-buffer ring needs the same DMA count in every wave");
 };
 
 struct SkParams {
@@ -104,7 +106,7 @@ LSA_DEVICE int fresh(int v) {
 }
 
 // 16 bytes a lane from base + off + at to LDS: the descriptor and ``at`` are scalars and off is one register (pointers took two a
-// block, two more to add the K offset in, and vector additions for that)
+// block and two more to add the K offset in, 20 registers of a 320 x 256 tile)
 LSA_DEVICE __amdgpu_buffer_rsrc_t dma_src(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, -1, 0x00020000);
 }
@@ -138,8 +140,8 @@ struct Kern {
   using G_ = Geo<BM, BN, NB>;
   static constexpr int WM = G_::WM, WN = G_::WN, TM = G_::TM, TN = G_::TN, FM = G_::FM, FN = G_::FN;
   static constexpr int AREG = G_::AREG, BREG = G_::BREG, BUF = G_::BUF, AGL = G_::AGL, BGL = G_::BGL,
-                       NPT = G_::NPT, NPT_LO = G_::NPT_LO, BGL_LO = G_::BGL_LO, BHI_WAVES = G_::BHI_WAVES,
-                       BBLK = G_::BBLK;
+                       NPT = G_::NPT, NPT_LO = G_::NPT_LO, AGL_LO = G_::AGL_LO, BGL_LO = G_::BGL_LO,
+                       HI_WAVES = G_::HI_WAVES, ABLK = G_::ABLK, BBLK = G_::BBLK;
   static constexpr int HM = FM / 2, HN = FN / 2;  // quadrant size in 16x16 tiles
 
   unsigned char* smem;
@@ -155,29 +157,30 @@ struct Kern {
   // 16-B chunks XOR-swizzled by row%8; each DMA instruction fetches 8 whole rows (full lines)
   // Sources = wave-uniform segment base (SGPRs) + 32-bit per-lane offset (one VGPR per block).
   __amdgpu_buffer_rsrc_t a_seg, b_seg;
+  // block s of this wave in an A region (where every wave has as many, its blocks lie side by side)
+  LSA_DEVICE int a_block(int s) const { return AGL == AGL_LO ? w * AGL + s : s * 8 + w; }
   LSA_DEVICE void stage_a(int buf, int mh, const unsigned (&aoff)[2][AGL], int kt) {
+    if (w < HI_WAVES) stage_a_g<true>(buf, mh, aoff, kt); else stage_a_g<false>(buf, mh, aoff, kt);
+  }
+  LSA_DEVICE void stage_b(int buf, int nh, const unsigned (&boff)[2][BGL], int kt) {
+    if (w < HI_WAVES) stage_b_g<true>(buf, nh, boff, kt); else stage_b_g<false>(buf, nh, boff, kt);
+  }
+  // the same for a wave group known at compile time (HI: a wave w < HI_WAVES, which issues
+  // AGL A and BGL B blocks per region; else AGL_LO and BGL_LO): the main loop is instantiated per
+  // group, so neither the DMA issue nor the counted waits branch on the wave id inside it
+  template <bool HI>
+  LSA_DEVICE void stage_a_g(int buf, int mh, const unsigned (&aoff)[2][AGL], int kt) {
     unsigned char* dst = smem + buf * BUF + mh * AREG;
     if constexpr (LSA_SK_ABLATE == 6) return;
 #pragma unroll
-    for (int s = 0; s < AGL; ++s) glds16(a_seg, aoff[mh][s], kt * (BK * 2), dst + (w * AGL + s) * 1024);
+    for (int s = 0; s < (HI ? AGL : AGL_LO); ++s) glds16(a_seg, aoff[mh][s], kt * (BK * 2), dst + a_block(s) * 1024);
   }
-  LSA_DEVICE void stage_b(int buf, int nh, const unsigned (&boff)[2][BGL], int kt) {
-    unsigned char* dst = smem + buf * BUF + 2 * AREG + nh * BREG;
-    if constexpr (LSA_SK_ABLATE == 7) return;
-#pragma unroll
-    for (int s = 0; s < BGL; ++s)
-      if (s < BGL_LO || w < BHI_WAVES) glds16_w(b_seg, boff[nh][s], kt * 2048, dst + (s * 8 + w) * 1024);
-  }
-  // the same for a wave group known at compile time (HI: a wave w < BHI_WAVES, which issues
-  // BGL B blocks per region; else BGL_LO): the main loop is instantiated per group, so neither
-  // the DMA issue nor the counted waits branch on the wave id inside it
   template <bool HI>
   LSA_DEVICE void stage_b_g(int buf, int nh, const unsigned (&boff)[2][BGL], int kt) {
     unsigned char* dst = smem + buf * BUF + 2 * AREG + nh * BREG;
     if constexpr (LSA_SK_ABLATE == 7) return;
 #pragma unroll
-    for (int s = 0; s < BGL; ++s)
-      if (s < BGL_LO || HI) glds16_w(b_seg, boff[nh][s], kt * 2048, dst + (s * 8 + w) * 1024);
+    for (int s = 0; s < (HI ? BGL : BGL_LO); ++s) glds16_w(b_seg, boff[nh][s], kt * 2048, dst + (s * 8 + w) * 1024);
   }
   template <bool HI>
   LSA_DEVICE void wait_tile_g() {
@@ -189,7 +192,7 @@ struct Kern {
     if constexpr (NPT == NPT_LO) {
       vm_wait<NPT + EXTRA>();
     } else {
-      if (w < BHI_WAVES) vm_wait<NPT + EXTRA>(); else vm_wait<NPT_LO + EXTRA>();
+      if (w < HI_WAVES) vm_wait<NPT + EXTRA>(); else vm_wait<NPT_LO + EXTRA>();
     }
   }
   // counted wait leaving one A and one B region of this wave's DMA in flight
@@ -197,7 +200,7 @@ struct Kern {
     if constexpr (NPT == NPT_LO) {
       vm_wait<AGL + BGL>();
     } else {
-      if (w < BHI_WAVES) vm_wait<AGL + BGL>(); else vm_wait<AGL + BGL_LO>();
+      if (w < HI_WAVES) vm_wait<AGL + BGL>(); else vm_wait<AGL_LO + BGL_LO>();
     }
   }
 
@@ -219,7 +222,7 @@ struct Kern {
         // block b = 8 whole 128-B rows (full cache lines) of the region's row-major image, rows
         // ordered (wr', i, r16); lane -> row b*8 + lane/8, physical 16-B chunk lane%8 holding
         // logical chunk (lane%8) ^ (row%8) (XOR swizzle: conflict-free fragment reads in rd_a)
-        const int b = w * AGL + s, wi = b >> 1, r16 = (b & 1) * 8 + (lane >> 3);
+        const int b = a_block(s) % ABLK, wi = b >> 1, r16 = (b & 1) * 8 + (lane >> 3);
         const int wr_ = wi / HM, i = wi % HM, ch = (lane & 7) ^ ((lane >> 3) & 7);
         if constexpr (LSA_SK_ABLATE == 5) {  // (pre-swizzle fragment-order gather, half lines)
           const int row = min(m0 + wr_ * TM + mh * (TM / 2) + i * 16 + (lane & 15), P.M - 1) - m0;
@@ -333,12 +336,12 @@ struct Kern {
           mma(0, b0, 0);
           loop_barrier();
           rd_b(cur, 1, b1);
-          if constexpr (S1) { stage_a(nxt, 1, aoff, t + 1); wait_tile_g<HI>(); } else vm_wait<0>();
+          if constexpr (S1) { stage_a_g<HI>(nxt, 1, aoff, t + 1); wait_tile_g<HI>(); } else vm_wait<0>();
           loop_barrier();
           mma(0, b1, 1);
           loop_barrier();
           rd_a(cur, 1);
-          if constexpr (S2) { stage_a(cur, 0, aoff, t + 2); wait_tile_g<HI>(); } else vm_wait<0>();
+          if constexpr (S2) { stage_a_g<HI>(cur, 0, aoff, t + 2); wait_tile_g<HI>(); } else vm_wait<0>();
           loop_barrier();
           mma(1, b1, 1);
           loop_barrier();
@@ -362,7 +365,7 @@ struct Kern {
           constexpr bool ST = decltype(st_c)::value;
           rd_a(cur, 0);
           rd_b(cur, 0, b0);
-          if constexpr (ST) { stage_a(nx2, 0, aoff, t + 2); vm_wait<NPT + 2 * AGL>(); } else vm_wait<0>();
+          if constexpr (ST) { stage_a_g<true>(nx2, 0, aoff, t + 2); vm_wait<NPT + 2 * AGL>(); } else vm_wait<0>();
           loop_barrier();
           mma(0, b0, 0);
           loop_barrier();
@@ -376,7 +379,7 @@ struct Kern {
           loop_barrier();
           mma(1, b1, 1);
           loop_barrier();
-          if constexpr (ST) { stage_a(nx2, 1, aoff, t + 2); vm_wait<NPT + AGL + BGL>(); } else vm_wait<0>();
+          if constexpr (ST) { stage_a_g<true>(nx2, 1, aoff, t + 2); vm_wait<NPT + AGL + BGL>(); } else vm_wait<0>();
           loop_barrier();
           mma(1, b0, 0);
           loop_barrier();
@@ -391,7 +394,7 @@ struct Kern {
     if constexpr (NPT == NPT_LO) {
       main_loop(T_);
     } else {
-      if (w < BHI_WAVES) main_loop(T_); else main_loop(F_);
+      if (w < HI_WAVES) main_loop(T_); else main_loop(F_);
     }
     if (!group) barrier();  // re-align the two wave groups; every LDS read has retired
   }

@@ -266,6 +266,42 @@ def test_gemm_sk_fused_rmsnorm_across_gemms(M, bn, bm, ws):
     assert rel_err(vc[0, :, pl].transpose(0, 1), (xn @ wv.float().T).view(M, nkv, hd)) < 1e-2
 
 
+@pytest.mark.parametrize("bm,bn", [(320, 256), (192, 256), (384, 192), (384, 128)])
+@pytest.mark.parametrize("K", [64, 128, 704])
+def test_gemm_sk_other_heights(bm, bn, K, ws):
+    """Tiles of 192, 320 and 384 rows: their edges, one K step to several, whole, in equal splits and by stream-K, every kind of
+    store (fp32 columns beside bf16 ones and alone), the gated unit and the fused norm's sums."""
+    h = hip()
+    N = 768
+    for M in (1, bm - 1, bm, bm + 1, 2 * bm + 17):
+        a, w, r = _rnd(M, K), _rnd(N, K, scale=0.05), _rnd(M, N)
+        ref = a.float() @ w.float().T
+        wp = packing.pack_b(w)
+        tiles = -(-M // bm) * -(-N // bn)
+        for split in {0, 1, min(3, K // 64)}:
+            kw = dict(bm=bm, bn=bn, grid=max(256, tiles), split=split, ws=ws)
+            out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+            h.gemm_sk(a, wp, M, N, K, h.EPI_STORE, h.make_epi(out=out, ldo=N), **kw)
+            assert rel_err(out, ref) < 8e-3, (M, split)
+            o32 = torch.full((M, N), float("nan"), device=DEV)
+            bias = torch.randn(N, device=DEV)
+            h.gemm_sk(a, wp, M, N, K, h.EPI_STORE, h.make_epi(out32=o32, ldo=N, bias=bias), **kw)
+            assert rel_err(o32, ref + bias) < 1e-5, (M, split)  # sums of K products of bf16, rounded in fp32
+            out, o32 = torch.zeros(M, 272, dtype=torch.bfloat16, device=DEV), torch.zeros(M, N - 272, device=DEV)
+            h.gemm_sk(a, wp, M, N, K, h.EPI_STORE, h.make_epi(out=out, ldo=272, out32=o32, col32=272, ldo32=N - 272), **kw)
+            assert rel_err(out, ref[:, :272]) < 8e-3 and rel_err(o32, ref[:, 272:]) < 1e-5, (M, split)
+            out = torch.zeros(M, N // 2, dtype=torch.bfloat16, device=DEV)
+            h.gemm_sk(a, wp, M, N, K, h.EPI_SWIGLU, h.make_epi(out=out, ldo=N // 2), **kw)
+            u = ref.view(M, N // 32, 2, 16)
+            assert rel_err(out, (F.silu(u[:, :, 0]) * u[:, :, 1]).reshape(M, -1)) < 1e-2, (M, split)
+            hb, ss = r.clone(), torch.full((M, N // 64), float("nan"), device=DEV) if bn != 192 else None
+            h.gemm_sk(a, wp, M, N, K, h.EPI_RESID, h.make_epi(out=hb, resid=hb, ldo=N, ldr=N, ss_out=ss), **kw)
+            assert rel_err(hb, r.float() + ref) < 8e-3, (M, split)
+            if ss is not None:
+                assert rel_err(ss, hb.float().pow(2).view(M, N // 64, 64).sum(-1)) < 1e-5, (M, split)
+    assert int(ws.counters.abs().sum()) == 0
+
+
 @pytest.mark.parametrize("name,N,K,epi", [("qkv", 10240, 8192, "store"), ("o", 8192, 8192, "resid"),
                                           ("gate_up", 57344, 8192, "swiglu"), ("down", 8192, 28672, "resid")])
 def test_gemm_llama70b_projections_at_512_rows(name, N, K, epi):
