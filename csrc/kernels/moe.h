@@ -9,7 +9,17 @@
 #include "elem.h"
 
 struct MoeTile {  // pairs [start, start + count) of the sorted list, all of one expert; expert < 0: none (after all others)
-  int expert, start, count, used;  // used: how many of the table's tiles there are, in each of them
+  int expert, start, count, used;  // used: how many of the table's tiles there are, in each of them; from MOE_HEIGHT on: MoePick
+};
+constexpr int MOE_HEIGHT = 24;
+
+// Tiles of the height, of these four, whose rounds on 256 CUs take least in both products, chosen when the experts' pairs are
+// counted. nt: columns of tiles of a product; step, own: us of a round's K steps, of its start and end. nt[0] = 0: the height is given.
+// Mirrored by llm_sharding_amd/ops/moe.py::Pick.
+constexpr int MOE_ROWS[4] = {128, 192, 256, 320};
+struct MoePick {
+  int nt[2];
+  float step[4][2], own[4];
 };
 
 // How experts are chosen. Mirrored by llm_sharding_amd/ops/moe.py::RouteArgs.

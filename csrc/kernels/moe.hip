@@ -124,13 +124,46 @@ LSA_DEVICE MoeSpan expert_spans(int c, int nt, int (*s_w)[16], int* s_n) {
   return MoeSpan{ba + a - c, bb + b - nt, *s_n};
 }
 // the tile table: expert tid's tiles, and the rest of the table
-LSA_DEVICE void write_tiles(MoeTile* __restrict__ tiles, const MoeSpan& sp, int E, int c, int nt, int tile_rows, int max_tiles) {
-  const int tid = threadIdx.x;
+LSA_DEVICE void write_tiles(MoeTile* __restrict__ tiles, const MoeSpan& sp, int E, int c, int nt, int tile_rows, int h, int max_tiles) {
+  const int tid = threadIdx.x, used = sp.used | h << MOE_HEIGHT;
   if (tid < E)
     for (int t = 0; t < nt; ++t)
       if (sp.tiles + t < max_tiles)
-        tiles[sp.tiles + t] = MoeTile{tid, sp.pairs + t * tile_rows, min(tile_rows, c - t * tile_rows), sp.used};
-  for (int t = sp.used + tid; t < max_tiles; t += 1024) tiles[t] = MoeTile{-1, 0, 0, sp.used};
+        tiles[sp.tiles + t] = MoeTile{tid, sp.pairs + t * tile_rows, min(tile_rows, c - t * tile_rows), used};
+  for (int t = sp.used + tid; t < max_tiles; t += 1024) tiles[t] = MoeTile{-1, 0, 0, used};
+}
+// The height of the tiles (MoePick), thread tid with expert tid's pairs c; tile_rows becomes it. CUs without a tile in the last
+// round leave the others more of the clock (ops/hip.py gemm_sk_cost).
+LSA_DEVICE int pick_height(const MoePick& pick, int c, int& tile_rows, int (*s_w)[16]) {
+  if (!pick.nt[0]) return 0;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int n[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) n[i] = wave_sum((c + MOE_ROWS[i] - 1) / MOE_ROWS[i]);
+  if (lane < 4) s_w[lane][w] = lane & 2 ? (lane & 1 ? n[3] : n[2]) : (lane & 1 ? n[1] : n[0]);
+  __syncthreads();
+  int h = 0;
+  float best = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int all = 0;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) all += s_w[i][x];
+    float us = 0.f;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int tiles = all * pick.nt[p], rem = tiles & 255;
+      us += (float)(tiles >> 8) * (pick.step[i][p] + pick.own[i]);
+      us += rem ? pick.step[i][p] * (1.f - 0.47f * (1.f - (float)rem / 256.f)) + pick.own[i] : 0.f;
+    }
+    if (i == 0 || us < best) {
+      best = us;
+      h = i;
+    }
+  }
+  tile_rows = h & 2 ? (h & 1 ? MOE_ROWS[3] : MOE_ROWS[2]) : (h & 1 ? MOE_ROWS[1] : MOE_ROWS[0]);
+  __syncthreads();  // s_w is read
+  return h;
 }
 
 // One workgroup: counting sort of the pairs by expert, and the tile table. NE > 0: few rows, whose routing
@@ -138,9 +171,9 @@ LSA_DEVICE void write_tiles(MoeTile* __restrict__ tiles, const MoeSpan& sp, int 
 template <int NE>
 __global__ __launch_bounds__(1024) void group_kernel(RouteArgs ra, const float* __restrict__ logits, int ldl, int top,
                                                      float* __restrict__ weight, int* expert, int pairs, int E,
-                                                     int tile_rows, int max_tiles, int* __restrict__ order,
+                                                     int tile_rows, MoePick pick, int max_tiles, int* __restrict__ order,
                                                      int* __restrict__ place, MoeTile* __restrict__ tiles) {
-  __shared__ int s_cnt[MAX_E], s_off[MAX_E], s_n[1], s_w[2][16];
+  __shared__ int s_cnt[MAX_E], s_off[MAX_E], s_n[1], s_w[4][16];
   const int tid = threadIdx.x;
   s_cnt[tid] = 0;
   if constexpr (NE > 0) {
@@ -161,11 +194,11 @@ __global__ __launch_bounds__(1024) void group_kernel(RouteArgs ra, const float* 
       if (i0 + u * 1024 < pairs) place[i0 + u * 1024] = atomicAdd(&s_cnt[e[u]], 1);  // rank within its expert
   }
   __syncthreads();
-  const int c = tid < E ? s_cnt[tid] : 0, nt = (c + tile_rows - 1) / tile_rows;
+  const int c = tid < E ? s_cnt[tid] : 0, hi = pick_height(pick, c, tile_rows, s_w), nt = (c + tile_rows - 1) / tile_rows;
   const MoeSpan sp = expert_spans(c, nt, s_w, s_n);
   s_off[tid] = sp.pairs;
   __syncthreads();
-  write_tiles(tiles, sp, E, c, nt, tile_rows, max_tiles);
+  write_tiles(tiles, sp, E, c, nt, tile_rows, hi, max_tiles);
   for (int i0 = tid; i0 < pairs; i0 += 1024 * U) {
     int e[U], rank[U];  // this thread's own ranks
 #pragma unroll
@@ -203,10 +236,10 @@ __global__ __launch_bounds__(1024) void count_kernel(const int* __restrict__ exp
   __syncthreads();
   if (tid < E) counts[(size_t)blockIdx.x * E + tid] = s_cnt[tid];
 }
-__global__ __launch_bounds__(1024) void place_kernel(const int* __restrict__ expert, int pairs, int E, int tile_rows, int max_tiles,
-                                                     int* __restrict__ order, int* __restrict__ place,
+__global__ __launch_bounds__(1024) void place_kernel(const int* __restrict__ expert, int pairs, int E, int tile_rows, MoePick pick,
+                                                     int max_tiles, int* __restrict__ order, int* __restrict__ place,
                                                      const int* __restrict__ counts, MoeTile* __restrict__ tiles) {
-  __shared__ int s_all[MAX_E], s_before[MAX_E], s_n[1], s_w[2][16];
+  __shared__ int s_all[MAX_E], s_before[MAX_E], s_n[1], s_w[4][16];
   const int tid = threadIdx.x, i0 = blockIdx.x * GROUP_PAIRS + tid, i1 = i0 + 1024;
   const int j0 = min(i0, pairs - 1), j1 = min(i1, pairs - 1);
   const int e0 = expert[j0], e1 = expert[j1], r0 = place[j0], r1 = place[j1];
@@ -219,11 +252,12 @@ __global__ __launch_bounds__(1024) void place_kernel(const int* __restrict__ exp
     if (i < mine) atomicAdd(&s_before[e], c);
   }
   __syncthreads();
-  const int c = tid < E ? s_all[tid] : 0, nt = (c + tile_rows - 1) / tile_rows;
+  const int c = tid < E ? s_all[tid] : 0, hi = blockIdx.x == 0 ? pick_height(pick, c, tile_rows, s_w) : 0;  // (it writes the tiles)
+  const int nt = (c + tile_rows - 1) / tile_rows;
   const MoeSpan sp = expert_spans(c, nt, s_w, s_n);
   s_before[tid] += sp.pairs;
   __syncthreads();
-  if (blockIdx.x == 0) write_tiles(tiles, sp, E, c, nt, tile_rows, max_tiles);
+  if (blockIdx.x == 0) write_tiles(tiles, sp, E, c, nt, tile_rows, hi, max_tiles);
   if (i0 < pairs) {
     const int at = s_before[e0] + r0;
     place[i0] = at;
@@ -434,21 +468,26 @@ extern "C" int lsa_moe_route(const RouteArgs* ra, const float* logits, int ldl, 
   return LSA_OK;
 }
 
-// max_tiles >= min(E, pairs) + pairs / tile_rows; counts: n_counts ints of scratch, or none
+// max_tiles >= min(E, pairs) + pairs / tile_rows; counts: n_counts ints of scratch, or none; heights: tiles of the height that the
+// pairs make best (tile_rows: the lowest, 128), or null
 extern "C" int lsa_moe_group(const int* expert, int pairs, int E, int tile_rows, int max_tiles, int* order, int* place,
-                             void* tiles, int* counts, int n_counts, hipStream_t s) {
+                             void* tiles, int* counts, int n_counts, const MoePick* heights, hipStream_t s) {
   if (pairs < 1 || E < 1 || E > MAX_E || tile_rows < 1 || max_tiles < (E < pairs ? E : pairs) + pairs / tile_rows ||
       (!counts && n_counts))
+    return LSA_BAD_SHAPE;
+  const MoePick pick = heights ? *heights : MoePick{};
+  if (heights && (tile_rows != MOE_ROWS[0] || max_tiles >= 1 << MOE_HEIGHT || pick.nt[0] < 1 || pick.nt[1] < 1 ||
+                  pick.nt[0] > 4096 || pick.nt[1] > 4096 || (long long)max_tiles * 4096 >= 1ll << 31))
     return LSA_BAD_SHAPE;
   const int wg = (pairs + GROUP_PAIRS - 1) / GROUP_PAIRS;
   if (pairs >= GROUP_MANY && (long long)wg * E <= n_counts) {
     count_kernel<<<wg, 1024, 0, s>>>(expert, pairs, E, place, counts);
-    place_kernel<<<wg, 1024, 0, s>>>(expert, pairs, E, tile_rows, max_tiles, order, place, counts, (MoeTile*)tiles);
+    place_kernel<<<wg, 1024, 0, s>>>(expert, pairs, E, tile_rows, pick, max_tiles, order, place, counts, (MoeTile*)tiles);
     LSA_CHECK_LAUNCH();
     return LSA_OK;
   }
   group_kernel<0><<<1, 1024, 0, s>>>(RouteArgs{}, nullptr, 0, 1, nullptr, const_cast<int*>(expert), pairs, E, tile_rows,
-                                     max_tiles, order, place, (MoeTile*)tiles);
+                                     pick, max_tiles, order, place, (MoeTile*)tiles);
   LSA_CHECK_LAUNCH();
   return LSA_OK;
 }
@@ -463,7 +502,7 @@ extern "C" int lsa_moe_route_group(const RouteArgs* ra, const float* logits, int
     return LSA_BAD_SHAPE;
   const size_t lds = (size_t)16 * (E + ra->groups) * 4;
 #define LSA_RG(NE)                                                                                                  \
-  group_kernel<NE><<<1, 1024, lds, s>>>(*ra, logits, ldl, top, weight, expert, pairs, E, tile_rows, max_tiles, order, \
+  group_kernel<NE><<<1, 1024, lds, s>>>(*ra, logits, ldl, top, weight, expert, pairs, E, tile_rows, MoePick{}, max_tiles, order, \
                                         place, (MoeTile*)tiles)
   if (E <= 64) LSA_RG(1);
   else LSA_RG(4);

@@ -5,6 +5,7 @@ stream, nothing falls back to another implementation."""
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional
 
 import torch
@@ -25,6 +26,27 @@ DOWN, GLU, RELU2 = 0, 1, 2  # MoeUp in csrc/kernels/moe.h
 class RouteArgs(ctypes.Structure):
     _fields_ = [("correction", ctypes.c_void_p), ("sigmoid", ctypes.c_int), ("groups", ctypes.c_int), ("keep", ctypes.c_int),
                 ("scale", ctypes.c_float)]
+
+
+class Pick(ctypes.Structure):  # csrc/kernels/moe.h MoePick
+    _fields_ = [("nt", ctypes.c_int * 2), ("step", (ctypes.c_float * 2) * 4), ("own", ctypes.c_float * 4)]
+
+
+HEIGHTS = (128, 192, 256, 320)  # of the bf16 kernel's tiles of 256 columns (MOE_ROWS)
+
+
+@functools.lru_cache(maxsize=256)
+def pick(*products) -> Optional[Pick]:
+    """What :func:`group` chooses a height from for both of the experts' products [(columns, k)]: the projection GEMM's costs of a
+    round of such tiles, a little more for low ones (they read an expert's weights more often); None: not for these."""
+    if any(n % 256 or k % 64 for n, k in products):
+        return None
+    p = Pick(tuple(n // 256 for n, _ in products))
+    for i, (h, more) in enumerate(zip(HEIGHTS, (1.06, 1.03, 1.0, 1.0))):
+        step, own = hip.SK_COST[(h, 256)]
+        p.step[i] = tuple(more * (k // 64 * step) for _, k in products)
+        p.own[i] = more * own
+    return p
 
 
 def route_args(s=None, correction=None) -> RouteArgs:
@@ -95,25 +117,26 @@ def route(logits, rows: int, experts: int, top: int, expert, weight, how: Option
            "lsa_moe_route")
 
 
-def group(expert, pairs: int, experts: int, rows: int, order, place, tiles, spare=None) -> int:
+def group(expert, pairs: int, experts: int, rows: int, order, place, tiles, spare=None, heights: Optional[Pick] = None) -> int:
     """Pairs sorted by expert (``order``; ``place`` is its inverse) and their tiles; returns the table's length. ``spare``: int32
-    scratch, as long as the pairs, that lets many of them have several workgroups."""
+    scratch, as long as the pairs, that lets many of them have several workgroups. ``heights`` (:func:`pick`): the tiles are as high
+    as the pairs make best, ``rows`` is the lowest; for :func:`gemm` with ``rows`` 0."""
     n = max_tiles(pairs, experts, rows)
     _req(all(t.dtype == torch.int32 for t in (expert, order, place, tiles)) and tiles.numel() >= 4 * n
          and min(expert.numel(), order.numel(), place.numel()) >= pairs, "group: shapes")
     _req(spare is None or (spare.dtype == torch.int32 and spare.is_contiguous()), "group: scratch")
     _check(lib().lsa_moe_group(_p(expert), pairs, experts, rows, n, _p(order), _p(place), _p(tiles), _p(spare),
-                               0 if spare is None else spare.numel(), _stream()), "lsa_moe_group")
+                               0 if spare is None else spare.numel(), heights, _stream()), "lsa_moe_group")
     return n
 
 
 def route_group(logits, rows: int, experts: int, top: int, tile: int, expert, weight, order, place, tiles,
-                how: Optional[RouteArgs] = None, spare=None) -> int:
-    """:func:`route` and :func:`group`, in one launch where there are few rows."""
+                how: Optional[RouteArgs] = None, spare=None, heights: Optional[Pick] = None) -> int:
+    """:func:`route` and :func:`group`, in one launch where there are few rows (and the height is given)."""
     pairs, how = rows * top, how or route_args()
-    if rows > 16 or experts > 256:
+    if rows > 16 or experts > 256 or heights is not None:
         route(logits, rows, experts, top, expert, weight, how)
-        return group(expert, pairs, experts, tile, order, place, tiles, spare)
+        return group(expert, pairs, experts, tile, order, place, tiles, spare, heights)
     n = max_tiles(pairs, experts, tile)
     _req(logits.dtype == torch.float32 and logits.stride(1) == 1 and logits.shape[0] >= rows
          and logits.shape[1] >= experts and weight.dtype == torch.float32 and weight.numel() >= pairs, "route: shapes")
@@ -126,13 +149,13 @@ def route_group(logits, rows: int, experts: int, top: int, tile: int, expert, we
 
 def gemm(tiles, n_tiles: int, rows: int, order, top: int, a, w, n: int, k: int, out, pairs: int, up: int) -> None:
     """One product of every tile's expert: ``up`` (GLU / RELU2) from rows of h (``a``) to out [pairs, n / 2 or n], or
-    DOWN from the sorted pairs (``a`` [pairs, k]) to out [pairs, n]."""
+    DOWN from the sorted pairs (``a`` [pairs, k]) to out [pairs, n]. ``rows`` 0: tiles of the height that :func:`group` chose."""
     _req(a.dtype == w.dtype == out.dtype and a.stride(1) == 1 and a.shape[1] >= k and out.stride(1) == 1
          and out.shape[0] >= pairs and out.shape[1] >= (n // 2 if up == GLU else n) and order.numel() >= pairs
          and (a.shape[0] * top >= pairs if up else a.shape[0] >= pairs), "moe: shapes")
     _req(w[0].numel() == n * k and w.is_contiguous(), "moe: weights")
     f32 = is_f32(a.dtype)
-    if rows > 64 and not f32:
+    if (rows > 64 or not rows) and not f32:
         _check(lib().lsa_moe_gemm_big(up, _p(tiles), n_tiles, rows, _p(order), top, _p(a), a.shape[0] if up else 0,
                                       a.stride(0), _p(w), n, k, _p(out), out.stride(0), _stream()), "lsa_moe_gemm_big")
         return
@@ -146,7 +169,7 @@ def declare(L: ctypes.CDLL) -> None:
     vp, i, ra = ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(RouteArgs)
     hip.set_signatures(L, {
         "lsa_moe_route": [ra, vp, i, i, i, i, vp, vp, vp],
-        "lsa_moe_group": [vp, i, i, i, i, vp, vp, vp, vp, i, vp],
+        "lsa_moe_group": [vp, i, i, i, i, vp, vp, vp, vp, i, ctypes.POINTER(Pick), vp],
         "lsa_moe_route_group": [ra, vp, i, i, i, i, vp, vp, i, i, vp, vp, vp, vp],
         "lsa_moe_gemm_big": [i, vp, i, i, vp, i, vp, i, i, vp, i, i, vp, i, vp],
         "lsa_moe_gemm": [i, i, vp, i, i, i, vp, i, vp, i, vp, i, i, vp, i, vp],

@@ -143,8 +143,10 @@ class Moe:
         weight, tiles = eng.scratch_view("pair_w", rows, s.top).reshape(-1), eng.scratch_view("tiles", rows, 8 * s.top)
         act, ye = eng.scratch_view("act", pairs, x.ff), eng.scratch_view("ye", pairs, x.width)
         tr = X.tile_rows(pairs, s.experts, x.f32, min(x.up_n, x.width))
-        nt = X.route_group(in32[:, col["router"]:], rows, s.experts, s.top, tr, expert, weight, order, place, tiles,
-                           self.how, spare)
+        heights = X.pick((x.up_n, x.width), (x.width, x.ff)) if tr >= 128 and not x.f32 else None
+        nt = X.route_group(in32[:, col["router"]:], rows, s.experts, s.top, tr if heights is None else X.HEIGHTS[0], expert, weight,
+                           order, place, tiles, self.how, spare, heights)
+        tr = tr if heights is None else 0
         X.gemm(tiles, nt, tr, order, s.top, h, x.up, x.up_n, x.width, act, pairs, x.kind)
         X.gemm(tiles, nt, tr, order, s.top, act, x.down, x.width, x.ff, ye, pairs, X.DOWN)
         out = {"experts": (ye, weight, place, s.top)}

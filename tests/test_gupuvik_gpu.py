@@ -728,6 +728,57 @@ def test_experts_share_out_the_tiles_there_are(pairs, experts, rows):
     assert torch.equal(*outs) and bool((outs[0].abs().sum(1) > 0).all())
 
 
+# pairs of each expert; on which tiles have the fewest rounds: a few rows over a tile's, one below, none, one expert for all
+DEALS = [[129] * 8, [193] * 40 + [0, 1], [257, 256, 255, 0, 1], [321, 320, 319] * 20, [640] * 16, [5000], [1] * 7 + [700], [797] * 32]
+
+
+@pytest.mark.parametrize("deal", range(len(DEALS)))
+@pytest.mark.parametrize("up", ["glu", "relu2"])
+def test_experts_tiles_of_the_height_that_the_pairs_make_best(deal, up):
+    """The height is the cheapest by the costs given, the table that of this height, and both products give what tiles of 128 and 256
+    rows give, bit for bit (a pair's sums run in the same order)."""
+    from llm_sharding_amd.ops import moe as X
+    from llm_sharding_amd.ops.packing import pack_b
+    counts = torch.tensor(DEALS[deal])
+    experts, pairs = len(counts), int(counts.sum())
+    g = torch.Generator().manual_seed(deal)
+    e = torch.repeat_interleave(torch.arange(experts), counts)[torch.randperm(pairs, generator=g)].int()
+    kind, n, k = (X.GLU, 512, 192) if up == "glu" else (X.RELU2, 256, 192)
+    width, ff = 256, n // 2 if up == "glu" else n
+    assert X.pick((n + 128, k), (width, ff)) is None
+    heights = X.pick((n, k), (width, ff))
+
+    def us(i):
+        total = 0.0
+        for p in range(2):
+            tiles = int(((counts + X.HEIGHTS[i] - 1) // X.HEIGHTS[i]).sum()) * heights.nt[p]
+            full, rem = divmod(tiles, 256)
+            last = heights.step[i][p] * (1 - 0.47 * (1 - rem / 256)) + heights.own[i] if rem else 0.0
+            total += full * (heights.step[i][p] + heights.own[i]) + last
+        return total
+    cost = [us(i) for i in range(4)]
+    wu = torch.stack([pack_b(_rand(n, k, seed=i, scale=k ** -0.5).to(DEV)) for i in range(experts)])
+    wd = torch.stack([pack_b(_rand(width, ff, seed=i + 99, scale=ff ** -0.5).to(DEV)) for i in range(experts)])
+    h = _rand(pairs, k, seed=7).to(DEV)
+    for spare in (None, torch.zeros(pairs + 1024, dtype=torch.int32, device=DEV)):
+        order, place = (torch.empty(pairs, dtype=torch.int32, device=DEV) for _ in range(2))
+        outs = []
+        for rows in (0, 128, 256):
+            tiles = torch.full((X.max_tiles(pairs, experts, rows or 128), 4), -7, dtype=torch.int32, device=DEV)
+            nt = X.group(e.to(DEV), pairs, experts, rows or 128, order, place, tiles, spare, None if rows else heights)
+            if not rows:
+                i, used = divmod(int(tiles[0, 3]), 1 << 24)
+                assert cost[i] <= min(cost) * (1 + 1e-5), (i, cost)
+                assert used == int(((counts + X.HEIGHTS[i] - 1) // X.HEIGHTS[i]).sum()) and bool((tiles[used:, 0] == -1).all())
+                assert int(tiles[:used, 2].max()) <= X.HEIGHTS[i] and int(tiles[:used, 2].sum()) == pairs
+            act, ye = (torch.full((pairs, c), float("nan"), dtype=BF, device=DEV) for c in (ff, width))
+            X.gemm(tiles, nt, rows, order, 1, h, wu, n, k, act, pairs, kind)
+            X.gemm(tiles, nt, rows, order, 1, act, wd, width, ff, ye, pairs, X.DOWN)
+            outs.append((act[place.long()], ye[place.long()]))  # (the order within an expert is not the same every time)
+        for a, y in outs[1:]:
+            assert torch.equal(a, outs[0][0]) and torch.equal(y, outs[0][1])
+
+
 @pytest.mark.parametrize("pairs", [10239, 10240, 12287, 12288, 12289, 40961])
 @pytest.mark.parametrize("experts", [1, 7, 32, 1024])
 def test_many_pairs_are_sorted_by_several_workgroups(pairs, experts):
