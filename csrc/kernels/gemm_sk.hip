@@ -105,7 +105,9 @@ __global__ __launch_bounds__(NTHR) void gemm_sk_kernel(const bf16_raw* __restric
     int mt, nt;
     tile_coords(prm, tile, mt, nt);
     zero();
-    k.run_segment(acc, mt * BM, nt, ka, kb);
+    k.run_segment(acc, mt * BM, nt, ka, kb, [&]() {
+      if (K_::SS_IN && ep.ss_in) k.row_scales(ep, mt * BM);
+    });
     LSA_STAMP(k.stamp_base + 2);
     bool do_epi = true;
     if (partial && EPI != EPI_PARTIAL) {
@@ -201,7 +203,7 @@ extern "C" int lsa_gemm_sk(const void* a, int lda, const void* wp, int M, int N,
   if (bn != 256 && bn != 192 && bn != 128) return LSA_UNSUPPORTED;
   if (bm != 256 && bm != 128 && !((bm == 320 || bm == 192) && bn == 256) && !(bm == 384 && bn != 256)) return LSA_UNSUPPORTED;
   const int BM = bm;
-  const bool three = bm <= 256 && bn == 128 || (bm == 128 && bn == 256);
+  const bool three = (bm <= 256 && bn == 128) || (bm == 128 && bn == 256);
   if (nb == 0) nb = three ? 3 : 2;
   if (nb != 2 && !(nb == 3 && three)) return LSA_UNSUPPORTED;
   if (bn == 192 ? (N % 16 || (epi_gated(epi) && N % 32)) : N % bn) return LSA_BAD_SHAPE;

@@ -205,8 +205,10 @@ struct Kern {
   }
 
   // ---- one segment: K-tiles [ka, kb) of output tile (mt, nt), accumulated into acc -------------
+  // meanwhile(): run while the first DMA is on its way
   int stamp_base = 0;
-  LSA_DEVICE void run_segment(f32x4_t (&acc)[FM][FN], int m0, int nt, int ka, int kb) {
+  template <typename F>
+  LSA_DEVICE void run_segment(f32x4_t (&acc)[FM][FN], int m0, int nt, int ka, int kb, F meanwhile) {
     LSA_STAMP(stamp_base + 0);
     const SkParams& P = *p;
     const int n = kb - ka;
@@ -257,10 +259,11 @@ struct Kern {
       if (NB == 3) {
         stage_b(1, 1, boff, 1);
         stage_a(1, 1, aoff, 1);
-        vm_wait<BGL + AGL + NPT>();
-      } else {
-        wait_tile();
       }
+    }
+    meanwhile();  // (what it loads comes after the DMA: waits for it are longer than what follows asks)
+    if (n > 1) {
+      if (NB == 3) vm_wait<BGL + AGL + NPT>(); else wait_tile();
     } else {
       wait_ab();
     }
@@ -476,38 +479,42 @@ struct Kern {
     }
   }
 
+  // fused RMSNorm: the rstd of each of the tile's BM rows from the producer's 64-column partials, computed
+  // ONCE per workgroup (one thread per row, all of its partials' loads in flight) and summed in the same
+  // order as before (bitwise-identical rstd). Before, every wave column recomputed its rows' rstd per
+  // pass: 4x the partials traffic, +23 us on a 2048-row gate_up (scripts/epi_cost_probe.py). Made while the
+  // tile's first DMA is on its way and not behind its last product, where nothing hid its loads: five
+  // 3072-wide prompts of 301 tokens 1250 -> 1236 us, four 4096-wide ones of 2048 10673 -> 10619. (One copy
+  // of it: with a second one in the epilogue the main loop's registers are laid out worse, 0.7 % the other way.)
+  static constexpr bool SS_IN = EPI == EPI_QKV || EPI == EPI_SWIGLU;
+  LSA_DEVICE void row_scales(const EpiArgs& ep, int m0) {
+    const int tid = fresh(this->tid);
+    float* s_rs = reinterpret_cast<float*>(smem + G_::RS_OFF);
+    for (int r = tid; r < BM; r += NTHR) {
+      const int m = min(m0 + r, p->M - 1);
+      const float* sp = ep.ss_in + (size_t)m * ep.ss_n;
+      float t = 0.f;
+      for (int i0 = 0; i0 < ep.ss_n; i0 += 64) {
+        f32x4_t q4[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          q4[j] = i0 + 4 * j < ep.ss_n ? *reinterpret_cast<const f32x4_t*>(sp + i0 + 4 * j)
+                                        : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          if (i0 + 4 * j < ep.ss_n) t += (q4[j][0] + q4[j][1]) + (q4[j][2] + q4[j][3]);
+      }
+      s_rs[r] = rsqrtf(t / (float)(64 * ep.ss_n) + ep.ss_eps);
+    }
+  }
+
   // ---- fused epilogue through an LDS transpose -------------------------------------------------
   LSA_DEVICE void epilogue(const EpiArgs& ep, const f32x4_t (&acc)[FM][FN], int m0, int nt, int sp) {
-    const int lane = fresh(this->lane), tid = fresh(this->tid);
+    const int lane = fresh(this->lane);
     const SkParams& P = *p;
     constexpr int EROWS = G_::EROWS, ELD = G_::ELD, FPP = EROWS / 16;  // rows / fragments per pass
     float* img = reinterpret_cast<float*>(smem) + w * (EROWS * ELD);
-    // fused RMSNorm: the rstd of each of the tile's BM rows from the producer's 64-column
-    // partials, computed ONCE per workgroup (one thread per row, all of its partials' loads in
-    // flight) and summed in the same order as before (bitwise-identical rstd). Before, every
-    // wave column recomputed its rows' rstd per pass: 4x the partials traffic, +23 us on a
-    // 2048-row gate_up (scripts/epi_cost_probe.py)
-    float* s_rs = reinterpret_cast<float*>(smem + G_::RS_OFF);
-    constexpr bool SS_IN = EPI == EPI_QKV || EPI == EPI_SWIGLU;
-    if (SS_IN && ep.ss_in) {
-      for (int r = tid; r < BM; r += NTHR) {
-        const int m = min(m0 + r, P.M - 1);
-        const float* sp = ep.ss_in + (size_t)m * ep.ss_n;
-        float t = 0.f;
-        for (int i0 = 0; i0 < ep.ss_n; i0 += 64) {
-          f32x4_t q4[16];
-#pragma unroll
-          for (int j = 0; j < 16; ++j)
-            q4[j] = i0 + 4 * j < ep.ss_n ? *reinterpret_cast<const f32x4_t*>(sp + i0 + 4 * j)
-                                          : f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int j = 0; j < 16; ++j)
-            if (i0 + 4 * j < ep.ss_n) t += (q4[j][0] + q4[j][1]) + (q4[j][2] + q4[j][3]);
-        }
-        s_rs[r] = rsqrtf(t / (float)(64 * ep.ss_n) + ep.ss_eps);
-      }
-      __syncthreads();
-    }
+    const float* s_rs = reinterpret_cast<const float*>(smem + G_::RS_OFF);
     constexpr int PASSES = TM / EROWS;
 #pragma unroll
     for (int ps = 0; ps < PASSES; ++ps) {

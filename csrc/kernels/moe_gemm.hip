@@ -34,7 +34,7 @@ LSA_DEVICE void moe_tile(unsigned char* smem, const MoeTile* __restrict__ tiles,
   for (int i = 0; i < K_::FM; ++i)
 #pragma unroll
     for (int j = 0; j < K_::FN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  k.run_segment(acc, tile.start, nt, 0, prm.NKT);
+  k.run_segment(acc, tile.start, nt, 0, prm.NKT, []() {});
   k.epilogue(ep, acc, tile.start, nt, 0);
 }
 
