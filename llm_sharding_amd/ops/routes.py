@@ -56,12 +56,11 @@ ROUTES = (
     Route(15360, 5120, 320, 384, "gemm_wr", {"bn": 192}, _WR_EPIS, "profiles/r4_gemm_wr_shapes.jsonl"),
     Route(15360, 5120, 448, 512, "gemm_wr", {"bn": 256}, _WR_EPIS, "profiles/r4_gemm_wr_shapes.jsonl"),
     # Llama-3.2-3B qkv and gate_up (SwiGLU epilogue)
-    Route(5120, 3072, 193, 512, "gemm_wr", {"bn": 128}, _WR_EPIS, "profiles/r4_gemm_wr_engine_ab.txt"),
+    # (up to 384 rows gemm_sk is faster since: 256 rows 22.9 us beside 29.9, 384 26.0 and 29.7; 448 30.5 and 25.9)
+    Route(5120, 3072, 385, 512, "gemm_wr", {"bn": 128}, _WR_EPIS, "profiles/r4_gemm_wr_engine_ab.txt"),
     Route(16384, 3072, 193, 256, "gemm_wr", {"bn": 128}, _WR_EPIS, "profiles/r4_gemm_wr_engine_ab.txt"),
     Route(16384, 3072, 320, 512, "gemm_wr", {"bn": 256}, _WR_EPIS, "profiles/r4_gemm_wr_engine_ab.txt"),
-    # 7B / 13B gate_up at 193-256 rows
-    Route(22016, 4096, 193, 256, "gemm_wr", {"bn": 256}, _WR_EPIS, "profiles/r4_gemm_wr_shapes.jsonl"),
-    Route(27648, 5120, 193, 256, "gemm_wr", {"bn": 256}, _WR_EPIS, "profiles/r4_gemm_wr_shapes.jsonl"),
+    # (7B / 13B gate_up at 193-256 rows had one until gemm_sk was faster: 256 rows 61 us beside 65, 86 and 94)
     # ---- the MFMA GEMMs below the GEMV limit: Llama-2-13B's 65-128-row decode (-4.6..5.6 % per
     # step on three boxes); the 7B (+6 %), 3B (+65 %) and 70B stage (+6-10 %) measured slower there
     Route(15360, 5120, 65, 128, "gemm_sk", {}, (), "profiles/r5_gemv_max_rows_ab.md"),
