@@ -312,91 +312,118 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(DeltaArgs a, const Del
   }
 }
 
-LSA_DEVICE void glds16(const void* src, unsigned char* lds_base) {
-  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)lds_base, 16, 0, 0);
+LSA_DEVICE __amdgpu_buffer_rsrc_t bytes_of(const void* p, int n) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, n, 0x00020000);
+}
+LSA_DEVICE void glds16(__amdgpu_buffer_rsrc_t src, int off, unsigned char* lds_base) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)lds_base, 16, off, 0, 0, 0);
 }
 
 // One workgroup per (run, head, NW 16 value channels): the state in registers (a wave has 16 channels of it), a
-// chunk's operands by LDS-DMA into a double buffer. Leaves the read-outs in fp32 for delta_norm_kernel.
+// chunk's operands by LDS-DMA two chunks ahead. Leaves the read-outs in fp32 for delta_norm_kernel.
+//
+// A chunk is one serial chain (operands from LDS, W S, u, the state's own products) on a CU that one workgroup fills.
+// Where a head has 64 keys or more they are halved between two waves for each 16 channels, which exchange their W S
+// and half of their read-outs through LDS; and the channels lie with as many workgroups as there are CUs (lsa_delta_chunked),
+// so that a CU reads the operands out of LDS for fewer waves. Three runs of 34 chunks, 16 heads of 128 x 128: 93 us with
+// all keys in a wave, 84 halved (96 workgroups), 65 with half of the channels each (192); 50 of them stay without the DMA.
 template <int DK, int DV, int NW>
-__global__ __launch_bounds__(NW * 64) void delta_scan_kernel(DeltaArgs a, const DeltaSpan* __restrict__ spans,
-                                                             const unsigned char* __restrict__ ws,
-                                                             float* __restrict__ o32) {
+__global__ __launch_bounds__(NW * (DK > 32 ? 128 : 64)) void delta_scan_kernel(DeltaArgs a,
+                                                                                const DeltaSpan* __restrict__ spans,
+                                                                                const unsigned char* __restrict__ ws,
+                                                                                float* __restrict__ o32) {
   using PC = Pieces<DK>;
+  constexpr int KS = DK > 32 ? 2 : 1, NWV = NW * KS;  // key parts, waves
   constexpr int KF = DK / 32, MT = DK / 16, NP = PC::U;
-  constexpr int NDMA = (NP + NW - 1) / NW, LESS = NP % NW;  // DMA instructions per wave; waves >= LESS > 0: one less
+  constexpr int KFW = KF / KS, MTW = MT / KS;  // of one wave
+  constexpr int NDMA = (NP + NWV - 1) / NWV, NST = 8 / KS;  // DMA instructions and stores of a wave per chunk
   constexpr size_t STRIDE = (size_t)(PC::U + DV / 8) * 1024;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[3 * NP * 1024];
+  // the exchange: 3 KiB a wave, in place of the chunk's W and q e^G (read by then) where LDS is full
+  constexpr int EX = KS > 1 ? NWV * 3072 : 0;
+  constexpr bool EX_OWN = 3 * NP * 1024 + EX <= 160 * 1024;
+  static_assert(EX_OWN || EX <= PC::K * 1024, "room for the exchange");
+  __shared__ __attribute__((aligned(16))) unsigned char smem[3 * NP * 1024 + (EX_OWN ? EX : 0)];
   const DeltaSpan sp = spans[blockIdx.x];
   const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, q4 = lane >> 4;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), vt = blockIdx.z * NW + w;  // this wave's channels: 16 vt ..
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), kh = w / NW;  // kh: this wave's keys
+  const int vt = blockIdx.z * NW + w % NW;                              // its channels: 16 vt ..
   const unsigned char* src = ws + ((size_t)sp.chunk0 * a.heads + h) * STRIDE;
   const size_t step = (size_t)a.heads * STRIDE;
 
-  f32x4_t S[MT], U0[2], U1[2];
-  float* st = a.state + ((size_t)sp.slot * a.heads + h) * DK * DV + vt * 16 + l16;
+  f32x4_t S[MTW], U0[2], U1[2];
+  float* st = a.state + (((size_t)sp.slot * a.heads + h) * DK + kh * (DK / KS)) * DV + vt * 16 + l16;
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int m = 0; m < MTW; ++m)
 #pragma unroll
     for (int r = 0; r < 4; ++r) S[m][r] = st[(size_t)(m * 16 + q4 * 4 + r) * DV];
   if (sp.pos0 == 0) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MTW; ++m) S[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  auto stage = [&](int c, int buf) {
-    const unsigned char* p = src + c * step + lane * 16;
+  // Chunk c, nothing where there is none: every wave has the same instructions in flight at the same place of each
+  // chunk, so that waits can be counted (what is left over of the pieces is requested twice).
+  int off[NDMA];
+#pragma unroll
+  for (int i = 0; i < NDMA; ++i) off[i] = min(i * NWV + w, NP - 1) * 1024 + lane * 16;
+  auto stage = [&](int c, int buf, f32x4_t (&U)[2]) {
+    const __amdgpu_buffer_rsrc_t r = bytes_of(src + c * step, c < sp.chunks ? (int)STRIDE : 0);
 #pragma unroll
     for (int i = 0; i < NDMA; ++i)
-      if (LESS == 0 || i * NW + w < NP) glds16(p + (i * NW + w) * 1024, smem + (buf * NP + i * NW + w) * 1024);
-  };
-  auto load_u = [&](int c, f32x4_t (&U)[2]) {
-    const unsigned char* p = src + c * step + (PC::U + vt * 2) * 1024 + lane * 16;
+      glds16(r, off[i], smem + (buf * NP + min(i * NWV + w, NP - 1)) * 1024);
 #pragma unroll
-    for (int m = 0; m < 2; ++m) U[m] = *reinterpret_cast<const f32x4_t*>(p + m * 1024);
+    for (int m = 0; m < 2; ++m)
+      U[m] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, (PC::U + vt * 2 + m) * 1024 + lane * 16, 0, 0));
+    asm volatile("" ::: "memory");
   };
-  const int v = vt * 16 + l16;
-  float* op = o32 + (size_t)sp.row0 * a.heads * a.vdim + h * a.vdim + min(v, a.vdim - 1);
-  const int ldo = a.heads * a.vdim;
+  const int v = vt * 16 + l16, ldo = a.heads * a.vdim;
+  const int row_at = v < a.vdim ? ((kh * 16 + q4 * 4) * ldo + v) * 4 : 0x40000000;
+  // a chunk's read-outs: rows past the run's last and channels past the head's lie behind the descriptor's end
+  auto put = [&](int c, const f32x4_t (&O)[2]) {
+    const int left = min(C, sp.n - c * C);
+    const __amdgpu_buffer_rsrc_t r =
+        bytes_of(o32 + ((size_t)sp.row0 + c * C) * ldo + h * a.vdim, c >= 0 ? ((left - 1) * ldo + a.vdim) * 4 : 0);
+#pragma unroll
+    for (int m = 0; m < 2 / KS; ++m)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(O[m][e]), r, row_at + (m * 16 + e) * ldo * 4, 0, 0);
+    asm volatile("" ::: "memory");
+  };
 
-  // Chunk c + 2 is requested while chunk c runs: operands into the buffer chunk c - 1 used, U into the
-  // registers chunk c's has left. The counted wait leaves those of chunk c + 1 in flight (the read-outs'
-  // stores come after them, so it waits for a few of them at most).
+  // Chunk c + 2 is requested while chunk c runs: operands into the buffer chunk c - 1 used, U into the registers
+  // chunk c's has left. The counted wait leaves what came after chunk c's in flight: the stores of two chunks and the
+  // requests for the next one.
   int buf = 0, buf2 = 2;
   auto chunk = [&](int c, f32x4_t (&U)[2]) {
-    if (c + 1 < sp.chunks) {
-      if (LESS == 0 || w < LESS) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(NDMA + 2) : "memory");
-      else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(NDMA + 1) : "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    }
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(NDMA + 2 + 2 * NST) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const unsigned char* p = smem + buf * NP * 1024 + lane * 16;
+    unsigned char* const at = smem + buf * NP * 1024;
+    const unsigned char* p = at + lane * 16;
     // operands are read a whole group ahead of their products; pin() is where the wait for a group goes
-    auto fetch = [&](auto& r, int first) {
+    auto fetch = [&](u32x4_t* r, int n, int first) {
 #pragma unroll
-      for (int i = 0; i < (int)(sizeof(r) / sizeof(r[0])); ++i) r[i] = *reinterpret_cast<const u32x4_t*>(p + (first + i) * 1024);
+      for (int i = 0; i < n; ++i) r[i] = *reinterpret_cast<const u32x4_t*>(p + (first + i) * 1024);
     };
     auto pin = [](auto& r) {
 #pragma unroll
       for (int i = 0; i < (int)(sizeof(r) / sizeof(r[0])); ++i) asm volatile("" : "+v"(r[i]));
     };
-    u32x4_t wf[4 * KF], qf[4 * KF], kf_[4 * KF], pf[4];
-    f32x4_t ef[MT];
-    fetch(wf, PC::W);
-    fetch(qf, PC::Q);
+    u32x4_t wf[4 * KFW], qf[4 * KFW], kf_[2 * MTW], pf[4];  // [rows or hi / lo][this wave's keys]
+    f32x4_t ef[MTW];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) fetch(wf + m * KFW, KFW, PC::W + m * KF + kh * KFW);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) fetch(qf + m * KFW, KFW, PC::Q + m * KF + kh * KFW);
     float u[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) u[j] = U[j >> 2][j & 3];
 #pragma unroll
     for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(u[j]));
-    if (c + 2 < sp.chunks) {
-      stage(c + 2, buf2);
-      load_u(c + 2, U);
-    }
-    u32x4_t sh[KF], sl[KF];
+    stage(c + 2, buf2, U);
+    u32x4_t sh[KFW], sl[KFW];
 #pragma unroll
-    for (int kf = 0; kf < KF; ++kf) {
+    for (int kf = 0; kf < KFW; ++kf) {
       float f[8];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -410,19 +437,44 @@ __global__ __launch_bounds__(NW * 64) void delta_scan_kernel(DeltaArgs a, const 
     for (int m = 0; m < 2; ++m) V[m] = O[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     pin(wf);
 #pragma unroll
-    for (int kf = 0; kf < KF; ++kf)
+    for (int kf = 0; kf < KFW; ++kf)
 #pragma unroll
-      for (int m = 0; m < 2; ++m) V[m] = mfma_pair(wf[m * KF + kf], wf[(2 + m) * KF + kf], sh[kf], sl[kf], V[m]);
-    fetch(kf_, PC::K);
-    fetch(pf, PC::P);
+      for (int m = 0; m < 2; ++m) V[m] = mfma_pair(wf[m * KFW + kf], wf[(2 + m) * KFW + kf], sh[kf], sl[kf], V[m]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-      ef[m] = *reinterpret_cast<const f32x4_t*>(smem + (buf * NP + PC::E) * 1024 + (m * 16 + q4 * 4) * 4);
+    for (int m = 0; m < 2; ++m) fetch(kf_ + m * MTW, MTW, PC::K + m * MT + kh * MTW);
+    if (KS == 1) {
+      fetch(pf, 4, PC::P);
+    } else {  // read-outs of rows 16 kh ..: one row tile of P
+      fetch(pf, 1, PC::P + kh);
+      fetch(pf + 2, 1, PC::P + 2 + kh);
+    }
+#pragma unroll
+    for (int m = 0; m < MTW; ++m)
+      ef[m] = *reinterpret_cast<const f32x4_t*>(at + PC::E * 1024 + ((kh * MTW + m) * 16 + q4 * 4) * 4);
     pin(qf);
+    unsigned char* const ex = (EX_OWN ? smem + 3 * NP * 1024 : at) + lane * 16;
+    if (KS > 1) {
+      if (!EX_OWN) {  // every wave has its W and q e^G
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      }
 #pragma unroll
-    for (int kf = 0; kf < KF; ++kf)
+      for (int m = 0; m < 2; ++m) *reinterpret_cast<f32x4_t*>(ex + (w * 3 + m) * 1024) = V[m];
+    }
 #pragma unroll
-      for (int m = 0; m < 2; ++m) O[m] = mfma_pair(qf[m * KF + kf], qf[(2 + m) * KF + kf], sh[kf], sl[kf], O[m]);
+    for (int kf = 0; kf < KFW; ++kf)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) O[m] = mfma_pair(qf[m * KFW + kf], qf[(2 + m) * KFW + kf], sh[kf], sl[kf], O[m]);
+    if (KS > 1) {
+      *reinterpret_cast<f32x4_t*>(ex + (w * 3 + 2) * 1024) = kh ? O[0] : O[1];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const unsigned char* other = ex + ((w + (kh ? -NW : NW)) * 3) * 1024;
+#pragma unroll
+      for (int m = 0; m < 2; ++m) V[m] += *reinterpret_cast<const f32x4_t*>(other + m * 1024);
+      O[0] = (kh ? O[1] : O[0]) + *reinterpret_cast<const f32x4_t*>(other + 2048);
+    }
     u32x4_t vh, vl;
 #pragma unroll
     for (int j = 0; j < 8; ++j) u[j] -= V[j >> 2][j & 3];
@@ -430,31 +482,28 @@ __global__ __launch_bounds__(NW * 64) void delta_scan_kernel(DeltaArgs a, const 
     pin(kf_);
     pin(ef);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) S[m] = mfma_pair(kf_[m], kf_[MT + m], vh, vl, S[m] * ef[m]);
+    for (int m = 0; m < MTW; ++m) S[m] = mfma_pair(kf_[m], kf_[MTW + m], vh, vl, S[m] * ef[m]);
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      O[m] = mfma_pair(pf[m], pf[2 + m], vh, vl, O[m]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = c * C + m * 16 + q4 * 4 + r;
-        if (t < sp.n && v < a.vdim) op[(size_t)t * ldo] = O[m][r];
-      }
-    }
+    for (int m = 0; m < 2 / KS; ++m) O[m] = mfma_pair(pf[m], pf[2 + m], vh, vl, O[m]);
+    put(c, O);
     buf = buf == 2 ? 0 : buf + 1;
     buf2 = buf2 == 2 ? 0 : buf2 + 1;
   };
-  stage(0, 0);
-  load_u(0, U0);
-  if (sp.chunks > 1) {
-    stage(1, 1);
-    load_u(1, U1);
-  }
-  for (int c = 0; c < sp.chunks; c += 2) {
+  // (what a chunk's products read and write has no fixed place in flight before the loop: stores of nothing stand in)
+  const f32x4_t none[2] = {};
+  stage(0, 0, U0);
+  put(-1, none);
+  stage(1, 1, U1);
+  put(-1, none);
+  int c = 0;
+  for (; c + 1 < sp.chunks; c += 2) {
     chunk(c, U0);
-    if (c + 1 < sp.chunks) chunk(c + 1, U1);
+    chunk(c + 1, U1);
   }
+  if (c < sp.chunks) chunk(c, U0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int m = 0; m < MTW; ++m)
 #pragma unroll
     for (int r = 0; r < 4; ++r) st[(size_t)(m * 16 + q4 * 4 + r) * DV] = S[m][r];
 }
@@ -508,19 +557,21 @@ extern "C" int lsa_delta_chunk_bytes(int dk, int dv) {
 }
 
 // chunks: n_chunks DeltaChunk; spans: n_spans DeltaSpan over them; ws: n_chunks * heads * lsa_delta_chunk_bytes;
-// o32: [rows][heads * vdim]
+// o32: [rows][heads * vdim]. The scan's workgroups have 32 value channels where those are no more than the 256 CUs (one fits on each) and
+// 64 otherwise: a second round of the narrow ones, 65 us each, costs more than one of the wide ones, 84.
 extern "C" int lsa_delta_chunked(const DeltaArgs* a, const void* chunks, int n_chunks, const void* spans, int n_spans,
                                  void* ws, float* o32, hipStream_t s) {
   if (!a || bad_delta(a) || !a->gate || n_chunks < 1 || n_spans < 1 || !chunks || !spans || !ws || !o32 || (uintptr_t)ws % 16)
     return LSA_BAD_SHAPE;
 #define LSA_S(K, V, NW)                                                                                                  \
-  delta_scan_kernel<K, V, NW><<<dim3(n_spans, a->heads, V / (NW * 16)), NW * 64, 0, s>>>(*a, (const DeltaSpan*)spans,     \
-                                                                                       (const unsigned char*)ws, o32)
+  delta_scan_kernel<K, V, NW><<<dim3(n_spans, a->heads, V / (NW * 16)), NW * (K > 32 ? 128 : 64), 0, s>>>(                \
+      *a, (const DeltaSpan*)spans, (const unsigned char*)ws, o32)
 #define LSA_C(K, V)                                                                                                       \
   if (a->dk == K && a->dv == V) {                                                                                         \
     delta_chunk_kernel<K, V><<<dim3(n_chunks, a->heads), 256, 0, s>>>(*a, (const DeltaChunk*)chunks, (unsigned char*)ws); \
     LSA_CHECK_LAUNCH();                                                                                                   \
-    LSA_S(K, V, (V == 32 ? 2 : 4));                                                                                       \
+    if (K > 32 && V > 32 && n_spans * a->heads * (V / 32) <= 256) LSA_S(K, V, 2);                                         \
+    else LSA_S(K, V, (V == 32 ? 2 : 4));                                                                                  \
     LSA_CHECK_LAUNCH();                                                                                                   \
     delta_norm_kernel<<<dim3(n_chunks, a->heads), 256, 0, s>>>(*a, (const DeltaChunk*)chunks, o32);                       \
     LSA_CHECK_LAUNCH();                                                                                                   \

@@ -418,6 +418,17 @@ def test_delta_forgets_and_remembers():
         assert (case.got[0][139].abs().max() > 0.3) == kept
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(64, 128, 128), (65, 128, 128), (128, 64, 40), (129, 64, 40), (3, 64, 128)])
+def test_delta_scan_of_few_and_many_heads(heads, dim, vdim):
+    """Value channels to 256 workgroups or fewer, and past that; a ragged last chunk and a state carried on. Limits as above."""
+    case = DeltaCase(DeltaSpec(heads, 1, dim, vdim, 4, 8, 8, dim ** -0.5, 1e-6), [103], BF, fast=0.3)
+    case.step([(0, 97)], "chunks")
+    case.step([(0, 6)], "chunks")
+    out, S = case.want(0)
+    close(case.got[0], out, 6e-3, "outputs")
+    close(case.state[0][0, :, :dim, :vdim], S, 3e-5, "state")
+
+
 def test_idle_rows_leave_state_alone():
     from llm_sharding_amd.ops import delta as D
     s = DELTA["small"]
