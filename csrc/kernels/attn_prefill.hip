@@ -261,8 +261,8 @@ __global__ __launch_bounds__(NTHR) void flash_prefill_kernel(
 #pragma unroll
   for (int d = 0; d < DT; ++d) {
     // this lane holds O[row][d*16 + 4g + r], r = 0..3
-    const unsigned lo = (unsigned)f2bf(o[d][0] * inv) | ((unsigned)f2bf(o[d][1] * inv) << 16);
-    const unsigned hi = (unsigned)f2bf(o[d][2] * inv) | ((unsigned)f2bf(o[d][3] * inv) << 16);
+    const unsigned lo = f2bf2(o[d][0] * inv, o[d][1] * inv);
+    const unsigned hi = f2bf2(o[d][2] * inv, o[d][3] * inv);
     *reinterpret_cast<unsigned long long*>(orow + d * 16 + g * 4) = (unsigned long long)lo | ((unsigned long long)hi << 32);
   }
 }

@@ -30,6 +30,14 @@ LSA_DEVICE bf16_raw f2bf(float f) {
   return __builtin_bit_cast(bf16_raw, b);
 }
 
+// Two of them, a in the low half, in the one instruction that converts two (f2bf(a) | f2bf(b) << 16 took it twice, a shift and an or:
+// 64 instead of 16 instructions in 230 of a flash-attention block of 32 rows x 64 keys a wave).
+LSA_DEVICE unsigned f2bf2(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
 LSA_DEVICE u32x4_t ld16(const void* p) { return *reinterpret_cast<const u32x4_t*>(p); }
 LSA_DEVICE void st16(void* p, u32x4_t v) { *reinterpret_cast<u32x4_t*>(p) = v; }
 
@@ -49,8 +57,7 @@ LSA_DEVICE void unpack8(u32x4_t v, float* f) {
 LSA_DEVICE u32x4_t pack8(const float* f) {
   u32x4_t r;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    r[i] = (unsigned)f2bf(f[2 * i]) | ((unsigned)f2bf(f[2 * i + 1]) << 16);
+  for (int i = 0; i < 4; ++i) r[i] = f2bf2(f[2 * i], f[2 * i + 1]);
   return r;
 }
 

@@ -9,8 +9,8 @@ LSA_DEVICE void st1(float* p, float v) { *p = v; }
 LSA_DEVICE void st1(bf16_raw* p, float v) { *p = f2bf(v); }
 LSA_DEVICE void st4(float* p, f32x4_t v) { *reinterpret_cast<f32x4_t*>(p) = v; }
 LSA_DEVICE void st4(bf16_raw* p, f32x4_t v) {
-  const unsigned lo = (unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16);
-  const unsigned hi = (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16);
+  const unsigned lo = f2bf2(v[0], v[1]);
+  const unsigned hi = f2bf2(v[2], v[3]);
   *reinterpret_cast<u32x2_t*>(p) = u32x2_t{lo, hi};
 }
 
