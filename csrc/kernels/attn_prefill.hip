@@ -5,9 +5,14 @@
 // HF LlamaDecoderLayer) with one kernel that never materialises the score matrix.
 //
 // Work unit: one query tile of ONE sequence (host-built tile table) x one KV head's group of
-// HPW query heads (HPW = G = n_heads / n_kv when it divides 8, else 1): 8 waves, each owning
-// 16 query rows of one head (positions (w / HPW) * 16 ..), so a tile holds 128 / HPW
+// HPW query heads (HPW = G = n_heads / n_kv when it divides 8, else 1): 4 waves, each owning two
+// groups of 16 query rows of one head (group i: head i % HPW, positions (i / HPW) * 16 ..), so a tile holds 128 / HPW
 // positions and every staged K/V block serves the whole GQA group (no re-staging per head).
+// A wave with one group (8 waves, before) reads twice as much of LDS for a product and waits as often. In tiles of up to 64
+// rows each of the four waves has one group. With the packing of bf16 pairs in one conversion: one causal prompt, 32 heads, 512
+// tokens 19.0 -> 12.9 us, 2048 70.5 -> 62.4, 8192 735 -> 667 (825 TFLOP/s); 64 heads on 8 2048 108 -> 99, 8192 1351 -> 1192
+// (922). What bounds it now: a wave's chain of products, exponents and products for a block, with two waves on a
+// SIMD (2048 tokens take 57 us without the DMA).
 // Per 64-key block:
 //   * K and V arrive by LDS-DMA (global_load_lds, 16 B/lane) into an NBUF-deep ring, blocks
 //     kb+1 .. kb+NBUF-1 in flight (counted vmcnt) while block kb is computed; one barrier per block. The swizzle is
@@ -26,7 +31,8 @@
 
 namespace {
 
-constexpr int BKV = 64, NWV = 8, NTHR = NWV * 64;  // 64-key blocks, 8 waves x 16 query rows
+constexpr int BKV = 64, NWV = 4, NTHR = NWV * 64;  // 64-key blocks, 4 waves x 32 query rows
+constexpr int GROUPS = 2 * NWV;                    // groups of 16 rows of one head in a tile
 // K/V ring depth. 2 (block kb+1 in flight while kb is computed) keeps the workgroup at 64 KiB of
 // LDS, two per CU; a 4-deep ring (128 KiB, one per CU) measured 6-16 % slower at S >= 2048
 // and no faster at S = 512 (scripts/prefill_attn_bench.py)
@@ -65,57 +71,57 @@ LSA_DEVICE void glds16_nt(const void* src, unsigned char* lds_base) {
   __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)lds_base, 16, 0, 2);
 }
 
-template <int HD, int HPW>
-__global__ __launch_bounds__(NTHR) void flash_prefill_kernel(
-    const bf16_raw* __restrict__ q, int ldq, const bf16_raw* __restrict__ kc, const bf16_raw* __restrict__ vc,
-    const PrefillTile* __restrict__ tiles, int n_heads, int n_kv, int t_max, float scale_log2, int causal,
-    bf16_raw* __restrict__ out, int ldo) {
+// The schedule of N operands of READS LDS reads each, for M products each: A operands are read ahead of their products. (The compiler
+// reads one or two and waits for them, every time: 65.5 us of 2048 tokens instead of 62.4. Eight and four ahead no better.)
+template <int A, int N, int READS, int M>
+LSA_DEVICE void ahead() {
+  constexpr int AA = A < N ? A : N;
+  __builtin_amdgcn_sched_group_barrier(0x100, AA * READS, 0);
+#pragma unroll
+  for (int i = AA; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, M, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x008, AA * M, 0);
+}
+constexpr int AHEAD_K = 6, AHEAD_V = 6;
+
+// The tile of a workgroup with RT groups of 16 rows a wave, each of one head: what is read of K and V from LDS is used for all of them.
+template <int HD, int HPW, int RT>
+LSA_DEVICE void prefill_tile(unsigned char* smem, const bf16_raw* __restrict__ q, int ldq, const bf16_raw* __restrict__ kc,
+                             const bf16_raw* __restrict__ vc, const PrefillTile& tile, int grp, int n_heads, int n_kv, int t_max,
+                             float scale_log2, int causal, bf16_raw* __restrict__ out, int ldo) {
   constexpr int KF = HD / 32;                 // 32-dim fragments of a query/key row
   constexpr int DT = HD / 16;                 // 16-dim output tiles
   constexpr int NC = HD / 8;                  // 16-B chunks per row
   constexpr int BLK = BKV * HD * 2;           // bytes of one K (or V) block
   constexpr int PPW = BLK / 1024 / NWV;       // 1 KiB DMA pieces per wave per operand
   constexpr int RPP = 1024 / (HD * 2);        // rows per piece
-  static_assert(PPW >= 1 && NWV % HPW == 0, "geometry");
-  __shared__ __attribute__((aligned(16))) unsigned char smem[NBUF * 2 * BLK];  // [buffer][K | V]
-
-  // work item -> (tile, head group). XCD-aware when the group count is a multiple of 8: XCD x
-  // (= blockIdx.x % 8 in dispatch order) owns groups x, x+8, ... so their K/V blocks stay in
-  // its L2, and walks its items tile-major (heaviest tiles of all its groups first)
-  const int n_groups = n_heads / HPW, n_tiles = gridDim.x / n_groups;
-  int tix, grp;
-  if (n_groups % 8 == 0) {
-    const int x = blockIdx.x % 8, j = blockIdx.x / 8, ngx = n_groups / 8;
-    tix = j / ngx;
-    grp = (j % ngx) * 8 + x;
-  } else {
-    tix = blockIdx.x % n_tiles;
-    grp = blockIdx.x / n_tiles;
-  }
-  const PrefillTile tile = tiles[tix];
+  static_assert(PPW >= 1 && (RT * NWV) % HPW == 0, "geometry");
   const int G = n_heads / n_kv;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int head = grp * HPW + w % HPW;
   const int kvh = grp * HPW / G;
-  const int prow0 = (w / HPW) * 16;
 
-  // ---- Q^T fragments for this wave's 16 rows (row = l16), kept for the whole tile
-  const int my_row = prow0 + l16;
-  const bool row_ok = my_row < tile.nrows;
-  const int my_pos = tile.pos0 + my_row;
-  u32x4_t qf[KF];
-  {
-    const bf16_raw* qrow = q + (size_t)(tile.row0 + (row_ok ? my_row : 0)) * ldq + head * HD;
-#pragma unroll
-    for (int kf = 0; kf < KF; ++kf) qf[kf] = ld16(qrow + kf * 32 + g * 8);
-  }
+  // ---- Q^T fragments for this wave's groups of 16 rows (row = l16), kept for the whole tile
   const int lim = causal ? min(tile.pos0 + tile.nrows, tile.kvlen) : tile.kvlen;  // keys any row needs
-  const int my_lim = causal ? min(my_pos + 1, tile.kvlen) : tile.kvlen;         // keys this row sees
-  const int wave_lim = causal ? min(tile.pos0 + min(prow0 + 16, tile.nrows), tile.kvlen) : tile.kvlen;
-  // blocks entirely below every row's limit need no mask (the wave's first row sees the fewest keys)
-  const int wave_min_lim = causal ? min(tile.pos0 + prow0 + 1, tile.kvlen) : tile.kvlen;
+  u32x4_t qf[RT][KF];
+  int head[RT], my_row[RT], my_lim[RT], lim1[RT], lim0[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const int id = w * RT + t, prow0 = (id / HPW) * 16;
+    head[t] = grp * HPW + id % HPW;
+    my_row[t] = prow0 + l16;
+    my_lim[t] = causal ? min(tile.pos0 + my_row[t] + 1, tile.kvlen) : tile.kvlen;  // keys this row sees
+    lim1[t] = causal ? min(tile.pos0 + min(prow0 + 16, tile.nrows), tile.kvlen) : tile.kvlen;  // ... any row of the group
+    // blocks entirely below every row's limit need no mask (the group's first row sees the fewest keys)
+    lim0[t] = causal ? min(tile.pos0 + prow0 + 1, tile.kvlen) : tile.kvlen;
+    const bf16_raw* qrow = q + (size_t)(tile.row0 + (my_row[t] < tile.nrows ? my_row[t] : 0)) * ldq + head[t] * HD;
+#pragma unroll
+    for (int kf = 0; kf < KF; ++kf) qf[t][kf] = ld16(qrow + kf * 32 + g * 8);
+  }
   const int nkb = (lim + BKV - 1) / BKV;
+  const bool none = (w * RT / HPW) * 16 >= tile.nrows;  // a wave past the tile's rows
 
   const size_t cache_base = ((size_t)tile.slot * n_kv + kvh) * (size_t)t_max * HD;
   const bf16_raw* kb_ptr = kc + cache_base;
@@ -136,10 +142,15 @@ __global__ __launch_bounds__(NTHR) void flash_prefill_kernel(
     }
   };
 
-  f32x4_t o[DT];
+  f32x4_t o[RT][DT];
+  float m_run[RT], l_run[RT];
 #pragma unroll
-  for (int d = 0; d < DT; ++d) o[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
+  for (int t = 0; t < RT; ++t) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d) o[t][d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    m_run[t] = -INFINITY;
+    l_run[t] = 0.f;
+  }
 
   // per-lane LDS offsets, hoisted out of the block loop (the swizzle term of a lane's reads is
   // the same in every block; rows differ by compile-time multiples folded into the reads)
@@ -149,6 +160,108 @@ __global__ __launch_bounds__(NTHR) void flash_prefill_kernel(
   const int key_lo = 4 * g + (l16 >> 2);                                    // + f2 * 32 (+ 16) rows
 #pragma unroll
   for (int d = 0; d < DT; ++d) v_off[d] = sw_off<HD>(key_lo, 2 * d + ((l16 & 3) >> 1)) + 8 * (l16 & 1);
+
+  // block kb, read from ks, for the groups FIRST .. RT - 1
+  auto block = [&](auto first, int kb, const unsigned char* ks) {
+    constexpr int FIRST = decltype(first)::value;
+    const unsigned char* vs = ks + BLK;
+    // S^T = K . Q^T : 4 key tiles of 16 (row kt*16 + l16: the swizzle term depends on l16 only)
+    f32x4_t s[RT][4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+      for (int t = FIRST; t < RT; ++t) s[t][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kf = 0; kf < KF; ++kf) {
+        const u32x4_t a = *reinterpret_cast<const u32x4_t*>(ks + kt * 16 * (HD * 2) + k_off[kf]);
+#pragma unroll
+        for (int t = FIRST; t < RT; ++t) s[t][kt] = mfma16(a, qf[t][kf], s[t][kt]);
+      }
+    }
+    ahead<AHEAD_K, 4 * KF, 1, RT - FIRST>();
+#pragma unroll
+    for (int t = FIRST; t < RT; ++t) {
+      // scale, mask (diagonal / tail blocks only), block row max (this lane: row my_row, keys
+      // kb*64 + kt*16 + 4g + r)
+      float mx = -INFINITY;
+      if ((kb + 1) * BKV <= lim0[t]) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            s[t][kt][r] *= scale_log2;
+            mx = fmaxf(mx, s[t][kt][r]);
+          }
+      } else {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int key = kb * BKV + kt * 16 + g * 4 + r;
+            const float v = key < my_lim[t] ? s[t][kt][r] * scale_log2 : -INFINITY;
+            s[t][kt][r] = v;
+            mx = fmaxf(mx, v);
+          }
+      }
+      mx = fmaxf(mx, lane_xor<16>(mx));
+      mx = fmaxf(mx, lane_xor<32>(mx));
+      const float m_new = fmaxf(m_run[t], mx);
+      // fully-masked rows so far (m_new = -inf) keep alpha = 1 and p = 0
+      const float m_use = m_new == -INFINITY ? 0.f : m_new;
+      // raw v_exp_f32 (arguments <= 0: no range reduction needed; -inf -> 0)
+      const float alpha = __builtin_amdgcn_exp2f(m_run[t] - m_use);
+      float psum = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float p = __builtin_amdgcn_exp2f(s[t][kt][r] - m_use);
+          s[t][kt][r] = p;
+          psum += p;
+        }
+      l_run[t] = l_run[t] * alpha + psum;  // per-lane partial (this lane's keys); reduced at the end
+      // rescale O only when some row's max moved (wave-uniform branch)
+      if (__builtin_amdgcn_ballot_w64(m_new != m_run[t])) {
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[t][d] *= alpha;
+      }
+      m_run[t] = m_new;
+    }
+
+    // O^T += V^T . P^T over two 32-key fragments; V^T by hardware-transposed reads: in each
+    // 16-lane group, lane 4q+p addresses key (base + q), dims 4p..4p+3 of the 16-dim tile
+#pragma unroll
+    for (int f2 = 0; f2 < 2; ++f2) {
+      u32x4_t b[RT];
+#pragma unroll
+      for (int t = FIRST; t < RT; ++t) {
+        float pf[8];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          pf[r] = s[t][2 * f2][r];
+          pf[4 + r] = s[t][2 * f2 + 1][r];
+        }
+        b[t] = pack8(pf);
+      }
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        // rows key_lo + f2*32 (+16): same swizzle term as key_lo (it depends on row & 15 only
+        // through row & 3 and (row >> 2) & 3, unchanged by multiples of 16; HD = 64: (row >> 1) & 7)
+        const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) v4s_t*)(vs + f2 * 32 * (HD * 2) + v_off[d]));
+        const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) v4s_t*)(vs + (f2 * 32 + 16) * (HD * 2) + v_off[d]));
+        u32x4_t a;
+        a[0] = __builtin_bit_cast(u32x2_t, lo)[0];
+        a[1] = __builtin_bit_cast(u32x2_t, lo)[1];
+        a[2] = __builtin_bit_cast(u32x2_t, hi)[0];
+        a[3] = __builtin_bit_cast(u32x2_t, hi)[1];
+#pragma unroll
+        for (int t = FIRST; t < RT; ++t) o[t][d] = mfma16(a, b[t], o[t][d]);
+      }
+    }
+    ahead<AHEAD_V, 2 * DT, 2, RT - FIRST>();
+  };
 
   // prologue: blocks 0 .. NBUF-2 in flight
   for (int b = 0; b < NBUF - 1 && b < nkb; ++b) stage(b, b);
@@ -163,108 +276,60 @@ __global__ __launch_bounds__(NTHR) void flash_prefill_kernel(
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();  // ... every wave's; every wave's reads of block kb-1 done
     if (kb + NBUF - 1 < nkb) stage(kb + NBUF - 1, (kb + NBUF - 1) % NBUF);  // into block kb-1's buffer
-    if (kb * BKV >= wave_lim) continue;                 // wave-uniform: all keys above the diagonal
     const unsigned char* ks = smem + cur * (2 * BLK);
-    const unsigned char* vs = ks + BLK;
-
-    // S^T = K . Q^T : 4 key tiles of 16 (row kt*16 + l16: the swizzle term depends on l16 only)
-    f32x4_t s[4];
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-      s[kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kf = 0; kf < KF; ++kf) {
-        const u32x4_t a = *reinterpret_cast<const u32x4_t*>(ks + kt * 16 * (HD * 2) + k_off[kf]);
-        s[kt] = mfma16(a, qf[kf], s[kt]);
-      }
-    }
-    // scale, mask (diagonal / tail blocks only), block row max (this lane: row my_row, keys
-    // kb*64 + kt*16 + 4g + r)
-    float mx = -INFINITY;
-    if ((kb + 1) * BKV <= wave_min_lim) {
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[kt][r] *= scale_log2;
-          mx = fmaxf(mx, s[kt][r]);
-        }
-    } else {
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = kb * BKV + kt * 16 + g * 4 + r;
-          const float v = key < my_lim ? s[kt][r] * scale_log2 : -INFINITY;
-          s[kt][r] = v;
-          mx = fmaxf(mx, v);
-        }
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m_run, mx);
-    // fully-masked rows so far (m_new = -inf) keep alpha = 1 and p = 0
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    // raw v_exp_f32 (arguments <= 0: no range reduction needed; -inf -> 0)
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
-    float psum = 0.f;
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float p = __builtin_amdgcn_exp2f(s[kt][r] - m_use);
-        s[kt][r] = p;
-        psum += p;
-      }
-    l_run = l_run * alpha + psum;  // per-lane partial (this lane's keys); reduced at the end
-    // rescale O only when some row's max moved (wave-uniform branch)
-    if (__builtin_amdgcn_ballot_w64(m_new != m_run)) {
-#pragma unroll
-      for (int d = 0; d < DT; ++d) o[d] *= alpha;
-    }
-    m_run = m_new;
-
-    // O^T += V^T . P^T over two 32-key fragments; V^T by hardware-transposed reads: in each
-    // 16-lane group, lane 4q+p addresses key (base + q), dims 4p..4p+3 of the 16-dim tile
-#pragma unroll
-    for (int f2 = 0; f2 < 2; ++f2) {
-      float pf[8];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        pf[r] = s[2 * f2][r];
-        pf[4 + r] = s[2 * f2 + 1][r];
-      }
-      const u32x4_t b = pack8(pf);
-#pragma unroll
-      for (int d = 0; d < DT; ++d) {
-        // rows key_lo + f2*32 (+16): same swizzle term as key_lo (it depends on row & 15 only
-        // through row & 3 and (row >> 2) & 3, unchanged by multiples of 16; HD = 64: (row >> 1) & 7)
-        const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) v4s_t*)(vs + f2 * 32 * (HD * 2) + v_off[d]));
-        const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) v4s_t*)(vs + (f2 * 32 + 16) * (HD * 2) + v_off[d]));
-        u32x4_t a;
-        a[0] = __builtin_bit_cast(u32x2_t, lo)[0];
-        a[1] = __builtin_bit_cast(u32x2_t, lo)[1];
-        a[2] = __builtin_bit_cast(u32x2_t, hi)[0];
-        a[3] = __builtin_bit_cast(u32x2_t, hi)[1];
-        o[d] = mfma16(a, b, o[d]);
-      }
-    }
+    // wave-uniform: groups whose rows end above the block take no part (the last group's rows end last)
+    if (none || kb * BKV >= lim1[RT - 1]) continue;
+    if (RT == 1 || kb * BKV < lim1[0]) block(std::integral_constant<int, 0>{}, kb, ks);
+    else block(std::integral_constant<int, RT - 1>{}, kb, ks);
   }
 
-  l_run += __shfl_xor(l_run, 16, 64);
-  l_run += __shfl_xor(l_run, 32, 64);
-  if (!row_ok) return;
-  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  bf16_raw* orow = out + (size_t)(tile.row0 + my_row) * ldo + head * HD;
 #pragma unroll
-  for (int d = 0; d < DT; ++d) {
-    // this lane holds O[row][d*16 + 4g + r], r = 0..3
-    const unsigned lo = f2bf2(o[d][0] * inv, o[d][1] * inv);
-    const unsigned hi = f2bf2(o[d][2] * inv, o[d][3] * inv);
-    *reinterpret_cast<unsigned long long*>(orow + d * 16 + g * 4) = (unsigned long long)lo | ((unsigned long long)hi << 32);
+  for (int t = 0; t < RT; ++t) {
+    l_run[t] += lane_xor<16>(l_run[t]);
+    l_run[t] += lane_xor<32>(l_run[t]);
+    if (my_row[t] >= tile.nrows) continue;
+    const float inv = l_run[t] > 0.f ? 1.f / l_run[t] : 0.f;
+    bf16_raw* orow = out + (size_t)(tile.row0 + my_row[t]) * ldo + head[t] * HD;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      // this lane holds O[row][d*16 + 4g + r], r = 0..3
+      const unsigned lo = f2bf2(o[t][d][0] * inv, o[t][d][1] * inv);
+      const unsigned hi = f2bf2(o[t][d][2] * inv, o[t][d][3] * inv);
+      *reinterpret_cast<unsigned long long*>(orow + d * 16 + g * 4) = (unsigned long long)lo | ((unsigned long long)hi << 32);
+    }
   }
+}
+
+template <int HD, int HPW>
+__global__ __launch_bounds__(NTHR, 2) void flash_prefill_kernel(
+    const bf16_raw* __restrict__ q, int ldq, const bf16_raw* __restrict__ kc, const bf16_raw* __restrict__ vc,
+    const PrefillTile* __restrict__ tiles, int n_heads, int n_kv, int t_max, float scale_log2, int causal,
+    bf16_raw* __restrict__ out, int ldo) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[NBUF * 2 * BKV * HD * 2];  // [buffer][K | V]
+
+  // work item -> (tile, head group). XCD-aware when the group count is a multiple of 8: XCD x
+  // (= blockIdx.x % 8 in dispatch order) owns groups x, x+8, ... so their K/V blocks stay in
+  // its L2, and walks its items tile-major (heaviest tiles of all its groups first)
+  const int n_groups = n_heads / HPW, n_tiles = gridDim.x / n_groups;
+  int tix, grp;
+  if (n_groups % 8 == 0) {
+    const int x = blockIdx.x % 8, ngx = n_groups / 8;
+    const int j = pair_up(blockIdx.x / 8, n_tiles * ngx);
+    tix = j / ngx;
+    grp = (j % ngx) * 8 + x;
+  } else {
+    tix = blockIdx.x % n_tiles;
+    grp = blockIdx.x / n_tiles;
+  }
+  const PrefillTile tile = tiles[tix];
+  // groups of 16 rows for half of the waves at most: one each, on all four SIMDs
+  if constexpr (HPW <= NWV) {
+    if (tile.nrows * HPW <= NWV * 16) {
+      prefill_tile<HD, HPW, 1>(smem, q, ldq, kc, vc, tile, grp, n_heads, n_kv, t_max, scale_log2, causal, out, ldo);
+      return;
+    }
+  }
+  prefill_tile<HD, HPW, 2>(smem, q, ldq, kc, vc, tile, grp, n_heads, n_kv, t_max, scale_log2, causal, out, ldo);
 }
 
 template <int HD, int HPW>
@@ -518,7 +583,7 @@ int launch_gqa_decode(int nw, const bf16_raw* q, int ldq, const bf16_raw* k, con
 extern "C" int lsa_prefill_tile_rows(int n_heads, int n_kv) {
   if (n_kv < 1 || n_heads % n_kv) return 0;
   const int g = n_heads / n_kv;
-  return NTHR / 64 * 16 / ((NWV % g == 0) ? g : 1);
+  return GROUPS * 16 / ((GROUPS % g == 0) ? g : 1);
 }
 
 extern "C" int lsa_attn_prefill(const void* q, int ldq, const void* kc, const void* vc, const void* tiles, int n_tiles,
@@ -526,7 +591,7 @@ extern "C" int lsa_attn_prefill(const void* q, int ldq, const void* kc, const vo
                                 int ldo, hipStream_t stream) {
   if (n_tiles < 1 || n_kv < 1 || n_heads % n_kv || n_heads < 1) return LSA_BAD_SHAPE;
   const float sl2 = scale * 1.4426950408889634f;
-  const int g = n_heads / n_kv, hpw = (NWV % g == 0) ? g : 1;
+  const int g = n_heads / n_kv, hpw = (GROUPS % g == 0) ? g : 1;
   const auto* t = static_cast<const PrefillTile*>(tiles);
   const auto* qq = static_cast<const bf16_raw*>(q);
   const auto* k = static_cast<const bf16_raw*>(kc);

@@ -619,6 +619,26 @@ def test_attention_prefill_long_sequence(nh, nkv):
     assert float(per_row.max()) < 2e-2, per_row
 
 
+@pytest.mark.parametrize("nh,nkv,hd", [(24, 8, 128), (8, 8, 128), (16, 8, 64), (8, 2, 128), (16, 2, 128), (16, 2, 64)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_attention_prefill_edges_of_tiles(nh, nkv, hd, causal):
+    """Tiles of one, a half and all of their rows, and one more or less: one or two groups of 16 rows a wave, some with none; from
+    positions that lie anywhere in a block of keys. Limits as above."""
+    h = hip()
+    most = h.prefill_tile_rows(nh, nkv)
+    sizes = sorted({1, 15, 16, 17, most // 2 - 1, most // 2, most // 2 + 1, most - 1, most, most + 1, 2 * most + 33} - {0})
+    starts = [(37 * i) % 130 for i in range(len(sizes))]
+    slot = [i for i, n in enumerate(sizes) for _ in range(n)]
+    pos = [p + j for n, p in zip(sizes, starts) for j in range(n)]
+    kvl = None if causal else [p + n + 5 for n, p in zip(sizes, starts) for _ in range(n)]
+    T = max(pos) + 8
+    kc, vc, q = _rnd(len(sizes), nkv, T, hd), _rnd(len(sizes), nkv, T, hd), _rnd(len(pos), nh * hd)
+    out = torch.zeros(len(pos), nh * hd, dtype=torch.bfloat16, device=DEV)
+    h.attn_prefill(q, kc, vc, h.build_prefill_tiles(slot, pos, kvl, device=DEV, tile_rows=most), nh, nkv, hd, out, causal=causal)
+    ref = _prefill_ref(q, kc, vc, slot, pos, nh, nkv, hd, kvl)
+    assert float(((out.float() - ref).norm(dim=1) / ref.norm(dim=1)).max()) < 3e-2
+
+
 @pytest.mark.parametrize("cfg", packing.FP8_CONFIGS)
 def test_gemv_fp8_every_config(cfg):
     """W8A16 GEMV (OCP e4m3 weights, per-row scales, bf16 MFMA after in-register conversion)
