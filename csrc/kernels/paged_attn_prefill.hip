@@ -41,7 +41,7 @@ __global__ __launch_bounds__(NTHR, DK + DV <= 256 ? 4 : 2) void attn_tiles_kerne
   const int H = a.heads, n_tiles = gridDim.x / H;
   int tix, head;
   if (H % 8 == 0) {  // one XCD's workgroups share heads of one kv head: its pages stay in that L2
-    const int x = blockIdx.x % 8, j = blockIdx.x / 8, hx = H / 8;
+    const int x = blockIdx.x % 8, hx = H / 8, j = DK + DV <= 256 ? pair_up(blockIdx.x / 8, n_tiles * hx) : blockIdx.x / 8;
     tix = j / hx;
     head = x * hx + j % hx;
   } else {

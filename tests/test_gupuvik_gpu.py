@@ -247,6 +247,23 @@ def test_attention_of_query_tiles(name):
         A.check_tiles(torch.tensor([[0, 10, 0, 250]]), 200, 2, 4)
 
 
+@pytest.mark.parametrize("rows", [768, 769, 1537])
+def test_attention_of_query_tiles_in_two_rows(rows):
+    """40 heads: 30, 35 and 65 tiles an XCD, of which 32 have a CU each and the rest the second place. Limit as above."""
+    from llm_sharding_amd.ops import paged_attn as A
+    from llm_sharding_amd.runtime.attn_mixer import Attention
+    s = SIZES["many_heads"]
+    case = Case(s, [rows], BF, seed=4).fill()
+    q = _rand(rows, s.heads, s.dim, seed=9)
+    eng = type("Eng", (), {"device": DEV})
+    tiles = Attention._tiles(type("Plan", (), {"eng": eng}), [(0, rows, 0, 0)], rows, case.table)
+    out = torch.full((rows, s.heads * s.dvp), float("nan"), dtype=BF, device=DEV)
+    A.tiles(case.args([0] * rows, list(range(rows))), tiles, case.padded(q, s.dkp).to(DEV), None, out)
+    pick = list(range(5, rows, 61)) + [rows - 1]
+    assert not out.isnan().any()
+    close(case.unpad(out).cpu()[pick], case.want(q[pick], [0] * len(pick), pick), 1.5e-2, "rows")
+
+
 @pytest.mark.parametrize("dtype", [BF, F32])
 @pytest.mark.parametrize("window,keep", [(40, 5), (64, 0), (1, 64), (100, 1), (65, 130)])
 def test_one_key_stands_out(dtype, window, keep):
