@@ -35,6 +35,7 @@ from ..models import gpt2 as G2
 from ..models import weights as W
 from ..models.rope import rope_table
 from ..ops import packing
+from .recording import collector_held
 
 
 # ---------------------------------------------------------------------------- weight sources
@@ -1131,7 +1132,7 @@ class DecodeGraph:
                 self._body()
         torch.cuda.current_stream(self.eng.device).wait_stream(s)
         g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g, stream=s):
+        with collector_held(), torch.cuda.graph(g, stream=s):
             if self.pre_comm is not None:
                 self.pre_comm()
             self._body()
