@@ -21,6 +21,7 @@ once. Hidden states go rank r -> r+1 over xGMI, token ids go last -> 0 (the ring
 from __future__ import annotations
 
 import contextlib
+import functools
 import os
 import time
 from typing import Optional
@@ -428,19 +429,20 @@ class PipelineStage:
         return all(self.p2p.fits(t) for t in probe)
 
     def _attach_comm(self, g: DecodeGraph) -> None:
+        # (what is attached holds the graph's buffers and not the graph: a cycle would keep it until the cyclic collector comes by)
         p2p, r = self.p2p, self.rank
         if self.mode in ("mid", "last"):
-            g.pre_comm = lambda: p2p.recv(g.h_in, r - 1)
+            g.pre_comm = functools.partial(p2p.recv, g.h_in, r - 1)
         if self.mode == "last" and self.split:
-            def post():
-                p2p.isend(g.out_hidden, 0)
-                p2p.isend(g.keys, 0)
+            sends = ((g.out_hidden, 0), (g.keys, 0))
         elif self.mode == "last":
-            def post():
-                p2p.isend(g.tokens, 0)
+            sends = ((g.tokens, 0),)
         else:
-            def post():
-                p2p.isend(g.out_hidden, r + 1)
+            sends = ((g.out_hidden, r + 1),)
+
+        def post():
+            for t, dst in sends:
+                p2p.isend(t, dst)
         g.post_comm = post
         g.in_graph_comm = True
 

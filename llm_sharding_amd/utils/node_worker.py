@@ -45,6 +45,7 @@ import threading
 import os
 import sys
 import time
+import weakref
 from typing import Optional
 
 import torch
@@ -64,13 +65,15 @@ def _log(msg: str) -> None:
 
 
 class _EngineKV:
-    """``past_key_value`` view of the worker's static cache (``get_seq_length``)."""
+    """``past_key_value`` view of the worker's static cache (``get_seq_length``; 0 without one). The worker keeps the view and not the
+    view the worker: in a cycle a dropped worker's engine and captured graphs would live until the cyclic collector comes by."""
 
     def __init__(self, worker: "NodeWorker"):
-        self.w = worker
+        self._worker = weakref.ref(worker)
 
     def get_seq_length(self, layer_idx: int = 0) -> int:
-        return 0 if self.w.engine is None else int(self.w.engine.seq_len[0])
+        engine = getattr(self._worker(), "engine", None)
+        return 0 if engine is None else int(engine.seq_len[0])
 
 
 class NodeWorker:
