@@ -224,6 +224,14 @@ def test_full_depth_tripwire_catches_one_layer_perturbation(model):
 # fixture was made with them, and is not made again.
 EARLIER_PLANS = {(800, 4096, 4096): (256, 256, 1, 4, 256), (800, 22016, 4096): (256, 256, 1, 2, 256),
                  (800, 4096, 11008): (256, 256, 1, 4, 256)}
+# What both recordings below were made with, and a later table and model chose otherwise.
+KEPT_PLANS = {(800, 12288, 4096): (192, 256, 1, 0, 256), (160, 12288, 4096): (128, 256, 1, 8, 256),
+              (160, 4096, 4096): (128, 256, 1, 0, 128), (160, 22016, 4096): (128, 256, 1, 8, 256),
+              (160, 4096, 11008): (128, 256, 1, 0, 128), (160, 32000, 4096): (128, 256, 1, 1, 256)}
+EARLIER_PLANS.update(KEPT_PLANS)
+# The first choice of the fitted model, of tiles of 128 and 256 rows.
+FITTED_PLANS = {(800, 4096, 4096): (256, 256, 1, 2, 128), (800, 22016, 4096): (256, 256, 1, 2, 128),
+                (800, 4096, 11008): (256, 256, 1, 2, 128), **KEPT_PLANS}
 
 
 @pytest.mark.skipif(RECORD, reason="compared with a recording that stays")
@@ -242,3 +250,16 @@ def test_full_depth_7b_big_batch_in_earlier_plans(model, monkeypatch):
     cfg, eng, ref = model
     _compare("big_batch in earlier plans", _run(cfg, eng, ref, **BIG), fx)
     assert set(EARLIER_PLANS) <= used
+
+
+@pytest.mark.skipif(RECORD, reason="compared with a recording that stays")
+def test_full_depth_7b_big_batch_in_fitted_plans(model, monkeypatch):
+    """The same for the recording from before tiles of other heights were chosen."""
+    from llm_sharding_amd.ops import hip
+    plan, used = hip.gemm_sk_plan, set()
+    monkeypatch.setattr(hip, "gemm_sk_plan", lambda *a, **kw: (used.add(a[:3]), FITTED_PLANS.get(a[:3]) or plan(*a, **kw))[1])
+    with open(os.path.join(os.path.dirname(os.path.abspath(__file__)), "fixtures", "full_depth_7b_fitted_plans.json")) as fh:
+        fx = json.load(fh)["big_batch"]
+    cfg, eng, ref = model
+    _compare("big_batch in fitted plans", _run(cfg, eng, ref, **BIG), fx)
+    assert set(FITTED_PLANS) <= used
