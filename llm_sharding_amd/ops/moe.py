@@ -33,17 +33,19 @@ class Pick(ctypes.Structure):  # csrc/kernels/moe.h MoePick
 
 
 HEIGHTS = (128, 192, 256, 320)  # of the bf16 kernel's tiles of 256 columns (MOE_ROWS)
+# us of such a tile on every CU, as measured in the projection GEMM: a 64-deep K step, and its start and end; and what low ones take
+# more because they read an expert's weights more often
+HEIGHT_COST = ((0.84, 3.8, 1.06), (1.09, 6.1, 1.03), (1.36, 7.9, 1.0), (1.70, 9.9, 1.0))
 
 
 @functools.lru_cache(maxsize=256)
 def pick(*products) -> Optional[Pick]:
-    """What :func:`group` chooses a height from for both of the experts' products [(columns, k)]: the projection GEMM's costs of a
-    round of such tiles, a little more for low ones (they read an expert's weights more often); None: not for these."""
+    """What :func:`group` chooses a height from for both of the experts' products [(columns, k)]: what a round of such tiles takes;
+    None: not for these."""
     if any(n % 256 or k % 64 for n, k in products):
         return None
     p = Pick(tuple(n // 256 for n, _ in products))
-    for i, (h, more) in enumerate(zip(HEIGHTS, (1.06, 1.03, 1.0, 1.0))):
-        step, own = hip.SK_COST[(h, 256)]
+    for i, (step, own, more) in enumerate(HEIGHT_COST):
         p.step[i] = tuple(more * (k // 64 * step) for _, k in products)
         p.own[i] = more * own
     return p

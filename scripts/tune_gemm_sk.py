@@ -3,11 +3,11 @@
 runs (QKV: RoPE + KV append, o/down: residual add, gate_up: SwiGLU), weights rotated over
 > 600 MB of copies so they stream from HBM as in a decode step. Residual projections are also
 timed as split-K partials summed by the following norm (EPI_PARTIAL + resid_rmsnorm_partials)
-against the fused EPI_RESID + rmsnorm pair; the winner goes in the entry's "partial" field. Both row-tile
-heights (bm 256 / 128) are swept. Writes the winners to
-llm_sharding_amd/ops/gemm_sk_tuning.json, which hip.gemm_sk_plan consults before its cost model.
+against the fused EPI_RESID + rmsnorm pair; the winner goes in the entry's "partial" field. Every tile of
+hip.SK_COST is swept. Writes llm_sharding_amd/ops/gemm_sk_tuning.json, which hip.gemm_sk_plan consults before its
+cost model: a winner ("cfg") only where it is more than 1 % faster than that model's choice.
 
-usage: tune_gemm_sk.py [--rows 256,512,...] [--models llama2-7b,...] [--out PATH] [--iters N]
+usage: tune_gemm_sk.py [--rows 256,512,...] [--models llama2-7b,...] [--out PATH] [--iters N] [--no-partial]
 One JSON line per (model, shape, M) on stdout with every candidate's time."""
 import argparse
 import json
@@ -80,20 +80,19 @@ def main():
                     out = torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
                     ep = hip.make_epi(out=out, resid=out, ldo=N, ldr=N)
                 res = []
-                for bm in (256, 128):
-                    for bn in (256, 192, 128):
-                        if N % (16 if bn == 192 else bn):
+                plan = hip.gemm_sk_plan(M, N, K, tuned=False)
+                for bm, bn in hip.SK_COST:
+                    if N % (16 if bn == 192 else bn):
+                        continue
+                    # whole-tile rounds first, the remainder by split / stream-K, as a plan is launched
+                    for sp in sorted({*SPLITS, plan[3]} if (bm, bn) == (plan[4], plan[0]) else SPLITS):
+                        try:
+                            us = timeit(lambda i: hip.gemm_sk(x, ws[i % nbuf], M, N, K, epi, ep, bn=bn, grid=hip.N_CU,
+                                                              split=sp, ws=sk_ws, bm=bm), a.iters)
+                        except (RuntimeError, ValueError) as e:  # a config the host rejects for this shape
+                            print(f"# skip bm={bm} bn={bn} split={sp}: {e}", file=sys.stderr)
                             continue
-                        # dp 1: whole-tile rounds first, the remainder by split / stream-K; dp 0 (split 0):
-                        # pure stream-K over the whole grid (every CU busy when the tiles do not fill a round)
-                        for dp, sp in [(1, s_) for s_ in SPLITS] + [(0, 0)]:
-                            try:
-                                us = timeit(lambda i: hip.gemm_sk(x, ws[i % nbuf], M, N, K, epi, ep, bn=bn, grid=hip.N_CU,
-                                                                  dp=dp, split=sp, ws=sk_ws, bm=bm), a.iters)
-                            except (RuntimeError, ValueError) as e:  # a config the host rejects for this shape
-                                print(f"# skip bm={bm} bn={bn} dp={dp} split={sp}: {e}", file=sys.stderr)
-                                continue
-                            res.append((round(us, 2), bn, sp, bm, dp))
+                        res.append((round(us, 2), bn, sp, bm, 1))
                 res.sort()
                 partial = None
                 if epi == hip.EPI_RESID and 128 < M <= hip.PARTIAL_MAX_ROWS and not a.no_partial:
@@ -125,27 +124,31 @@ def main():
                             pres.append((round(timeit(part, a.iters), 2), bn, sp))
                     pres.sort()
                     partial = {"fused_us": round(t_fused, 2), "best": pres[0] if pres else None, "all": pres}
-                plan = hip.gemm_sk_plan(M, N, K, tuned=False)
-                model_us = next((r[0] for r in res if (r[1], r[2], r[3], r[4]) == (plan[0], plan[3], plan[4], plan[2])),
-                                None)
+                model_us = next(r[0] for r in res if (r[1], r[2], r[3], r[4]) == (plan[0], plan[3], plan[4], plan[2]))
                 fl = 2.0 * M * N * K
                 line = {"model": model, "shape": name, "N": N, "K": K, "M": M, "epi": epi,
                         "best_us": res[0][0], "best": [res[0][1], hip.N_CU, res[0][4], res[0][2], res[0][3]],
                         "best_tflops": round(fl / res[0][0] / 1e6, 1), "cost_model_us": model_us,
                         "all": res, "partial": partial}
                 print(json.dumps(line), flush=True)
-                entries = [e for e in entries if (e["N"], e["K"], e["M"]) != (N, K, M)]
-                ent = {"N": N, "K": K, "M": M, "cfg": line["best"], "us": res[0][0]}
+                before = [e for e in entries if (e["N"], e["K"], e["M"]) == (N, K, M)]
+                entries = [e for e in entries if e not in before]
+                ent = {"N": N, "K": K, "M": M}
+                if res[0][0] < 0.99 * model_us:
+                    ent.update(cfg=line["best"], us=res[0][0])
+                ent.update({"partial": e["partial"] for e in before if "partial" in e})  # (kept with --no-partial)
                 if partial is not None:  # [bn, split] when partials + fused norm beat EPI_RESID + norm
                     pb = partial["best"]
                     ent["partial"] = [pb[1], pb[2]] if pb and pb[0] < partial["fused_us"] else None
-                entries.append(ent)
+                if len(ent) > 3:
+                    entries.append(ent)
             del ws
             torch.cuda.empty_cache()
     entries.sort(key=lambda e: (e["N"], e["K"], e["M"]))
-    with open(a.out, "w") as f:
-        json.dump({"note": "gemm_sk (bn, grid, dp, split) per (N, K, M), measured by scripts/tune_gemm_sk.py "
-                           "on MI355X with the engine's epilogues", "entries": entries}, f, indent=0)
+    with open(a.out, "w") as f:  # an entry a line
+        f.write('{"note": "gemm_sk (bn, grid, dp, split, bm) per (N, K, M) where it beats the cost model\'s choice, measured by '
+                'scripts/tune_gemm_sk.py on MI355X with the engine\'s epilogues",\n"entries": [\n'
+                + ",\n".join(map(json.dumps, entries)) + "\n]}\n")
 
 
 if __name__ == "__main__":

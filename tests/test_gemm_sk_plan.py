@@ -75,3 +75,38 @@ def test_cost_model_takes_the_cheapest_of_what_the_kernel_accepts():
                 cost = hip.gemm_sk_cost(M, N, K, bm, bn, split)
                 for b in (x for x in hip.SK_COST if N % (16 if x[1] == 192 else x[1]) == 0 and not (whole64 and x[1] == 192)):
                     assert cost <= hip.gemm_sk_cost(M, N, K, *b, 1) + 1e-6
+
+
+def test_choice_is_no_slower_than_the_one_of_two_heights():
+    """Every product that the model was fitted to, by its measured times (profiles/cost_gemm_sk.csv): against the choice of the model
+    before, of tiles of 128 and 256 rows, none takes more than 1.05 times as long, and all together take 0.984 of it at most."""
+    import csv
+    import math
+    import os
+    tiles = {(256, 256): (1.39, 6.3), (256, 192): (1.12, 4.7), (256, 128): (0.83, 2.9),
+             (128, 256): (0.85, 2.9), (128, 192): (0.72, 2.4), (128, 128): (0.55, 1.5)}
+
+    def before(M, N, K, bm, bn, split):
+        (step, own), nkt, slab = tiles[(bm, bn)], K // 64, bm * bn * 4 / 1e5
+        rounds, rem = divmod(-(-M // bm) * -(-N // bn), 256)
+        us = 5.5 + rounds * (nkt * step + own)
+        if rem and split:
+            us += -(-nkt // split) * step * (1 - 0.36 * (1 - min(256, rem * split) / 256)) + own
+            us += 2.1 + 1.5 * slab * (split if split > 2 else 1) if split > 1 else 0
+        elif rem:
+            us += rem * nkt / 256 * step * 1.6 + own * max(1.0, rem / 256) + 2.1 + 1.5 * slab * min(max(256 / rem, 1.0), 8.0)
+        return max(us, 5.5 + N * K * 2 / 5e6)
+    times = {}
+    with open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "profiles", "cost_gemm_sk.csv")) as fh:
+        for r in csv.DictReader(fh):
+            times.setdefault(tuple(int(r[c]) for c in "mnk"), {})[int(r["bm"]), int(r["bn"]), int(r["split"])] = float(r["us"])
+    ratio = {}
+    for (M, N, K), t in times.items():
+        bn, _, _, split, bm = hip.gemm_sk_plan(M, N, K, tuned=False)
+        if -(-M // bm) * -(-N // bn) % hip.N_CU == 0:
+            split = 1
+        old = min((c for c in t if c[:2] in tiles), key=lambda c: before(M, N, K, *c))
+        ratio[M, N, K] = t[bm, bn, split] / t[old]
+    assert len(ratio) == 378
+    assert max(ratio.values()) <= 1.05, sorted(ratio.items(), key=lambda x: -x[1])[:5]
+    assert math.exp(sum(map(math.log, ratio.values())) / len(ratio)) <= 0.984
