@@ -422,8 +422,8 @@ struct Kern {
   LSA_DEVICE void slab_add(const float* slab, size_t slot, f32x4_t (&acc)[FM][FN]) {
     const int lane = fresh(this->lane);
     // RP tile rows (PB blocks) per pass, NP passes, DB ring buffers per wave: as much in flight
-    // as this geometry's LDS allows (the ring must stay below the flag word at SMEM - 16)
-    constexpr int AVAIL = G_::SMEM - 16;
+    // as this geometry's LDS allows (the ring must end at the tile's row scales, which are made before the sum is)
+    constexpr int AVAIL = G_::RS_OFF;
     constexpr int RP = (FN <= 4 && FM % 2 == 0 && 8 * 2 * 2 * FN * 1024 <= AVAIL) ? 2 : 1;
     constexpr int NP = FM / RP, PB = RP * FN;
     constexpr int DB = (NP > 1 && 8 * 2 * PB * 1024 <= AVAIL) ? 2 : 1;
