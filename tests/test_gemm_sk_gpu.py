@@ -331,3 +331,43 @@ def test_gemm_llama70b_projections_at_512_rows(name, N, K, epi):
         want = F.silu(g) * u
     torch.cuda.synchronize()
     assert rel_err(out, want) < 1e-2, name
+
+
+@pytest.mark.parametrize("split", [0, 1, 2, 4])
+@pytest.mark.parametrize("bm,bn", [(320, 256), (192, 256), (384, 192), (384, 128), (256, 256)])
+def test_gemm_sk_row_scales_over_several_tiles(bm, bn, split, ws):
+    """The fused norm's row scales where a workgroup has two whole tiles and then a part of a third: they are made at the start of
+    each tile, outlive the sum of its partial sums and give way to the next tile's. Neighbouring rows differ by powers of two, and
+    every row is compared by itself. Outputs are rounded to bf16 once (2^-9 of a value); twice that and the sums are 8e-3."""
+    from llm_sharding_amd.config import tiny
+    from llm_sharding_amd.models.rope import rope_table
+    h = hip()
+    M, K, nh, nkv, hd, T, eps = 2 * bm + 17, 1024, 8, 2, 128, 1024, 1e-5
+    N = (nh + 2 * nkv) * hd
+    tiles = 3 * (N // bn)
+    kw = dict(ws=ws, bm=bm, bn=bn, grid=(tiles - 2) // 2, split=split)  # two rounds, and two tiles in ``split`` parts
+    hb = (_rnd(M, K).float() * torch.pow(2.0, (torch.arange(M, device=DEV) * 7 % 9 - 4).float())[:, None]).bfloat16()
+    ss = hb.float().pow(2).view(M, K // 64, 64).sum(-1)
+    xn = hb.float() * torch.rsqrt(hb.float().pow(2).mean(-1, keepdim=True) + eps)
+
+    def off(got, want):
+        return ((got.float() - want).norm(dim=-1) / want.norm(dim=-1)).max().item()
+    wg, wu = _rnd(N // 2, K, scale=0.03), _rnd(N // 2, K, scale=0.03)
+    out = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+    h.gemm_sk(hb, packing.pack_b(packing.fuse_gate_up(wg, wu)), M, N, K, h.EPI_SWIGLU,
+              h.make_epi(out=out, ldo=N // 2, ss_in=ss, ss_eps=eps), **kw)
+    assert off(out, F.silu(xn @ wg.float().T) * (xn @ wu.float().T)) < 8e-3
+    wq, wk, wv = (_rnd(n * hd, K, scale=0.03) for n in (nh, nkv, nkv))
+    cos, sin = rope_table(tiny(head_dim=hd), T, DEV)
+    slot, pos = torch.zeros(M, dtype=torch.int32, device=DEV), torch.randperm(T, device=DEV)[:M].to(torch.int32)
+    q = torch.full((M, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    kc, vc = (torch.zeros(1, nkv, T, hd, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    h.gemm_sk(hb, packing.pack_b(packing.fuse_qkv(wq, wk, wv, nh, nkv, hd)), M, N, K, h.EPI_QKV,
+              h.make_epi(out=q, k_cache=kc, v_cache=vc, slot=slot, pos=pos, cos=cos, sin=sin, ldo=nh * hd, n_heads=nh, n_kv=nkv,
+                         head_dim=hd, t_max=T, ss_in=ss, ss_eps=eps), **kw)
+    pl = pos.long()
+    assert off(q, _rope_ref((xn @ wq.float().T).view(M, nh, hd), pl, cos, sin).reshape(M, -1)) < 8e-3
+    assert off(kc[0, :, pl].transpose(0, 1).reshape(M, -1),
+               _rope_ref((xn @ wk.float().T).view(M, nkv, hd), pl, cos, sin).reshape(M, -1)) < 8e-3
+    assert off(vc[0, :, pl].transpose(0, 1).reshape(M, -1), xn @ wv.float().T) < 8e-3
+    assert int(ws.counters.abs().sum()) == 0
