@@ -304,7 +304,7 @@ template <int HD, int HPW>
 __global__ __launch_bounds__(NTHR, 2) void flash_prefill_kernel(
     const bf16_raw* __restrict__ q, int ldq, const bf16_raw* __restrict__ kc, const bf16_raw* __restrict__ vc,
     const PrefillTile* __restrict__ tiles, int n_heads, int n_kv, int t_max, float scale_log2, int causal,
-    bf16_raw* __restrict__ out, int ldo) {
+    bf16_raw* __restrict__ out, int ldo, int paired) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[NBUF * 2 * BKV * HD * 2];  // [buffer][K | V]
 
   // work item -> (tile, head group). XCD-aware when the group count is a multiple of 8: XCD x
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(NTHR, 2) void flash_prefill_kernel(
   int tix, grp;
   if (n_groups % 8 == 0) {
     const int x = blockIdx.x % 8, ngx = n_groups / 8;
-    const int j = pair_up(blockIdx.x / 8, n_tiles * ngx);
+    const int j = pair_up(blockIdx.x / 8, paired);
     tix = j / ngx;
     grp = (j % ngx) * 8 + x;
   } else {
@@ -334,21 +334,23 @@ __global__ __launch_bounds__(NTHR, 2) void flash_prefill_kernel(
 
 template <int HD, int HPW>
 void launch_prefill(const bf16_raw* q, int ldq, const bf16_raw* k, const bf16_raw* v, const PrefillTile* t,
-                    int n_tiles, int n_heads, int n_kv, int t_max, float sl2, int causal, bf16_raw* o, int ldo,
+                    int n_tiles, int n_heads, int n_kv, int t_max, float sl2, int causal, bf16_raw* o, int ldo, int keys,
                     hipStream_t stream) {
-  dim3 grid(n_tiles * (n_heads / HPW)), block(NTHR);
-  flash_prefill_kernel<HD, HPW><<<grid, block, 0, stream>>>(q, ldq, k, v, t, n_heads, n_kv, t_max, sl2, causal, o, ldo);
+  const int n_groups = n_heads / HPW;
+  dim3 grid(n_tiles * n_groups), block(NTHR);
+  flash_prefill_kernel<HD, HPW><<<grid, block, 0, stream>>>(q, ldq, k, v, t, n_heads, n_kv, t_max, sl2, causal, o, ldo,
+                                                            n_groups % 8 ? 0 : pairs((long long)n_tiles * (n_groups / 8), keys));
 }
 
 template <int HD>
 int dispatch_hpw(int hpw, const bf16_raw* q, int ldq, const bf16_raw* k, const bf16_raw* v, const PrefillTile* t,
-                 int n_tiles, int n_heads, int n_kv, int t_max, float sl2, int causal, bf16_raw* o, int ldo,
+                 int n_tiles, int n_heads, int n_kv, int t_max, float sl2, int causal, bf16_raw* o, int ldo, int keys,
                  hipStream_t stream) {
   switch (hpw) {
-    case 1: launch_prefill<HD, 1>(q, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, stream); break;
-    case 2: launch_prefill<HD, 2>(q, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, stream); break;
-    case 4: launch_prefill<HD, 4>(q, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, stream); break;
-    case 8: launch_prefill<HD, 8>(q, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, stream); break;
+    case 1: launch_prefill<HD, 1>(q, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, keys, stream); break;
+    case 2: launch_prefill<HD, 2>(q, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, keys, stream); break;
+    case 4: launch_prefill<HD, 4>(q, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, keys, stream); break;
+    case 8: launch_prefill<HD, 8>(q, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, keys, stream); break;
     default: return LSA_UNSUPPORTED;
   }
   return LSA_OK;
@@ -579,7 +581,7 @@ int launch_gqa_decode(int nw, const bf16_raw* q, int ldq, const bf16_raw* k, con
 }  // namespace
 
 // tiles: device array of n_tiles PrefillTile {row0, nrows, slot, pos0, kvlen, pad x3}; nrows <=
-// lsa_prefill_tile_rows(n_heads, n_kv) (128 / heads-per-workgroup).
+// lsa_prefill_tile_rows(n_heads, n_kv) (128 / heads-per-workgroup). keys: the most that a tile has (pairs, common.h).
 extern "C" int lsa_prefill_tile_rows(int n_heads, int n_kv) {
   if (n_kv < 1 || n_heads % n_kv) return 0;
   const int g = n_heads / n_kv;
@@ -588,7 +590,7 @@ extern "C" int lsa_prefill_tile_rows(int n_heads, int n_kv) {
 
 extern "C" int lsa_attn_prefill(const void* q, int ldq, const void* kc, const void* vc, const void* tiles, int n_tiles,
                                 int n_heads, int n_kv, int head_dim, int t_max, float scale, int causal, void* out,
-                                int ldo, hipStream_t stream) {
+                                int ldo, int keys, hipStream_t stream) {
   if (n_tiles < 1 || n_kv < 1 || n_heads % n_kv || n_heads < 1) return LSA_BAD_SHAPE;
   const float sl2 = scale * 1.4426950408889634f;
   const int g = n_heads / n_kv, hpw = (GROUPS % g == 0) ? g : 1;
@@ -599,9 +601,9 @@ extern "C" int lsa_attn_prefill(const void* q, int ldq, const void* kc, const vo
   auto* o = static_cast<bf16_raw*>(out);
   int rc;
   if (head_dim == 128)
-    rc = dispatch_hpw<128>(hpw, qq, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, stream);
+    rc = dispatch_hpw<128>(hpw, qq, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, keys, stream);
   else if (head_dim == 64)
-    rc = dispatch_hpw<64>(hpw, qq, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, stream);
+    rc = dispatch_hpw<64>(hpw, qq, ldq, k, v, t, n_tiles, n_heads, n_kv, t_max, sl2, causal, o, ldo, keys, stream);
   else
     return LSA_UNSUPPORTED;
   if (rc != LSA_OK) return rc;

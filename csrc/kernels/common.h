@@ -61,10 +61,15 @@ LSA_DEVICE u32x4_t pack8(const float* f) {
   return r;
 }
 
-// Item for the i-th workgroup of n of an XCD, items by falling work: where its 32 CUs take them in two rows (two workgroups a CU),
-// the second row comes in rising order, so that the heaviest shares its CU with the lightest (flash attention of one prompt of 2048,
-// 32 heads: 67.0 -> 65.5 us; by turns heavy and light, as if neighbours shared a CU, 70; paged attention of three of 1100, 16 heads, 51 -> 47).
-LSA_DEVICE int pair_up(int i, int n) { return n > 32 && n <= 64 && i >= 32 ? n + 31 - i : i; }
+// Item for the i-th workgroup of an XCD, items by falling keys: where its 32 CUs take them in two rows, the second row comes in
+// rising order, so that the heaviest shares its CU with the lightest. n: the items, 0 where they are not 33 to 64 or where no tile has
+// PAIR_KEYS keys (pairs, on the host). One prompt of 2048, flash attention of 32 heads of 128: 58.7 -> 56.0 us, 32 on 8 of 64 dimensions, of
+// which three or four workgroups share a CU, 43.2 -> 41.2; paged attention, three of 1100 with 16 heads, 45 -> 42.5. Below the line the tiles
+// with most keys are the prompts' short last ones: five prompts of 301 took 16.9 us instead of 16.2 (paged: 20.0, 18.2).
+// By turns heavy and light, as if neighbours shared a CU, is slower (70 us where the plain order took 67).
+constexpr int PAIR_KEYS = 1024;
+LSA_DEVICE int pair_up(int i, int n) { return i >= 32 && i < n ? n + 31 - i : i; }
+inline int pairs(long long items, int keys) { return items > 32 && items <= 64 && keys >= PAIR_KEYS ? (int)items : 0; }
 
 LSA_DEVICE bf16x8_t as_frag(u32x4_t v) { return __builtin_bit_cast(bf16x8_t, v); }
 

@@ -31,7 +31,7 @@ LSA_DEVICE void glds16(const void* src, unsigned char* lds_base) {
 template <int DK, int DV, bool SIG>
 __global__ __launch_bounds__(NTHR, DK + DV <= 256 ? 4 : 2) void attn_tiles_kernel(
     AttnArgs a, const AttTile* __restrict__ tiles, const bf16_raw* __restrict__ q, int ldq,
-    const bf16_raw* __restrict__ gate, int ldg, bf16_raw* __restrict__ out, int ldo) {
+    const bf16_raw* __restrict__ gate, int ldg, bf16_raw* __restrict__ out, int ldo, int paired) {
   constexpr int KF = DK / 32, DT = DV / 16, NCK = DK / 8, NCV = ATT_PAGE / 8;
   constexpr int KBLK = ATT_PAGE * DK * 2, VBLK = ATT_PAGE * DV * 2;
   constexpr int KPW = KBLK / 1024 / NWV, VPW = VBLK / 1024 / NWV;  // DMA pieces per wave
@@ -41,7 +41,7 @@ __global__ __launch_bounds__(NTHR, DK + DV <= 256 ? 4 : 2) void attn_tiles_kerne
   const int H = a.heads, n_tiles = gridDim.x / H;
   int tix, head;
   if (H % 8 == 0) {  // one XCD's workgroups share heads of one kv head: its pages stay in that L2
-    const int x = blockIdx.x % 8, hx = H / 8, j = DK + DV <= 256 ? pair_up(blockIdx.x / 8, n_tiles * hx) : blockIdx.x / 8;
+    const int x = blockIdx.x % 8, hx = H / 8, j = pair_up(blockIdx.x / 8, paired);
     tix = j / hx;
     head = x * hx + j % hx;
   } else {
@@ -234,8 +234,8 @@ __global__ __launch_bounds__(NTHR, DK + DV <= 256 ? 4 : 2) void attn_tiles_kerne
 
 }  // namespace
 
-// tiles: n_tiles {row0, nrows <= 128, slot, pos0}; every position's page is in the table
-extern "C" int lsa_attn_tiles(const AttnArgs* a, const void* tiles, int n_tiles, const void* q, int ldq, const void* gate,
+// tiles: n_tiles {row0, nrows <= 128, slot, pos0}; every position's page is in the table; keys: the most that a tile has
+extern "C" int lsa_attn_tiles(const AttnArgs* a, const void* tiles, int n_tiles, int keys, const void* q, int ldq, const void* gate,
                               int ldg, void* out, int ldo, hipStream_t s) {
   if (!a || !a->k || !a->v || !a->table || !a->hscale || n_tiles < 1 || a->max_pages < 1 || a->n_pages < 1 ||
       a->heads < 1 || a->kv_heads < 1 || a->heads % a->kv_heads || a->window < 1 || a->keep < 0 || a->softcap < 0.f ||
@@ -246,11 +246,12 @@ extern "C" int lsa_attn_tiles(const AttnArgs* a, const void* tiles, int n_tiles,
       ((uintptr_t)q | (uintptr_t)a->k | (uintptr_t)a->v) % 16 || (uintptr_t)out % 8)
     return LSA_BAD_SHAPE;
   const dim3 grid(n_tiles * a->heads);
+  const int paired = a->dkp + a->dvp > 256 || a->heads % 8 ? 0 : pairs((long long)n_tiles * (a->heads / 8), keys);  // two a CU
 #define LSA_T(K, V)                                                                                                   \
   if (a->dkp == K && a->dvp == V) {                                                                                   \
     auto* f = a->sig ? attn_tiles_kernel<K, V, true> : attn_tiles_kernel<K, V, false>;                                \
     f<<<grid, NTHR, 0, s>>>(*a, (const AttTile*)tiles, (const bf16_raw*)q, ldq, (const bf16_raw*)gate, ldg,           \
-                            (bf16_raw*)out, ldo);                                                                     \
+                            (bf16_raw*)out, ldo, paired);                                                             \
     LSA_CHECK_LAUNCH();                                                                                               \
     return LSA_OK;                                                                                                    \
   }

@@ -169,11 +169,11 @@ def rows(a: AttnArgs, n: int, q, gate, out, ns: int, po, pm) -> None:
         _check(lib().lsa_attn_merge(ctypes.byref(a), n, _p(po), _p(pm), ns, *io[2:], _stream()), "lsa_attn_merge")
 
 
-def tiles(a: AttnArgs, tiles_dev, q, gate, out) -> None:
-    """Attention of the rows of checked tiles [row0, rows, slot, pos0], bf16."""
+def tiles(a: AttnArgs, tiles_dev, q, gate, out, keys: int = ALL) -> None:
+    """Attention of the rows of checked tiles [row0, rows, slot, pos0], those with most keys first, bf16. ``keys``: of the first."""
     _req(tiles_dev.dtype == torch.int32 and tiles_dev.dim() == 2 and tiles_dev.shape[1] == 4 and tiles_dev.is_contiguous(),
          "attention tiles: table")
-    _check(lib().lsa_attn_tiles(ctypes.byref(a), _p(tiles_dev), tiles_dev.shape[0],
+    _check(lib().lsa_attn_tiles(ctypes.byref(a), _p(tiles_dev), tiles_dev.shape[0], keys,
                                 *_shapes(a, q, gate, out, torch.bfloat16), _stream()), "lsa_attn_tiles")
 
 
@@ -190,5 +190,5 @@ def declare(L: ctypes.CDLL) -> None:
         "lsa_attn_plain": [i, aa, i, i] + io + [vp],
         "lsa_attn_rows": [aa, i] + io + [i, vp, vp, vp],
         "lsa_attn_merge": [aa, i, vp, vp, i, vp, i, vp, i, vp],
-        "lsa_attn_tiles": [aa, vp, i] + io + [vp],
+        "lsa_attn_tiles": [aa, vp, i, i] + io + [vp],
     })

@@ -129,7 +129,7 @@ class Attention:
             if m:
                 A.pool(a if done is None else args(done), inp.dtype, m)
         if long:
-            A.tiles(a, tiles, q, gate, ao)
+            A.tiles(a, tiles, q, gate, ao, plan.longest)
         if n and self.tuned:
             A.rows(b, n, q, gate, ao, self.key_splits(eng, n, plan.longest), eng.part_o, eng.part_ml)
         elif n:

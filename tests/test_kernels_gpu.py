@@ -639,6 +639,21 @@ def test_attention_prefill_edges_of_tiles(nh, nkv, hd, causal):
     assert float(((out.float() - ref).norm(dim=1) / ref.norm(dim=1)).max()) < 3e-2
 
 
+@pytest.mark.parametrize("rows", [1023, 1024, 1537])
+@pytest.mark.parametrize("nh,hd", [(40, 64), (32, 128), (8, 64)])
+def test_attention_prefill_of_tiles_in_two_rows(nh, hd, rows):
+    """Tiles that share their CU with another one are taken in an order of their own from 1024 keys on: 40 to 65 of an XCD, and fewer
+    than it has CUs. Limits as above."""
+    h = hip()
+    kc, vc, q = _rnd(1, nh, rows, hd), _rnd(1, nh, rows, hd), _rnd(rows, nh * hd)
+    out = torch.full((rows, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    h.attn_prefill(q, kc, vc, h.build_prefill_tiles([0] * rows, list(range(rows)), device=DEV), nh, nh, hd, out)
+    assert not out.isnan().any()
+    idx = torch.tensor(list(range(3, rows, 64)) + [rows - 1])
+    ref = _prefill_ref(q[idx], kc, vc, [0] * len(idx), idx.tolist(), nh, nh, hd, None)
+    assert float(((out[idx].float() - ref).norm(dim=1) / ref.norm(dim=1)).max()) < 2e-2
+
+
 @pytest.mark.parametrize("cfg", packing.FP8_CONFIGS)
 def test_gemv_fp8_every_config(cfg):
     """W8A16 GEMV (OCP e4m3 weights, per-row scales, bf16 MFMA after in-register conversion)
