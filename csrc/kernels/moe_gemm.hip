@@ -59,9 +59,9 @@ __global__ __launch_bounds__(NTHR) void moe_gemm_kernel(const MoeTile* __restric
 // they are counted and not before: 32 experts of 1024 x 2048 with 900 pairs each are 127 tiles of 256 rows, four rounds in either
 // product, and 96 of 320, three (365 -> 330 us); with 700 each 96 and 96. One workgroup a CU takes tile after tile of its
 // XCD's (as above): with one for as many as there could be of the lowest, those too many held a CU for 1.5 us each and made 470 us of 64
-// experts with 1100 pairs 495. Four lists of experts, 200 to 1500 pairs each, evenly and unevenly drawn: 0.93 times the
-// time of 128 rows up to 320 pairs an expert and 256 above, which the host chose (0.70 to 1.03 times; by the mean it could get to
-// 0.98). Tiles of several heights in one table, to fill all but 64 rows of an expert's, were slower on average (0.97).
+// experts with 1100 pairs 495. Four lists of experts, 200 to 1500 pairs each, evenly and unevenly drawn (profiles/cost_moe_bf16.csv): 0.94
+// times the time of 128 rows up to 320 pairs an expert and 256 above, which the host chose (0.72 to 1.03 times; by the mean it could
+// get to 0.98). Tiles of several heights in one table, to fill all but 64 rows of an expert's, were slower on average (0.97).
 template <int BM, int UP>
 LSA_DEVICE void moe_tiles(unsigned char* smem, const MoeTile* __restrict__ tiles, const int* __restrict__ order, int top,
                           const bf16_raw* __restrict__ A, const bf16_raw* __restrict__ W, SkParams& prm, const EpiArgs& ep) {

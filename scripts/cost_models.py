@@ -107,6 +107,17 @@ def main() -> None:
         off = [float(r[name + "_us"]) / float(r["two_heights_us"]) for r in rows]
         print(f"gemm_sk, products it was not fitted to, {name} / two_heights: {math.exp(sum(map(math.log, off)) / len(off)):.3f}, "
               f"worst {max(off):.2f}, {sum(x > 1.05 for x in off)} of {len(off)} more than 1.05")
+    def against(name, file, now, other):
+        with open(os.path.join(ROOT, "profiles", file)) as fh:
+            off = [float(now(r)) / float(other(r)) for r in csv.DictReader(fh)]
+        print(f"{name}: {math.exp(sum(map(math.log, off)) / len(off)):.3f}, {min(off):.2f} to {max(off):.2f}, {len(off)} cases")
+    for what, other in (("two heights by the mean", lambda r: r["us_two_heights"]),
+                        ("the fastest of four", lambda r: min(float(r[f"us_{h}"]) for h in (128, 192, 256, 320)))):
+        against(f"experts' height picked / {what}", "cost_moe_bf16.csv", lambda r: r["us_picked"], other)
+    for w in ("32", "64"):
+        against(f"delta rule's scan by its rule / always {w} channels", "delta_scan_width.csv", lambda r: r["us_by_the_rule"],
+                lambda r: r[f"us_{w}"])
+    against("prompt attention by its rule / plain order", "prompt_order.csv", lambda r: r["us_by_the_rule"], lambda r: r["us_plain_order"])
     products = load("cost_coop.csv", 3)
     for name, pick in (("the model", coop), ("smallest split that fills", fills)):
         for rows in (24, 48, 65, 96, 100, 128):
