@@ -51,6 +51,12 @@ def pick(*products) -> Optional[Pick]:
     return p
 
 
+def heights(pairs: int, experts: int, rows: int, f32, *products) -> Optional[Pick]:
+    """:func:`pick` where the height is picked when the pairs are counted: bf16 tiles of ``rows`` >= 128, in tables that lsa_moe_group
+    takes with heights (2^19 tiles of the lowest). None: tiles of ``rows``."""
+    return pick(*products) if rows >= 128 and not f32 and max_tiles(pairs, experts, HEIGHTS[0]) < 1 << 19 else None
+
+
 def route_args(s=None, correction=None) -> RouteArgs:
     """How the experts of ``s`` (a MoeSpec; None: softmax over the largest logits) are chosen."""
     if s is None:

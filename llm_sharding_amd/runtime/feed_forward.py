@@ -143,7 +143,7 @@ class Moe:
         weight, tiles = eng.scratch_view("pair_w", rows, s.top).reshape(-1), eng.scratch_view("tiles", rows, 8 * s.top)
         act, ye = eng.scratch_view("act", pairs, x.ff), eng.scratch_view("ye", pairs, x.width)
         tr = X.tile_rows(pairs, s.experts, x.f32, min(x.up_n, x.width))
-        heights = X.pick((x.up_n, x.width), (x.width, x.ff)) if tr >= 128 and not x.f32 else None
+        heights = X.heights(pairs, s.experts, tr, x.f32, (x.up_n, x.width), (x.width, x.ff))
         nt = X.route_group(in32[:, col["router"]:], rows, s.experts, s.top, tr if heights is None else X.HEIGHTS[0], expert, weight,
                            order, place, tiles, self.how, spare, heights)
         tr = tr if heights is None else 0

@@ -272,3 +272,14 @@ def test_row_tables_from_runs(runs):
     assert s.tolist() == slot and p.tolist() == pos
     with pytest.raises(RuntimeError):
         hip.row_tables(np.array([0, 0]), np.array([5, 2 ** 31]), "cuda")
+
+
+def test_expert_tables_too_long_for_a_picked_height():
+    """The sorting kernel takes 2^19 - 1 tiles with heights; longer tables have tiles of 256 rows, as without them."""
+    from llm_sharding_amd.ops import moe as X
+    products = (512, 256), (256, 256)
+    most = ((1 << 19) - 1 - 32) * 128
+    assert X.heights(most, 32, 256, False, *products) is not None and X.heights(most + 128, 32, 256, False, *products) is None
+    assert X.max_tiles(most + 128, 32, 256) <= 1 << 20  # (of the experts' products)
+    for rows, f32, cols in ((64, False, 512), (256, True, 512), (256, False, 640)):
+        assert X.heights(4096, 32, rows, f32, (cols, 256), (256, 256)) is None
