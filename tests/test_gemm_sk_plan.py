@@ -78,8 +78,9 @@ def test_cost_model_takes_the_cheapest_of_what_the_kernel_accepts():
 
 
 def test_choice_is_no_slower_than_the_one_of_two_heights():
-    """Every product that the model was fitted to, by its measured times (profiles/cost_gemm_sk.csv): against the choice of the model
-    before, of tiles of 128 and 256 rows, none takes more than 1.05 times as long, and all together take 0.984 of it at most."""
+    """Every product that the model was fitted to and the planner is asked for (gemm_wr has some), by its measured times
+    (profiles/cost_gemm_sk.csv): against the choice of the model before, of tiles of 128 and 256 rows, none takes more than 1.05 times
+    as long, and all 378 together take 0.984 of it at most."""
     import csv
     import math
     import os
@@ -108,5 +109,6 @@ def test_choice_is_no_slower_than_the_one_of_two_heights():
         old = min((c for c in t if c[:2] in tiles), key=lambda c: before(M, N, K, *c))
         ratio[M, N, K] = t[bm, bn, split] / t[old]
     assert len(ratio) == 378
-    assert max(ratio.values()) <= 1.05, sorted(ratio.items(), key=lambda x: -x[1])[:5]
+    asked = {k: r for k, r in ratio.items() if hip.gemm_wr_plan(*k, hip.EPI_STORE, hip.EpiArgs()) is None}
+    assert max(asked.values()) <= 1.05, sorted(asked.items(), key=lambda x: -x[1])[:5]
     assert math.exp(sum(map(math.log, ratio.values())) / len(ratio)) <= 0.984
