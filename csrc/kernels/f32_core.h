@@ -4,7 +4,7 @@
 // From row-major weights (16 pieces of 64 bytes) 16 rows took N = K = 2048 10.5 instead of 8.3 us, N = 8704 27.7 instead of 20.3,
 // N = 32000 72 instead of 50. The sum over k runs in the order of that layout, the same for A and W.
 //
-// Three forms, chosen by the caller:
+// Two forms, chosen by the caller:
 //   F32Stream  few rows, on the fp32 matrix instructions (v_mfma_f32_*_f32: true fp32 products and sums): a lane loads four
 //              consecutive k and gives them to four instructions in turn; the weights go once from memory to operand registers;
 //              the waves of a workgroup share K and meet in LDS. Bound by launch and one round trip, then by reading the weights:
@@ -18,12 +18,6 @@
 //              Errors against 64 bits are lower than those of fp32 instructions, since a sum is rounded once for 32 k instead
 //              of once for 2 (the five smaller products have sums of their own): K = 2048 3.3e-7 to 5.7e-7 -> 1.1e-7 to 2.7e-7 of the
 //              result's norm, K = 8192 6.6e-7 to 1.15e-6 -> 2.2e-7 to 5.7e-7. With all six in one sum it was 7e-7.
-//   F32Pair    the same in two fp16 pieces of values scaled row by row and column by column, three products and half of the splitting:
-//              for sums long enough to be no further off. Of the same products 812 -> 508 us (306 -> 338 TFLOP/s at K = 4096), 963
-//              rows, N = 16384 311 -> 208, N = 2048 52.7 -> 41.1, K = 8192 175 -> 128, with 4 to 12 us for the rows' exponents; errors
-//              2.7e-7 -> 1.45e-7 (K = 2048), 2.8e-7 -> 1.6e-7 (8192). Bound by the chip's power (zeros instead of random numbers 384 us at the
-//              full clock), and then by the LDS and vector instructions beside a matrix unit that is busy for 53 % of the time: reads from
-//              LDS further ahead, the compiler's own order and raised priorities of half of the waves made no difference.
 #pragma once
 #include "elem.h"
 #include "mfma_pair.h"
@@ -140,13 +134,7 @@ struct F32Split {
     for (int n = 0; n < NT; ++n) w2[n] = wr[n] + from * 16;
     sums([&](int r) { return row(r) + from; }, w2, steps, mine, last, lds + grp * 2 * BUF);
     whole([&](int r) { return row(r) + from; }, w2, mine * 32);
-    gather(lds);
-  }
-
-  // every group gets the others' sums of its rows
-  LSA_DEVICE void gather(u32x4_t* lds) {
-    if constexpr (KG > 1) {
-      const int grp = group();
+    if constexpr (KG > 1) {  // every group gets the others' sums of its rows
       static_assert(KG * (KG - 1) * MO * NT * NW * 64 <= LDS);
       const int at = wave() * 64 + (threadIdx.x & 63);
       auto part = [&](int to, int from, int m, int n) -> u32x4_t& {  // from: groups behind `to`
@@ -334,165 +322,5 @@ struct F32Split {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         f((group() * MO + m) * 16 + (lane >> 4) * 4 + r, wave() * 32 + (lane & 15), acc[m][0][r], acc[m][1][r]);
-  }
-};
-
-// How a row or column of a product in two pieces is scaled: by 2^exp, so that its largest value is from 2^14 up to 2^15. F32_WIDE: not to
-// be taken apart in two pieces; a tile that has such a row or column is made of three (F32Split). It holds infinities or NaN, its largest
-// value is under 2^-109, or more than a sixteenth of its values are not zero and less than 2^-17 of the largest, where the second piece
-// is in steps of 2^-25 and not of its value.
-constexpr int F32_WIDE = 1 << 20, F32_TOP = 14;
-// Of 32 k: in the shortest sum that is made of two pieces; in a sum of three pieces from which on two are no further off. Errors of
-// 2-norm, random operands: K = 2048 in one sum 2.7e-7 in three pieces and 1.45e-7 in two, of 32 1.9e-7 and 1.3e-7, of 16 1.27e-7 and
-// 1.1e-7, of 8 1.1e-7 and 1.3e-7.
-constexpr int PAIR_UNITS = 8, THREE_LONG = 16;
-
-// The tile of F32Split in two fp16 pieces, 11 + 11 bits and a sign between them, of values scaled by their row's and column's power of
-// two, and three products: 2^-24.3 of a product is lost in the pieces and 2^-24.8 with the product of the second ones (root mean
-// squares), together 0.6e-7 of a result of random operands. What the sums round is less than there in turn: the six products of 64 k are
-// a sum of their own, the small ones first, which then joins the others in one fp32 addition (K = 2048 in one sum: 64 additions on the
-// matrix unit, each rounded several times, are 2.7e-7). Sums of fewer than PAIR_UNITS steps would be further off than in three pieces.
-template <int MT, int NW, int KG>
-struct F32Pair : F32Split<MT, NW, KG> {
-  using B = F32Split<MT, NW, KG>;
-  using B::acc;
-  using B::SF;
-  static constexpr int NT = B::NT;
-  static constexpr int UNITS = 2 * (SF + NT);  // fragments of 32 k that a wave takes apart for a step of 64, the rows' first
-  static constexpr int AHEAD = 6;              // pairs of products between a fragment's read from LDS and its use
-  static constexpr int BUF = MT * 4 * 64;      // 64 k of the rows: fragments of (32 k, piece), 16 bytes a lane
-  static constexpr int EXPS = KG * 2 * BUF > B::LDS ? KG * 2 * BUF : B::LDS, LDS = EXPS + B::BM / 4;
-
-  typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
-  typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-  typedef float f2_t __attribute__((ext_vector_type(2)));
-
-  // as F32Split::run; re(r), ce(n): the exponents of row r of the tile and of this lane's column of block n
-  template <typename R, typename RE, typename CE>
-  LSA_DEVICE void run(R row, RE re, CE ce, const float* const (&wr)[NT], int K, u32x4_t* lds0) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    int* rows = reinterpret_cast<int*>(lds0 + EXPS);  // their exponents
-    int e[NT], wide = 0;
-#pragma unroll
-    for (int n = 0; n < NT; ++n) wide |= (e[n] = ce(n)) == F32_WIDE;
-    for (int r = tid; r < B::BM; r += B::THREADS) wide |= (rows[r] = re(r)) == F32_WIDE;
-    if (__syncthreads_or(wide)) return B::run(row, wr, K, lds0);
-    const auto rexp = [&](int r) { return rows[r]; };
-    const int grp = B::group(), blocks = (K + 63) / 64, u = blocks * grp / KG, mine = blocks * (grp + 1) / KG - u;
-    const int from = mine ? u * 64 : 0, len = mine ? min(K - from, mine * 64) : 32;
-    const float* w2[NT];
-#pragma unroll
-    for (int n = 0; n < NT; ++n) w2[n] = wr[n] + from * 16;
-    sums([&](int r) { return row(r) + from; }, rexp, w2, e, (blocks + KG - 1) / KG, mine, len, lds0 + grp * 2 * BUF);
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int x = rows[m * 16 + 4 * (lane >> 4) + r];
-#pragma unroll
-        for (int n = 0; n < NT; ++n) acc[m][n][r] = ldexpf(acc[m][n][r], -(x + e[n]));
-      }
-    // (finite operands overflow only as weights that have grown since their exponents were found)
-    B::whole([&](int r) { return row(r) + from; }, w2, min(len, mine * 64));
-    B::gather(lds0);
-  }
-
-  template <typename R, typename RE>
-  LSA_DEVICE void sums(R row, RE re, const float* const (&wr)[NT], const int (&e)[NT], int steps, int mine, int len, u32x4_t* lds) {
-    const int lane = threadIdx.x & 63, w = B::wave();
-    const float* p[SF + NT];
-#pragma unroll
-    for (int i = 0; i < SF + NT; ++i)
-      p[i] = i < SF ? row((w + NW * i) * 16 + (lane & 15)) + 4 * (lane >> 4) : wr[i < SF ? 0 : i - SF];
-    f32x4_t g[UNITS][2];  // 8 k of a row or column: from 4 (lane / 16) on and from 16 behind that
-    // unit i: fragment i / 2 of the rows', then i / 2 of the columns'; its half i % 2 of the 64 k
-    auto load = [&](int i, int step) {
-      const int f = i >> 1, k = min(step * 64 + (i & 1) * 32, len - 32);  // past the end: the last ones again
-      const float* q = p[f] + (f < SF ? k : k * 16);
-      g[i][0] = *reinterpret_cast<const f32x4_t*>(q);
-      g[i][1] = *reinterpret_cast<const f32x4_t*>(q + (f < SF ? 16 : 256));
-    };
-#pragma unroll
-    for (int i = 0; i < UNITS; ++i) load(i, 0);
-    float scale[SF + NT];
-#pragma unroll
-    for (int i = 0; i < SF + NT; ++i)
-      scale[i] = ldexpf(1.f, i < SF ? re((w + NW * (i < SF ? i : 0)) * 16 + (lane & 15)) : e[i < SF ? 0 : i - SF]);
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int n = 0; n < NT; ++n) acc[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    u32x4_t to[2], b[2][NT][2][2], a[4][2][2];  // [][half][piece]
-    float s, x, y;
-    unsigned h;
-    // Half of the split of two values of a step's (scaling, rounding and difference in one v_fma_mix{lo,hi}_f16 each, four instructions for
-    // six, are 2 % slower); after the last of a fragment it goes to LDS (rows) and the next is requested. The
-    // values behind the last 32 k of an odd number of them are zeros.
-    constexpr int HALVES = 8 * UNITS;
-    static_assert(16 * SF * 6 * MT <= HALVES * (6 * MT - AHEAD));  // the rows are in LDS before the barrier
-    auto half = [&](int z, int step, u32x4_t* nxt, u32x4_t (&bn)[NT][2][2]) {
-      const int i = z / 8, j = z / 2 % 4, f = i >> 1;
-      if (z % 8 == 0) s = (i & 1) && step * 64 + 32 >= len ? 0.f : scale[f];
-      if (z % 2 == 0) {
-        x = g[i][j >> 1][2 * j & 3] * s, y = g[i][j >> 1][(2 * j & 3) + 1] * s;
-        h = __builtin_bit_cast(unsigned, __builtin_convertvector((f2_t{x, y}), h2_t));
-        to[0][j] = h;
-        return;
-      }
-      const h2_t r = __builtin_bit_cast(h2_t, h);
-      to[1][j] = __builtin_bit_cast(unsigned, __builtin_convertvector((f2_t{x - (float)r[0], y - (float)r[1]}), h2_t));
-      if (z % 8 < 7) return;
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        if (f < SF) nxt[(((w + NW * f) * 2 + (i & 1)) * 2 + c) * 64 + lane] = to[c];
-        else bn[f < SF ? 0 : f - SF][i & 1][c] = to[c];
-      }
-      load(i, step + 1);
-    };
-    auto mul = [](const u32x4_t& u, const u32x4_t& v, const f32x4_t& c) {
-      return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, u), __builtin_bit_cast(h8_t, v), c, 0, 0, 0);
-    };
-    // 64 k that are split already, as F32Split's step: `step` is the one whose operands are split meanwhile.
-    f32x4_t c[2][NT];
-    constexpr int hh[6] = {0, 0, 1, 1, 0, 1}, pa[6] = {1, 0, 1, 0, 0, 0}, pb[6] = {0, 1, 0, 1, 0, 0};
-    // a fragment's pieces in the order of their first use, from product z of a step's (or the next one's) on
-    auto read = [&](int z, const u32x4_t* cur, const u32x4_t* nxt) {
-      const int m = z / 6, o = z % 6 ^ 1;
-      if (z % 6 < 4) a[m & 3][o >> 1][o & 1] = m < MT ? cur[(m * 4 + o) * 64 + lane] : nxt[((m - MT) * 4 + o) * 64 + lane];
-    };
-    auto step = [&](int at, const u32x4_t* cur, u32x4_t* nxt, const u32x4_t (&b)[NT][2][2], u32x4_t (&bn)[NT][2][2]) {
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-#pragma unroll
-        for (int q = 0; q < 6; ++q) {
-          const int z = m * 6 + q;
-          if (z == 6 * MT - AHEAD) __syncthreads();
-          read(z + AHEAD, cur, nxt);
-#pragma unroll
-          for (int n = 0; n < NT; ++n)
-            c[m & 1][n] = mul(a[m & 3][hh[q]][pa[q]], b[n][hh[q]][pb[q]], q ? c[m & 1][n] : f32x4_t{0.f, 0.f, 0.f, 0.f});
-          if (q == 2 && m)
-#pragma unroll
-            for (int n = 0; n < NT; ++n) acc[m ? m - 1 : 0][n] += c[(m - 1) & 1][n];
-#pragma unroll
-          for (int v = z * HALVES / (6 * MT); v < (z + 1) * HALVES / (6 * MT); ++v) half(v, at, nxt, bn);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-#pragma unroll
-      for (int n = 0; n < NT; ++n) acc[MT - 1][n] += c[(MT - 1) & 1][n];
-    };
-#pragma unroll
-    for (int z = 0; z < HALVES; ++z) half(z, 0, lds, b[0]);
-    __syncthreads();
-#pragma unroll
-    for (int z = 0; z < AHEAD; ++z) read(z, lds, lds);
-    for (int t = 0; t < steps; t += 2) {
-      if (t < mine) step(t + 1, lds, lds + BUF, b[0], b[1]);
-      else __syncthreads();
-      if (t + 1 >= steps) break;
-      if (t + 1 < mine) step(t + 2, lds + BUF, lds, b[1], b[0]);
-      else __syncthreads();
-    }
   }
 };

@@ -3,9 +3,6 @@
 // EPI_SWIGLU / EPI_GEGLU of the bf16 GEMMs.
 #include "epilogue.h"
 #include "f32_core.h"
-#include <algorithm>
-#include <cmath>
-#include <type_traits>
 
 namespace {
 
@@ -55,12 +52,11 @@ __global__ __launch_bounds__(NW * 64) void stream_f32_kernel(const float* __rest
   }
 }
 
-// ea, ew: exponents of the rows and columns, for two pieces (PAIR)
-template <int EPI, int MT, int NW, int KG, bool PAIR>
+template <int EPI, int MT, int NW, int KG>
 __global__ __launch_bounds__(NW * KG * 64) void tile_f32_kernel(
     const float* __restrict__ A, int lda, const float* __restrict__ W, int M, int N, int K, int mt, int nt, int whole, int S,
-    float* slab, unsigned* counters, EpiArgs ep, const int* __restrict__ ea, const int* __restrict__ ew) {
-  using T = std::conditional_t<PAIR, F32Pair<MT, NW, KG>, F32Split<MT, NW, KG>>;
+    float* slab, unsigned* counters, EpiArgs ep) {
+  using T = F32Split<MT, NW, KG>;
   __shared__ u32x4_t lds[T::LDS];
   __shared__ int s_last;
   // workgroups of one XCD get consecutive work; 8 row tiles share a sweep over the columns
@@ -73,13 +69,7 @@ __global__ __launch_bounds__(NW * KG * 64) void tile_f32_kernel(
 #pragma unroll
   for (int n = 0; n < T::NT; ++n) wr[n] = f32_block(W, min(n0 / 16 + T::wave() * T::NT + n, N / 16 - 1), K) + u0 * 512;
   T t;  // of a tile past the whole ones one of the S parts of K
-  const auto row = [&](int i) { return A + (size_t)min(m0 + i, M - 1) * lda + u0 * 32; };
-  if constexpr (PAIR) {
-    t.run(row, [&](int i) { return ea[min(m0 + i, M - 1)]; },
-          [&](int n) { return ew[min(n0 / 16 + T::wave() * T::NT + n, N / 16 - 1) * 16 + (threadIdx.x & 15)]; }, wr, (u1 - u0) * 32, lds);
-  } else {
-    t.run(row, wr, (u1 - u0) * 32, lds);
-  }
+  t.run([&](int i) { return A + (size_t)min(m0 + i, M - 1) * lda + u0 * 32; }, wr, (u1 - u0) * 32, lds);
   if (part >= 0 && !t.meet(p, S, slab + (size_t)(part / S) * S * (T::BM * T::BN), counters + part / S, &s_last)) return;
   t.each([&](int m, int n, float v, float u) {
     if (m0 + m >= M || n0 + n >= N) return;
@@ -92,105 +82,21 @@ __global__ __launch_bounds__(NW * KG * 64) void tile_f32_kernel(
   });
 }
 
-// Of a row whose largest magnitude is `top` (bits): what is too small for two pieces, up to `low`; its exponent if `small` values are
-LSA_DEVICE unsigned exp_low(unsigned top) { return top >> 23 > 17 ? top - (17u << 23) : 0; }  // (under 2^-109 the row is wide)
-LSA_DEVICE int exp_of(unsigned top, int small, int K) {
-  const int at = (int)(top >> 23) - 127;  // under 2^-126: -127; infinities and NaN: 128
-  return !top ? 0 : at > 127 || at < -109 || small > K / 16 ? F32_WIDE : F32_TOP - at;
-}
-
-// The exponents of rows (F32Pair), a wave a row: its largest value, then how many there are under 2^-17 of that. Bound by the
-// launch (1000 rows of 2048 4.4 us), then by the read.
-__global__ __launch_bounds__(256) void row_exps_kernel(const float* __restrict__ A, int lda, int M, int K, int* __restrict__ e) {
-  constexpr int U = 8;  // requested together
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (row >= M) return;
-  const float* a = A + (size_t)row * lda;
-  u32x4_t v[U];
-  auto load = [&](int k) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int at = k + u * 256 + lane * 4;
-      v[u] = *reinterpret_cast<const u32x4_t*>(a + min(at, K - 4));
-      if (at >= K) v[u] = u32x4_t{0, 0, 0, 0};
-    }
-  };
-  unsigned top = 0;  // of magnitudes, which order as the bits do; NaN are largest
-  for (int k = 0; k < K; k += U * 256) {
-    load(k);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) top = max(top, v[u][j] & 0x7fffffffu);
-  }
-  top = wave_max(top);
-  const unsigned low = exp_low(top);
-  int small = 0;
-  for (int k = 0; k < K; k += U * 256) {
-    if (K > U * 256) load(k);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) small += (v[u][j] & 0x7fffffffu) - 1u < low;  // zeros are none
-  }
-#pragma unroll
-  for (int o = 32; o; o >>= 1) small += __shfl_xor(small, o);
-  if (lane == 0) e[row] = exp_of(top, small, K);
-}
-
-// The same of packed weights' columns, 16 to a workgroup, each wave with a quarter of K
-__global__ __launch_bounds__(256) void col_exps_kernel(const float* __restrict__ W, int K, int* __restrict__ e) {
-  __shared__ unsigned s_top[4][16];
-  __shared__ int s_small[4][16];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = lane & 15, k0 = K / 16 * w / 4, k1 = K / 16 * (w + 1) / 4;
-  const u32x4_t* p = reinterpret_cast<const u32x4_t*>(W + (size_t)blockIdx.x * 16 * K) + lane;
-  unsigned top = 0;
-#pragma unroll 4
-  for (int k = k0; k < k1; ++k) {
-    const u32x4_t v = p[k * 64];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) top = max(top, v[j] & 0x7fffffffu);
-  }
-  top = max(top, __shfl_xor(top, 16));
-  s_top[w][c] = max(top, __shfl_xor(top, 32));  // four lanes the same
-  __syncthreads();
-  top = max(max(s_top[0][c], s_top[1][c]), max(s_top[2][c], s_top[3][c]));
-  const unsigned low = exp_low(top);
-  int small = 0;
-#pragma unroll 4
-  for (int k = k0; k < k1; ++k) {
-    const u32x4_t v = p[k * 64];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) small += (v[j] & 0x7fffffffu) - 1u < low;
-  }
-  small += __shfl_xor(small, 16);
-  s_small[w][c] = small + __shfl_xor(small, 32);
-  __syncthreads();
-  if (threadIdx.x < 16) e[blockIdx.x * 16 + c] = exp_of(top, s_small[0][c] + s_small[1][c] + s_small[2][c] + s_small[3][c], K);
-}
-
 // A product's tiles, and how many parts of K for each of the last `rem` ones, which fill the CUs only in part (S; `whole` before
 // them that fill them). Modelled us: a round of tiles its steps of 32 k and 5.2 to begin and end, a part its share of the steps;
 // the meeting by the parts of a tile and by their bytes. Fitted to 176 products (11 of 512 to 8192 k by 640 to 16384 columns at 20
 // to 2567 rows, all forms and splits): what it takes is 1.005 times the fastest (geometric mean; worst 1.08; timed without the operands' scaling, which adds 2 %
 // to the large tiles' products and up to 9 % to the others). The largest tiles
 // split least and read least (1.14 us for 128 x 128 of 32 k against 1.52 of the smallest), the smallest leave the fewest CUs idle.
-// In two pieces a round takes 10 us to begin and end, and a launch before it finds the rows' exponents: 4 us and a us for each million of
-// values. They are taken where they cost less by this and where most tiles' sums are long enough (THREE_LONG). 192 tiles of 128 x 256 at
-// K = 8192 take 337 us, 384 of 128 x 128 394; half of a remainder's 10 us passes beside the round before it.
 struct Plan {
   int rows, cols, whole, S;
-  double us;
-  int units;  // of 32 k in a sum: of most tiles
 };
-struct Form {
-  int rows, cols;
-  double busy, idle;  // us for 32 k: all CUs at it, few
-  int groups;         // a workgroup's parts of K
-};
-constexpr Form THREE[] = {{128, 256, 2.08, 1.74, 1}, {128, 128, 1.14, 0.92, 2}, {64, 128, 0.635, 0.525, 2}, {64, 64, 0.38, 0.31, 4}};
-constexpr Form TWO[] = {{128, 256, 1.29, 0.91, 1}, {128, 128, 0.73, 0.573, 2}, {64, 128, 0.43, 0.357, 2}, {64, 64, 0.30, 0.29, 4}};
-Plan plan(const Form (&forms)[4], int least_units, double own, int M, int N, int K, long long slab_floats, int counters) {
+Plan plan(int M, int N, int K, long long slab_floats, int counters) {
+  struct Form {
+    int rows, cols;
+    double busy, idle;  // us for 32 k: all CUs at it, few
+  };
+  constexpr Form forms[] = {{128, 256, 2.08, 1.74}, {128, 128, 1.14, 0.92}, {64, 128, 0.635, 0.525}, {64, 64, 0.38, 0.31}};
   Plan best{};
   double least = 0;
   for (const Form& f : forms) {
@@ -198,16 +104,14 @@ Plan plan(const Form (&forms)[4], int least_units, double own, int M, int N, int
     const double kb = f.rows * f.cols / 256.0;
     for (int S : {1, 2, 3, 4, 6, 8, 12, 16}) {
       const long long parts = (long long)rem * S;
-      if (K / 32 < least_units * S * f.groups) continue;
       if (S > 1 && (!rem || K / 32 < 2 * S || parts > 1024 || parts * f.rows * f.cols > slab_floats || rem > counters)) continue;
-      const double full = std::min(parts / 256.0, 1.0);  // of the CUs; in two pieces those that idle leave the others more of the clock
-      double us = rounds * (K / 32 * f.busy + own);
+      double us = rounds * (K / 32 * f.busy + 5.2);
       if (rem) {
         const int n = (int)((parts + 255) / 256), per = (K / 32 + S - 1) / S;
-        us += n * (per * (rounds ? f.busy : f.idle + (f.busy - f.idle) * (least_units && S == 1 ? std::pow(full, 1.7) : full)) + (least_units && rounds ? 0.5 : 1.0) * own);
+        us += n * (per * (rounds || n > 1 ? f.busy : f.idle + (f.busy - f.idle) * parts / 256) + 5.2);
         if (S > 1) us += (0.28 + S * (0.22 + 0.0065 * kb) + 0.00051 * kb * parts) * (rounds ? 1.42 : 1.0);
       }
-      if (!best.rows || us < least) best = Plan{f.rows, f.cols, S > 1 ? tiles - rem : tiles, S, us, K / 32 / ((S > 1 && tiles > rem ? 1 : S) * f.groups)}, least = us;
+      if (!best.rows || us < least) best = Plan{f.rows, f.cols, S > 1 ? tiles - rem : tiles, S}, least = us;
     }
   }
   return best;
@@ -225,10 +129,9 @@ int stream_tiles(int M, int N, int K, bool gated) {
   return K % 32 || (M <= 32 && (long long)N * K <= 1 << 24) ? 2 : 0;
 }
 
-// we: the columns' exponents, or null
 template <int EPI>
-void launch(const float* a, int lda, const float* w, const int* we, int M, int N, int K, const EpiArgs& ep, float* slab,
-            long long slab_floats, unsigned* counters, int n_counters, hipStream_t s) {
+void launch(const float* a, int lda, const float* w, int M, int N, int K, const EpiArgs& ep, float* slab, long long slab_floats,
+            unsigned* counters, int n_counters, hipStream_t s) {
 #define LSA_STREAM(MT, NT) \
   stream_f32_kernel<EPI, MT, NT, 8><<<dim3((t + NT - 1) / NT, (M + MT * 16 - 1) / (MT * 16)), 512, 0, s>>>(a, lda, w, M, N, K, ep)
   // A CU takes 3 us for a tile's products, so that the tiles are as many per workgroup as the fullest CU has anyway:
@@ -251,79 +154,35 @@ void launch(const float* a, int lda, const float* w, const int* we, int M, int N
     return;
   }
 #undef LSA_STREAM
-  Plan p = plan(THREE, 0, 5.2, M, N, K, slab_floats, n_counters);
-  int* ea = nullptr;
-  if (const long long rest = (slab_floats - M) & ~3ll; we && rest >= 0 && p.units >= THREE_LONG) {
-    const Plan two = plan(TWO, PAIR_UNITS, 10.0, M, N, K, rest, n_counters);
-    if (two.rows && two.us + 4.0 + M * (double)K * 1e-6 < p.us) p = two, ea = (int*)(slab + rest);  // at the end of the slab
-  }
-  const bool pair = ea;
-  if (pair) row_exps_kernel<<<(M + 3) / 4, 256, 0, s>>>(a, lda, M, K, ea);
+  const Plan p = plan(M, N, K, slab_floats, n_counters);
   const int mt = (M + p.rows - 1) / p.rows, nt = (N + p.cols - 1) / p.cols, grid = p.whole + (mt * nt - p.whole) * p.S;
-#define LSA_TILE_(MT, NW, KG, PAIR)                                                                                              \
-  tile_f32_kernel<EPI, MT, NW, KG, PAIR><<<grid, NW * KG * 64, 0, s>>>(a, lda, w, M, N, K, mt, nt, p.whole, p.S, slab, counters, \
-                                                                       ep, ea, we)
-#define LSA_TILE(MT, NW, KG)            \
-  if (pair) LSA_TILE_(MT, NW, KG, true); \
-  else LSA_TILE_(MT, NW, KG, false)
-  if (p.cols == 256) {
-    LSA_TILE(8, 8, 1);
-  } else if (p.rows == 128) {
-    LSA_TILE(8, 4, 2);
-  } else if (p.cols == 128) {
-    LSA_TILE(4, 4, 2);
-  } else {
-    LSA_TILE(4, 2, 4);
-  }
+#define LSA_TILE(MT, NW, KG)                                                                                               \
+  tile_f32_kernel<EPI, MT, NW, KG><<<grid, NW * KG * 64, 0, s>>>(a, lda, w, M, N, K, mt, nt, p.whole, p.S, slab, counters, ep)
+  if (p.cols == 256) LSA_TILE(8, 8, 1);
+  else if (p.rows == 128) LSA_TILE(8, 4, 2);
+  else if (p.cols == 128) LSA_TILE(4, 4, 2);
+  else LSA_TILE(4, 2, 4);
 #undef LSA_TILE
-#undef LSA_TILE_
 }
 
 }  // namespace
 
-// we: the columns' exponents (lsa_row_exps_f32), for products in two pieces where there is scratch, or null
 // slab (16-byte aligned floats) and counters (zeros, left so): scratch of this stream for products in parts; none: whole tiles
-static int linear_f32(const float* a, int lda, const float* w, const int* we, int M, int N, int K, int epi, const EpiArgs* ep,
+extern "C" int lsa_linear_f32(const float* a, int lda, const float* w, int M, int N, int K, int epi, const EpiArgs* ep,
                               float* slab, long long slab_floats, unsigned* counters, int n_counters, hipStream_t stream) {
   if (M < 1 || N < 16 || N % 16 || K < 16 || K % 16 || lda < K || lda % 4 || !ep || !(ep->out32 || ep->out)) return LSA_BAD_SHAPE;
   if (((uintptr_t)a | (uintptr_t)w | (uintptr_t)slab) % 16 || (!slab && slab_floats) || (!counters && n_counters))
     return LSA_BAD_SHAPE;
   if (epi_gated(epi)) {
     if (N % 32 || ep->ldo < N / 2 || !ep->out32) return LSA_BAD_SHAPE;
-    if (epi == EPI_GEGLU) launch<EPI_GEGLU>(a, lda, w, we, M, N, K, *ep, slab, slab_floats, counters, n_counters, stream);
-    else launch<EPI_SWIGLU>(a, lda, w, we, M, N, K, *ep, slab, slab_floats, counters, n_counters, stream);
+    if (epi == EPI_GEGLU) launch<EPI_GEGLU>(a, lda, w, M, N, K, *ep, slab, slab_floats, counters, n_counters, stream);
+    else launch<EPI_SWIGLU>(a, lda, w, M, N, K, *ep, slab, slab_floats, counters, n_counters, stream);
   } else if (epi == EPI_STORE) {
     if (bad_store(*ep, N)) return LSA_BAD_SHAPE;
-    launch<EPI_STORE>(a, lda, w, we, M, N, K, *ep, slab, slab_floats, counters, n_counters, stream);
+    launch<EPI_STORE>(a, lda, w, M, N, K, *ep, slab, slab_floats, counters, n_counters, stream);
   } else {
     return LSA_UNSUPPORTED;
   }
-  LSA_CHECK_LAUNCH();
-  return LSA_OK;
-}
-
-extern "C" int lsa_linear_f32(const float* a, int lda, const float* w, int M, int N, int K, int epi, const EpiArgs* ep,
-                              float* slab, long long slab_floats, unsigned* counters, int n_counters, hipStream_t stream) {
-  return linear_f32(a, lda, w, nullptr, M, N, K, epi, ep, slab, slab_floats, counters, n_counters, stream);
-}
-extern "C" int lsa_linear_f32_pair(const float* a, int lda, const float* w, const int* we, int M, int N, int K, int epi,
-                                   const EpiArgs* ep, float* slab, long long slab_floats, unsigned* counters, int n_counters,
-                                   hipStream_t stream) {
-  return we ? linear_f32(a, lda, w, we, M, N, K, epi, ep, slab, slab_floats, counters, n_counters, stream) : LSA_BAD_SHAPE;
-}
-
-// e[i]: the exponent of row i of A, for products in two pieces
-extern "C" int lsa_row_exps_f32(const float* a, long long lda, long long M, int K, int* e, hipStream_t stream) {
-  if (M < 1 || M > 1ll << 30 || K < 4 || K % 4 || lda < K || lda % 4 || lda >= 1ll << 31 || (uintptr_t)a % 16 || !e) return LSA_BAD_SHAPE;
-  row_exps_kernel<<<(M + 3) / 4, 256, 0, stream>>>(a, lda, M, K, e);
-  LSA_CHECK_LAUNCH();
-  return LSA_OK;
-}
-
-// e[i]: that of column i of weights packed in blocks (f32_core.h)
-extern "C" int lsa_col_exps_f32(const float* w, long long columns, int K, int* e, hipStream_t stream) {
-  if (columns < 16 || columns % 16 || columns >= 1ll << 31 || K < 16 || K % 16 || (uintptr_t)w % 16 || !e) return LSA_BAD_SHAPE;
-  col_exps_kernel<<<columns / 16, 256, 0, stream>>>(w, K, e);
   LSA_CHECK_LAUNCH();
   return LSA_OK;
 }
@@ -333,7 +192,7 @@ extern "C" int lsa_col_exps_f32(const float* w, long long columns, int K, int* e
 extern "C" int lsa_linear_f32_form(int M, int N, int K, int gated, long long slab_floats, int n_counters, int* form) {
   if (M < 1 || N < 16 || N % 16 || K < 16 || K % 16 || (gated && N % 32) || !form) return LSA_BAD_SHAPE;
   const int m = stream_tiles(M, N, K, gated);
-  const Plan p = m ? Plan{16 * m, 0, 0, 1} : plan(THREE, 0, 5.2, M, N, K, slab_floats, n_counters);
+  const Plan p = m ? Plan{16 * m, 0, 0, 1} : plan(M, N, K, slab_floats, n_counters);
   form[0] = p.rows;
   form[1] = p.cols;
   form[2] = p.whole;

@@ -1,7 +1,6 @@
 // Mixture of experts (moe.h): routing, grouping and the expert products (bf16 on MFMA, and fp32 for the
 // fp32 engine).
 #include "f32_core.h"
-#include <type_traits>
 #include "moe.h"
 
 namespace {
@@ -394,14 +393,12 @@ __global__ __launch_bounds__(NW * 64) void moe_stream_f32_kernel(const MoeTile* 
 // many: MT x 16 pairs x NW x 32 columns. 20536 pairs, 32 experts of 2048 x 1024: up 776 -> 477, down 769 -> 465 us (64 x 64 tiles
 // on the fp32 matrix instructions before); about 90 pairs an expert, gated, of 1024 columns 509 -> 346 in 64 x 128 tiles; 8 experts
 // of 1024 x 2048, 40 pairs each 35 -> 29 in 64 x 64 (64 x 128 44, 128 x 256 117: which of them, ops/moe.py).
-// ea, ew: exponents of A's rows and of the experts' columns, for two pieces (PAIR)
-template <int UP, int MT, int NW, int KG, bool PAIR>
+template <int UP, int MT, int NW, int KG>
 __global__ __launch_bounds__(NW * KG * 64) void moe_tile_f32_kernel(const MoeTile* __restrict__ tiles, const int* __restrict__ order,
                                                                     int top, const float* __restrict__ A, int lda,
                                                                     const float* __restrict__ W, int N, int K,
-                                                                    float* __restrict__ out, int ldo, const int* __restrict__ ea,
-                                                                    const int* __restrict__ ew) {
-  using T = std::conditional_t<PAIR, F32Pair<MT, NW, KG>, F32Split<MT, NW, KG>>;
+                                                                    float* __restrict__ out, int ldo) {
+  using T = F32Split<MT, NW, KG>;
   __shared__ u32x4_t lds[T::LDS];
   // Workgroups of one XCD get consecutive work, 8 tiles (mostly of one expert) share a sweep over the columns.
   const int nx = gridDim.x, b = blockIdx.y * nx + blockIdx.x, told = tiles[0].used;
@@ -418,18 +415,10 @@ __global__ __launch_bounds__(NW * KG * 64) void moe_tile_f32_kernel(const MoeTil
   for (int n = 0; n < T::NT; ++n)
     wr[n] = f32_block(W + (size_t)tile.expert * N * K, min(n0 / 16 + T::wave() * T::NT + n, N / 16 - 1), K);
   T t;
-  const auto at = [&](int i) {
-    const int p = tile.start + min(i, tile.count - 1);  // rows past the count are not stored
-    return UP ? order[p] / top : p;
-  };
-  const auto row = [&](int i) { return A + (size_t)at(i) * lda; };
-  if constexpr (PAIR) {
-    t.run(row, [&](int i) { return ea[at(i)]; }, [&](int n) {
-      return ew[(size_t)tile.expert * N + min(n0 / 16 + T::wave() * T::NT + n, N / 16 - 1) * 16 + (threadIdx.x & 15)];
-    }, wr, K, lds);
-  } else {
-    t.run(row, wr, K, lds);
-  }
+  t.run([&](int i) {
+    const int at = tile.start + min(i, tile.count - 1);  // rows past the count are not stored
+    return A + (size_t)(UP ? order[at] / top : at) * lda;
+  }, wr, K, lds);
   t.each([&](int m, int n, float v, float u) {
     if (m >= tile.count || n0 + n >= N) return;
     float* o = out + (size_t)(tile.start + m) * ldo;
@@ -442,33 +431,20 @@ __global__ __launch_bounds__(NW * KG * 64) void moe_tile_f32_kernel(const MoeTil
   });
 }
 
-// we: the columns' exponents, ea: of A's rows; or null
 template <int UP>
 int launch_f32(const MoeTile* t, int max_tiles, int tile_rows, bool narrow, const int* order, int top, const float* A, int lda,
-               const float* W, int N, int K, float* out, int ldo, const int* ea, const int* we, hipStream_t s) {
+               const float* W, int N, int K, float* out, int ldo, hipStream_t s) {
   constexpr int NT = UP == MOE_GLU ? 2 : 1;
   const dim3 grid((N + NT * 16 - 1) / (NT * 16), max_tiles);
-#define LSA_TILE(MT, NW, KG)                                                                                                       \
-  if (we && K / 32 / KG >= THREE_LONG)                                                                                             \
-    moe_tile_f32_kernel<UP, MT, NW, KG, true><<<dim3((N + NW * 32 - 1) / (NW * 32), max_tiles), 512, 0, s>>>(t, order, top, A, lda, W, N, \
-                                                                                                             K, out, ldo, ea, we); \
-  else                                                                                                                             \
-    moe_tile_f32_kernel<UP, MT, NW, KG, false><<<dim3((N + NW * 32 - 1) / (NW * 32), max_tiles), 512, 0, s>>>(t, order, top, A, lda, W,   \
-                                                                                                              N, K, out, ldo, ea, we)
-  if (tile_rows <= 16) {
-    moe_stream_f32_kernel<UP, 1, NT, 8><<<grid, 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
-  } else if (tile_rows <= 32) {
-    moe_stream_f32_kernel<UP, 2, NT, 8><<<grid, 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
-  } else if (tile_rows <= 64 && narrow) {
-    LSA_TILE(4, 2, 4);
-  } else if (tile_rows <= 64) {
-    LSA_TILE(4, 4, 2);
-  } else if (tile_rows <= 128) {
-    LSA_TILE(8, 8, 1);
-  } else {
-    return LSA_UNSUPPORTED;
-  }
-#undef LSA_TILE
+  if (tile_rows <= 16) moe_stream_f32_kernel<UP, 1, NT, 8><<<grid, 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
+  else if (tile_rows <= 32) moe_stream_f32_kernel<UP, 2, NT, 8><<<grid, 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
+  else if (tile_rows <= 64 && narrow)
+    moe_tile_f32_kernel<UP, 4, 2, 4><<<dim3((N + 63) / 64, max_tiles), 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
+  else if (tile_rows <= 64)
+    moe_tile_f32_kernel<UP, 4, 4, 2><<<dim3((N + 127) / 128, max_tiles), 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
+  else if (tile_rows <= 128)
+    moe_tile_f32_kernel<UP, 8, 8, 1><<<dim3((N + 255) / 256, max_tiles), 512, 0, s>>>(t, order, top, A, lda, W, N, K, out, ldo);
+  else return LSA_UNSUPPORTED;
   LSA_CHECK_LAUNCH();
   return LSA_OK;
 }
@@ -537,8 +513,8 @@ extern "C" int lsa_moe_route_group(const RouteArgs* ra, const float* logits, int
 
 // up (MoeUp): A = h rows, out [pairs][ldo >= N / 2 (glu) or N]; down: A = act [pairs], out [pairs][ldo >= N]
 // narrow (fp32, tiles of 64 rows): 64 columns a workgroup instead of 128
-static int moe_gemm(int f32, int up, const void* tiles, int max_tiles, int tile_rows, int narrow, const int* order, int top,
-                            const void* A, int lda, const void* W, int N, int K, void* out, int ldo, const int* ea, const int* we, hipStream_t s) {
+extern "C" int lsa_moe_gemm(int f32, int up, const void* tiles, int max_tiles, int tile_rows, int narrow, const int* order, int top,
+                            const void* A, int lda, const void* W, int N, int K, void* out, int ldo, hipStream_t s) {
   if (max_tiles < 1 || max_tiles > 65535 || top < 1 || N < 32 || N % 32 || K < 32 || K % 32 || lda < K || lda % 8 ||
       up < MOE_DOWN || up > MOE_RELU2 || ldo < (up == MOE_GLU ? N / 2 : N) || ldo % 4 ||
       ((uintptr_t)A | (uintptr_t)W | (uintptr_t)out) % 16)
@@ -547,7 +523,7 @@ static int moe_gemm(int f32, int up, const void* tiles, int max_tiles, int tile_
   const MoeTile* t = (const MoeTile*)tiles;
   if (f32) {
     auto* f = up == MOE_GLU ? launch_f32<MOE_GLU> : up ? launch_f32<MOE_RELU2> : launch_f32<MOE_DOWN>;
-    return f(t, max_tiles, tile_rows, narrow, order, top, (const float*)A, lda, (const float*)W, N, K, (float*)out, ldo, ea, we, s);
+    return f(t, max_tiles, tile_rows, narrow, order, top, (const float*)A, lda, (const float*)W, N, K, (float*)out, ldo, s);
   }
 #define LSA_M(MT)                                                                                                     \
   if (tile_rows == MT * 16) {                                                                                         \
@@ -559,17 +535,4 @@ static int moe_gemm(int f32, int up, const void* tiles, int max_tiles, int tile_
   LSA_M(1) LSA_M(2) LSA_M(4)
 #undef LSA_M
   return LSA_UNSUPPORTED;
-}
-
-extern "C" int lsa_moe_gemm(int f32, int up, const void* tiles, int max_tiles, int tile_rows, int narrow, const int* order, int top,
-                            const void* A, int lda, const void* W, int N, int K, void* out, int ldo, hipStream_t s) {
-  return moe_gemm(f32, up, tiles, max_tiles, tile_rows, narrow, order, top, A, lda, W, N, K, out, ldo, nullptr, nullptr, s);
-}
-// fp32 in two pieces where the tiles are made for many pairs: ea, we: exponents of A's rows and of the experts' columns [E][N]
-// (lsa_row_exps_f32)
-extern "C" int lsa_moe_gemm_pair(int up, const void* tiles, int max_tiles, int tile_rows, int narrow, const int* order, int top,
-                                 const void* A, int lda, const void* W, int N, int K, void* out, int ldo, const int* ea,
-                                 const int* we, hipStream_t s) {
-  if (!ea || !we) return LSA_BAD_SHAPE;
-  return moe_gemm(1, up, tiles, max_tiles, tile_rows, narrow, order, top, A, lda, W, N, K, out, ldo, ea, we, s);
 }

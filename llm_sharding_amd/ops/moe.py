@@ -6,7 +6,6 @@ from __future__ import annotations
 
 import ctypes
 import functools
-import math
 from typing import Optional
 
 import torch
@@ -14,7 +13,7 @@ import torch
 from . import hip
 from .hip import _check, _p, _req, _stream, lib
 from .packing import fuse_gate_up, pack_b, pack_f32
-from .stream import column_exps, is_f32, pad2, row_exps
+from .stream import is_f32, pad2
 
 
 def pad128(n: int) -> int:
@@ -84,32 +83,15 @@ class Experts:
         self.up_n = ups[0].shape[0]
         self.down = torch.stack([lay(pad2(d, self.width, self.ff)) for d in down])
         self.experts = len(up)
-        pair = self.f32 and self.up.is_cuda  # exponents of the columns, for products in two pieces
-        self.up_exps, self.down_exps = (column_exps(w) if pair else None for w in (self.up, self.down))
-
-    @property
-    def two_pieces(self) -> bool:
-        """Whether tiles of 128 rows are made in two pieces (:func:`gemm`)."""
-        return self.up_exps is not None and min(self.width, self.ff) >= 512
 
     def tensors(self) -> list:
-        return [self.up, self.down] + [e for e in (self.up_exps, self.down_exps) if e is not None]
+        return [self.up, self.down]
 
 
-def tile_rows(pairs: int, experts: int, f32: bool, cols: Optional[int] = None, wide: Optional[int] = None) -> int:
+def tile_rows(pairs: int, experts: int, f32: bool, cols: Optional[int] = None) -> int:
     """Pairs per tile: what an expert gets on average, rounded to a kernel's size. ``cols``: of the narrower of the two products (None:
-    wide enough); ``wide`` (fp32): of the wider one, where both are made in two pieces (:attr:`Experts.two_pieces`)."""
+    wide enough)."""
     mean = pairs / experts  # (a second tile of an expert reads its weights again)
-    if f32 and wide is not None and mean > 16:
-        # 128 rows x 256 columns in two pieces read an expert's weights faster than the others, however few of the rows are used, if there is
-        # half a round of them and no round that is nearly empty. 32 experts of 2048 x 1024, us of both products in 32 (up to 24 pairs
-        # each), 64 and 128 rows: 18 pairs 223, 197 and 175, 42 390, 207 and 174, 75 268 and 185, 95 280 and 210; 64 of 1024 x 512, 42
-        # pairs 197, 108 and 94; 16 of 2048 x 1024 (128 tiles) 50 pairs 87 and 123, 70 126 and 123; 24 of 2048 x 1408 (264 tiles) 50
-        # pairs 214 and 270; 8 of 2048 x 2048 (64 tiles and more) 100 pairs 125 and 161, 125 181 and 161.
-        many = [experts * max(1.0, mean / 128 + 0.5) * -(-n // 256) for n in (cols, wide)]
-        full = experts * -(-wide // 256) / 256
-        if many[0] >= (90 if mean > 112 else 130) and (mean > 112 or full <= 1 or math.ceil(full) <= 1.35 * full):
-            return 128
     if f32:  # 64 x 128 and 128 rows x 256 columns: 90 pairs an expert 3907 and 4155 us a pass (Runidra 2k), 183 6000 and 5662, 104
         # 3780 and 3804 (Dumizen 2k), 141 4568 and 4440. The large ones keep a CU for more than twice as long and are for products with as
         # many as 160 of them: 8 experts of 1024 x 2048, 136 pairs each 51 and 122 us, 32 experts 145 and 138. With narrow ones (gemm)
@@ -173,11 +155,9 @@ def route_group(logits, rows: int, experts: int, top: int, tile: int, expert, we
     return n
 
 
-def gemm(tiles, n_tiles: int, rows: int, order, top: int, a, w, n: int, k: int, out, pairs: int, up: int, exps=None, spare=None) -> None:
+def gemm(tiles, n_tiles: int, rows: int, order, top: int, a, w, n: int, k: int, out, pairs: int, up: int) -> None:
     """One product of every tile's expert: ``up`` (GLU / RELU2) from rows of h (``a``) to out [pairs, n / 2 or n], or
-    DOWN from the sorted pairs (``a`` [pairs, k]) to out [pairs, n]. ``rows`` 0: tiles of the height that :func:`group` chose. ``exps``
-    (fp32): the columns' exponents [experts, n], with which tiles of more than 32 pairs are made in two pieces; ``spare``: int32 scratch,
-    as long as the rows of ``a`` that are used."""
+    DOWN from the sorted pairs (``a`` [pairs, k]) to out [pairs, n]. ``rows`` 0: tiles of the height that :func:`group` chose."""
     _req(a.dtype == w.dtype == out.dtype and a.stride(1) == 1 and a.shape[1] >= k and out.stride(1) == 1
          and out.shape[0] >= pairs and out.shape[1] >= (n // 2 if up == GLU else n) and order.numel() >= pairs
          and (a.shape[0] * top >= pairs if up else a.shape[0] >= pairs), "moe: shapes")
@@ -188,17 +168,6 @@ def gemm(tiles, n_tiles: int, rows: int, order, top: int, a, w, n: int, k: int, 
                                       a.stride(0), _p(w), n, k, _p(out), out.stride(0), _stream()), "lsa_moe_gemm_big")
         return
     narrow = bool(f32) and narrow_tiles(pairs, w.shape[0], rows, n)
-    used = -(-pairs // top) if up else pairs
-    # as long sums as two pieces need (f32_core.h THREE_LONG) in each of a workgroup's parts of K
-    pair = bool(f32) and exps is not None and spare is not None and spare.numel() >= used and 32 < rows <= 128 \
-        and k >= 512 * (1 if rows > 64 else 4 if narrow else 2)
-    _req(not pair or (exps.dtype == torch.int32 and exps.is_contiguous() and exps.numel() == w.shape[0] * n
-                      and spare.dtype == torch.int32 and spare.is_contiguous()), "moe: exponents")
-    if pair:
-        row_exps(a[:used, :k], spare)
-        _check(lib().lsa_moe_gemm_pair(up, _p(tiles), n_tiles, rows, narrow, _p(order), top, _p(a), a.stride(0), _p(w), n, k,
-                                       _p(out), out.stride(0), _p(spare), _p(exps), _stream()), "lsa_moe_gemm_pair")
-        return
     _check(lib().lsa_moe_gemm(f32, up, _p(tiles), n_tiles, rows, narrow, _p(order), top, _p(a), a.stride(0), _p(w),
                               n, k, _p(out), out.stride(0), _stream()), "lsa_moe_gemm")
 
@@ -211,6 +180,5 @@ def declare(L: ctypes.CDLL) -> None:
         "lsa_moe_group": [vp, i, i, i, i, vp, vp, vp, vp, i, ctypes.POINTER(Pick), vp],
         "lsa_moe_route_group": [ra, vp, i, i, i, i, vp, vp, i, i, vp, vp, vp, vp],
         "lsa_moe_gemm_big": [i, vp, i, i, vp, i, vp, i, i, vp, i, i, vp, i, vp],
-        "lsa_moe_gemm_pair": [i, vp, i, i, i, vp, i, vp, i, vp, i, i, vp, i, vp, vp, vp],
         "lsa_moe_gemm": [i, i, vp, i, i, i, vp, i, vp, i, vp, i, i, vp, i, vp],
     })

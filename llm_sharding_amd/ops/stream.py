@@ -28,23 +28,6 @@ def pad2(w: torch.Tensor, n: int, k: int) -> torch.Tensor:
     return out
 
 
-def row_exps(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """The exponents with which rows of fp32 ``x`` are taken apart in two pieces (csrc/kernels/f32_core.h F32Pair), int32."""
-    _req(x.dtype == torch.float32 and x.is_cuda and x.dim() == 2 and x.stride(1) == 1, "row_exps: fp32 cuda rows")
-    out = torch.empty(x.shape[0], dtype=torch.int32, device=x.device) if out is None else out
-    _req(out.dtype == torch.int32 and out.is_contiguous() and out.numel() >= x.shape[0], "row_exps: output")
-    _check(lib().lsa_row_exps_f32(_p(x), x.stride(0), x.shape[0], x.shape[1], _p(out), _stream()), "lsa_row_exps_f32")
-    return out
-
-
-def column_exps(wp: torch.Tensor) -> torch.Tensor:
-    """The same of the columns of packed weights [..., N / 16, K / 16, 64, 4] (packing.pack_f32) -> [..., N]."""
-    _req(wp.dtype == torch.float32 and wp.is_cuda and wp.is_contiguous() and wp.shape[-2:] == (64, 4), "column_exps: packed fp32 weights")
-    out = torch.empty(wp.shape[:-4] + (wp.shape[-4] * 16,), dtype=torch.int32, device=wp.device)
-    _check(lib().lsa_col_exps_f32(_p(wp), out.numel(), wp.shape[-3] * 16, _p(out), _stream()), "lsa_col_exps_f32")
-    return out
-
-
 class Linear:
     """One projection of a stack engine in the engine's type: N and K padded to whole 128-wide
     blocks with zeros, so that every kernel configuration takes it; weights packed for the
@@ -56,7 +39,6 @@ class Linear:
         wp = w if w.shape == (self.n, self.k) else pad2(w, self.n, self.k)
         self.f32 = is_f32(w.dtype)
         self.w = (pack_f32(wp) if self.f32 else pack_b(wp)).contiguous()
-        self.exps = column_exps(self.w) if self.f32 and wp.is_cuda else None
 
     @staticmethod
     def glu(gate: torch.Tensor, up: torch.Tensor) -> "Linear":
@@ -72,7 +54,7 @@ class Linear:
         return fuse_gate_up(pad2(gate[:, None], n, 1), pad2(up[:, None], n, 1)).reshape(-1).contiguous()
 
     def tensors(self) -> list:
-        return [self.w] + ([self.exps] if self.exps is not None else [])
+        return [self.w]
 
     def __call__(self, x: torch.Tensor, rows: int, out: Optional[torch.Tensor], ws=None, sk_ws=None, glu=None, keys=None,
                  bias=None, col_offset: int = 0, out32: Optional[torch.Tensor] = None, col32: int = 0,
@@ -117,12 +99,9 @@ class Linear:
             if ws is None and not torch.cuda.is_current_stream_capturing():
                 ws = hip.default_workspace(x.device)
             slab, counters = (None, None) if ws is None else (ws.slab, ws.counters)
-            rest = (rows, self.n, self.k, epi, ctypes.byref(ep), _p(slab), 0 if ws is None else slab.numel(), _p(counters),
-                    0 if ws is None else counters.numel(), _stream())
-            if self.exps is None:
-                _check(lib().lsa_linear_f32(_p(x), x.stride(0), _p(self.w), *rest), "lsa_linear_f32")
-            else:
-                _check(lib().lsa_linear_f32_pair(_p(x), x.stride(0), _p(self.w), _p(self.exps), *rest), "lsa_linear_f32_pair")
+            _check(lib().lsa_linear_f32(_p(x), x.stride(0), _p(self.w), rows, self.n, self.k, epi, ctypes.byref(ep), _p(slab),
+                                        0 if ws is None else slab.numel(), _p(counters), 0 if ws is None else counters.numel(),
+                                        _stream()), "lsa_linear_f32")
         elif rows <= 128:
             hip.gemv(x, self.w, rows, self.n, self.k, epi, ep, ws=ws)
         else:
@@ -313,8 +292,5 @@ def declare(L: ctypes.CDLL) -> None:
         "lsa_stream_renorm": [i, ctypes.POINTER(RenormArgs), i, i, vp, i, vp, i, vp],
         "lsa_logits_argmax": [vp, i, i, i, i, vp, vp],
         "lsa_linear_f32_form": [i, i, i, i, ctypes.c_longlong, i, vp],
-        "lsa_row_exps_f32": [vp, ctypes.c_longlong, ctypes.c_longlong, i, vp, vp],
-        "lsa_col_exps_f32": [vp, ctypes.c_longlong, i, vp, vp],
-        "lsa_linear_f32_pair": [vp, i, vp, vp, i, i, i, i, ctypes.POINTER(hip.EpiArgs), vp, ctypes.c_longlong, vp, i, vp],
         "lsa_linear_f32": [vp, i, vp, i, i, i, i, ctypes.POINTER(hip.EpiArgs), vp, ctypes.c_longlong, vp, i, vp],
     })

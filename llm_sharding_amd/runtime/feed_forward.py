@@ -127,7 +127,7 @@ class Moe:
     def scratch(self) -> dict:
         top = self.spec.top
         own = {"sact": self.shared.k} if self.shared_glu is not None else {}
-        return {**own, "act": top * self.experts.ff, "ye": top * self.experts.width, "pairs": (5 * top, torch.int32),
+        return {**own, "act": top * self.experts.ff, "ye": top * self.experts.width, "pairs": (4 * top, torch.int32),
                 "tiles": (8 * top, torch.int32), "pair_w": (top, torch.float32)}
 
     def projections(self) -> list:
@@ -139,16 +139,16 @@ class Moe:
         from ..ops import moe as X
         s, x = self.spec, self.experts
         pairs = rows * s.top
-        expert, order, place, spare, exps = eng.scratch_view("pairs", rows, 5 * s.top).reshape(5, pairs)
+        expert, order, place, spare = eng.scratch_view("pairs", rows, 4 * s.top).reshape(4, pairs)
         weight, tiles = eng.scratch_view("pair_w", rows, s.top).reshape(-1), eng.scratch_view("tiles", rows, 8 * s.top)
         act, ye = eng.scratch_view("act", pairs, x.ff), eng.scratch_view("ye", pairs, x.width)
-        tr = X.tile_rows(pairs, s.experts, x.f32, min(x.up_n, x.width), max(x.up_n, x.width) if x.two_pieces else None)
+        tr = X.tile_rows(pairs, s.experts, x.f32, min(x.up_n, x.width))
         heights = X.heights(pairs, s.experts, tr, x.f32, (x.up_n, x.width), (x.width, x.ff))
         nt = X.route_group(in32[:, col["router"]:], rows, s.experts, s.top, tr if heights is None else X.HEIGHTS[0], expert, weight,
                            order, place, tiles, self.how, spare, heights)
         tr = tr if heights is None else 0
-        X.gemm(tiles, nt, tr, order, s.top, h, x.up, x.up_n, x.width, act, pairs, x.kind, x.up_exps, exps)
-        X.gemm(tiles, nt, tr, order, s.top, act, x.down, x.width, x.ff, ye, pairs, X.DOWN, x.down_exps, exps)
+        X.gemm(tiles, nt, tr, order, s.top, h, x.up, x.up_n, x.width, act, pairs, x.kind)
+        X.gemm(tiles, nt, tr, order, s.top, act, x.down, x.width, x.ff, ye, pairs, X.DOWN)
         out = {"experts": (ye, weight, place, s.top)}
         if gate is not None:
             out["gate2"] = gate

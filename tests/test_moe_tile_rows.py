@@ -4,14 +4,10 @@ import pytest
 from llm_sharding_amd.ops.moe import tile_rows
 
 
-@pytest.mark.parametrize("mean,experts,cols,wide,rows", [
-    (16, 32, 2048, 2048, 32), (17, 32, 2048, 2048, 128), (42, 32, 2048, 2048, 128), (95, 64, 1024, 1024, 128), (50, 16, 2048, 2048, 64),
-    (70, 16, 2048, 2048, 128), (50, 24, 2048, 2816, 64), (115, 24, 2048, 2816, 128), (100, 8, 2048, 4096, 64), (125, 8, 2048, 4096, 128),
-    (200, 32, 2048, 2048, 128)])
-def test_two_pieces(mean, experts, cols, wide, rows):
-    """Tall tiles where there are enough of them for the CUs and no round is nearly empty; as before without two pieces."""
-    assert tile_rows(mean * experts, experts, True, cols, wide) == rows
-    before = 128 if mean > 112 and experts * max(1.0, mean / 128 + 0.5) * -(-cols // 256) >= 160 else \
-        16 if mean <= 12 else 32 if mean <= 24 else 64
-    assert tile_rows(mean * experts, experts, True, cols) == before
-    assert tile_rows(mean * experts, experts, False, cols, wide) == tile_rows(mean * experts, experts, False, cols)
+@pytest.mark.parametrize("mean,experts,cols,rows", [
+    (12, 32, 2048, 16), (16, 32, 2048, 32), (24, 32, 2048, 32), (25, 32, 2048, 64), (42, 32, 2048, 64), (95, 64, 1024, 64), (112, 64, 1024, 64),
+    (50, 16, 2048, 64), (70, 16, 2048, 64), (115, 24, 2048, 128), (125, 8, 2048, 64), (125, 8, 4096, 128), (200, 32, 2048, 128)])
+def test_fp32_tiles(mean, experts, cols, rows):
+    """Tall tiles from 113 pairs an expert on, where there are 160 of them."""
+    assert tile_rows(mean * experts, experts, True, cols) == rows
+    assert tile_rows(mean * experts, experts, True) == (128 if mean > 112 else rows)
