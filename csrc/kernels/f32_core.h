@@ -30,7 +30,6 @@ template <int MT, int NT, int NW>
 struct F32Stream {
   static constexpr int UN = MT + NT <= 2 ? 4 : 2;  // units requested together (another UN are in flight meanwhile)
   static constexpr int LD = NT * 16 + 4, LDS = NW * MT * 16 * LD;
-  static constexpr int CH = MT * NT <= 2 ? 4 : 2;  // (four sums of 32 x 32 would leave room for one workgroup a CU)
   struct Unit {
     f32x4_t a[UN][MT], w[UN][NT];
   };
@@ -40,14 +39,11 @@ struct F32Stream {
   LSA_DEVICE static void run(const float* const (&ar)[MT], const float* const (&wr)[NT], int K, float* s_acc) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int u0 = (K / 16) * w / NW, u1 = (K / 16) * (w + 1) / NW;
-    // sums of every CH-th instruction: shorter ones round less, at K = 2048 1.6e-7 of the result in four, 2.1e-7 in two, 2.9e-7 in one
-    f32x4_t acc[CH][MT][NT];
+    f32x4_t acc[2][MT][NT];  // of every other instruction: half as long sums round less, 2.1e-7 of the result at K = 2048 for 2.9e-7
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int n = 0; n < NT; ++n)
-#pragma unroll
-        for (int j = 0; j < CH; ++j) acc[j][m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int n = 0; n < NT; ++n) acc[0][m][n] = acc[1][m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     auto load = [&](int u, Unit& x) {
 #pragma unroll
       for (int i = 0; i < UN; ++i) {
@@ -68,7 +64,7 @@ struct F32Stream {
           for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int n = 0; n < NT; ++n)
-              acc[j % CH][m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a[i][m][j], x.w[i][n][j], acc[j % CH][m][n], 0, 0, 0);
+              acc[j & 1][m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a[i][m][j], x.w[i][n][j], acc[j & 1][m][n], 0, 0, 0);
       }
     };
     Unit x0, x1;
@@ -85,11 +81,8 @@ struct F32Stream {
 #pragma unroll
       for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float v = acc[0][m][n][r] + acc[1][m][n][r];
-          if constexpr (CH == 4) v += acc[2][m][n][r] + acc[3][m][n][r];
-          s_acc[(w * MT * 16 + m * 16 + (lane >> 4) * 4 + r) * LD + n * 16 + (lane & 15)] = v;
-        }
+        for (int r = 0; r < 4; ++r)
+          s_acc[(w * MT * 16 + m * 16 + (lane >> 4) * 4 + r) * LD + n * 16 + (lane & 15)] = acc[0][m][n][r] + acc[1][m][n][r];
     __syncthreads();
   }
   LSA_DEVICE static float sum(const float* s_acc, int m, int n) {
