@@ -112,3 +112,27 @@ def test_choice_is_no_slower_than_the_one_of_two_heights():
     asked = {k: r for k, r in ratio.items() if hip.gemm_wr_plan(*k, hip.EPI_STORE, hip.EpiArgs()) is None}
     assert max(asked.values()) <= 1.05, sorted(asked.items(), key=lambda x: -x[1])[:5]
     assert math.exp(sum(map(math.log, ratio.values())) / len(ratio)) <= 0.984
+
+
+def test_an_entry_is_taken_where_it_is_the_nearest_measured(monkeypatch):
+    """Of the rows with as many tiles of 128: entries at both ends, one of which says that the model's choice stands."""
+    hip.gemm_sk_plan.cache_clear()
+    monkeypatch.setattr(hip, "_SK_TUNED", {(4096, 11008): [(256, (128, 256, 1, 6, 256))]})
+    monkeypatch.setattr(hip, "_SK_MODELLED", {(4096, 11008): [160, 384]})
+    try:
+        for M in (129, 160, 207):
+            assert hip.gemm_sk_plan(M, 4096, 11008) == hip.gemm_sk_plan(M, 4096, 11008, tuned=False) != (128, 256, 1, 6, 256), M
+        for M in (208, 256):
+            assert hip.gemm_sk_plan(M, 4096, 11008) == (128, 256, 1, 6, 256), M
+        for M in (128, 257):  # other numbers of tiles
+            assert hip.gemm_sk_plan(M, 4096, 11008) == hip.gemm_sk_plan(M, 4096, 11008, tuned=False)
+    finally:
+        hip.gemm_sk_plan.cache_clear()
+
+
+def test_residual_projections_of_few_row_tiles_at_both_ends():
+    """Rows whose plan was another entry's, measured at its other end: 7B's and 70B's residual projections."""
+    for M, N, K in [(129, 4096, 11008), (160, 4096, 11008), (257, 4096, 4096), (288, 4096, 4096), (513, 8192, 8192), (544, 8192, 8192)]:
+        assert hip.gemm_sk_plan(M, N, K, whole64=True) == hip.gemm_sk_plan(M, N, K, tuned=False, whole64=True)
+    assert hip.gemm_sk_partial_plan(160, 8192, 28672) == (256, 7) and hip.gemm_sk_partial_plan(256, 8192, 28672) is None
+    assert hip.gemm_sk_partial_plan(512, 8192, 28672) == (256, 4) and hip.gemm_sk_partial_plan(400, 8192, 28672) is None
