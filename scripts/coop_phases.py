@@ -40,12 +40,10 @@ def main():
     from llm_sharding_amd.ops import hip, packing
     from scripts.bench_kernels import timeit
     rows = [int(v) for v in sys.argv[1:]] or [32, 64, 128]
-    vp, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
     libs = {}
     for v in VARIANTS:
         L = ctypes.CDLL(so(v))
-        L.lsa_gemv_coop.argtypes = [vp, i, vp, vp, i, i, i, i, f, i, ctypes.POINTER(hip.EpiArgs), i, i, i, i, i, vp,
-                                    vp, vp]
+        L.lsa_gemv_coop.argtypes = hip.lib().lsa_gemv_coop.argtypes
         libs[v] = L
     ws = hip.CoopWorkspace("cuda", slab_floats=1 << 25)
     for name, (N, K, epi) in {"qkv": (12288, 4096, hip.EPI_STORE), "o": (4096, 4096, hip.EPI_RESID),
@@ -59,14 +57,14 @@ def main():
             algo, cfg = packing.proj_config(N // 16, M, need_even=epi == hip.EPI_SWIGLU, k=K)
             if algo != "coop":
                 continue
-            tnw, nw, kf, sk, kw = cfg
+            tnw, nw, kf, sk, kw, depth = cfg
             res = {}
             for v in VARIANTS:
                 L = libs[v]
 
                 def run(j):
                     rc = L.lsa_gemv_coop(x.data_ptr(), K, None, wps[j % nbuf].data_ptr(), M, N, K, 0, 1e-5, epi,
-                                         ctypes.byref(ep), tnw, nw, kf, sk, kw, ws.slab.data_ptr(),
+                                         ctypes.byref(ep), tnw, nw, kf, sk, kw, depth, ws.slab.data_ptr(),
                                          ws.counters.data_ptr(), torch.cuda.current_stream().cuda_stream)
                     assert rc == 0, rc
                 res[v] = round(timeit(run), 2)

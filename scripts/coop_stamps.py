@@ -27,8 +27,7 @@ def main():
     from llm_sharding_amd.ops import hip, packing
     rows = [int(v) for v in sys.argv[1:]] or [64, 128]
     L = ctypes.CDLL(SO)
-    vp, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
-    L.lsa_gemv_coop.argtypes = [vp, i, vp, vp, i, i, i, i, f, i, ctypes.POINTER(hip.EpiArgs), i, i, i, i, i, vp, vp, vp]
+    L.lsa_gemv_coop.argtypes = hip.lib().lsa_gemv_coop.argtypes
     ws = hip.CoopWorkspace("cuda", slab_floats=1 << 25)
     st = torch.zeros(4096 * 16, dtype=torch.int64, device="cuda")
     L.lsa_coop_set_stamps(ctypes.c_void_p(st.data_ptr()))
@@ -43,14 +42,14 @@ def main():
             algo, cfg = packing.proj_config(N // 16, M, k=K)
             if algo != "coop":
                 continue
-            tnw, nw, kf, sk, kw = cfg
+            tnw, nw, kf, sk, kw, depth = cfg
             G = N // 16 // (tnw * nw)
             grid = G * sk
             acc = {}
             for rep in range(6):
                 st.zero_()
                 rc = L.lsa_gemv_coop(x.data_ptr(), K, None, wps[rep % nbuf].data_ptr(), M, N, K, 0, 1e-5, epi,
-                                     ctypes.byref(ep), tnw, nw, kf, sk, kw, ws.slab.data_ptr(), ws.counters.data_ptr(),
+                                     ctypes.byref(ep), tnw, nw, kf, sk, kw, depth, ws.slab.data_ptr(), ws.counters.data_ptr(),
                                      torch.cuda.current_stream().cuda_stream)
                 assert rc == 0
                 torch.cuda.synchronize()

@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """A/B of two gemm_sk builds in ONE process on ONE box (box-to-box spread is ~10 %): the in-tree
 library against llm_sharding_amd/_native/liblsa_gemm_sk_prev.so (a build of an older
-gemm_sk.hip), interleaved rounds, cold weights, hipGraph-timed; engine epilogues.
+gemm_sk.hip whose entry takes the same arguments), interleaved rounds, cold weights, hipGraph-timed; engine epilogues.
 
 usage: gemm_sk_ab.py M N K epi bn split bm [...]   (epi: 1 resid, 2 swiglu, 3 qkv-as-store)"""
 import ctypes
@@ -19,7 +19,6 @@ from scripts.bench_kernels import timeit  # noqa: E402
 
 def main():
     args = [int(v) for v in sys.argv[1:]]
-    vp, i = ctypes.c_void_p, ctypes.c_int
     libs = {"new": hip.lib(), "prev": ctypes.CDLL(os.path.join(ROOT, "llm_sharding_amd", "_native",
                                                                "liblsa_gemm_sk_prev.so"))}
     libs["prev"].lsa_gemm_sk.argtypes = hip.lib().lsa_gemm_sk.argtypes
@@ -40,7 +39,8 @@ def main():
                 def run(j, L=L):
                     rc = L.lsa_gemm_sk(x.data_ptr(), K, wps[j % nbuf].data_ptr(), M, N, K, e, ctypes.byref(ep), bm, bn,
                                        0, hip.N_CU, 1, split, 8, ws.slab.data_ptr(), ws.counters.data_ptr(),
-                                       ws.slab.numel(), ws.counters.numel(), torch.cuda.current_stream().cuda_stream)
+                                       ws.slab.numel(), ws.counters.numel(), hip.HANDOFF_LOOKS,
+                                       torch.cuda.current_stream().cuda_stream)
                     assert rc == 0, rc
                 res[name].append(timeit(run))
                 if rnd == 0:

@@ -33,9 +33,7 @@ def main():
     reps = int(sys.argv[8]) if len(sys.argv) > 8 else 5
     bm = int(sys.argv[9]) if len(sys.argv) > 9 else 256
     L = ctypes.CDLL(SO)
-    vp, i = ctypes.c_void_p, ctypes.c_int
-    L.lsa_gemm_sk.argtypes = [vp, i, vp, i, i, i, i, ctypes.POINTER(hip.EpiArgs), i, i, i, i, i, i, i, vp, vp,
-                              ctypes.c_longlong, i, i, vp]
+    L.lsa_gemm_sk.argtypes = hip.lib().lsa_gemm_sk.argtypes
     nbuf = max(2, (600 << 20) // (N * K * 2) + 1)
     wps = [packing.pack_b(torch.randn(N, K, device="cuda").mul_(0.02).to(torch.bfloat16)) for _ in range(nbuf)]
     x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
@@ -49,7 +47,8 @@ def main():
         rc = L.lsa_gemm_sk(ctypes.c_void_p(x.data_ptr()), x.stride(0), ctypes.c_void_p(wps[r % nbuf].data_ptr()), M, N, K,
                            hip.EPI_STORE, ctypes.byref(ep), bm, bn, 0, grid, dp, split, 8,
                            ctypes.c_void_p(ws.slab.data_ptr()), ctypes.c_void_p(ws.counters.data_ptr()),
-                           ws.slab.numel(), ws.counters.numel(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+                           ws.slab.numel(), ws.counters.numel(), hip.HANDOFF_LOOKS,
+                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
         assert rc == 0, rc
         torch.cuda.synchronize()
     s = st.view(-1, 32).cpu().double()
