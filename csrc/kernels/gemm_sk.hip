@@ -115,6 +115,7 @@ __global__ __launch_bounds__(NTHR) void gemm_sk_kernel(const bf16_raw* __restric
     unsigned todo = 1, mine = 0;
     int shares = 1;
     bool last = false;
+    static_assert(!K_::SHARED || K_::FM <= HO_SHARES, "a share for a strip at most");
     const bool shared = K_::SHARED && partial && EPI != EPI_PARTIAL && prm.split && prm.looks >= 0;
     if (partial && EPI != EPI_PARTIAL) {
       // contributors of this tile, in K order: split mode - workgroups ts + s * sk_tiles; stream-K - the workgroups whose iteration ranges intersect the tile's

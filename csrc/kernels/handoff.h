@@ -6,7 +6,10 @@
 // us, by 4096 x 4096 in four 36.1 -> 28.0 and in two 29.1 -> 26.9, 1256 by 3072 x 8192 in two 65.2 -> 61.2, and 1984 products in parts
 // within one round of tiles 0.89 of their time (geometric mean); whole steps of 512 sequences (Llama-2-7B) 6993 -> 6884.
 // Nobody waits for a workgroup that may have no place to run: after ``looks`` looks at the counter a workgroup leaves its share to the
-// last to arrive, who finds that in the counter it arrives at. (Two streams' launches that wait for each other's places end this way.)
+// last to arrive, who finds that in the counter it arrives at. Two streams' launches that wait for each other's places end this way. A pair of
+// products beside each other, with 64 looks and with none (and through the last to arrive alone): 512 rows by 4096 x 11008 in four parts 105 and 117
+// us (118), by 4096 x 4096 in two 53.4 and 55.2 (54.8), 384 by 4096 x 11008 in five 98.4 and 100 (103), 128 by 3072 x 3072 in four 22.8 and 24.0
+// (24.6); in six parts of 256 x 128, 256 by 4096 x 11008, the wait costs 2 of 73.
 // The sums are the same whoever makes them: parts are added in their order.
 #pragma once
 #include "common.h"
@@ -16,9 +19,8 @@ constexpr unsigned HO_PARTS = 4095u, HO_LEFT = 12, HO_DONE = 20;
 // From one tile's counter to the next, in words: lines and channels of their own. With 64 counters in two lines the looks of all tiles'
 // workgroups held up each other's arrivals: 3072 x 3072 of 128 rows in four parts 16.8 us instead of 13.0 from first start to last end.
 constexpr int HO_STRIDE = 64;
-constexpr int HO_SHARES = 8;  // at most
-constexpr int HO_LOOKS = 64;  // some 40 us
-constexpr int HO_LAST = -1;   // instead of looks: the last to arrive finishes all, for launches with more workgroups than CUs
+constexpr int HO_SHARES = HO_DONE - HO_LEFT;  // at most
+constexpr int HO_LAST = -1;                   // instead of looks: the last to arrive finishes all, for launches with more workgroups than CUs
 
 // One thread, what other shares need of its workgroup's part written through: arrives at ``c`` with part ``s`` of ``S``. The shares that
 // are this workgroup's to finish, as bits; ``last``: all other parts had arrived. HO_TIRED: it has looked often enough. Then all of its part
@@ -29,7 +31,7 @@ LSA_DEVICE unsigned ho_arrive(unsigned* c, int s, int S, int ns, int looks, bool
   last = (v & HO_PARTS) == (unsigned)S;
   if (looks < 0) return last ? (1u << ns) - 1u : 0u;
   const unsigned mine = s < ns ? 1u << s : 0u;
-  if (last) return mine | ((v >> HO_LEFT) & 255u);
+  if (last) return mine | ((v >> HO_LEFT) & ((1u << HO_SHARES) - 1u));
   if (!mine) return 0u;
   for (int i = 0; i < looks; ++i) {
     __builtin_amdgcn_s_sleep(1);
@@ -47,7 +49,8 @@ LSA_DEVICE unsigned ho_leave(unsigned* c, int s, int S) {
   return 1u << s;
 }
 
-// One thread, its workgroup's shares read: the last one through leaves the counter as it was.
+// One thread: the last one through leaves the counter as it was. Other waves of its workgroup may still be reading parts: neither they nor
+// the counter are used for anything else before the launch has ended.
 LSA_DEVICE void ho_through(unsigned* c, int s, int ns, int looks, unsigned mine, bool last) {
   if (looks < 0) {
     if (last) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -57,7 +60,7 @@ LSA_DEVICE void ho_through(unsigned* c, int s, int ns, int looks, unsigned mine,
   const unsigned own = (s < ns ? (mine >> s) & 1u : 0u) + (last ? 1u : 0u);
   if (!own) return;
   const unsigned v = __hip_atomic_fetch_add(c, own << HO_DONE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if ((v >> HO_DONE) + own + __builtin_popcount((v >> HO_LEFT) & 255u) == (unsigned)ns + 1u)
+  if ((v >> HO_DONE) + own + __builtin_popcount((v >> HO_LEFT) & ((1u << HO_SHARES) - 1u)) == (unsigned)ns + 1u)
     __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

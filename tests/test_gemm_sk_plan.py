@@ -136,3 +136,11 @@ def test_residual_projections_of_few_row_tiles_at_both_ends():
         assert hip.gemm_sk_plan(M, N, K, whole64=True) == hip.gemm_sk_plan(M, N, K, tuned=False, whole64=True)
     assert hip.gemm_sk_partial_plan(160, 8192, 28672) == (256, 7) and hip.gemm_sk_partial_plan(256, 8192, 28672) is None
     assert hip.gemm_sk_partial_plan(512, 8192, 28672) == (256, 4) and hip.gemm_sk_partial_plan(400, 8192, 28672) is None
+
+
+def test_counters_lie_as_the_kernel_has_them():
+    import os
+    import re
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    with open(os.path.join(root, "csrc", "kernels", "handoff.h")) as fh:
+        assert int(re.search(r"constexpr int HO_STRIDE = (\d+);", fh.read()).group(1)) == hip.HANDOFF_STRIDE
