@@ -100,13 +100,15 @@ def fit(products):
 
 def main() -> None:
     packing._TUNED = {}
-    print("gemm_sk:", regret(load("cost_gemm_sk.csv", 3), sk))
-    with open(os.path.join(ROOT, "profiles", "cost_gemm_sk_checks.csv")) as fh:
-        rows = list(csv.DictReader(fh))
-    for name in ("one_hand_off", "present"):
-        off = [float(r[name + "_us"]) / float(r["two_heights_us"]) for r in rows]
-        print(f"gemm_sk, products it was not fitted to, {name} / two_heights: {math.exp(sum(map(math.log, off)) / len(off)):.3f}, "
-              f"worst {max(off):.2f}, {sum(x > 1.05 for x in off)} of {len(off)} more than 1.05")
+    for what, file in (("", ""), (" (split tiles finished by all their workgroups)", "_shared")):
+        print(f"gemm_sk{what}:", regret(load(f"cost_gemm_sk{file}.csv", 3), sk))
+        with open(os.path.join(ROOT, "profiles", f"cost_gemm_sk_checks{file}.csv")) as fh:
+            rows = list(csv.DictReader(fh))
+        for name in ("one_hand_off", "present"):
+            off = [float(r[name + "_us"]) / float(r["two_heights_us"]) for r in rows]
+            print(f"gemm_sk{what}, products it was not fitted to, {name} / two_heights: {math.exp(sum(map(math.log, off)) / len(off)):.3f}, "
+                  f"worst {max(off):.2f}, {sum(x > 1.05 for x in off)} of {len(off)} more than 1.05")
+
     def against(name, file, now, other):
         with open(os.path.join(ROOT, "profiles", file)) as fh:
             off = [float(now(r)) / float(other(r)) for r in csv.DictReader(fh)]
